@@ -36,23 +36,134 @@ static_assert(SD_TABLE_USED <= SD_TABLE_BYTES, "table layout");
 constexpr int SD_BLOCK = 256;
 constexpr int SD_WAVES = SD_BLOCK / 64;
 constexpr int SORT_N = 2048;
+constexpr int SORT_PER = SORT_N / SD_BLOCK;   // keys per lane
 
-// Block-wide bitonic sort of 2048 uint64 keys in LDS, ascending.
-__device__ void bitonic_sort_2048(unsigned long long* keys) {
-  for (int k = 2; k <= SORT_N; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      __syncthreads();
-      for (int i = threadIdx.x; i < SORT_N; i += SD_BLOCK) {
-        const int ixj = i ^ j;
-        if (ixj > i) {
-          const unsigned long long x = keys[i], y = keys[ixj];
-          const bool up = (i & k) == 0;
-          if ((x > y) == up) { keys[i] = y; keys[ixj] = x; }
-        }
-      }
-    }
+// The value of lane (lane ^ MASK): DPP where the pattern has one, a lane permute otherwise.
+template <int MASK>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  if constexpr (MASK == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1,0,3,2
+  else if constexpr (MASK == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2,3,0,1
+  else if constexpr (MASK == 3) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x1B, 0xF, 0xF, true);   // quad_perm 3,2,1,0
+  else if constexpr (MASK == 7) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+  else if constexpr (MASK == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);  // row_ror:8
+  else if constexpr (MASK == 15) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true); // row_mirror
+  else return (uint32_t)__shfl_xor((int)v, MASK, P2_WAVE);
+}
+
+__device__ __forceinline__ void order_pair(uint32_t& lo, uint32_t& hi) {
+  const uint32_t x = lo < hi ? lo : hi, y = lo < hi ? hi : lo;
+  lo = x;
+  hi = y;
+}
+
+// Merge steps at distances that stay inside a lane's eight keys.
+template <int J>
+__device__ __forceinline__ void merge_in_lane(uint32_t (&v)[SORT_PER]) {
+  if constexpr (J >= 1) {
+#pragma unroll
+    for (int r = 0; r < SORT_PER; ++r)
+      if (!(r & J)) order_pair(v[r], v[r | J]);
+    merge_in_lane<J / 2>(v);
   }
-  __syncthreads();
+}
+// ... and at distances of LJ lanes and less inside a wave.
+template <int LJ>
+__device__ __forceinline__ void merge_in_wave(uint32_t (&v)[SORT_PER]) {
+  if constexpr (LJ >= 1) {
+    const bool low = !(threadIdx.x & LJ);
+#pragma unroll
+    for (int r = 0; r < SORT_PER; ++r) {
+      const uint32_t o = lane_xor<LJ>(v[r]);
+      v[r] = (v[r] < o) == low ? v[r] : o;
+    }
+    merge_in_wave<LJ / 2>(v);
+  } else {
+    merge_in_lane<SORT_PER / 2>(v);
+  }
+}
+// Sorted runs of K / 2 keys -> runs of K keys, K = 16 .. 512 (2 .. 64 lanes): every key against its mirror image in
+// the run (all comparisons ascending), then halving distances.
+template <int K>
+__device__ __forceinline__ void merge_runs(uint32_t (&v)[SORT_PER]) {
+  constexpr int LANES = K / SORT_PER;
+  const bool low = !(threadIdx.x & (LANES / 2));
+  uint32_t o[SORT_PER];
+#pragma unroll
+  for (int r = 0; r < SORT_PER; ++r) o[r] = lane_xor<LANES - 1>(v[SORT_PER - 1 - r]);
+#pragma unroll
+  for (int r = 0; r < SORT_PER; ++r) v[r] = (v[r] < o[r]) == low ? v[r] : o[r];
+  merge_in_wave<LANES / 4>(v);
+}
+
+// Block-wide bitonic sort of 2048 distinct (or all-ones) 32-bit keys, ascending: lane t holds keys 8 t .. 8 t + 7 before
+// and after.  Distances under eight keys are register min / max, under a wave lane permutes; only the three steps
+// that cross waves go through LDS (`keys`, which holds the sorted keys at the end, behind a barrier).
+__device__ __forceinline__ void sort_2048(uint32_t (&v)[SORT_PER], uint32_t* keys) {
+  const int t = threadIdx.x;
+  // runs of 2, 4, 8 inside a lane
+#pragma unroll
+  for (int r = 0; r < SORT_PER; r += 2) order_pair(v[r], v[r + 1]);
+#pragma unroll
+  for (int r = 0; r < SORT_PER; r += 4) {
+    order_pair(v[r], v[r + 3]);
+    order_pair(v[r + 1], v[r + 2]);
+  }
+  merge_in_lane<1>(v);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) order_pair(v[r], v[7 - r]);
+  merge_in_lane<2>(v);
+  merge_runs<16>(v);
+  merge_runs<32>(v);
+  merge_runs<64>(v);
+  merge_runs<128>(v);
+  merge_runs<256>(v);
+  merge_runs<512>(v);
+  auto put = [&]() {
+#pragma unroll
+    for (int r = 0; r < SORT_PER; r += 4)
+      *reinterpret_cast<uint4*>(keys + t * SORT_PER + r) = make_uint4(v[r], v[r + 1], v[r + 2], v[r + 3]);
+  };
+  auto take = [&](int lane_mask, bool mirrored, bool low) {
+    uint32_t o[SORT_PER];
+#pragma unroll
+    for (int r = 0; r < SORT_PER; r += 4) {
+      const uint4 x = *reinterpret_cast<const uint4*>(keys + (t ^ lane_mask) * SORT_PER + r);
+      o[r] = x.x; o[r + 1] = x.y; o[r + 2] = x.z; o[r + 3] = x.w;
+    }
+#pragma unroll
+    for (int r = 0; r < SORT_PER; ++r) {
+      const uint32_t w = mirrored ? o[SORT_PER - 1 - r] : o[r];
+      v[r] = (v[r] < w) == low ? v[r] : w;
+    }
+  };
+  put();
+  p2_sync_lds();
+  take(127, true, !(t & 64));                 // runs of 512 -> 1024
+  merge_in_wave<32>(v);
+  p2_sync_lds();
+  put();
+  p2_sync_lds();
+  take(255, true, !(t & 128));                // -> 2048
+  p2_sync_lds();
+  put();
+  p2_sync_lds();
+  take(64, false, !(t & 64));
+  merge_in_wave<32>(v);
+  p2_sync_lds();
+  put();
+  p2_sync_lds();
+}
+
+// A packed score (ranker.hip: type 1..9 and five kicker nibbles of 0..14, the last zero outside high cards and
+// flushes) as a number of 21 bits in the same order, so that score and combo index share one 32-bit sort key.
+constexpr uint32_t SC_V4 = 15u * 15u * 15u * 15u, SC_V5 = SC_V4 * 15u;
+static_assert(2u * SC_V5 + 7u * SC_V4 < (1u << 21), "score codes fit 21 bits");
+__device__ __forceinline__ uint32_t score_code(int32_t sc) {
+  const uint32_t s = (uint32_t)sc, type = s >> 20;
+  const uint32_t v4 = (((s >> 16 & 15u) * 15u + (s >> 12 & 15u)) * 15u + (s >> 8 & 15u)) * 15u + (s >> 4 & 15u);
+  const bool five = type == 1u || type == 6u;                          // high card, flush: five kickers
+  const uint32_t below4 = type <= 1u ? 0u : (type >= 7u ? type - 3u : type - 2u);   // four-kicker types below this one
+  return (five ? v4 * 15u + (s & 15u) : v4) + below4 * SC_V4 + ((type > 1u ? 1u : 0u) + (type > 6u ? 1u : 0u)) * SC_V5;
 }
 
 // Per-card lists: clist[c][j] = sorted position of the j-th weakest of the 51 combos holding card
@@ -85,6 +196,27 @@ __device__ __forceinline__ int board_card(const void* boards, int64_t m, int j) 
   return (int)reinterpret_cast<const T*>(boards)[m * 5 + j];
 }
 
+// Positions of a table as bits: which sorted positions start a tie group, and which hold a combo of a card.
+constexpr int SD_WORDS = (P2_H + 31) / 32;     // 42
+constexpr int SD_WPITCH = 43;                  // words per card in LDS (odd: the cards' rows start in different banks)
+constexpr int SD_HWORDS = (P2_H + 63) / 64;    // 21
+
+struct SetupLds {
+  __align__(16) uint32_t keys[SORT_N];
+  uint32_t bits[P2_CARDS][SD_WPITCH];          // bit k: the combo at sorted position k holds the card
+  uint8_t pre[P2_CARDS][SD_WORDS + 2];         // bits of the card in the words before
+  unsigned long long heads[SD_HWORDS];         // bit k: a tie group starts at sorted position k
+  uint16_t head_before[SD_HWORDS], head_after[SD_HWORDS], heads_in[SD_HWORDS];
+  __align__(4) uint16_t clist[P2_CARDS * 51];
+  int bcards[5];
+};
+
+// Combos of card c at sorted positions below `bound`.
+__device__ __forceinline__ int card_below(const SetupLds& S, int c, int bound) {
+  const int w = bound >> 5;
+  return (int)S.pre[c][w] + __popc(S.bits[c][w] & ((1u << (bound & 31)) - 1u));
+}
+
 // One workgroup per board.
 //   mode 0: score = union of hole and board planes (a combo touching the board is a
 //           6-card hand), rules.py:86-102; ranks_out = dense 1-based group ids
@@ -92,32 +224,39 @@ __device__ __forceinline__ int board_card(const void* boards, int64_t m, int j) 
 //           rules_triton.py:139-148; ranks_out = packed scores
 // ranks_out [M,1326] int32, order_out [M,1326] int64 (stable ascending argsort) and
 // table_out are each optional.
+// Bound by vector issue and LDS.  Sorting 64-bit keys through LDS (66 steps with a barrier each), ranking every card's
+// combos against each other (52 x 51 x 51 look-ups) and binary searches for the tie groups took 544 us for 4096
+// boards; keys of 32 bits sorted in registers, and positions kept as bit sets whose prefix counts answer "how
+// many below", take 100 us (1 board: 20 us).
 __global__ __launch_bounds__(SD_BLOCK) void showdown_setup_kernel(const void* __restrict__ boards, int elem_size,
                                                                    int mode, int32_t* __restrict__ ranks_out,
                                                                    int64_t* __restrict__ order_out,
                                                                    uint8_t* __restrict__ table_out) {
-  __shared__ unsigned long long keys[SORT_N];
-  __shared__ uint16_t pos_of[P2_H];       // combo -> sorted position
-  __shared__ uint16_t clist[P2_CARDS][52];
-  __shared__ int scan_tmp[SD_WAVES];
-  __shared__ int bcards[5];
+  __shared__ SetupLds S;
   const int64_t m = blockIdx.x;
-  if (threadIdx.x < 5) {
-    int c = elem_size == 1 ? board_card<int8_t>(boards, m, threadIdx.x)
-          : elem_size == 2 ? board_card<int16_t>(boards, m, threadIdx.x)
-          : elem_size == 4 ? board_card<int32_t>(boards, m, threadIdx.x)
-                           : board_card<int64_t>(boards, m, threadIdx.x);
-    bcards[threadIdx.x] = c;
+  const int t = threadIdx.x, lane = t & 63;
+  if (t < 5) {
+    int c = elem_size == 1 ? board_card<int8_t>(boards, m, t)
+          : elem_size == 2 ? board_card<int16_t>(boards, m, t)
+          : elem_size == 4 ? board_card<int32_t>(boards, m, t)
+                           : board_card<int64_t>(boards, m, t);
+    S.bcards[t] = c;
   }
+  for (int i = t; i < P2_CARDS * SD_WPITCH; i += SD_BLOCK) (&S.bits[0][0])[i] = 0u;
   __syncthreads();
   uint32_t bs[4] = {0, 0, 0, 0};
   unsigned long long board_bits = 0;
+  CardAcc board_acc;
   for (int j = 0; j < 5; ++j) {
-    const uint32_t c = (uint32_t)bcards[j];
+    const uint32_t c = (uint32_t)S.bcards[j];
     if (c < 52u) { bs[c / 13u] |= 1u << (c % 13u); board_bits |= 1ull << c; }
+    if (c < 52u && mode != 0) board_acc.add((int)c);   // the order of the cards does not matter: the board goes first, once
   }
-  for (int h = threadIdx.x; h < SORT_N; h += SD_BLOCK) {
-    unsigned long long key = ~0ull;
+  uint32_t key[SORT_PER];
+#pragma unroll
+  for (int i = 0; i < SORT_PER; ++i) {
+    const int h = t + i * SD_BLOCK;              // any order does: the keys are distinct
+    key[i] = ~0u;
     if (h < P2_H) {
       const int a = p2_combo.a[h], b = p2_combo.b[h];
       int32_t sc;
@@ -127,91 +266,99 @@ __global__ __launch_bounds__(SD_BLOCK) void showdown_setup_kernel(const void* __
         s[b / 13] |= 1u << (b % 13);
         sc = score_hand(hand_from_suits(s[0], s[1], s[2], s[3]), false);
       } else {
-        CardAcc acc;
+        CardAcc acc = board_acc;
         acc.add(a);
         acc.add(b);
-        for (int j = 0; j < 5; ++j)
-          if ((uint32_t)bcards[j] < 52u) acc.add(bcards[j]);
         sc = score_hand(acc.finish(), true);
+        if (ranks_out) ranks_out[m * P2_H + h] = sc;
       }
-      key = ((unsigned long long)(uint32_t)sc << 11) | (unsigned long long)h;
+      key[i] = (score_code(sc) << 11) | (uint32_t)h;
     }
-    keys[h] = key;
   }
-  bitonic_sort_2048(keys);  // ties resolve by combo index: a stable argsort
+  sort_2048(key, S.keys);  // ties resolve by combo index: a stable argsort
 
-  for (int k = threadIdx.x; k < P2_H; k += SD_BLOCK) {
-    const unsigned long long key = keys[k];
-    const int h = (int)(key & 2047ull);
-    pos_of[h] = (uint16_t)k;
-    if (order_out) order_out[m * P2_H + k] = h;
-    if (mode == 1 && ranks_out) ranks_out[m * P2_H + h] = (int32_t)(key >> 11);
+  uint32_t hk[6], ab[6];   // this lane's positions t + 256 i
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const int k = t + i * SD_BLOCK;
+    const bool in = k < P2_H;
+    const uint32_t mine = S.keys[k];
+    hk[i] = in ? mine & 2047u : 0u;
+    const bool head = in && (k == 0 || (S.keys[k - 1] >> 11) != (mine >> 11));
+    const unsigned long long word = __ballot(head);
+    if (lane == 0 && k < P2_H) S.heads[k >> 6] = word;
+    ab[i] = (uint32_t)p2_combo.a[hk[i]] | ((uint32_t)p2_combo.b[hk[i]] << 8);
+    if (in) {
+      atomicOr(&S.bits[ab[i] & 0xFFu][k >> 5], 1u << (k & 31));
+      atomicOr(&S.bits[ab[i] >> 8][k >> 5], 1u << (k & 31));
+      if (order_out) order_out[m * P2_H + k] = hk[i];
+    }
   }
   __syncthreads();
-
-  // dense group ids (mode 0): 1 + number of group starts at sorted positions 1..k
-  if (mode == 0 && ranks_out) {
-    // each thread owns 6 consecutive sorted positions (256*6 = 1536 >= 1326)
-    const int k0 = threadIdx.x * 6;
-    int flags[6], local = 0;
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-      const int k = k0 + i;
-      flags[i] = (k > 0 && k < P2_H && (keys[k] >> 11) != (keys[k - 1] >> 11)) ? 1 : 0;
-      local += flags[i];
+  // prefix counts of the cards' words: four lanes per card, eleven words each
+  {
+    const int c = t >> 2, sub = t & 3, w0 = sub * 11, w1 = w0 + 11 < SD_WORDS ? w0 + 11 : SD_WORDS;
+    int n = 0;
+    if (c < P2_CARDS)
+      for (int w = w0; w < w1; ++w) n += __popc(S.bits[c][w]);
+    const int n1 = __shfl_up(n, 1, 4), n2 = __shfl_up(n, 2, 4), n3 = __shfl_up(n, 3, 4);
+    int run = (sub > 0 ? n1 : 0) + (sub > 1 ? n2 : 0) + (sub > 2 ? n3 : 0);
+    if (c < P2_CARDS)
+      for (int w = w0; w < w1; ++w) {
+        S.pre[c][w] = (uint8_t)run;
+        run += __popc(S.bits[c][w]);
+      }
+  }
+  // tie groups: the last start in the words before, the first one in the words behind, starts in the words before
+  if (t < 64) {
+    const unsigned long long w = lane < SD_HWORDS ? S.heads[lane] : 0ull;
+    int last = w ? lane * 64 + 63 - __clzll((long long)w) : -1, first = w ? lane * 64 + __ffsll(w) - 1 : P2_H;
+    int count = __popcll(w);
+    for (int off = 1; off < 32; off <<= 1) {
+      const int a = __shfl_up(last, off), c = __shfl_up(count, off), b = __shfl_down(first, off);
+      if (lane >= off) {
+        last = a > last ? a : last;
+        count += c;
+      }
+      if (lane + off < 64) first = b < first ? b : first;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = local;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      int o = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += o;
+    const int before = __shfl_up(last, 1), in_before = __shfl_up(count, 1), after = __shfl_down(first, 1);
+    if (lane < SD_HWORDS) {
+      S.head_before[lane] = (uint16_t)(lane > 0 ? before : 0);
+      S.heads_in[lane] = (uint16_t)(lane > 0 ? in_before : 0);
+      S.head_after[lane] = (uint16_t)after;
     }
-    if (lane == 63) scan_tmp[wave] = incl;
-    __syncthreads();
-    int base = 0;
-    for (int w = 0; w < wave; ++w) base += scan_tmp[w];
-    int run = base + incl - local;
+  }
+  __syncthreads();
+  const int64_t tab = m * SD_TABLE_BYTES;
+  uint16_t* t_perm = reinterpret_cast<uint16_t*>(table_out + tab + SD_OFF_PERM);
+  uint32_t* t_lr = reinterpret_cast<uint32_t*>(table_out + tab + SD_OFF_LR);
+  uint32_t* t_cidx = reinterpret_cast<uint32_t*>(table_out + tab + SD_OFF_CIDX);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-      const int k = k0 + i;
-      run += flags[i];
-      if (k < P2_H) ranks_out[m * P2_H + (int)(keys[k] & 2047ull)] = run + 1;
-    }
+  for (int i = 0; i < 6; ++i) {
+    const int k = t + i * SD_BLOCK;
+    if (k >= P2_H) break;
+    const int w = k >> 6;
+    const unsigned long long heads = S.heads[w], upto = heads & (~0ull >> (63 - (k & 63)));
+    if (mode == 0 && ranks_out) ranks_out[m * P2_H + hk[i]] = (int)S.heads_in[w] + __popcll(upto);
+    if (!table_out) continue;
+    const unsigned long long behind = heads & ~(~0ull >> (63 - (k & 63)));
+    const int L = upto ? w * 64 + 63 - __clzll((long long)upto) : (int)S.head_before[w];
+    const int R = behind ? w * 64 + __ffsll(behind) - 1 : (int)S.head_after[w];
+    const int a = (int)(ab[i] & 0xFFu), b = (int)(ab[i] >> 8);
+    const bool blocked = ((board_bits >> a) | (board_bits >> b)) & 1ull;
+    t_perm[k] = (uint16_t)(hk[i] | (blocked ? 0x8000u : 0u));
+    t_lr[k] = (uint32_t)L | ((uint32_t)R << 16);
+    t_cidx[k] = (uint32_t)card_below(S, a, L) | ((uint32_t)card_below(S, a, R) << 8) |
+                ((uint32_t)card_below(S, b, L) << 16) | ((uint32_t)card_below(S, b, R) << 24);
+    // the list of a board card is masked out as a whole
+    S.clist[a * 51 + card_below(S, a, k)] = (board_bits >> a) & 1ull ? (uint16_t)0xFFFF : (uint16_t)k;
+    S.clist[b * 51 + card_below(S, b, k)] = (board_bits >> b) & 1ull ? (uint16_t)0xFFFF : (uint16_t)k;
   }
   if (!table_out) return;
-  uint16_t* t_perm = reinterpret_cast<uint16_t*>(table_out + m * SD_TABLE_BYTES + SD_OFF_PERM);
-  uint16_t* t_lr = reinterpret_cast<uint16_t*>(table_out + m * SD_TABLE_BYTES + SD_OFF_LR);
-
-  fill_card_lists(pos_of, clist);
-  uint16_t* t_clist = reinterpret_cast<uint16_t*>(table_out + m * SD_TABLE_BYTES + SD_OFF_CLIST);
-  for (int e = threadIdx.x; e < P2_CARDS * 51; e += SD_BLOCK) {
-    const int c = e / 51, j = e % 51;
-    const bool on_board = (board_bits >> c) & 1ull;
-    t_clist[e] = on_board ? (uint16_t)0xFFFF : clist[c][j];
-  }
-  uint8_t* t_cidx = table_out + m * SD_TABLE_BYTES + SD_OFF_CIDX;
-  for (int k = threadIdx.x; k < P2_H; k += SD_BLOCK) {
-    const unsigned long long key = keys[k];
-    const unsigned long long sc = key >> 11;
-    const int h = (int)(key & 2047ull);
-    // [L, R): first position with this score, first position with a larger one
-    int lo = 0, hi = k;
-    while (lo < hi) { int mid = (lo + hi) >> 1; if ((keys[mid] >> 11) < sc) lo = mid + 1; else hi = mid; }
-    const int L = lo;
-    lo = k + 1; hi = P2_H;
-    while (lo < hi) { int mid = (lo + hi) >> 1; if ((keys[mid] >> 11) <= sc) lo = mid + 1; else hi = mid; }
-    const int R = lo;
-    const int a = p2_combo.a[h], b = p2_combo.b[h];
-    const bool blocked = ((board_bits >> a) | (board_bits >> b)) & 1ull;
-    t_perm[k] = (uint16_t)(h | (blocked ? 0x8000 : 0));
-    t_lr[2 * k] = (uint16_t)L;
-    t_lr[2 * k + 1] = (uint16_t)R;
-    t_cidx[4 * k + 0] = (uint8_t)card_list_below(clist[a], L);
-    t_cidx[4 * k + 1] = (uint8_t)card_list_below(clist[a], R);
-    t_cidx[4 * k + 2] = (uint8_t)card_list_below(clist[b], L);
-    t_cidx[4 * k + 3] = (uint8_t)card_list_below(clist[b], R);
-  }
+  __syncthreads();
+  uint32_t* t_clist = reinterpret_cast<uint32_t*>(table_out + tab + SD_OFF_CLIST);
+  for (int e = t; e < P2_CARDS * 51 / 2; e += SD_BLOCK) t_clist[e] = reinterpret_cast<const uint32_t*>(S.clist)[e];
 }
 
 // The same table from hands that are ALREADY in strength order: row m lists, per sorted position,

@@ -170,6 +170,7 @@ def rank_7_cards_single_batch_triton(cards_batch: torch.Tensor) -> torch.Tensor:
 
 
 def _rank_boards(board: torch.Tensor, mode: int, want_table: bool):
+    """(ranks, order, None), or with ``want_table`` (None, None, table): what is not asked for is not written."""
     _require_backend()
     if board.dim() != 2 or board.shape[1] != 5:
         raise ValueError(f"board must be [M, 5], got {tuple(board.shape)}")
@@ -179,11 +180,12 @@ def _rank_boards(board: torch.Tensor, mode: int, want_table: bool):
         board = board.to(torch.int64)
     board = board.contiguous()
     m = board.shape[0]
-    ranks = torch.empty((m, NUM_HANDS), device=board.device, dtype=torch.int32)
-    order = torch.empty((m, NUM_HANDS), device=board.device, dtype=torch.int64)
-    table = None
+    ranks = order = table = None
     if want_table:
         table = torch.empty((m, showdown_table_bytes()), device=board.device, dtype=torch.uint8)
+    else:
+        ranks = torch.empty((m, NUM_HANDS), device=board.device, dtype=torch.int32)
+        order = torch.empty((m, NUM_HANDS), device=board.device, dtype=torch.int64)
     _lib.call("p2hip_showdown_setup", _lib.ptr(board), board.element_size(), m, mode, _lib.ptr(ranks),
               _lib.ptr(order), _lib.ptr(table), _lib.stream_ptr())
     return ranks, order, table
