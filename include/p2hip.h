@@ -427,6 +427,25 @@ typedef struct P2HipIterArgs {
 int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max_children, int phases,
                         void* stream);
 
+/* p2hip_cfr_iteration that moves fewer bytes where rows of the state repeat one another.
+ *
+ * range_rows (optional, [total], from p2hip_range_rows): reach, reach_avg, beliefs and beliefs_avg of the player
+ *   who did not act on the way into a row are the numbers of an earlier row, bit for bit, back to that player's
+ *   last action (or to the row right under the root).  range_rows[c] names it in the [total*2] row space.  With it
+ *   every iteration reads those rows there and a lean iteration (bit 4) stores them only there; leaves a network
+ *   is asked about (node_flags 8 without 1) and beliefs_avg under enforce_zero_sum keep both rows.
+ * phases bit 5 (32): rows flagged 16 in node_flags (fold leaves: one number per player in latest and values_avg,
+ *   whatever the hand) are read through their first two entries; a lean iteration stores only those two of
+ *   values_avg.  After lean iterations with the bit, one iteration with the bit and without bit 4 makes every
+ *   row whole again.
+ * The state after that last iteration is bit-identical to p2hip_cfr_iteration's. */
+int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* range_rows, int64_t n_items,
+                               int max_children, int phases, void* stream);
+
+/* range_rows of a tree: parent_index [total] (rows numbered top-down, the n_roots roots first), to_act [total]. */
+int p2hip_range_rows(const int64_t* parent_index, const int64_t* to_act, int64_t n_roots, int64_t total, int32_t* out,
+                     void* stream);
+
 /* Copy 8 floats and 8 int64 from HOST arrays into the device arrays fscal[8] / iscal[8] read by
  * p2hip_cfr_iteration.  The values travel as kernel arguments: the host arrays may be reused as
  * soon as the call returns.  Plays the role of TScalars.update, search/fused_cfr_triton.py:2131-2158. */

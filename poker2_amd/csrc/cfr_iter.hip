@@ -43,6 +43,7 @@ constexpr uint8_t NODE_SHOWDOWN = 1;  // river showdown leaf: value from the sho
 constexpr uint8_t NODE_DONE = 2;      // terminal node: excluded from the zero-sum shift
 constexpr uint8_t NODE_PARENT = 4;    // the row has children
 constexpr uint8_t NODE_LEAF_EVAL = 8; // childless row whose ranges feed a leaf evaluation (showdown, leaf network)
+constexpr uint8_t NODE_CONST = 16;    // fold leaf: values and average values are one number per player, whatever the hand
 // vectors card-summed per batch: what the LDS union holds next to the showdown buffers, and
 // never less than one family (parent + children)
 template <int MAXC>
@@ -89,6 +90,12 @@ struct IterArgs {
   const int64_t* item_root;
   const uint8_t* item_top;
   int phases;            // PHASE_* bits
+  // [total] or null: for the player who did not act on the way into row c, the row of the [total*2] row space
+  // where that player's reach, average reach and ranges are kept.  They are the same numbers, bit for bit, at
+  // every node since that player's last action (only the actor's reach changes, and a range is a function of
+  // the reach alone), so a lean iteration stores them once, and every iteration reads them there.
+  const int32_t* range_rows;
+  int const_rows;        // rows flagged NODE_CONST: read the first pair only, store only that in a lean iteration
 };
 
 // Which sweeps a launch runs.  Sweep 1 of a family reads its parent's beliefs, values and reach_avg
@@ -111,6 +118,12 @@ constexpr int PHASE_12 = 1, PHASE_3 = 2, PHASE_1 = 4, PHASE_2 = 8;
 // swaps from iteration to iteration, sweep 2 reads it from the buffer of the previous iteration
 // instead: one row read per parent in place of a read, a write and a re-read.
 constexpr int PHASE_LEAN = 16;
+// What range_rows and const_rows are for: the kernel is bound by the bytes it moves, and these move fewer.  Per
+// root of the three-raise river tree (105 nodes: 34 parents, 35 showdown and 36 fold leaves) a lean iteration
+// touches about 2420 rows of 5304 bytes; the unchanged player's rows are 134 of the writes (reach, reach_avg,
+// beliefs of a node with children, beliefs of a showdown leaf), the fold leaves' values 180 of the reads and 72 of
+// the writes (latest once per player and once more in the regret part, values_avg both ways).
+constexpr int PHASE_CONST = 32;
 
 constexpr int IT_VSTRIDE = P2_H + 2;  // floats between vectors staged in LDS
 constexpr int IT_RED = 20;            // block-reduction slots: 2 + 2 * 8 children, rounded up
@@ -170,6 +183,11 @@ __device__ __forceinline__ void lane_init(Lane& ln) {
 __device__ __forceinline__ void ld(float2 (&dst)[IT_PPT], const float* base, int64_t row, const Lane& ln) {
   const float2* s = p2_row2(base, row);
   IT_FOR(j) dst[j] = s[ln.idx[j]];
+  dst[2] = ln.ok2 ? dst[2] : make_float2(0.f, 0.f);
+}
+__device__ __forceinline__ void ld_masked(float2 (&dst)[IT_PPT], const float* base, int64_t row, const Lane& ln, int mask) {
+  const float2* s = p2_row2(base, row);
+  IT_FOR(j) dst[j] = s[ln.idx[j] & mask];
   dst[2] = ln.ok2 ? dst[2] : make_float2(0.f, 0.f);
 }
 __device__ __forceinline__ void st(float* base, int64_t row, const float2 (&src)[IT_PPT], const Lane& ln) {
@@ -261,11 +279,14 @@ __device__ __forceinline__ float2 mul2(float2 a, float2 b) { return make_float2(
 // row of its first child, the child count and who acts.  The kernel broadcasts an entry with a lane
 // read, so walking the tree costs no dependent global loads per family; every wave keeps its own copy.
 struct FamWin {
-  int p, first, ca;   // ca = child count | actor << 8 | kinds << 16
+  int p, first, ca;   // ca = child count | actor << 8
+  int kinds;          // see below
+  int rs;             // the range row of the player who did not act on the way into p (IterArgs::range_rows)
   int base;           // list position (relative to the item's first family) held by lane 0
 };
-// KINDS: also collect, per child k, bit 2k = the child has children, bit 2k + 1 = its ranges feed a
-// leaf evaluation (what a lean iteration decides its stores by).
+// KINDS: also collect what a lean iteration decides its stores by, per child k: bit 2k = the child has children,
+// bit 2k + 1 = its ranges feed a leaf evaluation, bit 16 + 2k = that evaluation reads both of the child's own
+// range rows (a leaf network), bit 17 + 2k = the child's values do not depend on the hand.
 template <int MAXC, bool KINDS>
 __device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t pp0, int nfam, int base) {
   const int l = base + (int)(threadIdx.x & 63);
@@ -273,22 +294,32 @@ __device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t p
   F.p = 0;
   F.first = 0;
   F.ca = 0;
+  F.kinds = 0;
+  F.rs = 0;
   if (l < nfam) {
     const int64_t p = A.root_parents[pp0 + l];
     const int64_t first = A.child_offsets[p];
     const int cnt = (int)A.child_count[p];
     F.p = (int)p;
     F.first = (int)first;
-    int kinds = 0;
-    if (KINDS) {
+    F.rs = A.range_rows ? A.range_rows[p] : 2 * (int)p;
+    if (KINDS || A.const_rows) {
+      uint32_t kinds = 0;
 #pragma unroll
-      for (int k = 0; k < MAXC; ++k)
-        if (k < cnt) kinds |= (((int)A.node_flags[first + k] >> 2) & 3) << (2 * k);
+      for (int k = 0; k < MAXC; ++k) {
+        if (k < cnt) {
+          const uint32_t fl = A.node_flags[first + k];
+          kinds |= ((fl >> 2) & 3u) << (2 * k);
+          if ((fl & (NODE_LEAF_EVAL | NODE_SHOWDOWN)) == NODE_LEAF_EVAL) kinds |= 0x10000u << (2 * k);
+          if ((fl & NODE_CONST) && A.const_rows) kinds |= 0x20000u << (2 * k);
+        }
+      }
+      F.kinds = (int)kinds;
     }
-    F.ca = cnt | ((int)A.to_act[p] << 8) | (kinds << 16);
+    F.ca = cnt | ((int)A.to_act[p] << 8);
   }
 }
-struct Fam { int64_t p, first; int cnt, actor, kinds; };
+struct Fam { int64_t p, first; int cnt, actor, kinds, rs; };
 __device__ __forceinline__ Fam fam_get(const FamWin& F, int i) {
   const int s = i - F.base;
   Fam f;
@@ -297,25 +328,36 @@ __device__ __forceinline__ Fam fam_get(const FamWin& F, int i) {
   const int ca = __builtin_amdgcn_readlane(F.ca, s);
   f.cnt = ca & 0xFF;
   f.actor = (ca >> 8) & 0xFF;
-  f.kinds = (int)((unsigned)ca >> 16);
+  f.kinds = __builtin_amdgcn_readlane(F.kinds, s);
+  f.rs = __builtin_amdgcn_readlane(F.rs, s);
   return f;
+}
+// Row (of the [total*2] row space) that holds player q's reach / ranges of the family's parent.
+__device__ __forceinline__ int64_t range_row(const Fam& f, int q) {
+  return ((f.rs ^ q) & 1) ? f.p * 2 + q : (int64_t)f.rs;
+}
+// All ones, or zero for a child whose row is the same number for every hand: ANDed to the lanes' pair indices it
+// makes every lane read the row's first pair (one line instead of 42, no branch around the load).
+__device__ __forceinline__ int const_mask(const Fam& f, int k) {
+  return ((f.kinds >> (17 + 2 * k)) & 1) ? 0 : -1;
 }
 
 // The same for the item's showdown rows: row, chips at stake for either player, scale.
 struct SdWin {
-  int c;
+  int c, rs;
   float pot0, pot1, scale;
   int base;
 };
 __device__ __forceinline__ void sd_load(SdWin& S, const IterArgs& A, int64_t sd0, int nsd, int base) {
   const int l = base + (int)(threadIdx.x & 63);
   S.base = base;
-  S.c = 0;
+  S.c = S.rs = 0;
   S.pot0 = S.pot1 = 0.f;
   S.scale = 1.f;
   if (l < nsd) {
     const int64_t c = A.root_showdown_nodes[sd0 + l];
     S.c = (int)c;
+    S.rs = A.range_rows ? A.range_rows[c] : 2 * (int)c;
     S.pot0 = A.potential[2 * c];
     S.pot1 = A.potential[2 * c + 1];
     S.scale = A.scale[c];
@@ -393,8 +435,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           for (int uu = 0; uu < SB; ++uu) {
             const int u = u0 + uu < nch ? u0 + uu : nch - 1;
             const Fam f = fam_get(F, i0 + u);
-            ld(bo[uu], leaf_beliefs, f.p * 2 + (1 - f.actor), ln);
-            if (stash) ld(ra[uu], A.reach_avg, f.p * 2 + f.actor, ln);  // the mix in sweep 2 needs the pre-update value
+            ld(bo[uu], leaf_beliefs, range_row(f, 1 - f.actor), ln);
+            if (stash) ld(ra[uu], A.reach_avg, range_row(f, f.actor), ln);  // the mix in sweep 2 needs the pre-update value
           }
 #pragma unroll
           for (int uu = 0; uu < SB; ++uu) {
@@ -433,7 +475,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
               const int k = g0 + kk;
               if (k < MAXC && k < cnt) {
                 const int64_t c = first + k;
-                ld(ach[kk], A.latest, c * 2 + actor, ln);
+                ld_masked(ach[kk], A.latest, c * 2 + actor, ln, const_mask(f, k));
                 ld(cu[kk], A.cum, c, ln);
                 ld(ws[kk], A.wsum, c, ln);
               }
@@ -540,15 +582,21 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // a leaf evaluation; an ordinary iteration keeps every row
       const int has_children = LEAN ? f.kinds & 0x5555 : 0x5555, leaf_eval = LEAN ? (f.kinds >> 1) & 0x5555 : 0x5555;
       const int keep_b = cfr_avg ? has_children : (has_children | leaf_eval);
+      // The player who does not act keeps the rows of the parent's range row: a lean iteration stores them
+      // again only right under the root (whose own rows are given, not computed) and where a leaf network
+      // reads a leaf's two rows side by side.
+      const int opp_all = !LEAN || !A.range_rows || (top && i == 0) ? 0x5555 : 0;
+      const int opp_rows = opp_all | (f.kinds >> 16);
       const int keep_ba = bavg_all ? 0x5555 : (cfr_avg ? (has_children | leaf_eval) : 0);
       float2 rn[2][IT_PPT], ran[2][IT_PPT], ra_old[IT_PPT];
       float2 cur[MAXC][IT_PPT], pav[MAXC][IT_PPT];
-      ld(rn[0], A.reach, p * 2, ln);
-      ld(rn[1], A.reach, p * 2 + 1, ln);
-      ld(ran[0], A.reach_avg, p * 2, ln);
-      ld(ran[1], A.reach_avg, p * 2 + 1, ln);
+      const int64_t row0 = range_row(f, 0), row1 = range_row(f, 1);
+      ld(rn[0], A.reach, row0, ln);
+      ld(rn[1], A.reach, row1, ln);
+      ld(ran[0], A.reach_avg, row0, ln);
+      ld(ran[1], A.reach_avg, row1, ln);
       if (stash) ld(ra_old, A.scratch, p, ln);
-      else ld(ra_old, A.reach_avg_prev, p * 2 + actor, ln);
+      else ld(ra_old, A.reach_avg_prev, actor == 0 ? row0 : row1, ln);
 #pragma unroll
       for (int k = 0; k < MAXC; ++k)
         if (k < cnt) ld(cur[k], A.policy, first + k, ln);
@@ -678,8 +726,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           const int64_t c = first + k;
           float2 xa[IT_PPT];
           from_lds(xa, L.u.vecs[k], ln);
-          if (actor == 0) { st(A.reach, c * 2, xa, ln); st(A.reach, c * 2 + 1, rn_opp, ln); }
-          else { st(A.reach, c * 2, rn_opp, ln); st(A.reach, c * 2 + 1, xa, ln); }
+          st(A.reach, c * 2 + actor, xa, ln);
+          if (opp_all) st(A.reach, c * 2 + 1 - actor, rn_opp, ln);
         }
       }
       // reach_avg
@@ -687,8 +735,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       for (int k = 0; k < MAXC; ++k) {
         if (k < cnt && ((has_children >> (2 * k)) & 1)) {
           const int64_t c = first + k;
-          if (actor == 0) { st(A.reach_avg, c * 2, pav[k], ln); st(A.reach_avg, c * 2 + 1, ran_opp, ln); }
-          else { st(A.reach_avg, c * 2, ran_opp, ln); st(A.reach_avg, c * 2 + 1, pav[k], ln); }
+          st(A.reach_avg, c * 2 + actor, pav[k], ln);
+          if (opp_all) st(A.reach_avg, c * 2 + 1 - actor, ran_opp, ln);
         }
       }
       // beliefs
@@ -709,8 +757,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
             const float2 vb = mul2(rb_act[j], xa[j]);
             o[j] = sa > 1e-5f ? make_float2(vb.x / sa, vb.y / sa) : ap[j];
           }
-          if (actor == 0) { st(A.beliefs, c * 2, o, ln); st(A.beliefs, c * 2 + 1, bo, ln); }
-          else { st(A.beliefs, c * 2, bo, ln); st(A.beliefs, c * 2 + 1, o, ln); }
+          st(A.beliefs, c * 2 + actor, o, ln);
+          if ((opp_rows >> (2 * k)) & 1) st(A.beliefs, c * 2 + 1 - actor, bo, ln);
         }
       }
       // beliefs_avg
@@ -724,8 +772,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
             const float2 vba = mul2(rba_act[j], pav[k][j]);
             oa[j] = saa > 1e-5f ? make_float2(vba.x / saa, vba.y / saa) : ap[j];
           }
-          if (actor == 0) { st(A.beliefs_avg, c * 2, oa, ln); st(A.beliefs_avg, c * 2 + 1, boa, ln); }
-          else { st(A.beliefs_avg, c * 2, boa, ln); st(A.beliefs_avg, c * 2 + 1, oa, ln); }
+          st(A.beliefs_avg, c * 2 + actor, oa, ln);
+          if (bavg_all || ((opp_rows >> (2 * k)) & 1)) st(A.beliefs_avg, c * 2 + 1 - actor, boa, ln);
         }
       }
     }
@@ -747,7 +795,13 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // global memory, hence a full barrier
       __syncthreads();
       float vk[2][SD_PPT];
-      showdown_gather(leaf_beliefs + (int64_t)__builtin_amdgcn_readlane(S.c, 0) * 2 * P2_H, sdr, vk);
+      // both players' range rows of showdown row c: the last actor's is c's own
+      auto gather = [&](int c, int rs, float (&v)[2][SD_PPT]) {
+        const int64_t own = (int64_t)c * 2;
+        const int64_t b0 = rs & 1 ? own : (int64_t)rs, b1 = rs & 1 ? (int64_t)rs : own + 1;
+        showdown_gather(leaf_beliefs + b0 * P2_H, leaf_beliefs + b1 * P2_H, sdr, v);
+      };
+      gather(__builtin_amdgcn_readlane(S.c, 0), __builtin_amdgcn_readlane(S.rs, 0), vk);
       for (int i = 0; i < nsd; ++i) {
         if (i >= S.base + 64) sd_load(S, A, sd0, nsd, i);
         const int sl = i - S.base;
@@ -755,9 +809,12 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
         const float pot0 = readlane_f(S.pot0, sl), pot1 = readlane_f(S.pot1, sl), scl = readlane_f(S.scale, sl);
         float vnext[2][SD_PPT];
         if (i + 1 < nsd) {
-          const int64_t cn = sl + 1 < 64 ? (int64_t)__builtin_amdgcn_readlane(S.c, (sl + 1) & 63)
-                                         : A.root_showdown_nodes[sd0 + i + 1];
-          showdown_gather(leaf_beliefs + cn * 2 * P2_H, sdr, vnext);
+          int cn = __builtin_amdgcn_readlane(S.c, (sl + 1) & 63), rsn = __builtin_amdgcn_readlane(S.rs, (sl + 1) & 63);
+          if (sl + 1 >= 64) {
+            cn = (int)A.root_showdown_nodes[sd0 + i + 1];
+            rsn = A.range_rows ? A.range_rows[cn] : 2 * cn;
+          }
+          gather(cn, rsn, vnext);
         }
         // the EVs land in the sorted-range buffers, which the evaluation no longer needs by then
         showdown_eval(vk, sdr, L.u.sd, L.u.sd.v, pot0, pot1, scl);
@@ -791,7 +848,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // actor beliefs at the parent and the marginal of every action, card-summed in one pass
       PROF_BEGIN(t_c3);
       float2 ab[IT_PPT], dn[IT_PPT], polk[MAXC][IT_PPT];
-      ld(ab, A.beliefs, p * 2 + actor, ln);
+      ld(ab, A.beliefs, range_row(f, actor), ln);
 #pragma unroll
       for (int k = 0; k < MAXC; ++k)
         if (k < cnt) ld(polk[k], A.policy, first + k, ln);
@@ -817,12 +874,14 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           float2 v[GRP3][2][IT_PPT], av[GRP3][2][IT_PPT];
 #pragma unroll
           for (int kk = 0; kk < GRP3; ++kk) {
-            const int64_t c = first + (g0 + kk < cnt ? g0 + kk : cnt - 1);
-            ld(v[kk][0], A.latest, c * 2, ln);
-            ld(v[kk][1], A.latest, c * 2 + 1, ln);
+            const int k = g0 + kk < cnt ? g0 + kk : cnt - 1;
+            const int64_t c = first + k;
+            const int m = const_mask(f, k);
+            ld_masked(v[kk][0], A.latest, c * 2, ln, m);
+            ld_masked(v[kk][1], A.latest, c * 2 + 1, ln, m);
             if (update_avg) {
-              ld(av[kk][0], A.values_avg, c * 2, ln);
-              ld(av[kk][1], A.values_avg, c * 2 + 1, ln);
+              ld_masked(av[kk][0], A.values_avg, c * 2, ln, m);
+              ld_masked(av[kk][1], A.values_avg, c * 2 + 1, ln, m);
             }
           }
           if (g0 == 0) {
@@ -856,7 +915,11 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 #pragma unroll
                 for (int pl = 0; pl < 2; ++pl) {
                   IT_FOR(j) av[kk][pl][j] = make_float2(av[kk][pl][j].x - shift, av[kk][pl][j].y - shift);
-                  st(A.values_avg, c * 2 + pl, av[kk][pl], ln);
+                  if (LEAN && const_mask(f, k) == 0) {
+                    if (threadIdx.x == 0) p2_row2(A.values_avg, c * 2 + pl)[0] = av[kk][pl][0];
+                  } else {
+                    st(A.values_avg, c * 2 + pl, av[kk][pl], ln);
+                  }
                 }
               }
               float2 nm[IT_PPT], occ[IT_PPT];
@@ -916,6 +979,27 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
     }
     PROF_END(2, t_s3);
   }
+}
+
+// IterArgs::range_rows of every row.  Rows are numbered top-down (a parent before its children), so the walk
+// towards the root ends; a row whose parent index does not fit that keeps its own row.
+__global__ __launch_bounds__(256) void range_rows_kernel(const int64_t* __restrict__ parent,
+                                                         const int64_t* __restrict__ to_act, int64_t n_roots,
+                                                         int64_t total, int32_t* __restrict__ out) {
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= total) return;
+  int64_t row = 2 * c;
+  if (c >= n_roots && parent[c] >= 0 && parent[c] < c) {
+    const int o = to_act[parent[c]] == 0 ? 1 : 0;
+    int64_t y = c;
+    while (true) {
+      const int64_t p = parent[y];
+      if (p < n_roots || p >= y || to_act[p] == o) break;   // right under the root, or o's own last action
+      y = p;
+    }
+    row = 2 * y + o;
+  }
+  out[c] = (int32_t)row;
 }
 
 struct ScalarPack {
@@ -979,9 +1063,9 @@ int p2hip_upload_floats(float* dst, const float* host_values, int n, void* strea
 
 // P2HipIterArgs (include/p2hip.h) mirrors p2::IterArgs field by field.
 
-int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max_children, int phases,
-                        void* stream) {
-  if (!host_args || n_items < 0 || n_items > 0x7FFFFFFF || max_children < 1 || max_children > 8 || (phases & ~31) ||
+static int p2_launch_iteration(const P2HipIterArgs* host_args, const int32_t* range_rows, int64_t n_items,
+                               int max_children, int phases, void* stream) {
+  if (!host_args || n_items < 0 || n_items > 0x7FFFFFFF || max_children < 1 || max_children > 8 ||
       (phases & 15) == 0)
     return P2_EINVAL;
   if (n_items == 0) return 0;
@@ -1014,6 +1098,8 @@ int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max
   a.item_root = h.item_root; a.item_top = h.item_top;
   a.reach_avg_prev = h.reach_avg_prev;
   a.phases = phases & 15;
+  a.range_rows = range_rows;
+  a.const_rows = (phases & p2::PHASE_CONST) != 0;
   const bool lean = (phases & p2::PHASE_LEAN) != 0;
   const dim3 grid((unsigned)n_items), block(p2::IT_BLOCK);
   const bool alt = h.reach_avg_prev != nullptr;
@@ -1032,6 +1118,30 @@ int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max
 #undef P2_ITER_LAUNCH
   P2_LAUNCH_CHECK();
   return 0;
+}
+
+int p2hip_range_rows(const int64_t* parent_index, const int64_t* to_act, int64_t n_roots, int64_t total, int32_t* out,
+                     void* stream) {
+  if (total < 0 || total > 0x3FFFFFFF || n_roots < 0 || n_roots > total) return P2_EINVAL;
+  if (total == 0) return 0;
+  if (!parent_index || !to_act || !out || !p2_aligned8(parent_index) || !p2_aligned8(to_act) || !p2_aligned4(out))
+    return P2_EINVAL;
+  hipLaunchKernelGGL(p2::range_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                     parent_index, to_act, n_roots, total, out);
+  P2_LAUNCH_CHECK();
+  return 0;
+}
+
+int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max_children, int phases,
+                        void* stream) {
+  if (phases & ~31) return P2_EINVAL;
+  return p2_launch_iteration(host_args, nullptr, n_items, max_children, phases, stream);
+}
+
+int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* range_rows, int64_t n_items,
+                               int max_children, int phases, void* stream) {
+  if ((phases & ~63) || !p2_aligned4(range_rows)) return P2_EINVAL;
+  return p2_launch_iteration(host_args, range_rows, n_items, max_children, phases, stream);
 }
 
 }  // extern "C"

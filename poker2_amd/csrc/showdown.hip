@@ -488,16 +488,16 @@ __device__ __forceinline__ void showdown_load_regs(const uint8_t* __restrict__ t
   for (int i = 0; i < 13; ++i) R.clist[i] = lane < 51 ? cl[i] : 0xFFFFu;
 }
 
-// Gather both ranges of the node whose beliefs start at `bel` ([2,H]) into strength order:
+// Gather both ranges of a node (`bel0` / `bel1`: the rows of players 0 and 1) into strength order:
 // vk[p][i] = villain-of-hero-p mass at this lane's i-th sorted position.
-__device__ __forceinline__ void showdown_gather(const float* __restrict__ bel, const ShowdownRegs& R,
-                                                float (&vk)[2][SD_PPT]) {
+__device__ __forceinline__ void showdown_gather(const float* __restrict__ bel0, const float* __restrict__ bel1,
+                                                const ShowdownRegs& R, float (&vk)[2][SD_PPT]) {
 #pragma unroll
   for (int i = 0; i < SD_PPT; ++i) {
     const bool ok = R.perm[i] != 0xFFFFFFFFu;
     const int h = (int)(R.perm[i] & 0x7FFFu);
-    vk[0][i] = ok ? bel[P2_H + h] : 0.f;
-    vk[1][i] = ok ? bel[h] : 0.f;
+    vk[0][i] = ok ? bel1[h] : 0.f;
+    vk[1][i] = ok ? bel0[h] : 0.f;
   }
 }
 
@@ -647,7 +647,7 @@ __global__ __launch_bounds__(SD_BLOCK, 3) void showdown_both_kernel(const float*
   int64_t n = blockIdx.x;
   if (n < m) {
     showdown_load_regs(tables + (table_row ? table_row[n] : n) * SD_TABLE_BYTES, Rn, ab_lds);
-    showdown_gather(beliefs + n * 2 * P2_H, Rn, vkn);
+    showdown_gather(beliefs + n * 2 * P2_H, beliefs + n * 2 * P2_H + P2_H, Rn, vkn);
   }
   for (; n < m; n += gridDim.x) {
     R = Rn;
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(SD_BLOCK, 3) void showdown_both_kernel(const float*
     if (more) showdown_load_regs(tables + (table_row ? table_row[nn] : nn) * SD_TABLE_BYTES, Rn, ab_lds);
     const float mul0 = potential[2 * n], mul1 = potential[2 * n + 1], div = scale[n];
     showdown_scans(vk, R, s);
-    if (more) showdown_gather(beliefs + nn * 2 * P2_H, Rn, vkn);
+    if (more) showdown_gather(beliefs + nn * 2 * P2_H, beliefs + nn * 2 * P2_H + P2_H, Rn, vkn);
     // the EVs go over the sorted ranges, which are dead once the card scans are done
     showdown_finish(vk, R, s, s.v, mul0, mul1, div);
     p2_sync_lds();

@@ -50,7 +50,7 @@ STATE_NAMES = ("policy_probs", "policy_probs_avg", "policy_probs_sample", "cumul
                "regret_weight_sums", "self_reach", "self_reach_avg", "beliefs", "beliefs_avg",
                "latest_values", "values_avg")
 
-_NODE_SHOWDOWN, _NODE_DONE, _NODE_PARENT, _NODE_LEAF_EVAL = 1, 2, 4, 8
+_NODE_SHOWDOWN, _NODE_DONE, _NODE_PARENT, _NODE_LEAF_EVAL, _NODE_CONST = 1, 2, 4, 8, 16
 
 
 class _IterArgs(ctypes.Structure):
@@ -68,6 +68,8 @@ _PHASE_12, _PHASE_3, _PHASE_1, _PHASE_2 = 1, 2, 4, 8
 # Lean launch (include/p2hip.h): the reach / belief part stores only the rows that the rest of the
 # iteration or the next iteration reads.  ``evaluate_cfr`` runs every iteration but its last that way.
 _PHASE_LEAN = 16
+# Fold leaves are one number per player: read through their first pair (lean iterations, and the one that follows).
+_PHASE_CONST = 32
 # One workgroup per root fills the chip (256 CUs x 3 resident workgroups) from 768 roots on.  Below
 # SPLIT_ROOTS_BELOW roots each root's tree is cut at level SPLIT_CUT_LEVEL into work items (the top of
 # the tree, and one subtree per node of that level) that get a workgroup each.  Measured on the
@@ -494,7 +496,14 @@ class HipSparseCFREvaluator:
         flags[tree.showdown_mask & (tree.child_count == 0)] |= _NODE_LEAF_EVAL
         if self.model is not None:
             flags[model_mask & (tree.child_count == 0)] |= _NODE_LEAF_EVAL
+        flags[tree.fold_mask & (tree.child_count == 0)] |= _NODE_CONST
         self._node_flags = self._t(flags)
+        # rows of values_avg that lean iterations have left in their first pair only
+        self._const_rows_short = False
+        self._range_rows = torch.empty(T, dtype=torch.int32, device=dev)
+        code = _lib.load().p2hip_range_rows(_lib.ptr(self.parent_index), _lib.ptr(self.env.to_act), N, T,
+                                            _lib.ptr(self._range_rows), _lib.stream_ptr())
+        _lib.check(code, "p2hip_range_rows")
         def per_root(mask):
             """Rows selected by ``mask`` grouped by root (ascending inside a root) + offsets [N+1]."""
             rows = np.nonzero(mask)[0]
@@ -892,9 +901,9 @@ class HipSparseCFREvaluator:
     def _launch_items(self, args: _IterArgs, n_items: int, phases: int) -> None:
         if n_items == 0:
             return
-        code = _lib.load().p2hip_cfr_iteration(ctypes.byref(args), n_items, self._max_children, phases,
-                                               _lib.stream_ptr())
-        _lib.check(code, "p2hip_cfr_iteration")
+        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), _lib.ptr(self._range_rows), n_items,
+                                                      self._max_children, phases, _lib.stream_ptr())
+        _lib.check(code, "p2hip_cfr_iteration_shared")
 
     def _other_reach_avg(self) -> torch.Tensor:
         """The second reach_avg buffer of the alternating scheme (allocated on first use; root rows 1)."""
@@ -937,7 +946,9 @@ class HipSparseCFREvaluator:
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
         alternate = alternate and bool(phases & _PHASE_12)
         b = self._iter_bundle(alternate)
-        mode = _PHASE_LEAN if lean else 0
+        mode = _PHASE_LEAN | _PHASE_CONST if lean else (_PHASE_CONST if self._const_rows_short else 0)
+        if phases & _PHASE_3 and not self.use_final_policy_values:
+            self._const_rows_short = lean
         if self._items is None:
             self._launch_items(b.main, self.root_nodes, phases | mode)
         else:
