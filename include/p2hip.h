@@ -438,9 +438,18 @@ int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max
  *   whatever the hand) are read through their first two entries; a lean iteration stores only those two of
  *   values_avg.  After lean iterations with the bit, one iteration with the bit and without bit 4 makes every
  *   row whole again.
- * The state after that last iteration is bit-identical to p2hip_cfr_iteration's. */
-int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* range_rows, int64_t n_items,
-                               int max_children, int phases, void* stream);
+ * leaf_prev (optional, [total,2,H]): beliefs (beliefs_avg under cfr_avg) as the previous iteration left them, where
+ *   that was another buffer than the one in host_args.
+ * phases bit 6 (64): one walk per family instead of three (bit 7, 128, with it exactly if iscal[6] is set): regrets,
+ *   policy, ranges, the value of the showdown child, and the backup of families whose children are all leaves, with
+ *   phases bit 0; the backup of the others with bit 1.  Needs bits 4 and 5, range_rows, reach_avg_prev, at most five
+ *   children per parent, at most one showdown child among siblings (not checked here: it is a property of the
+ *   tree), no enforce_zero_sum, and two range buffers: leaf_prev is read and leaf_next written in place of
+ *   beliefs (beliefs_avg under cfr_avg) of host_args; both hold the roots' ranges (the walk copies them on).
+ *   Bits 2 and 3 do not apply: tiers of work items take bit 0 downwards and bit 1 upwards.
+ * The state after a closing iteration without bits 4 and 6 is bit-identical to p2hip_cfr_iteration's. */
+int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* range_rows, const float* leaf_prev,
+                               float* leaf_next, int64_t n_items, int max_children, int phases, void* stream);
 
 /* range_rows of a tree: parent_index [total] (rows numbered top-down, the n_roots roots first), to_act [total]. */
 int p2hip_range_rows(const int64_t* parent_index, const int64_t* to_act, int64_t n_roots, int64_t total, int32_t* out,

@@ -72,7 +72,7 @@ _SIGNATURES: dict[str, list] = {
     "p2hip_deep_beliefs": [_P, _P, _P, _P, _P, _L, _L, _F, _P],
     "p2hip_sample_snapshot": [_P, _P, _P, _P, _L, _P],
     "p2hip_cfr_iteration": [_P, _L, _I, _I, _P],
-    "p2hip_cfr_iteration_shared": [_P, _P, _L, _I, _I, _P],
+    "p2hip_cfr_iteration_shared": [_P, _P, _P, _P, _L, _I, _I, _P],
     "p2hip_range_rows": [_P, _P, _L, _L, _P, _P],
     "p2hip_write_scalars": [_P, _P, _P, _P, _P],
     "p2hip_stream_probe": [_P, _P, _L, _I, _I, _I, _P],

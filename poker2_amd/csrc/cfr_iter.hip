@@ -14,6 +14,7 @@
 // A "family" is a parent and its contiguous child rows.  Every thread owns the same
 // three float2 pairs (six hands) of every 1326-vector for the whole kernel, so all
 // per-hand work is register-to-register; only sums over hands go through LDS.
+#pragma once
 #include "common.h"
 #include "unblocked.hip"
 #include "showdown.hip"
@@ -95,6 +96,8 @@ struct IterArgs {
   // every node since that player's last action (only the actor's reach changes, and a range is a function of
   // the reach alone), so a lean iteration stores them once, and every iteration reads them there.
   const int32_t* range_rows;
+  const float* leaf_prev;  // null, or [total,2,H]: the ranges the regret part reads (beliefs; beliefs_avg under cfr_avg)
+                           // as the previous iteration left them, where that was another buffer
   int const_rows;        // rows flagged NODE_CONST: read the first pair only, store only that in a lean iteration
 };
 
@@ -435,7 +438,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           for (int uu = 0; uu < SB; ++uu) {
             const int u = u0 + uu < nch ? u0 + uu : nch - 1;
             const Fam f = fam_get(F, i0 + u);
-            ld(bo[uu], leaf_beliefs, range_row(f, 1 - f.actor), ln);
+            ld(bo[uu], A.leaf_prev ? A.leaf_prev : leaf_beliefs, range_row(f, 1 - f.actor), ln);
             if (stash) ld(ra[uu], A.reach_avg, range_row(f, f.actor), ln);  // the mix in sweep 2 needs the pre-update value
           }
 #pragma unroll
@@ -1063,8 +1066,9 @@ int p2hip_upload_floats(float* dst, const float* host_values, int n, void* strea
 
 // P2HipIterArgs (include/p2hip.h) mirrors p2::IterArgs field by field.
 
-static int p2_launch_iteration(const P2HipIterArgs* host_args, const int32_t* range_rows, int64_t n_items,
-                               int max_children, int phases, void* stream) {
+// The kernel's arguments from the caller's, after the checks every entry point makes.
+static int p2_iteration_args(const P2HipIterArgs* host_args, int64_t n_items, int max_children, int phases,
+                             p2::IterArgs& a) {
   if (!host_args || n_items < 0 || n_items > 0x7FFFFFFF || max_children < 1 || max_children > 8 ||
       (phases & 15) == 0)
     return P2_EINVAL;
@@ -1086,7 +1090,6 @@ static int p2_launch_iteration(const P2HipIterArgs* host_args, const int32_t* ra
                         h.reach_avg_prev};
   for (const void* p : rows)
     if (!p2_aligned8(p)) return P2_EINVAL;
-  p2::IterArgs a;
   a.child_offsets = h.child_offsets; a.child_count = h.child_count; a.to_act = h.to_act;
   a.node_flags = h.node_flags; a.root_parent_offsets = h.root_parent_offsets; a.root_parents = h.root_parents;
   a.root_showdown_offsets = h.root_showdown_offsets; a.root_showdown_nodes = h.root_showdown_nodes;
@@ -1098,11 +1101,16 @@ static int p2_launch_iteration(const P2HipIterArgs* host_args, const int32_t* ra
   a.item_root = h.item_root; a.item_top = h.item_top;
   a.reach_avg_prev = h.reach_avg_prev;
   a.phases = phases & 15;
-  a.range_rows = range_rows;
+  a.range_rows = nullptr;
+  a.leaf_prev = nullptr;
   a.const_rows = (phases & p2::PHASE_CONST) != 0;
+  return 0;
+}
+
+static int p2_launch_iteration(const p2::IterArgs& a, int64_t n_items, int max_children, int phases, void* stream) {
   const bool lean = (phases & p2::PHASE_LEAN) != 0;
   const dim3 grid((unsigned)n_items), block(p2::IT_BLOCK);
-  const bool alt = h.reach_avg_prev != nullptr;
+  const bool alt = a.reach_avg_prev != nullptr;
 #define P2_ITER_LAUNCH(MAXC, LEAN, ALT) \
   hipLaunchKernelGGL((p2::cfr_iteration_kernel<MAXC, LEAN, ALT>), grid, block, 0, (hipStream_t)stream, a)
 #define P2_ITER_MODES(MAXC)                                  \
@@ -1135,13 +1143,9 @@ int p2hip_range_rows(const int64_t* parent_index, const int64_t* to_act, int64_t
 int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max_children, int phases,
                         void* stream) {
   if (phases & ~31) return P2_EINVAL;
-  return p2_launch_iteration(host_args, nullptr, n_items, max_children, phases, stream);
-}
-
-int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* range_rows, int64_t n_items,
-                               int max_children, int phases, void* stream) {
-  if ((phases & ~63) || !p2_aligned4(range_rows)) return P2_EINVAL;
-  return p2_launch_iteration(host_args, range_rows, n_items, max_children, phases, stream);
+  p2::IterArgs a;
+  const int bad = p2_iteration_args(host_args, n_items, max_children, phases, a);
+  return bad || n_items == 0 ? bad : p2_launch_iteration(a, n_items, max_children, phases, stream);
 }
 
 }  // extern "C"

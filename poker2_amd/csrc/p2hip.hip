@@ -6,6 +6,7 @@
 #include "showdown.hip"
 #include "cfr_ops.hip"
 #include "cfr_iter.hip"
+#include "cfr_search.hip"
 #include "chance.hip"
 #include "best_response.hip"
 #include "tree.hip"

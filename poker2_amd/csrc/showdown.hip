@@ -575,7 +575,45 @@ __device__ __forceinline__ void showdown_scans(const float (&vk)[2][SD_PPT], con
   p2_sync_lds();
 }
 
-// Second half: eight 64-bit LDS reads per hand serve both players; EVs written in combo order to ev.
+// EVs (hero 0, hero 1) of one hand from the prefixes: eight 64-bit LDS reads serve both players.
+//   perm, lr, cidx, ab: the hand's entries of ShowdownRegs; vk0, vk1: its masses; r0, r1: potential / scale
+__device__ __forceinline__ float2 showdown_hand(const ShowdownLds& s, uint32_t perm, uint32_t lr, uint32_t cidx,
+                                                uint32_t ab, float vk0, float vk1, float r0, float r1) {
+  const bool live = !(perm & 0x8000u);   // not blocked by the board
+  const int L = (int)(lr & 0xFFFFu), Rr = (int)(lr >> 16);
+  const int a = (int)(ab & 0xFFu), b = (int)(ab >> 8);
+  const int iLa = (int)(cidx & 0xFFu), iRa = (int)((cidx >> 8) & 0xFFu);
+  const int iLb = (int)((cidx >> 16) & 0xFFu), iRb = (int)(cidx >> 24);
+  const float2 PL2 = s.P[L], PR2 = s.P[Rr];
+  const float2 aL2 = s.Pc[a][iLa], aR2 = s.Pc[a][iRa], bL2 = s.Pc[b][iLb], bR2 = s.Pc[b][iRb];
+  const float2 aT2 = s.Pc[a][51], bT2 = s.Pc[b][51];
+  float e[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const float v0 = p ? vk1 : vk0;
+    const float PL = p ? PL2.y : PL2.x, PR = p ? PR2.y : PR2.x;
+    const float aL = p ? aL2.y : aL2.x, aR = p ? aR2.y : aR2.x;
+    const float bL = p ? bL2.y : bL2.x, bR = p ? bR2.y : bR2.x;
+    const float win = PL - aL - bL;
+    const float tie = (PR - PL) - (aR - aL) - (bR - bL) + v0;
+    float den = 1.0f - (p ? aT2.y : aT2.x) - (p ? bT2.y : bT2.x) + v0;
+    den = fmaxf(den, 1e-8f);
+    // The kernel is VALU-issue bound and an IEEE division is about ten instructions, so both
+    // quotients share one hardware reciprocal and are corrected by one fused residual step
+    // each, which keeps x/x == 1 and 0/x == 0 exact (an all-tie board stays exactly zero).
+    // a hand the board blocks goes the way of an empty denominator: every quotient 0, EV 0
+    const bool valid = live && den > 1e-8f;
+    const float inv = valid ? __builtin_amdgcn_rcpf(den) : 0.f;
+    float wp = win * inv, tp = tie * inv;
+    wp = __builtin_fmaf(__builtin_fmaf(-wp, den, win), inv, wp);
+    tp = __builtin_fmaf(__builtin_fmaf(-tp, den, tie), inv, tp);
+    const float lp = valid ? 1.0f - wp - tp : 0.f;
+    e[p] = wp - lp;
+  }
+  return make_float2(e[0] * r0, e[1] * r1);
+}
+
+// Second half: EVs written in combo order to ev.
 __device__ __forceinline__ void showdown_finish(const float (&vk)[2][SD_PPT], const ShowdownRegs& R,
                                                 const ShowdownLds& s, float2* ev, float mul0, float mul1, float div) {
   const float r0 = mul0 / div, r1 = mul1 / div;  // potential / scale of the node, one division each
@@ -583,38 +621,7 @@ __device__ __forceinline__ void showdown_finish(const float (&vk)[2][SD_PPT], co
   for (int i = 0; i < SD_PPT; ++i) {
     if (R.perm[i] == 0xFFFFFFFFu) continue;
     const int h = (int)(R.perm[i] & 0x7FFFu);
-    const bool live = !(R.perm[i] & 0x8000u);   // not blocked by the board
-    const int L = (int)(R.lr[i] & 0xFFFFu), Rr = (int)(R.lr[i] >> 16);
-    const int a = (int)(R.ab[i] & 0xFFu), b = (int)(R.ab[i] >> 8);
-    const int iLa = (int)(R.cidx[i] & 0xFFu), iRa = (int)((R.cidx[i] >> 8) & 0xFFu);
-    const int iLb = (int)((R.cidx[i] >> 16) & 0xFFu), iRb = (int)(R.cidx[i] >> 24);
-    const float2 PL2 = s.P[L], PR2 = s.P[Rr];
-    const float2 aL2 = s.Pc[a][iLa], aR2 = s.Pc[a][iRa], bL2 = s.Pc[b][iLb], bR2 = s.Pc[b][iRb];
-    const float2 aT2 = s.Pc[a][51], bT2 = s.Pc[b][51];
-    float e[2];
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const float v0 = vk[p][i];
-      const float PL = p ? PL2.y : PL2.x, PR = p ? PR2.y : PR2.x;
-      const float aL = p ? aL2.y : aL2.x, aR = p ? aR2.y : aR2.x;
-      const float bL = p ? bL2.y : bL2.x, bR = p ? bR2.y : bR2.x;
-      const float win = PL - aL - bL;
-      const float tie = (PR - PL) - (aR - aL) - (bR - bL) + v0;
-      float den = 1.0f - (p ? aT2.y : aT2.x) - (p ? bT2.y : bT2.x) + v0;
-      den = fmaxf(den, 1e-8f);
-      // The kernel is VALU-issue bound and an IEEE division is about ten instructions, so both
-      // quotients share one hardware reciprocal and are corrected by one fused residual step
-      // each, which keeps x/x == 1 and 0/x == 0 exact (an all-tie board stays exactly zero).
-      // a hand the board blocks goes the way of an empty denominator: every quotient 0, EV 0
-      const bool valid = live && den > 1e-8f;
-      const float inv = valid ? __builtin_amdgcn_rcpf(den) : 0.f;
-      float wp = win * inv, tp = tie * inv;
-      wp = __builtin_fmaf(__builtin_fmaf(-wp, den, win), inv, wp);
-      tp = __builtin_fmaf(__builtin_fmaf(-tp, den, tie), inv, tp);
-      const float lp = valid ? 1.0f - wp - tp : 0.f;
-      e[p] = wp - lp;
-    }
-    ev[h] = make_float2(e[0] * r0, e[1] * r1);
+    ev[h] = showdown_hand(s, R.perm[i], R.lr[i], R.cidx[i], R.ab[i], vk[0][i], vk[1][i], r0, r1);
   }
 }
 

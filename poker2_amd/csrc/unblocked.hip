@@ -20,11 +20,14 @@ constexpr int UB_WAVES = UB_BLOCK / 64;
 // Four lanes share one (vector, card) task: each adds 13 partner cards, two shuffles
 // combine them.  Every thread must call it after an LDS barrier that covers the staged
 // vectors; it ends with an LDS barrier.
-__device__ __forceinline__ void card_sums_multi(const float* t, int stride, int nvec, double* cs) {
-  const int sub = threadIdx.x & 3;
+// `tid` is threadIdx.x; a caller inside a loop may pass a copy that the optimiser cannot see through, so that the
+// thirteen offsets of a task are not kept in registers from one call to the next.
+template <int BLOCK>
+__device__ __forceinline__ void card_sums_block(const float* t, int stride, int nvec, double* cs, int tid) {
+  const int sub = tid & 3;
   const int ntask = nvec * P2_CARDS;
-  for (int base = 0; base < ntask; base += UB_BLOCK / 4) {
-    const int task = base + (threadIdx.x >> 2);
+  for (int base = 0; base < ntask; base += BLOCK / 4) {
+    const int task = base + (tid >> 2);
     const bool valid = task < ntask;
     double v = 0.0;
     if (valid) {
@@ -45,6 +48,10 @@ __device__ __forceinline__ void card_sums_multi(const float* t, int stride, int 
     if (valid && sub == 0) cs[task] = v;
   }
   p2_sync_lds();
+}
+
+__device__ __forceinline__ void card_sums_multi(const float* t, int stride, int nvec, double* cs) {
+  card_sums_block<UB_BLOCK>(t, stride, nvec, cs, (int)threadIdx.x);
 }
 
 // Total mass of a vector from its 52 card sums (every combo is counted under both of its

@@ -70,6 +70,16 @@ _PHASE_12, _PHASE_3, _PHASE_1, _PHASE_2 = 1, 2, 4, 8
 _PHASE_LEAN = 16
 # Fold leaves are one number per player: read through their first pair (lean iterations, and the one that follows).
 _PHASE_CONST = 32
+# One walk per family (csrc/cfr_search.hip): lean iterations between two buffers of reach_avg and of the ranges the
+# leaves are evaluated with.  The kernel has registers for five children per parent.
+_PHASE_FUSED, _PHASE_FUSED_CFR_AVG = 64, 128
+FUSED_MAX_CHILDREN = 5
+# It shortens the chain of steps per family, at the cost of fewer workgroups per compute unit, so it is for launches
+# that leave the chip part empty: at most this many work items in a tier.  us per iteration, three walks -> one:
+# three-raise tree (9 items per root) 64 roots 386 -> 270, 96 roots 428 -> 380, 128 roots 465 -> 472, 192 roots 569 ->
+# 686; one-raise tree (4 per root) 128 roots 156 -> 134, 192 roots 171 -> 180; depth-2 tree (4 per root) 128 roots 110 ->
+# 95, 192 roots 128 -> 120, 300 roots 199 -> 223.
+FUSED_MAX_ITEMS = 640
 # One workgroup per root fills the chip (256 CUs x 3 resident workgroups) from 768 roots on.  Below
 # SPLIT_ROOTS_BELOW roots each root's tree is cut at level SPLIT_CUT_LEVEL into work items (the top of
 # the tree, and one subtree per node of that level) that get a workgroup each.  Measured on the
@@ -240,6 +250,7 @@ class HipSparseCFREvaluator:
         self._iscal_host = (ctypes.c_int64 * 8)()
         self._iter_bundles: dict = {}
         self._reach_avg_alt = None
+        self._leaf_alt = None
         self._chance_helper = None
         self.subgame_serial = 0
 
@@ -363,7 +374,7 @@ class HipSparseCFREvaluator:
 
     _STATE_TENSORS = ("policy_probs", "policy_probs_avg", "policy_probs_sample", "cumulative_regrets",
                       "regret_weight_sums", "beliefs", "beliefs_avg", "self_reach", "self_reach_avg", "latest_values",
-                      "values_avg", "_scratch", "_reach_avg_alt")
+                      "values_avg", "_scratch", "_reach_avg_alt", "_leaf_alt", "_leaf_home")
 
     def _drop_state(self) -> None:
         """Let go of the state tensors and their slabs (``reuse_state``), so that larger slabs can take
@@ -475,6 +486,9 @@ class HipSparseCFREvaluator:
         cc_dest = self.child_count[:tree.top].repeat_interleave(self.child_count[:tree.top])
         self.uniform_policy[N:] = (1.0 / cc_dest)[:, None].expand(-1, NUM_HANDS)
         self.beliefs, self.beliefs_avg = z2(), z2()
+        # the leaf ranges' own tensor: what every iteration but a one-walk one writes
+        self._leaf_home = self.beliefs_avg if self.cfr_avg else self.beliefs
+        self._walk_open = None         # the argument blocks of a one-walk iteration whose leaves a network evaluates
         self.root_pre_chance_beliefs = torch.zeros(N, 2, NUM_HANDS, dtype=self.float_dtype, device=dev)
         self.self_reach = z2()
         self.self_reach[:N] = 1.0
@@ -526,6 +540,12 @@ class HipSparseCFREvaluator:
         # (whole tree tops), which makes fewer and longer workgroups of the same work.
         self._items_regret = (self._split_items(tree) if self._items is not None and len(self._items.tiers) > 2
                               else self._items)
+        # the one-walk kernel: few work items, at most one showdown child among siblings
+        showdown_parents = tree.parent_index[tree.showdown_mask]
+        self._one_walk = (with_alt and T > N and self._max_children <= FUSED_MAX_CHILDREN
+                          and (max(self._items.tiers) if self._items is not None else N) <= FUSED_MAX_ITEMS
+                          and not bool((np.diff(showdown_parents) == 0).any()))
+        self._leaf_alt = torch.empty_like(self._leaf_home) if self._one_walk else None
         self._root_items = None
         if self._items is None and T:
             # Roots of unequal size (mixed streets, stacks, pots): one work item per root, largest tree first, so
@@ -885,7 +905,8 @@ class HipSparseCFREvaluator:
         a.potential, a.scale = p(self._potential_all), p(self.env.scale)
         a.policy, a.policy_avg, a.policy_sample = p(self.policy_probs), p(self.policy_probs_avg), p(self.policy_probs_sample)
         a.cum, a.wsum = p(self.cumulative_regrets), p(self.regret_weight_sums)
-        a.beliefs, a.beliefs_avg = p(self.beliefs), p(self.beliefs_avg)
+        a.beliefs = p(self.beliefs if self.cfr_avg else self._leaf_home)
+        a.beliefs_avg = p(self._leaf_home if self.cfr_avg else self.beliefs_avg)
         a.reach = p(self.self_reach)
         a.reach_avg = p(self.self_reach_avg if reach_avg is None else reach_avg)
         a.reach_avg_prev = p(reach_avg_prev)
@@ -898,12 +919,46 @@ class HipSparseCFREvaluator:
             a.item_root, a.item_top = p(it.item_root), p(it.item_top)
         return a
 
-    def _launch_items(self, args: _IterArgs, n_items: int, phases: int) -> None:
+    def _launch_items(self, args: _IterArgs, n_items: int, phases: int, leaf_prev: torch.Tensor | None = None,
+                      leaf_next: torch.Tensor | None = None) -> None:
         if n_items == 0:
             return
-        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), _lib.ptr(self._range_rows), n_items,
-                                                      self._max_children, phases, _lib.stream_ptr())
+        p = _lib.ptr
+        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), p(self._range_rows), p(leaf_prev), p(leaf_next),
+                                                      n_items, self._max_children, phases, _lib.stream_ptr())
         _lib.check(code, "p2hip_cfr_iteration_shared")
+
+    def _swap_leaf_ranges(self) -> torch.Tensor:
+        """Let the evaluator's name for the leaf ranges (``beliefs``, ``beliefs_avg`` with CFR-AVG) stand for the
+        other of the two buffers; returns the one it stood for."""
+        name = "beliefs_avg" if self.cfr_avg else "beliefs"
+        before = getattr(self, name)
+        setattr(self, name, self._leaf_alt)
+        self._leaf_alt = before
+        return before
+
+    def _launch_walk(self, phases: int) -> None:
+        """A lean iteration by the one-walk kernel (``_one_walk``); ``phases`` as in ``_launch_iteration``.  The
+        name of the leaf ranges and ``self_reach_avg`` stand for the buffers just written when this returns."""
+        mode = _PHASE_LEAN | _PHASE_CONST | _PHASE_FUSED | (_PHASE_FUSED_CFR_AVG if self.cfr_avg else 0)
+        if phases & _PHASE_12:
+            b = self._iter_bundle(True)
+            prev = self._swap_leaf_ranges()
+            self.self_reach_avg, self._reach_avg_alt = self._reach_avg_alt, self.self_reach_avg
+        else:
+            b, prev = self._walk_open
+        now = self.beliefs_avg if self.cfr_avg else self.beliefs
+        tiers = b.tiers if self._items is not None else [(b.main, self.root_nodes)]
+        down, up = phases & _PHASE_12, phases & _PHASE_3
+        if down:
+            for args, count in tiers[:-1]:
+                self._launch_items(args, count, _PHASE_12 | mode, prev, now)
+        args, count = tiers[-1]
+        self._launch_items(args, count, down | up | mode, prev, now)
+        if up:
+            for args, count in reversed(tiers[:-1]):
+                self._launch_items(args, count, _PHASE_3 | mode, prev, now)
+        self._walk_open = None if up else (b, prev)
 
     def _other_reach_avg(self) -> torch.Tensor:
         """The second reach_avg buffer of the alternating scheme (allocated on first use; root rows 1)."""
@@ -944,17 +999,28 @@ class HipSparseCFREvaluator:
         """``phases``: 1 = regrets, policy, reach, beliefs; 2 = leaf values and backup; 3 = both.
         ``lean``: store only what is read again (include/p2hip.h).  ``alternate``: write reach_avg into
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
+        if (self._walk_open is not None and not phases & _PHASE_12) or (
+                lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum):
+            self._launch_walk(phases)
+            if phases & _PHASE_3 and not self.use_final_policy_values:
+                self._const_rows_short = True
+            return
+        self._walk_open = None
         alternate = alternate and bool(phases & _PHASE_12)
+        # the three walks write the ranges' own tensor, wherever the one-walk iterations before left them
+        leaf_prev = None
+        if phases & _PHASE_12 and self._leaf_home is not (self.beliefs_avg if self.cfr_avg else self.beliefs):
+            leaf_prev = self._swap_leaf_ranges()
         b = self._iter_bundle(alternate)
         mode = _PHASE_LEAN | _PHASE_CONST if lean else (_PHASE_CONST if self._const_rows_short else 0)
         if phases & _PHASE_3 and not self.use_final_policy_values:
             self._const_rows_short = lean
         if self._items is None:
-            self._launch_items(b.main, self.root_nodes, phases | mode)
+            self._launch_items(b.main, self.root_nodes, phases | mode, leaf_prev)
         else:
             tiers = b.tiers
             if phases & _PHASE_12:
-                self._launch_items(*b.regret, _PHASE_1 | mode)                      # regrets of every family, all items at once
+                self._launch_items(*b.regret, _PHASE_1 | mode, leaf_prev)                      # regrets of every family, all items at once
                 for args, count in tiers[:-1]:
                     self._launch_items(args, count, _PHASE_2 | mode)                # upper tiers, top-down
             args, count = tiers[-1]

@@ -42,13 +42,15 @@ def test_range_rows_and_the_rows_they_stand_for(seed):
         assert torch.equal(x, x[:, :, :1].expand_as(x)), name
 
 
+@pytest.mark.parametrize("one_walk", [False, True])
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("seed", range(8))
-def test_rows_kept_elsewhere_are_never_read(seed, split):
+def test_rows_kept_elsewhere_are_never_read(seed, split, one_walk):
     variant = VARIANTS[(seed + 5) % len(VARIANTS)]
     iters = 5 + seed % 2
     plain = build(seed, variant, split, lean=False, iters=iters)
     lean = build(seed, variant, split, lean=True, iters=iters)
+    lean._one_walk = lean._one_walk and one_walk
     tree = lean.tree
     want = expected_range_rows(tree)
     network = tree.leaf_mask & ~np.asarray(tree.state["done"]) & (lean.model is not None)
@@ -70,3 +72,60 @@ def test_rows_kept_elsewhere_are_never_read(seed, split):
     lean.cfr_iteration(iters)
     for name in STATE:
         assert torch.equal(getattr(plain, name), getattr(lean, name)), name
+
+
+@pytest.mark.parametrize("cfr_type,cfr_avg,street", [("discounted", False, 3), ("linear", True, 3), ("discounted", False, 2)])
+def test_one_walk_over_long_family_lists(cfr_type, cfr_avg, street):
+    """More than 64 families per work item (the window of the family list moves), one root and three, with and
+    without showdown rows; the one-walk kernel against plain iterations, and against the three walks."""
+    from poker2_amd.config import river_dcfr_config
+    from poker2_amd.evaluator import HipSparseCFREvaluator
+    from poker2_amd.fused_cfr_hip import CFRType
+    from poker2_amd.tree import RootStates
+    from tests.helpers import random_boards, random_ranges
+    for n in (1, 3):
+        rng = np.random.default_rng(77 + n)
+        boards = random_boards(rng, n)
+        if street == 2:
+            boards[:, 4] = -1
+        beliefs = torch.from_numpy(random_ranges(rng, boards))
+        roots = RootStates.at_round_start(street, np.full(n, 200), np.full((n, 2), 4000), boards, bb=100)
+        runs = []
+        for lean, walk in ((False, False), (True, False), (True, True)):
+            cfg = river_dcfr_config(n, iterations=6, depth=8)
+            cfg.search.cfr_type, cfg.search.cfr_avg = CFRType[cfr_type], cfr_avg
+            cfg.env.bet_bins = [0.5, 1.0]
+            ev = HipSparseCFREvaluator(None, torch.device("cuda"), cfg, max_raises=4, split_small_batches=False,
+                                       lean_search=lean)
+            ev.initialize_subgame(roots, np.arange(n), beliefs)
+            assert ((ev.tree.child_count > 0).sum() > 64 * n) and (not lean or ev._one_walk)
+            ev._one_walk = walk
+            ev.prepare_search(t_sample=torch.full((ev.total_nodes,), 2))
+            ev.run_search_iterations()
+            runs.append(ev)
+        for ev in runs[1:]:
+            for name in STATE:
+                assert torch.equal(getattr(runs[0], name), getattr(ev, name)), f"{n} roots: {name}"
+
+
+def test_entry_point_refuses_what_the_one_walk_kernel_cannot_run():
+    import ctypes
+    from poker2_amd import _lib
+    ev = build(1, VARIANTS[0], False, lean=True, iters=4)
+    lib, stream, p = _lib.load(), _lib.stream_ptr(), _lib.ptr
+    args = ev._iter_bundle(True).main
+    rows, a, b = p(ev._range_rows), p(ev.beliefs), p(torch.empty_like(ev.beliefs))
+    walk = 64 | 32 | 16
+
+    def refused(*call):
+        return lib.p2hip_cfr_iteration_shared(*call, stream) != 0
+    n = ev.root_nodes
+    assert refused(ctypes.byref(args), rows, a, a, n, 4, walk | 3)             # one range buffer
+    assert refused(ctypes.byref(args), rows, a, None, n, 4, walk | 3)
+    assert refused(ctypes.byref(args), None, a, b, n, 4, walk | 3)             # no range rows
+    assert refused(ctypes.byref(args), rows, a, b, n, 6, walk | 3)             # six children
+    assert refused(ctypes.byref(args), rows, a, b, n, 4, walk | 8)             # a part of the first walk
+    assert refused(ctypes.byref(args), rows, a, b, n, 4, 64 | 16 | 3)
+    assert refused(ctypes.byref(ev._iter_bundle(False).main), rows, a, b, n, 4, walk | 3)   # reach_avg in place
+    assert refused(ctypes.byref(args), rows, None, b, n, 4, 3)                 # a second range buffer without the walk
+    torch.cuda.synchronize()
