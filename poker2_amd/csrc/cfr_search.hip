@@ -14,10 +14,11 @@
 // What bounds it: with few roots nothing fills the chip, and an iteration lasts as long as its longest chain of
 // families, each a chain of dependent steps.  Twelve waves take a family (one pair of hands per lane, four waves for
 // the prefix of the sorted ranges while eight take the card scans), every row is requested before the first barrier,
-// and five launches replace six.  Microseconds per iteration, three walks -> one: three-raise river tree (105 nodes)
-// 1 root 299 -> 211, 64 roots 386 -> 270, 96 roots 428 -> 380; depth-2 tree 1 root 81 -> 57, 128 roots 110 -> 95; 64
-// mixed roots to depth 5 368 -> 240.  Tried: all children's rows requested at once instead of one child ahead
-// (211 -> 231; with a branch per child 218).
+// and a tier of work items costs one launch downwards and one upwards.  Microseconds per iteration, three walks ->
+// one over the same work items: three-raise river tree (105 nodes) 1 root 299 -> 211 (141 with the tree cut at every
+// level), 64 roots 386 -> 270, 96 roots 428 -> 380; depth-2 tree 1 root 81 -> 57, 128 roots 110 -> 95; 64 mixed roots to
+// depth 5 368 -> 240.  Tried: all children's rows requested at once instead of one child ahead (211 -> 231; with a
+// branch per child 218).
 //
 // Why only few roots: the showdown's tables leave room for two workgroups per CU at most, and the barriers of a
 // family (fourteen) drain what rows are in flight.  4096 roots: 11.3 ms per iteration against 9.7 of the three walks,

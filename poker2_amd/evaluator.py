@@ -80,6 +80,12 @@ FUSED_MAX_CHILDREN = 5
 # 686; one-raise tree (4 per root) 128 roots 156 -> 134, 192 roots 171 -> 180; depth-2 tree (4 per root) 128 roots 110 ->
 # 95, 192 roots 128 -> 120, 300 roots 199 -> 223.
 FUSED_MAX_ITEMS = 640
+# While every family can have a compute unit of its own, the trees are cut at every level down to the fourth: the
+# chain of families inside an item goes (9 in the longest subtree of a three-raise tree), for two launches more per
+# level.  us per iteration, cut at levels 1 and 2 -> 1 to 4: three-raise tree 1 root 210 -> 141, 8 roots 218 -> 150, 24
+# roots (312 families in the widest level) 223 -> 178; 24 mixed roots to depth 5 233 -> 154; trees of two levels the same.
+FUSED_DEEP_CUT = 4
+FUSED_DEEP_MAX_ITEMS = 384
 # One workgroup per root fills the chip (256 CUs x 3 resident workgroups) from 768 roots on.  Below
 # SPLIT_ROOTS_BELOW roots each root's tree is cut at level SPLIT_CUT_LEVEL into work items (the top of
 # the tree, and one subtree per node of that level) that get a workgroup each.  Measured on the
@@ -542,9 +548,16 @@ class HipSparseCFREvaluator:
                               else self._items)
         # the one-walk kernel: few work items, at most one showdown child among siblings
         showdown_parents = tree.parent_index[tree.showdown_mask]
+        offs = tree.depth_offsets
+        families = [int((tree.child_count[a:b] > 0).sum()) for a, b in zip(offs[:-1], offs[1:])]   # per level
+        cuttable = split and self._items is not None
         self._one_walk = (with_alt and T > N and self._max_children <= FUSED_MAX_CHILDREN
-                          and (max(self._items.tiers) if self._items is not None else N) <= FUSED_MAX_ITEMS
+                          and (max(families[:SPLIT_CUT_LEVEL + 1]) if cuttable else N) <= FUSED_MAX_ITEMS
+                          and (cuttable or N < SPLIT_ROOTS_BELOW)
                           and not bool((np.diff(showdown_parents) == 0).any()))
+        self._items_walk = self._items
+        if self._one_walk and cuttable and max(families[:FUSED_DEEP_CUT + 1]) <= FUSED_DEEP_MAX_ITEMS:
+            self._items_walk = self._split_items(tree, list(range(1, FUSED_DEEP_CUT)), FUSED_DEEP_CUT)
         self._leaf_alt = torch.empty_like(self._leaf_home) if self._one_walk else None
         self._root_items = None
         if self._items is None and T:
@@ -569,12 +582,13 @@ class HipSparseCFREvaluator:
                                                    showdown_offsets=showdown_offsets, item_root=self._t(order),
                                                    item_top=self._t(np.ones(N, np.uint8)))
 
-    def _split_items(self, tree: SparseTree, mid_level: int | None = None):
+    def _split_items(self, tree: SparseTree, mid_level: int | list[int] | None = None, cut_level: int | None = None):
         """``tree.split_work_items`` with the arrays on the device (None if the tree is too shallow to cut)."""
         # equal trees: items in row order, the last rounds' items by size; roots of unequal size: all by size
         sizes = np.bincount(tree.root_index, minlength=self.root_nodes)
         tail = self._sorted_tail if sizes.min() == sizes.max() else tree.total
-        it = split_work_items(tree, self.root_nodes, SPLIT_CUT_LEVEL, mid_level, sorted_tail=tail)
+        it = split_work_items(tree, self.root_nodes, SPLIT_CUT_LEVEL if cut_level is None else cut_level, mid_level,
+                              sorted_tail=tail)
         if it is None:
             return None
         for name in ("parents", "parent_offsets", "showdown", "showdown_offsets", "item_root", "item_top"):
@@ -948,7 +962,7 @@ class HipSparseCFREvaluator:
         else:
             b, prev = self._walk_open
         now = self.beliefs_avg if self.cfr_avg else self.beliefs
-        tiers = b.tiers if self._items is not None else [(b.main, self.root_nodes)]
+        tiers = b.walk
         down, up = phases & _PHASE_12, phases & _PHASE_3
         if down:
             for args, count in tiers[:-1]:
@@ -967,6 +981,20 @@ class HipSparseCFREvaluator:
             self._reach_avg_alt[:self.root_nodes] = 1.0
         return self._reach_avg_alt
 
+    def _tier_args(self, items, **kw) -> list:
+        """One argument block per tier of ``items``, with its item count: the same lists entered behind the items of
+        the tiers before."""
+        tiers, first = [], 0
+        for count in items.tiers:
+            tier = self._build_iter_args(items, **kw)
+            tier.root_parent_offsets += 8 * first
+            tier.root_showdown_offsets += 8 * first
+            tier.item_root += 8 * first
+            tier.item_top += first
+            tiers.append((tier, count))
+            first += count
+        return tiers
+
     def _iter_bundle(self, alternate: bool) -> SimpleNamespace:
         """Argument blocks of the iteration kernel for the tensor ``self_reach_avg`` names right now:
         updated in place (the old row saved in the scratch tensor), or — ``alternate`` — read as the
@@ -979,19 +1007,12 @@ class HipSparseCFREvaluator:
             kw = dict(reach_avg=self._other_reach_avg(), reach_avg_prev=self.self_reach_avg)
         else:
             kw = {}
-        b = SimpleNamespace(main=self._build_iter_args(**kw), regret=None, tiers=None)
+        b = SimpleNamespace(main=self._build_iter_args(**kw), regret=None, tiers=None, walk=None)
         if self._items is not None:
             b.regret = (self._build_iter_args(self._items_regret, **kw), sum(self._items_regret.tiers))
-            # one argument block per tier: the same lists entered behind the items of the tiers before
-            b.tiers, first = [], 0
-            for count in self._items.tiers:
-                tier = self._build_iter_args(**kw)
-                tier.root_parent_offsets += 8 * first
-                tier.root_showdown_offsets += 8 * first
-                tier.item_root += 8 * first
-                tier.item_top += first
-                b.tiers.append((tier, count))
-                first += count
+            b.tiers = self._tier_args(self._items, **kw)
+        if alternate and self._one_walk:
+            b.walk = [(b.main, self.root_nodes)] if self._items_walk is None else self._tier_args(self._items_walk, **kw)
         self._iter_bundles[key] = b
         return b
 
