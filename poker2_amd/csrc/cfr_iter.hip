@@ -596,8 +596,12 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       const int64_t row0 = range_row(f, 0), row1 = range_row(f, 1);
       ld(rn[0], A.reach, row0, ln);
       ld(rn[1], A.reach, row1, ln);
-      ld(ran[0], A.reach_avg, row0, ln);
-      ld(ran[1], A.reach_avg, row1, ln);
+      // the average reach of the player who does not act is only handed on, or normalised into beliefs_avg
+      const bool opp_avg = (opp_all | keep_ba) != 0;
+      if (opp_avg || actor == 0) ld(ran[0], A.reach_avg, row0, ln);
+      else IT_FOR(j) ran[0][j] = make_float2(0.f, 0.f);
+      if (opp_avg || actor == 1) ld(ran[1], A.reach_avg, row1, ln);
+      else IT_FOR(j) ran[1][j] = make_float2(0.f, 0.f);
       if (stash) ld(ra_old, A.scratch, p, ln);
       else ld(ra_old, A.reach_avg_prev, actor == 0 ? row0 : row1, ln);
 #pragma unroll

@@ -121,6 +121,12 @@ SPLIT_MID_LEVEL = 1
 # and only the last rounds' items by size; two raises: 1024 roots 2.15 -> 2.07 ms, 4096 roots 7.93 -> 7.76 ms;
 # the 21-node trees lose 3-7 % above 400 roots).
 SPLIT_NODES_PER_ROOT = 50
+# Roots of unequal size: a launch of whole roots lasts at least as long as its largest tree, whatever the others
+# are.  They are cut while that tree holds more than this many times the nodes that a resident workgroup gets on
+# average (us per search iteration, whole -> cut, with the ratio): roots of mixed streets with unequal stacks to the end
+# of the street, three raises, 420 roots (5.4) 1350 -> 590, 1024 (2.3) 1583 -> 1143, 1300 (1.7) 1706 -> 1474, 1536 (1.5)
+# 1768 -> 1688, 2048 (1.1) 2111 -> 2267; two raises 600 (2.3) 703 -> 557, 768 (1.7) 755 -> 718, 900 (1.5) 789 -> 849.
+SPLIT_LARGEST_SHARE = 1.65
 
 
 def _cfr_type_name(x) -> str:
@@ -539,8 +545,11 @@ class HipSparseCFREvaluator:
         self._has_model_leaves = bool(model_mask.any())
         self._iter_bundles = {}
         split = self.split_small_batches
+        size = np.bincount(tree.root_index, minlength=N)
         if split is None:
-            split = N < SPLIT_ROOTS_BELOW or T >= SPLIT_NODES_PER_ROOT * N
+            slots = self._sorted_tail // 3
+            split = (N < SPLIT_ROOTS_BELOW or T >= SPLIT_NODES_PER_ROOT * N
+                     or (size.min() != size.max() and size.max() * slots > SPLIT_LARGEST_SHARE * T))
         self._items = self._split_items(tree, SPLIT_MID_LEVEL) if split else None
         # The regret part has no order among families: it runs over the coarser of the two partitions
         # (whole tree tops), which makes fewer and longer workgroups of the same work.
@@ -565,7 +574,6 @@ class HipSparseCFREvaluator:
             # that the launch does not end on a long root that started last.  (Row order with only the last
             # rounds by size, which wins for the work items of equal trees, loses here: 16 384 mixed roots 23.2 ms
             # per iteration against 22.3 ms.)
-            size = np.bincount(tree.root_index, minlength=N)
             if size.min() != size.max():
                 order = launch_order(size, N)
 

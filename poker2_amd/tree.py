@@ -391,9 +391,9 @@ def split_work_items(tree: "SparseTree", n_roots: int, cut_level: int, mid_level
         return rows[order], np.concatenate([[0], np.cumsum(counts)])
 
     def reordered(rows, offsets, order):
-        pieces = [rows[offsets[g]:offsets[g + 1]] for g in order]
-        lengths = np.array([len(x) for x in pieces], dtype=np.int64)
-        return (np.concatenate(pieces) if pieces else rows), np.concatenate([[0], np.cumsum(lengths)])
+        lengths = np.diff(offsets)[order]
+        at = np.concatenate([[0], np.cumsum(lengths)])
+        return rows[np.repeat(np.asarray(offsets)[:-1][order] - at[:-1], lengths) + np.arange(len(rows))], at
     roots = np.arange(N)
     # tier 0: families whose parent lies above the first cut, showdown rows down to that cut, per root
     upper = np.nonzero(has_children[:offs[cuts[0]]])[0]
@@ -414,10 +414,12 @@ def split_work_items(tree: "SparseTree", n_roots: int, cut_level: int, mid_level
         tp, tpo = grouped(parent_rows, anchor[parent_rows], heads)
         sd_rows = np.arange(offs[lo + 1], offs[hi + 1] if hi < n_levels else T)
         sd_rows = sd_rows[tree.showdown_mask[sd_rows]]
-        sd_rows = sd_rows[np.isin(anchor[sd_rows], heads)]
+        headed = np.zeros(T, dtype=bool)
+        headed[heads] = True                         # (rows above the level have no anchor and are not in these spans)
+        sd_rows = sd_rows[headed[anchor[sd_rows]]]
         ts, tso = grouped(sd_rows, anchor[sd_rows], heads)
         below = np.arange(offs[lo], offs[hi + 1] if hi < n_levels else T)
-        below = below[np.isin(anchor[below], heads)]
+        below = below[headed[anchor[below]]]
         size = np.bincount(np.searchsorted(heads, anchor[below]), minlength=len(heads))
         order = launch_order(size, sorted_tail)
         lists_p.append(reordered(tp, tpo, order))
