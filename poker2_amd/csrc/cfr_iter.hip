@@ -290,7 +290,8 @@ struct FamWin {
 // KINDS: also collect what a lean iteration decides its stores by, per child k: bit 2k = the child has children,
 // bit 2k + 1 = its ranges feed a leaf evaluation, bit 16 + 2k = that evaluation reads both of the child's own
 // range rows (a leaf network), bit 17 + 2k = the child's values do not depend on the hand.
-template <int MAXC, bool KINDS>
+// SH: the launch shares rows (range_rows or const_rows given); without, none of that costs anything.
+template <int MAXC, bool KINDS, bool SH>
 __device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t pp0, int nfam, int base) {
   const int l = base + (int)(threadIdx.x & 63);
   F.base = base;
@@ -305,8 +306,8 @@ __device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t p
     const int cnt = (int)A.child_count[p];
     F.p = (int)p;
     F.first = (int)first;
-    F.rs = A.range_rows ? A.range_rows[p] : 2 * (int)p;
-    if (KINDS || A.const_rows) {
+    if (SH) F.rs = A.range_rows ? A.range_rows[p] : 2 * (int)p;
+    if (KINDS || SH) {
       uint32_t kinds = 0;
 #pragma unroll
       for (int k = 0; k < MAXC; ++k) {
@@ -314,7 +315,7 @@ __device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t p
           const uint32_t fl = A.node_flags[first + k];
           kinds |= ((fl >> 2) & 3u) << (2 * k);
           if ((fl & (NODE_LEAF_EVAL | NODE_SHOWDOWN)) == NODE_LEAF_EVAL) kinds |= 0x10000u << (2 * k);
-          if ((fl & NODE_CONST) && A.const_rows) kinds |= 0x20000u << (2 * k);
+          if (SH && (fl & NODE_CONST) && A.const_rows) kinds |= 0x20000u << (2 * k);
         }
       }
       F.kinds = (int)kinds;
@@ -323,6 +324,7 @@ __device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t p
   }
 }
 struct Fam { int64_t p, first; int cnt, actor, kinds, rs; };
+template <bool KINDS, bool SH>
 __device__ __forceinline__ Fam fam_get(const FamWin& F, int i) {
   const int s = i - F.base;
   Fam f;
@@ -331,8 +333,8 @@ __device__ __forceinline__ Fam fam_get(const FamWin& F, int i) {
   const int ca = __builtin_amdgcn_readlane(F.ca, s);
   f.cnt = ca & 0xFF;
   f.actor = (ca >> 8) & 0xFF;
-  f.kinds = __builtin_amdgcn_readlane(F.kinds, s);
-  f.rs = __builtin_amdgcn_readlane(F.rs, s);
+  f.kinds = KINDS || SH ? __builtin_amdgcn_readlane(F.kinds, s) : 0;
+  f.rs = SH ? __builtin_amdgcn_readlane(F.rs, s) : 2 * (int)f.p;
   return f;
 }
 // Row (of the [total*2] row space) that holds player q's reach / ranges of the family's parent.
@@ -351,6 +353,7 @@ struct SdWin {
   float pot0, pot1, scale;
   int base;
 };
+template <bool SH>
 __device__ __forceinline__ void sd_load(SdWin& S, const IterArgs& A, int64_t sd0, int nsd, int base) {
   const int l = base + (int)(threadIdx.x & 63);
   S.base = base;
@@ -360,7 +363,7 @@ __device__ __forceinline__ void sd_load(SdWin& S, const IterArgs& A, int64_t sd0
   if (l < nsd) {
     const int64_t c = A.root_showdown_nodes[sd0 + l];
     S.c = (int)c;
-    S.rs = A.range_rows ? A.range_rows[c] : 2 * (int)c;
+    S.rs = SH && A.range_rows ? A.range_rows[c] : 2 * (int)c;
     S.pot0 = A.potential[2 * c];
     S.pot1 = A.potential[2 * c + 1];
     S.scale = A.scale[c];
@@ -370,7 +373,7 @@ __device__ __forceinline__ float readlane_f(float v, int s) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s));
 }
 
-template <int MAXC, bool LEAN, bool ALT>
+template <int MAXC, bool LEAN, bool ALT, bool SH>
 __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iteration_kernel(IterArgs A) {
   constexpr int IT_CHUNK = ItChunk<MAXC>::value;
   // how many rows are requested together: parents staged for the card sums, children of a family in
@@ -385,8 +388,10 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 
   Lane ln;
   lane_init(ln);
+  auto row_of = [](const Fam& f, int q) { return SH ? range_row(f, q) : f.p * 2 + q; };
+  auto mask_of = [](const Fam& f, int k) { return SH ? const_mask(f, k) : -1; };
   FamWin F;
-  fam_load<MAXC, LEAN>(F, A, pp0, nfam, 0);
+  fam_load<MAXC, LEAN, SH>(F, A, pp0, nfam, 0);
   constexpr bool stash = !ALT;   // the pre-update reach_avg of a parent goes through `scratch`
 
   const float f_an = A.fscal[0], f_bn = A.fscal[1], f_ad = A.fscal[2], f_bd = A.fscal[3];
@@ -425,7 +430,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
     }
     for (int i0 = 0; i0 < nfam; i0 += IT_CHUNK) {
       const int nch = (nfam - i0) < IT_CHUNK ? (nfam - i0) : IT_CHUNK;
-      if (i0 < F.base || i0 + nch > F.base + 64) fam_load<MAXC, LEAN>(F, A, pp0, nfam, i0);
+      if (i0 < F.base || i0 + nch > F.base + 64) fam_load<MAXC, LEAN, SH>(F, A, pp0, nfam, i0);
       // opponent beliefs of every parent of the chunk: requested together, staged together,
       // card-summed in one pass
       PROF_BEGIN(t_c1);
@@ -437,15 +442,15 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 #pragma unroll
           for (int uu = 0; uu < SB; ++uu) {
             const int u = u0 + uu < nch ? u0 + uu : nch - 1;
-            const Fam f = fam_get(F, i0 + u);
-            ld(bo[uu], A.leaf_prev ? A.leaf_prev : leaf_beliefs, range_row(f, 1 - f.actor), ln);
-            if (stash) ld(ra[uu], A.reach_avg, range_row(f, f.actor), ln);  // the mix in sweep 2 needs the pre-update value
+            const Fam f = fam_get<LEAN, SH>(F, i0 + u);
+            ld(bo[uu], A.leaf_prev ? A.leaf_prev : leaf_beliefs, row_of(f, 1 - f.actor), ln);
+            if (stash) ld(ra[uu], A.reach_avg, row_of(f, f.actor), ln);  // the mix in sweep 2 needs the pre-update value
           }
 #pragma unroll
           for (int uu = 0; uu < SB; ++uu) {
             const int u = u0 + uu;
             if (u < IT_CHUNK && u < nch) {
-              const Fam f = fam_get(F, i0 + u);
+              const Fam f = fam_get<LEAN, SH>(F, i0 + u);
               to_lds(L.u.vecs[u], bo[uu], ln);
               if (stash) st(A.scratch, f.p, ra[uu], ln);
             }
@@ -456,7 +461,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       card_sums_multi(L.u.vecs[0], IT_VSTRIDE, nch, L.cs);
       PROF_END(4, t_c1);
       for (int u = 0; u < nch; ++u) {
-        const Fam f = fam_get(F, i0 + u);
+        const Fam f = fam_get<LEAN, SH>(F, i0 + u);
         const int cnt = f.cnt, actor = f.actor;
         const int64_t first = f.first;
         if (take_sample) {
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
               const int k = g0 + kk;
               if (k < MAXC && k < cnt) {
                 const int64_t c = first + k;
-                ld_masked(ach[kk], A.latest, c * 2 + actor, ln, const_mask(f, k));
+                ld_masked(ach[kk], A.latest, c * 2 + actor, ln, mask_of(f, k));
                 ld(cu[kk], A.cum, c, ln);
                 ld(ws[kk], A.wsum, c, ln);
               }
@@ -577,8 +582,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       to_lds(L.u.vecs[MAXC + 3], rbak[1], ln);
     }
     for (int i = 0; i < nfam; ++i) {
-      if (i < F.base || i >= F.base + 64) fam_load<MAXC, LEAN>(F, A, pp0, nfam, i);
-      const Fam f = fam_get(F, i);
+      if (i < F.base || i >= F.base + 64) fam_load<MAXC, LEAN, SH>(F, A, pp0, nfam, i);
+      const Fam f = fam_get<LEAN, SH>(F, i);
       const int64_t p = f.p, first = f.first;
       const int cnt = f.cnt, actor = f.actor;
       // per child: does it have children (its reach rows are read by its own family), do its ranges feed
@@ -588,12 +593,12 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // The player who does not act keeps the rows of the parent's range row: a lean iteration stores them
       // again only right under the root (whose own rows are given, not computed) and where a leaf network
       // reads a leaf's two rows side by side.
-      const int opp_all = !LEAN || !A.range_rows || (top && i == 0) ? 0x5555 : 0;
+      const int opp_all = !LEAN || !SH || !A.range_rows || (top && i == 0) ? 0x5555 : 0;
       const int opp_rows = opp_all | (f.kinds >> 16);
       const int keep_ba = bavg_all ? 0x5555 : (cfr_avg ? (has_children | leaf_eval) : 0);
       float2 rn[2][IT_PPT], ran[2][IT_PPT], ra_old[IT_PPT];
       float2 cur[MAXC][IT_PPT], pav[MAXC][IT_PPT];
-      const int64_t row0 = range_row(f, 0), row1 = range_row(f, 1);
+      const int64_t row0 = row_of(f, 0), row1 = row_of(f, 1);
       ld(rn[0], A.reach, row0, ln);
       ld(rn[1], A.reach, row1, ln);
       // the average reach of the player who does not act is only handed on, or normalised into beliefs_avg
@@ -797,7 +802,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       ShowdownRegs sdr;
       SdWin S;
       showdown_load_regs(A.tables + r * SD_TABLE_BYTES, sdr);
-      sd_load(S, A, sd0, nsd, 0);
+      sd_load<SH>(S, A, sd0, nsd, 0);
       // beliefs written in sweep 2 are gathered by other lanes here: the one hand-off through
       // global memory, hence a full barrier
       __syncthreads();
@@ -810,7 +815,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       };
       gather(__builtin_amdgcn_readlane(S.c, 0), __builtin_amdgcn_readlane(S.rs, 0), vk);
       for (int i = 0; i < nsd; ++i) {
-        if (i >= S.base + 64) sd_load(S, A, sd0, nsd, i);
+        if (i >= S.base + 64) sd_load<SH>(S, A, sd0, nsd, i);
         const int sl = i - S.base;
         const int64_t c = __builtin_amdgcn_readlane(S.c, sl);
         const float pot0 = readlane_f(S.pot0, sl), pot1 = readlane_f(S.pot1, sl), scl = readlane_f(S.scale, sl);
@@ -819,7 +824,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           int cn = __builtin_amdgcn_readlane(S.c, (sl + 1) & 63), rsn = __builtin_amdgcn_readlane(S.rs, (sl + 1) & 63);
           if (sl + 1 >= 64) {
             cn = (int)A.root_showdown_nodes[sd0 + i + 1];
-            rsn = A.range_rows ? A.range_rows[cn] : 2 * cn;
+            rsn = SH && A.range_rows ? A.range_rows[cn] : 2 * cn;
           }
           gather(cn, rsn, vnext);
         }
@@ -847,15 +852,15 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 
     // ---------------- sweep 3b: backup, bottom-up ----------------
     for (int i = nfam - 1; i >= 0; --i) {
-      if (i < F.base || i >= F.base + 64) fam_load<MAXC, LEAN>(F, A, pp0, nfam, i > 63 ? i - 63 : 0);
-      const Fam f = fam_get(F, i);
+      if (i < F.base || i >= F.base + 64) fam_load<MAXC, LEAN, SH>(F, A, pp0, nfam, i > 63 ? i - 63 : 0);
+      const Fam f = fam_get<LEAN, SH>(F, i);
       const int64_t p = f.p, first = f.first;
       const int cnt = f.cnt, actor = f.actor;
 
       // actor beliefs at the parent and the marginal of every action, card-summed in one pass
       PROF_BEGIN(t_c3);
       float2 ab[IT_PPT], dn[IT_PPT], polk[MAXC][IT_PPT];
-      ld(ab, A.beliefs, range_row(f, actor), ln);
+      ld(ab, A.beliefs, row_of(f, actor), ln);
 #pragma unroll
       for (int k = 0; k < MAXC; ++k)
         if (k < cnt) ld(polk[k], A.policy, first + k, ln);
@@ -883,7 +888,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           for (int kk = 0; kk < GRP3; ++kk) {
             const int k = g0 + kk < cnt ? g0 + kk : cnt - 1;
             const int64_t c = first + k;
-            const int m = const_mask(f, k);
+            const int m = mask_of(f, k);
             ld_masked(v[kk][0], A.latest, c * 2, ln, m);
             ld_masked(v[kk][1], A.latest, c * 2 + 1, ln, m);
             if (update_avg) {
@@ -922,7 +927,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 #pragma unroll
                 for (int pl = 0; pl < 2; ++pl) {
                   IT_FOR(j) av[kk][pl][j] = make_float2(av[kk][pl][j].x - shift, av[kk][pl][j].y - shift);
-                  if (LEAN && const_mask(f, k) == 0) {
+                  if (LEAN && mask_of(f, k) == 0) {
                     if (threadIdx.x == 0) p2_row2(A.values_avg, c * 2 + pl)[0] = av[kk][pl][0];
                   } else {
                     st(A.values_avg, c * 2 + pl, av[kk][pl], ln);
@@ -1115,8 +1120,12 @@ static int p2_launch_iteration(const p2::IterArgs& a, int64_t n_items, int max_c
   const bool lean = (phases & p2::PHASE_LEAN) != 0;
   const dim3 grid((unsigned)n_items), block(p2::IT_BLOCK);
   const bool alt = a.reach_avg_prev != nullptr;
-#define P2_ITER_LAUNCH(MAXC, LEAN, ALT) \
-  hipLaunchKernelGGL((p2::cfr_iteration_kernel<MAXC, LEAN, ALT>), grid, block, 0, (hipStream_t)stream, a)
+  const bool shared = a.range_rows || a.const_rows;
+#define P2_ITER_LAUNCH(MAXC, LEAN, ALT)                                                                                  \
+  do {                                                                                                                   \
+    if (shared) hipLaunchKernelGGL((p2::cfr_iteration_kernel<MAXC, LEAN, ALT, true>), grid, block, 0, (hipStream_t)stream, a); \
+    else hipLaunchKernelGGL((p2::cfr_iteration_kernel<MAXC, LEAN, ALT, false>), grid, block, 0, (hipStream_t)stream, a); \
+  } while (0)
 #define P2_ITER_MODES(MAXC)                                  \
   do {                                                       \
     if (lean && alt) P2_ITER_LAUNCH(MAXC, true, true);       \

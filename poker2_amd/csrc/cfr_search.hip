@@ -253,7 +253,7 @@ __device__ __forceinline__ void search_window(SearchLds& L, const IterArgs& A, i
   p2_sync_lds();
   if (threadIdx.x < 64) {
     FamWin F;
-    fam_load<SR_MAXC, true>(F, A, pp0, nfam, base);
+    fam_load<SR_MAXC, true, true>(F, A, pp0, nfam, base);
     SearchFam f = {F.p, F.first, F.ca, F.kinds, F.rs, 0.f, 0.f, 1.f};
     const uint32_t k = (uint32_t)F.kinds, sd = (k >> 1) & 0x5555u & ~(k >> 16);
     if (base + (int)threadIdx.x < nfam && sd) {

@@ -524,8 +524,8 @@ class HipSparseCFREvaluator:
             flags[model_mask & (tree.child_count == 0)] |= _NODE_LEAF_EVAL
         flags[tree.fold_mask & (tree.child_count == 0)] |= _NODE_CONST
         self._node_flags = self._t(flags)
-        # rows of values_avg that lean iterations have left in their first pair only
-        self._const_rows_short = False
+        # whether the last iteration was lean: rows that repeat others are then kept once (``_range_rows``, fold rows)
+        self._rows_short = False
         self._range_rows = torch.empty(T, dtype=torch.int32, device=dev)
         code = _lib.load().p2hip_range_rows(_lib.ptr(self.parent_index), _lib.ptr(self.env.to_act), N, T,
                                             _lib.ptr(self._range_rows), _lib.stream_ptr())
@@ -946,8 +946,8 @@ class HipSparseCFREvaluator:
         if n_items == 0:
             return
         p = _lib.ptr
-        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), p(self._range_rows), p(leaf_prev), p(leaf_next),
-                                                      n_items, self._max_children, phases, _lib.stream_ptr())
+        shared = self._range_rows if phases & _PHASE_CONST else None      # every row is whole otherwise
+        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), p(shared), p(leaf_prev), p(leaf_next), n_items, self._max_children, phases, _lib.stream_ptr())
         _lib.check(code, "p2hip_cfr_iteration_shared")
 
     def _swap_leaf_ranges(self) -> torch.Tensor:
@@ -1030,9 +1030,8 @@ class HipSparseCFREvaluator:
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
         if (self._walk_open is not None and not phases & _PHASE_12) or (
                 lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum):
+            self._rows_short = True
             self._launch_walk(phases)
-            if phases & _PHASE_3 and not self.use_final_policy_values:
-                self._const_rows_short = True
             return
         self._walk_open = None
         alternate = alternate and bool(phases & _PHASE_12)
@@ -1041,9 +1040,10 @@ class HipSparseCFREvaluator:
         if phases & _PHASE_12 and self._leaf_home is not (self.beliefs_avg if self.cfr_avg else self.beliefs):
             leaf_prev = self._swap_leaf_ranges()
         b = self._iter_bundle(alternate)
-        mode = _PHASE_LEAN | _PHASE_CONST if lean else (_PHASE_CONST if self._const_rows_short else 0)
-        if phases & _PHASE_3 and not self.use_final_policy_values:
-            self._const_rows_short = lean
+        self._rows_short = self._rows_short or lean
+        mode = (_PHASE_LEAN if lean else 0) | (_PHASE_CONST if self._rows_short else 0)
+        if phases & _PHASE_3:
+            self._rows_short = lean
         if self._items is None:
             self._launch_items(b.main, self.root_nodes, phases | mode, leaf_prev)
         else:
