@@ -1064,7 +1064,9 @@ class HipSparseCFREvaluator:
         """One CFR iteration (fused_sparse_cfr_evaluator.py:478-533).  The two keywords are for
         ``evaluate_cfr`` (one-kernel path only): ``lean`` leaves rows unwritten that nothing reads before
         the next iteration rewrites them — the state is complete again after one ordinary iteration —
-        and ``alternate_reach_avg`` rebinds ``self_reach_avg`` to the other of two buffers."""
+        and ``alternate_reach_avg`` rebinds ``self_reach_avg`` to the other of two buffers.  With both, on few
+        roots, ``beliefs`` (``beliefs_avg`` with CFR-AVG) is rebound as well until the next iteration without ``lean``,
+        which leaves its values in the tensor it named before."""
         if not self._skip_t_scalars_update:
             self.prepare_replay(t)
         if self.fused_iteration:
