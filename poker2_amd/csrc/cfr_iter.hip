@@ -276,6 +276,12 @@ __device__ __forceinline__ int opaque(int x) {
   return x;
 }
 
+// Workgroup barrier that no wave enters with a load of its own still under way (p2_sync_lds orders LDS traffic only).
+__device__ __forceinline__ void sync_loads() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 __device__ __forceinline__ float2 mul2(float2 a, float2 b) { return make_float2(a.x * b.x, a.y * b.y); }
 
 // A window of 64 consecutive entries of a work item's family list, one per lane: the parent row, the
@@ -928,8 +934,12 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                 for (int pl = 0; pl < 2; ++pl) {
                   IT_FOR(j) av[kk][pl][j] = make_float2(av[kk][pl][j].x - shift, av[kk][pl][j].y - shift);
                   if (LEAN && mask_of(f, k) == 0) {
+                    // (the other waves read the pair for nothing: whichever of its two values they see is dropped)
                     if (threadIdx.x == 0) p2_row2(A.values_avg, c * 2 + pl)[0] = av[kk][pl][0];
                   } else {
+                    // Every wave mixes the row's first pair, which the first wave is about to overwrite: all of
+                    // them have read it, for both players, before the first of its two rows is stored.
+                    if (SH && pl == 0 && mask_of(f, k) == 0) sync_loads();
                     st(A.values_avg, c * 2 + pl, av[kk][pl], ln);
                   }
                 }

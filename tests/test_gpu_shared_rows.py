@@ -129,3 +129,38 @@ def test_entry_point_refuses_what_the_one_walk_kernel_cannot_run():
     assert refused(ctypes.byref(ev._iter_bundle(False).main), rows, a, b, n, 4, walk | 3)   # reach_avg in place
     assert refused(ctypes.byref(args), rows, None, b, n, 4, 3)                 # a second range buffer without the walk
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("bins", [[0.5, 1.0], [0.25, 0.5, 1.0, 2.0]])
+@pytest.mark.parametrize("one_walk", [False, True])
+def test_rows_of_one_number_at_any_child(bins, one_walk):
+    """Rows flagged as one number per player need not be fold leaves, nor the first of their siblings: here every leaf
+    at the depth limit is one too.  The closing iteration mixes a row's first pair in every wave and stores it in one."""
+    from poker2_amd.config import river_dcfr_config
+    from poker2_amd.evaluator import HipSparseCFREvaluator
+    from poker2_amd.tree import RootStates
+    from tests.helpers import random_boards, random_ranges
+    n = 48
+    rng = np.random.default_rng(31)
+    boards = random_boards(rng, n)
+    beliefs = torch.from_numpy(random_ranges(rng, boards))
+    roots = RootStates.at_round_start(3, np.full(n, 200), np.full((n, 2), 4000), boards, bb=100)
+    runs = []
+    for lean in (False, True):
+        cfg = river_dcfr_config(n, iterations=5, depth=3)
+        cfg.env.bet_bins = bins
+        ev = HipSparseCFREvaluator(None, torch.device("cuda"), cfg, lean_search=lean)
+        ev.initialize_subgame(roots, np.arange(n), beliefs)
+        ev.prepare_search(t_sample=torch.full((ev.total_nodes,), 2))
+        gen = torch.Generator(device="cuda").manual_seed(5)
+        for table in (ev.latest_values, ev.values_avg):
+            table[ev.model_indices] = torch.rand(ev.model_indices.numel(), 2, 1, generator=gen, device="cuda") - 0.5
+        if lean:
+            ev._node_flags[ev.model_indices] |= 16
+            ev._one_walk = ev._one_walk and one_walk
+        ev.run_search_iterations()
+        runs.append(ev)
+    siblings = runs[1].tree.parent_index[runs[1].model_indices.cpu().numpy()]
+    assert (np.diff(siblings) == 0).any() and (runs[1]._max_children > 5) == (len(bins) > 2)
+    for name in STATE:
+        assert torch.equal(getattr(runs[0], name), getattr(runs[1], name)), name
