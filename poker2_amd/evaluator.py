@@ -524,8 +524,9 @@ class HipSparseCFREvaluator:
             flags[model_mask & (tree.child_count == 0)] |= _NODE_LEAF_EVAL
         flags[tree.fold_mask & (tree.child_count == 0)] |= _NODE_CONST
         self._node_flags = self._t(flags)
-        # whether the last iteration was lean: rows that repeat others are then kept once (``_range_rows``, fold rows)
-        self._rows_short = False
+        # whether the last iteration was lean: rows that repeat others are then kept once (``_range_rows``, fold rows);
+        # and whether the one-walk kernel ran it: ranges of showdown leaves are then not kept at all
+        self._rows_short = self._walked = False
         self._range_rows = torch.empty(T, dtype=torch.int32, device=dev)
         code = _lib.load().p2hip_range_rows(_lib.ptr(self.parent_index), _lib.ptr(self.env.to_act), N, T,
                                             _lib.ptr(self._range_rows), _lib.stream_ptr())
@@ -757,6 +758,7 @@ class HipSparseCFREvaluator:
 
     def update_policy(self, t: int) -> None:
         """fused_sparse_cfr_evaluator.py:201-236."""
+        self._complete_rows()
         bottom, top = self.depth_offsets[1], self.depth_offsets[-2]
         if self._fused_positive_regrets_buf is None or \
                 self._fused_positive_regrets_buf.shape != self.cumulative_regrets.shape:
@@ -776,6 +778,7 @@ class HipSparseCFREvaluator:
 
     def update_average_policy(self, t: int) -> None:
         """fused_sparse_cfr_evaluator.py:355-398."""
+        self._complete_rows()
         if self._avg_policy_copies(t):
             self.policy_probs_avg[:] = self.policy_probs
             return
@@ -795,6 +798,7 @@ class HipSparseCFREvaluator:
     def compute_instantaneous_regrets(self, values_achieved: torch.Tensor,
                                       values_expected: torch.Tensor | None = None) -> torch.Tensor:
         """fused_sparse_cfr_evaluator.py:312-349."""
+        self._complete_rows()
         if values_expected is None:
             values_expected = values_achieved
         bottom, top = self.depth_offsets[1], self.depth_offsets[-2]
@@ -810,6 +814,7 @@ class HipSparseCFREvaluator:
 
     def compute_expected_values(self, policy=None, beliefs=None, leaf_values=None, values=None) -> None:
         """fused_sparse_cfr_evaluator.py:242-306."""
+        self._complete_rows()
         policy = self.policy_probs if policy is None else policy
         beliefs = self.beliefs if beliefs is None else beliefs
         leaf_values = self.latest_values if leaf_values is None else leaf_values
@@ -833,6 +838,7 @@ class HipSparseCFREvaluator:
 
     def update_average_values(self, t: int) -> None:
         """fused_sparse_cfr_evaluator.py:404-414."""
+        self._complete_rows()
         F.fused_avg_values_zero_sum_(values_avg=self.values_avg, latest_values=self.latest_values,
                                      beliefs=self.beliefs_avg, old=self._t_scalars.mix_old,
                                      new=self._t_scalars.mix_new, inv_total=self._t_scalars.mix_inv_total,
@@ -908,6 +914,8 @@ class HipSparseCFREvaluator:
     def set_leaf_values(self, t: int, beliefs: torch.Tensor | None = None, *, showdown: bool = True) -> None:
         """fused_sparse_cfr_evaluator.py:447-472: model rows through PyTorch, showdown rows
         through the showdown kernel; fold rows are constants set at construction."""
+        if showdown:                # (an iteration asks for the model rows alone, which are complete)
+            self._complete_rows()
         if beliefs is None:
             beliefs = self.beliefs_avg if self.cfr_avg else self.beliefs
         self._set_model_values_impl(t, beliefs)
@@ -982,6 +990,42 @@ class HipSparseCFREvaluator:
                 self._launch_items(args, count, _PHASE_3 | mode, prev, now)
         self._walk_open = None if up else (b, prev)
 
+    def _complete_rows(self) -> None:
+        """Give the rows that lean iterations leave out, and that an iteration without ``_range_rows`` or any other
+        reader of the state looks at, their values, and the leaf ranges their own tensor: a captured graph, a
+        snapshot and the single operations go on from the state of a lean iteration as from an ordinary one.  (Rows
+        that every lean iteration leaves stale stay so: reach and ranges of other childless rows, ``beliefs_avg``
+        without CFR-AVG.)  Does nothing after an ordinary iteration, or in the middle of a one-walk one."""
+        moved = self._leaf_home is not (self.beliefs_avg if self.cfr_avg else self.beliefs)
+        if self._walk_open is not None or not (moved or self._rows_short):
+            return
+        tree, n = self.tree, self.root_nodes
+        inner = np.nonzero(tree.child_count > 0)[0]
+        inner = self._t(inner[inner >= n])
+        leaves = self._t(np.nonzero(tree.showdown_mask & (tree.child_count == 0))[0])
+        if moved:
+            kept = torch.cat([torch.arange(n, device=self.device), inner, self.model_indices])
+            before = self._swap_leaf_ranges()
+            self._leaf_home[kept] = before[kept]
+        tables = [(self.self_reach, inner), (self.self_reach_avg, inner), (self._leaf_home, torch.cat([inner, leaves]))]
+        if self.cfr_avg:
+            tables.append((self.beliefs, inner))
+        for table, rows in tables:                     # the player who did not act on the way into the row
+            source = self._range_rows[rows].long()
+            flat = table.view(-1, NUM_HANDS)
+            flat[2 * rows + source % 2] = flat[source]
+        if self._walked:                               # the other player's range at the showdown leaves
+            reach, policy = ((self.self_reach_avg, self.policy_probs_avg) if self.cfr_avg
+                             else (self.self_reach, self.policy_probs))
+            actor = self.prev_actor[leaves]
+            own = reach[self.parent_index[leaves], actor] * policy[leaves] * self.allowed_hands[leaves]
+            own *= self._leaf_home[self._root_index[leaves], actor]
+            total = own.sum(dim=-1, keepdim=True)
+            self._leaf_home[leaves, actor] = torch.where(total > 1e-5, own / total, self.allowed_hands_prob[leaves])
+        folds = self._t(np.nonzero(tree.fold_mask & (tree.child_count == 0))[0])
+        self.values_avg[folds] = self.values_avg[folds, :, :1].expand(-1, -1, NUM_HANDS)
+        self._rows_short = self._walked = False
+
     def _other_reach_avg(self) -> torch.Tensor:
         """The second reach_avg buffer of the alternating scheme (allocated on first use; root rows 1)."""
         if self._reach_avg_alt is None or self._reach_avg_alt.shape != self.self_reach_avg.shape:
@@ -1030,10 +1074,11 @@ class HipSparseCFREvaluator:
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
         if (self._walk_open is not None and not phases & _PHASE_12) or (
                 lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum):
-            self._rows_short = True
+            self._rows_short = self._walked = True
             self._launch_walk(phases)
             return
         self._walk_open = None
+        self._walked = self._walked and not phases & _PHASE_12
         alternate = alternate and bool(phases & _PHASE_12)
         # the three walks write the ranges' own tensor, wherever the one-walk iterations before left them
         leaf_prev = None
@@ -1100,6 +1145,7 @@ class HipSparseCFREvaluator:
     def initialize_policy_and_beliefs(self) -> None:
         """cfr_evaluator.py:830-886: initial policy from the model's logits (uniform over the
         legal actions without a model), beliefs pushed down level by level."""
+        self._complete_rows()
         self.policy_probs.zero_()
         if self.tree_depth == 0:
             self._normalize_beliefs()
@@ -1204,6 +1250,7 @@ class HipSparseCFREvaluator:
 
     def update_average_values_final(self) -> None:
         """cfr_evaluator.py:1276-1292."""
+        self._complete_rows()
         self.set_leaf_values(0, beliefs=self.beliefs_avg)
         self.compute_expected_values(self.policy_probs_avg, self.beliefs_avg, self.latest_values, self.values_avg)
         if self.enforce_zero_sum:
@@ -1340,6 +1387,7 @@ class HipSparseCFREvaluator:
         Roots standing at the start of a betting round after a deal also give a sample for the
         state BEFORE that deal: its value is the network's answer averaged over the cards that
         could have come (single card on turn and river, canonical flops on the flop)."""
+        self._complete_rows()
         N = self.root_nodes
         top = self.depth_offsets[-2] if len(self.depth_offsets) > 1 else N
         dev = self.device
@@ -1426,6 +1474,7 @@ class HipSparseCFREvaluator:
         if n == 0:
             return ExploitabilityStats(torch.empty(0, device=self.device, dtype=self.float_dtype),
                                        torch.empty(0, 2, device=self.device, dtype=self.float_dtype))
+        self._complete_rows()
         policy, beliefs = self.policy_probs_avg, self.beliefs_avg
         leaf_values = self.values_avg.clamp(-1.0, 1.0)
         base_values = torch.zeros_like(leaf_values)
@@ -1441,6 +1490,7 @@ class HipSparseCFREvaluator:
                                    local_best_response_values=torch.stack(br_agg, dim=-1))
 
     def state_dict(self) -> dict:
+        self._complete_rows()
         return {n: getattr(self, n) for n in STATE_NAMES}
 
 
@@ -1462,9 +1512,11 @@ class _EvaluatorStateSnapshot:
 
     @classmethod
     def from_evaluator(cls, evaluator) -> "_EvaluatorStateSnapshot":
+        evaluator._complete_rows()
         return cls({name: getattr(evaluator, name).detach().clone() for name in STATE_NAMES})
 
     def restore_to(self, evaluator) -> None:
+        evaluator._complete_rows()         # the names stand for the tensors that a captured graph works on
         for name, kept in self._saved.items():
             getattr(evaluator, name).copy_(kept)
 
@@ -1485,6 +1537,7 @@ class GraphedCFRIteration:
         self.evaluator = evaluator
         self._graph = None
         self._captured_t = None
+        self._reach_avg = None
 
     def capture(self, t_capture: int, num_warmup: int = 2) -> None:
         ev = self.evaluator
@@ -1507,12 +1560,18 @@ class GraphedCFRIteration:
             ev._skip_t_scalars_update = prev
         self._graph = graph
         self._captured_t = t_capture
+        self._reach_avg = ev.self_reach_avg       # the one of two buffers that the graph updates in place
 
     def replay(self, t: int | None = None) -> None:
         if self._graph is None:
             raise RuntimeError("capture() must be called before replay().")
+        ev = self.evaluator
+        # the graph holds an ordinary iteration, on these tensors: what lean iterations left elsewhere comes back first
+        ev._complete_rows()
+        if ev._reach_avg_alt is self._reach_avg and self._reach_avg is not None:
+            ev._reach_avg_alt, ev.self_reach_avg = ev.self_reach_avg, self._reach_avg.copy_(ev.self_reach_avg)
         if t is not None:
-            self.evaluator.prepare_replay(t)
+            ev.prepare_replay(t)
         self._graph.replay()
 
     @property
