@@ -1084,6 +1084,7 @@ class HipSparseCFREvaluator:
         leaf_prev = None
         if phases & _PHASE_12 and self._leaf_home is not (self.beliefs_avg if self.cfr_avg else self.beliefs):
             leaf_prev = self._swap_leaf_ranges()
+            self._leaf_home[:self.root_nodes] = leaf_prev[:self.root_nodes]    # a caller may have written new ones
         b = self._iter_bundle(alternate)
         self._rows_short = self._rows_short or lean
         mode = (_PHASE_LEAN if lean else 0) | (_PHASE_CONST if self._rows_short else 0)

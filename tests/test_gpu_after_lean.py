@@ -1,6 +1,6 @@
 """GPU: what may follow a lean iteration besides another iteration of the same search.  A lean iteration keeps rows
-that repeat others once and, on few roots, leaves the ranges in a second buffer; a captured graph, a snapshot and
-the launch-per-operation path all go on from there as from a plain iteration, bit for bit."""
+that repeat others once and, on few roots, leaves the ranges in a second buffer; a captured graph, a snapshot, the
+launch-per-operation path and ranges written by the caller all go on from there as from a plain iteration, bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -84,6 +84,20 @@ def test_snapshot(cfr_type, cfr_avg, one_walk):
         graph.replay(t)
         for ev in (lean, other, graphed):
             assert_same(plain, ev)
+
+
+@pytest.mark.parametrize("one_walk", [False, True])
+@pytest.mark.parametrize("cfr_type,cfr_avg", CFR)
+def test_root_ranges_written_between_iterations(cfr_type, cfr_avg, one_walk):
+    plain, lean = (build(cfr_type, cfr_avg, one_walk=one_walk) for _ in range(2))
+    for t in range(6):                                 # one lean iteration, and two, before a plain one
+        plain.cfr_iteration(t)
+        lean.cfr_iteration(t, lean=t in (0, 2, 3), alternate_reach_avg=True)
+        if t in (1, 4, 5):
+            assert_same(plain, lean)
+        for ev in (plain, lean):
+            for table in (ev.beliefs, ev.beliefs_avg):
+                table[:ev.root_nodes] = table[:ev.root_nodes].flip(1)
 
 
 @pytest.mark.parametrize("one_walk", [False, True])
