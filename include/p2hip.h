@@ -350,7 +350,8 @@ int p2hip_sample_snapshot(const float* policy_probs, float* policy_probs_sample,
  * own (row-major over all nodes of all roots); the rest is derived once per subgame:
  *   node_flags [total] bytes: bit0 = river showdown row, bit1 = terminal row, bit2 = the row has children,
  *             bit3 = childless row whose ranges feed a leaf evaluation (a showdown row, or a row the caller's
- *             leaf network is asked about); bits 2 and 3 are read by lean launches only
+ *             leaf network is asked about); bits 2 and 3 are read by lean launches only; bit4 = latest and values_avg of the row are one number per
+ *             player, whatever the hand (a fold leaf; read by p2hip_cfr_iteration_shared only)
  *   root_parent_offsets [roots+1], root_parents: rows that have children, per root, ascending
  *   root_showdown_offsets [roots+1], root_showdown_nodes: river showdown rows per root
  *   tables [roots, p2hip_showdown_table_bytes()] (NULL when no row is a showdown)
@@ -447,6 +448,9 @@ int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max
  *   tree), no enforce_zero_sum, and two range buffers: leaf_prev is read and leaf_next written in place of
  *   beliefs (beliefs_avg under cfr_avg) of host_args; both hold the roots' ranges (the walk copies them on).
  *   Bits 2 and 3 do not apply: tiers of work items take bit 0 downwards and bit 1 upwards.
+ * phases bit 8 (256): a lean iteration stores the rows that range_rows and bit 5 spare all the same, for a caller
+ *   whose own code (a leaf network with the node table in hand) reads the state between the parts of an iteration;
+ *   reads are as without it.  Not with bit 6.
  * The state after a closing iteration without bits 4 and 6 is bit-identical to p2hip_cfr_iteration's. */
 int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* range_rows, const float* leaf_prev,
                                float* leaf_next, int64_t n_items, int max_children, int phases, void* stream);

@@ -99,6 +99,7 @@ struct IterArgs {
   const float* leaf_prev;  // null, or [total,2,H]: the ranges the regret part reads (beliefs; beliefs_avg under cfr_avg)
                            // as the previous iteration left them, where that was another buffer
   int const_rows;        // rows flagged NODE_CONST: read the first pair only, store only that in a lean iteration
+  int whole_rows;        // a lean iteration stores the rows that range_rows and const_rows spare all the same
 };
 
 // Which sweeps a launch runs.  Sweep 1 of a family reads its parent's beliefs, values and reach_avg
@@ -127,6 +128,9 @@ constexpr int PHASE_LEAN = 16;
 // beliefs of a node with children, beliefs of a showdown leaf), the fold leaves' values 180 of the reads and 72 of
 // the writes (latest once per player and once more in the regret part, values_avg both ways).
 constexpr int PHASE_CONST = 32;
+// PHASE_WHOLE: for an iteration between whose parts somebody else reads the state (a leaf model that is handed the
+// node table): a lean iteration then stores every row that PHASE_LEAN alone keeps.
+constexpr int PHASE_WHOLE = 256;
 
 constexpr int IT_VSTRIDE = P2_H + 2;  // floats between vectors staged in LDS
 constexpr int IT_RED = 20;            // block-reduction slots: 2 + 2 * 8 children, rounded up
@@ -599,7 +603,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // The player who does not act keeps the rows of the parent's range row: a lean iteration stores them
       // again only right under the root (whose own rows are given, not computed) and where a leaf network
       // reads a leaf's two rows side by side.
-      const int opp_all = !LEAN || !SH || !A.range_rows || (top && i == 0) ? 0x5555 : 0;
+      const int opp_all = !LEAN || !SH || !A.range_rows || A.whole_rows || (top && i == 0) ? 0x5555 : 0;
       const int opp_rows = opp_all | (f.kinds >> 16);
       const int keep_ba = bavg_all ? 0x5555 : (cfr_avg ? (has_children | leaf_eval) : 0);
       float2 rn[2][IT_PPT], ran[2][IT_PPT], ra_old[IT_PPT];
@@ -933,7 +937,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 #pragma unroll
                 for (int pl = 0; pl < 2; ++pl) {
                   IT_FOR(j) av[kk][pl][j] = make_float2(av[kk][pl][j].x - shift, av[kk][pl][j].y - shift);
-                  if (LEAN && mask_of(f, k) == 0) {
+                  if (LEAN && !A.whole_rows && mask_of(f, k) == 0) {
                     // (the other waves read the pair for nothing: whichever of its two values they see is dropped)
                     if (threadIdx.x == 0) p2_row2(A.values_avg, c * 2 + pl)[0] = av[kk][pl][0];
                   } else {
@@ -1123,6 +1127,7 @@ static int p2_iteration_args(const P2HipIterArgs* host_args, int64_t n_items, in
   a.range_rows = nullptr;
   a.leaf_prev = nullptr;
   a.const_rows = (phases & p2::PHASE_CONST) != 0;
+  a.whole_rows = (phases & p2::PHASE_WHOLE) != 0;
   return 0;
 }
 

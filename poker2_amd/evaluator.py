@@ -19,7 +19,10 @@ Leaf model protocol (the value network itself stays ordinary PyTorch): ``model``
 ``MockModel``) or an object with
     enforce_zero_sum: bool
     leaf_values(beliefs[K,2,1326], node_rows[K], evaluator) -> [K,2,1326]
+    leaf_values_from_nodes(table[T,2,1326], node_rows[K], evaluator) -> [K,2,1326]        (optional, asked instead)
     policy_logits(beliefs[T,2,1326], node_rows[K], evaluator) -> [K,1326,A]   (optional)
+A model may say that its answer depends on the rows it is asked about alone, by an attribute of these functions
+(``leaf_models.reads_given_rows_only``): a search then keeps fewer rows between the parts of an iteration.
 
 Also here, either side of the iterations: warm start (``warm_start``), leaf sampling
 (``sample_leaves``), training-data assembly (``training_data``) and the local best response /
@@ -70,6 +73,9 @@ _PHASE_12, _PHASE_3, _PHASE_1, _PHASE_2 = 1, 2, 4, 8
 _PHASE_LEAN = 16
 # Fold leaves are one number per player: read through their first pair (lean iterations, and the one that follows).
 _PHASE_CONST = 32
+# ... and stored in full all the same, like every other row that repeats one, where code from outside looks at the state
+# between the parts of an iteration (``HipSparseCFREvaluator._rows_are_watched``).
+_PHASE_WHOLE = 256
 # One walk per family (csrc/cfr_search.hip): lean iterations between two buffers of reach_avg and of the ranges the
 # leaves are evaluated with.  The kernel has registers for five children per parent.
 _PHASE_FUSED, _PHASE_FUSED_CFR_AVG = 64, 128
@@ -568,7 +574,7 @@ class HipSparseCFREvaluator:
         self._items_walk = self._items
         if self._one_walk and cuttable and max(families[:FUSED_DEEP_CUT + 1]) <= FUSED_DEEP_MAX_ITEMS:
             self._items_walk = self._split_items(tree, list(range(1, FUSED_DEEP_CUT)), FUSED_DEEP_CUT)
-        self._leaf_alt = torch.empty_like(self._leaf_home) if self._one_walk else None
+        self._leaf_alt = torch.zeros_like(self._leaf_home) if self._one_walk else None
         self._root_items = None
         if self._items is None and T:
             # Roots of unequal size (mixed streets, stacks, pots): one work item per root, largest tree first, so
@@ -1068,12 +1074,29 @@ class HipSparseCFREvaluator:
         self._iter_bundles[key] = b
         return b
 
+    # what an iteration calls by name
+    _ITERATION_HOOKS = ("cfr_iteration", "prepare_replay", "set_leaf_values", "_set_model_values_impl", "_model_leaf_values",
+                        "_launch_iteration")
+
+    def _rows_are_watched(self) -> bool:
+        """Whether code from outside this package runs between the parts of an iteration, and so may look at any row
+        that a lean iteration has to store: an overridden method, or a leaf model other than those that say of their
+        ``leaf_values`` / ``leaf_values_from_nodes`` (by ``reads_given_rows_only``) that they read no other row."""
+        if any(getattr(getattr(self, name), "__func__", None) is not getattr(HipSparseCFREvaluator, name)
+               for name in self._ITERATION_HOOKS):
+            return True
+        if self.model is None or not self._has_model_leaves:
+            return False
+        asked = [getattr(self.model, name, None) for name in ("leaf_values_from_nodes", "leaf_values")]
+        return not all(getattr(f, "reads_given_rows_only", False) for f in asked if f is not None)
+
     def _launch_iteration(self, phases: int, lean: bool = False, alternate: bool = False) -> None:
         """``phases``: 1 = regrets, policy, reach, beliefs; 2 = leaf values and backup; 3 = both.
         ``lean``: store only what is read again (include/p2hip.h).  ``alternate``: write reach_avg into
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
+        watched = lean and self._rows_are_watched()
         if (self._walk_open is not None and not phases & _PHASE_12) or (
-                lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum):
+                lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum and not watched):
             self._rows_short = self._walked = True
             self._launch_walk(phases)
             return
@@ -1087,7 +1110,7 @@ class HipSparseCFREvaluator:
             self._leaf_home[:self.root_nodes] = leaf_prev[:self.root_nodes]    # a caller may have written new ones
         b = self._iter_bundle(alternate)
         self._rows_short = self._rows_short or lean
-        mode = (_PHASE_LEAN if lean else 0) | (_PHASE_CONST if self._rows_short else 0)
+        mode = (_PHASE_LEAN if lean else 0) | (_PHASE_CONST if self._rows_short else 0) | (_PHASE_WHOLE if watched else 0)
         if phases & _PHASE_3:
             self._rows_short = lean
         if self._items is None:
@@ -1109,10 +1132,11 @@ class HipSparseCFREvaluator:
     def cfr_iteration(self, t: int, *, lean: bool = False, alternate_reach_avg: bool = False) -> None:
         """One CFR iteration (fused_sparse_cfr_evaluator.py:478-533).  The two keywords are for
         ``evaluate_cfr`` (one-kernel path only): ``lean`` leaves rows unwritten that nothing reads before
-        the next iteration rewrites them — the state is complete again after one ordinary iteration —
-        and ``alternate_reach_avg`` rebinds ``self_reach_avg`` to the other of two buffers.  With both, on few
-        roots, ``beliefs`` (``beliefs_avg`` with CFR-AVG) is rebound as well until the next iteration without ``lean``,
-        which leaves its values in the tensor it named before."""
+        the next iteration rewrites them, or that repeat others — the state is complete again after one
+        ordinary iteration, replayed from a graph or not, and as complete as lean iterations leave it in
+        ``state_dict`` and every method that reads it — and ``alternate_reach_avg`` rebinds ``self_reach_avg`` to
+        the other of two buffers.  With both, on few roots, ``beliefs`` (``beliefs_avg`` with CFR-AVG) is rebound
+        as well until the next iteration without ``lean``, which leaves its values in the tensor it named before."""
         if not self._skip_t_scalars_update:
             self.prepare_replay(t)
         if self.fused_iteration:

@@ -24,6 +24,14 @@ from .card_utils import NUM_HANDS
 from .chance_node_helper import ChanceNodeHelper, MLPFeatures
 
 
+def reads_given_rows_only(leaf_values):
+    """Marks a ``leaf_values`` / ``leaf_values_from_nodes`` whose answer depends on the rows it is asked about alone: it
+    reads no other row of the node table and no state tensor of the evaluator, and does not rely on the table's
+    address.  Between the parts of a lean iteration the evaluator then keeps rows that repeat others once."""
+    leaf_values.reads_given_rows_only = True
+    return leaf_values
+
+
 class RangeBoardMLP(torch.nn.Module):
     def __init__(self, hidden: int = 1536, layers: int = 3, seed: int = 42) -> None:
         super().__init__()
@@ -117,6 +125,7 @@ class NetworkLeafModel:
             return torch.zeros(rows.numel(), NUM_HANDS, ev.num_actions, dtype=torch.float32, device=self.device)
         return logits.reshape(rows.numel(), NUM_HANDS, ev.num_actions)
 
+    @reads_given_rows_only
     @torch.no_grad()
     def leaf_values(self, beliefs: torch.Tensor, rows: torch.Tensor, ev) -> torch.Tensor:
         # Context and board of a leaf are public state: encoded once per subgame, only the ranges
@@ -131,6 +140,7 @@ class NetworkLeafModel:
                             beliefs=beliefs.reshape(beliefs.shape[0], -1))
         return self._run(feats, False).hand_values
 
+    @reads_given_rows_only
     @torch.no_grad()
     def leaf_values_from_nodes(self, table: torch.Tensor, rows: torch.Tensor, ev) -> torch.Tensor:
         """The same answer from the whole node table ``table`` [total, 2, 1326]: for a network that
@@ -197,6 +207,7 @@ class ChanceLeafModel:
                         to_act=plan.to_act, board=plan.board, beliefs=beliefs.reshape(k, -1))
         return f if sel is None else f[sel]
 
+    @reads_given_rows_only
     @torch.no_grad()
     def leaf_values(self, beliefs: torch.Tensor, rows: torch.Tensor, ev) -> torch.Tensor:
         key = (id(ev), ev.subgame_serial, rows.data_ptr(), rows.numel())
