@@ -1171,7 +1171,7 @@ int p2hip_range_rows(const int64_t* parent_index, const int64_t* to_act, int64_t
 int p2hip_cfr_iteration(const P2HipIterArgs* host_args, int64_t n_items, int max_children, int phases,
                         void* stream) {
   if (phases & ~31) return P2_EINVAL;
-  p2::IterArgs a;
+  p2::IterArgs a = {};
   const int bad = p2_iteration_args(host_args, n_items, max_children, phases, a);
   return bad || n_items == 0 ? bad : p2_launch_iteration(a, n_items, max_children, phases, stream);
 }

@@ -613,7 +613,7 @@ int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* ra
                                float* leaf_next, int64_t n_items, int max_children, int phases, void* stream) {
   constexpr int FUSED = 64, FUSED_CFR_AVG = 128;
   if (phases & ~511) return P2_EINVAL;
-  p2::IterArgs a;
+  p2::IterArgs a = {};
   const int bad = p2_iteration_args(host_args, n_items, max_children, phases, a);
   if (bad) return bad;
   if (!p2_aligned4(range_rows) || !p2_aligned8(leaf_prev) || !p2_aligned8(leaf_next)) return P2_EINVAL;
@@ -626,7 +626,8 @@ int p2hip_cfr_iteration_shared(const P2HipIterArgs* host_args, const int32_t* ra
   }
   // one walk per family: a lean iteration between two reach_avg and two range buffers
   if (max_children > p2::SR_MAXC || (phases & 15 & ~3) || !(phases & p2::PHASE_LEAN) || !(phases & p2::PHASE_CONST) ||
-      (phases & p2::PHASE_WHOLE) || !range_rows || !leaf_prev || !leaf_next || leaf_prev == leaf_next || !a.reach_avg_prev)
+      (phases & p2::PHASE_WHOLE) || !range_rows || !leaf_prev || !leaf_next || leaf_prev == leaf_next ||
+      (n_items > 0 && !a.reach_avg_prev))
     return P2_EINVAL;
   if (n_items == 0) return 0;
   const p2::SearchRows rows = {leaf_prev, leaf_next};

@@ -121,3 +121,24 @@ def test_bench_refuses_more_than_one_gpu_and_has_the_contract_flags():
                               timeout=300).stdout
     for flag in ("--gpus", "--steps", "--warmup"):
         assert flag in helptext
+
+
+def test_an_iteration_without_work_items_is_no_error():
+    """No item, nothing to do, whatever the kind of iteration; a broken combination of arguments is refused all the same."""
+    import ctypes
+    from poker2_amd import _lib
+    from poker2_amd.evaluator import _IterArgs
+    lib, args = _lib.load(), _IterArgs()
+    rows, a, b = 4096, 8192, 12288                     # never dereferenced: nothing is launched
+    lean, const, walk, cfr_avg = 16, 32, 64, 128
+    for phases in (1, 3, lean | 3, lean | const | 3, lean | const | walk | 3, lean | const | walk | cfr_avg | 1):
+        leaf_next = b if phases & walk else None
+        code = lib.p2hip_cfr_iteration_shared(ctypes.byref(args), rows, a, leaf_next, 0, 4, phases, None)
+        assert code == 0, phases
+        if not phases & ~31:
+            assert lib.p2hip_cfr_iteration(ctypes.byref(args), 0, 4, phases, None) == 0
+    for refused in ((rows, a, a, 4, walk | const | lean | 3), (None, a, b, 4, walk | const | lean | 3),
+                    (rows, a, b, 6, walk | const | lean | 3), (rows, a, b, 4, walk | lean | 3), (rows, a, b, 4, 3),
+                    (rows, a, None, 4, cfr_avg | 3), (rows, a, b, 4, 256 | walk | const | lean | 3), (rows, a, None, 4, 512 | 3)):
+        *ptrs, children, phases = refused
+        assert lib.p2hip_cfr_iteration_shared(ctypes.byref(args), *ptrs, 0, children, phases, None) != 0, refused
