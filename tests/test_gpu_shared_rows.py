@@ -51,6 +51,8 @@ def test_rows_kept_elsewhere_are_never_read(seed, split, one_walk):
     plain = build(seed, variant, split, lean=False, iters=iters)
     lean = build(seed, variant, split, lean=True, iters=iters)
     lean._one_walk = lean._one_walk and one_walk
+    if one_walk and not (lean._one_walk and seed % 3 and not lean.enforce_zero_sum and not lean._rows_are_watched()):
+        pytest.skip("this search is not one of the one-walk kernel: the other half of the parametrisation runs it")
     tree = lean.tree
     want = expected_range_rows(tree)
     network = tree.leaf_mask & ~np.asarray(tree.state["done"]) & (lean.model is not None)
@@ -62,6 +64,7 @@ def test_rows_kept_elsewhere_are_never_read(seed, split, one_walk):
         last = t + 1 == iters
         lean.cfr_iteration(t, lean=not last, alternate_reach_avg=bool(seed % 3))
         if not last:
+            assert lean._walked == one_walk
             for name in ("self_reach", "self_reach_avg", "beliefs") + (() if lean.enforce_zero_sum else ("beliefs_avg",)):
                 getattr(lean, name).view(-1, 1326)[dead] = float("nan")
             lean.values_avg[folds, :, 2:] = float("nan")
@@ -164,3 +167,83 @@ def test_rows_of_one_number_at_any_child(bins, one_walk):
     assert (np.diff(siblings) == 0).any() and (runs[1]._max_children > 5) == (len(bins) > 2)
     for name in STATE:
         assert torch.equal(getattr(runs[0], name), getattr(runs[1], name)), name
+
+
+@pytest.mark.parametrize("split", [False, None])       # one tier of whole roots; the rule's own cut at every level
+@pytest.mark.parametrize("network", [False, True])
+@pytest.mark.parametrize("cfr_type,cfr_avg", [("discounted", False), ("linear", True)])
+def test_one_walk_reads_only_what_it_keeps(cfr_type, cfr_avg, network, split):
+    """The one-walk kernel on river trees with showdown leaves, alternating throughout: rows it leaves out, and all but
+    the roots' rows of the two buffers that its next iteration writes, hold NaN between iterations."""
+    from poker2_amd.config import river_dcfr_config
+    from poker2_amd.evaluator import HipSparseCFREvaluator
+    from poker2_amd.fused_cfr_hip import CFRType
+    from poker2_amd.leaf_models import NetworkLeafModel, RangeBoardMLP
+    from poker2_amd.tree import RootStates
+    from tests.helpers import random_boards, random_ranges
+    n, iters = 5, 6
+    rng = np.random.default_rng(41)
+    boards = random_boards(rng, n)
+    beliefs = torch.from_numpy(random_ranges(rng, boards))
+    stacks = np.full((n, 2), 4000 if network else 800)
+    roots = RootStates.at_round_start(3, np.full(n, 200), stacks, boards, button=rng.integers(0, 2, n), bb=100)
+    runs = []
+    for lean in (False, True):
+        model = (NetworkLeafModel(RangeBoardMLP(hidden=64, layers=2).cuda(), torch.device("cuda")) if network else None)
+        cfg = river_dcfr_config(n, iterations=iters, depth=4 if network else 16)
+        cfg.search.cfr_type, cfg.search.cfr_avg = CFRType[cfr_type], cfr_avg
+        cfg.env.bet_bins = [0.5, 1.0]
+        ev = HipSparseCFREvaluator(model, torch.device("cuda"), cfg, max_raises=None if network else 3,
+                                    split_small_batches=split, lean_search=lean)
+        ev.initialize_subgame(roots, np.arange(n), beliefs)
+        ev.prepare_search(t_sample=torch.full((ev.total_nodes,), 2))
+        runs.append(ev)
+    plain, ev = runs
+    tree = ev.tree
+    assert ev._one_walk and ev._has_model_leaves == network and tree.showdown_mask.any()
+    assert len(ev._iter_bundle(True).walk) == (1 if split is False else 4 if network else 5)
+    want = expected_range_rows(tree)
+    at_network = tree.leaf_mask & ~np.asarray(tree.state["done"])
+    moved = (want // 2 != np.arange(tree.total)) & ~at_network
+    passive = torch.from_numpy(np.nonzero(moved)[0] * 2 + want[moved] % 2).cuda()
+    showdown = torch.from_numpy(np.nonzero(tree.showdown_mask)[0]).cuda()
+    folds = torch.from_numpy(np.nonzero(tree.fold_mask)[0]).cuda()
+    for t in range(iters):
+        plain.cfr_iteration(t)
+        ev.cfr_iteration(t, lean=t + 1 < iters, alternate_reach_avg=True)
+        if t + 1 < iters:
+            assert ev._walked
+            for name in ("self_reach", "self_reach_avg", "beliefs", "beliefs_avg"):
+                getattr(ev, name).view(-1, 1326)[passive] = float("nan")
+            for name in ("beliefs", "beliefs_avg"):
+                getattr(ev, name)[showdown] = float("nan")
+            ev._leaf_alt[n:] = float("nan")
+            ev._reach_avg_alt[n:] = float("nan")
+            ev.values_avg[folds, :, 2:] = float("nan")
+    for name in STATE:
+        assert torch.equal(getattr(plain, name), getattr(ev, name)), name
+
+
+@pytest.mark.parametrize("lean", [False, True])
+@pytest.mark.parametrize("alternate", [False, True])
+@pytest.mark.parametrize("seed", [1, 2, 6])
+def test_the_entry_point_without_shared_rows(seed, alternate, lean):
+    """p2hip_cfr_iteration called directly, in place and between two reach_avg buffers, against the evaluator."""
+    import ctypes
+    from poker2_amd import _lib
+    lib = _lib.load()
+    iters = 6
+    want, got = (build(seed, VARIANTS[0], False, lean=False, iters=iters) for _ in range(2))
+    other = got.self_reach_avg.clone()
+    for t in range(iters):
+        want.cfr_iteration(t)
+        got.prepare_replay(t)
+        args = (got._build_iter_args(reach_avg=other, reach_avg_prev=got.self_reach_avg) if alternate
+                else got._build_iter_args())
+        code = lib.p2hip_cfr_iteration(ctypes.byref(args), got.root_nodes, got._max_children,
+                                       3 | (16 if lean and t + 1 < iters else 0), _lib.stream_ptr())
+        assert code == 0
+        if alternate:
+            got.self_reach_avg, other = other, got.self_reach_avg
+    for name in STATE:
+        assert torch.equal(getattr(want, name), getattr(got, name)), name

@@ -14,6 +14,8 @@ BOARDS = [[0, 1, 2, 3, 4],            # straight flush on the board: most hands 
           [12, 25, 38, 51, 0],        # quads
           [0, 13, 1, 14, 27],         # full house
           [3, 17, 31, 45, 7], [51, 50, 38, 20, 2], [0, 2, 4, 6, 8],
+          [7, 7, 20, 33, 50], [12, 12, 11, 10, 9], [12, 12, 12, 12, 25], [51, 51, 51, 51, 51],   # a card repeated: the suit
+          [0, 0, 1, 1, 2],            # masks of the card ranker carry, up to two bits past the ace
           [5, 18, 30, -1, -1], [-1, -1, -1, -1, -1]]   # flop only, nothing dealt
 
 
