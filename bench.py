@@ -8,8 +8,8 @@ A step is ONE CFR iteration over a batch of B seeded synthetic river subgames (r
 leaf a fold or a showdown; discounted CFR alpha 1.5 / beta 0 / gamma 2).  All inputs are
 resident in HBM before the timed region.  The steps run the way a search runs them
 (``HipSparseCFREvaluator.run_search_iterations``: every iteration but a search's last leaves rows
-unwritten that nothing reads before the next iteration rewrites them, and reach_avg alternates
-between two buffers; the final state of a search is bit-identical either way); ``--mode plain`` times
+unwritten that nothing reads before the next iteration rewrites them or that repeat other rows, and
+reach_avg alternates between two buffers; the final state of a search is bit-identical either way); ``--mode plain`` times
 the iteration that writes all eleven tensors in full, as ``cfr_iteration(t)`` does.  Both are in the line.
 Prints ONE JSON line:
   value        subgame-iterations per second (iterations/s x subgames)
@@ -47,10 +47,10 @@ TREES = {"depth2": (2, None), "raise1": (16, 1), "raise2": (16, 2), "raise3": (1
 # program: counters need the profiler, so these are constants taken from the summary file named
 # below, one per workload that has a counter run; None elsewhere.  (read bytes, written bytes)
 TRAFFIC_SOURCE = "profiles/cfr_iteration_kernel_river.hbm_counters.txt"
-MEASURED_TRAFFIC_BYTES = {("raise3", 4096, "plain"): (34.30e9, 35.73e9), ("raise3", 4096, "search"): (32.76e9, 23.10e9),
-                          ("depth2", 4096, "plain"): (5.87e9, 6.69e9), ("depth2", 4096, "search"): (5.68e9, 3.82e9),
-                          ("raise1", 4096, "plain"): (6.60e9, 7.02e9), ("raise1", 4096, "search"): (6.35e9, 4.61e9),
-                          ("raise3", 1024, "plain"): (8.58e9, 8.94e9), ("raise3", 1024, "search"): (8.20e9, 5.78e9)}
+MEASURED_TRAFFIC_BYTES = {("raise3", 4096, "plain"): (34.24e9, 35.68e9), ("raise3", 4096, "search"): (28.56e9, 18.85e9),
+                          ("depth2", 4096, "plain"): (5.85e9, 6.68e9), ("depth2", 4096, "search"): (5.34e9, 3.60e9),
+                          ("raise1", 4096, "plain"): (6.58e9, 7.01e9), ("raise1", 4096, "search"): (5.58e9, 4.00e9),
+                          ("raise3", 1024, "plain"): (8.57e9, 8.92e9), ("raise3", 1024, "search"): (7.15e9, 4.71e9)}
 # how the iterations of a search run (all but its last) / how cfr_iteration(t) runs one
 MODES = {"search": dict(lean=True, alternate_reach_avg=True), "plain": {}}
 
@@ -377,7 +377,8 @@ def main() -> None:
     flat = flat_stream_rate()
     moved = traffic if traffic else algo_bytes
     mode_text = {"search": "iterations as a search runs all but its last (rows nothing reads before the next iteration "
-                           "rewrites them are not stored; reach_avg alternates between two buffers)",
+                           "rewrites them, and rows that repeat others, are not stored; reach_avg alternates between "
+                           "two buffers)",
                  "plain": "every iteration writes all eleven tensors in full, as cfr_iteration(t) does"}
     result = {
         "metric": "river CFR iters/sec x subgames",
