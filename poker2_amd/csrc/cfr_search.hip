@@ -13,16 +13,17 @@
 //
 // What bounds it: with few roots nothing fills the chip, and an iteration lasts as long as its longest chain of
 // families, each a chain of dependent steps.  Twelve waves take a family (one pair of hands per lane, four waves for
-// the prefix of the sorted ranges while eight take the card scans), every row is requested before the first barrier,
-// and a tier of work items costs one launch downwards and one upwards.  Microseconds per iteration, three walks ->
-// one over the same work items: three-raise river tree (105 nodes) 1 root 299 -> 211 (141 with the tree cut at every
-// level), 64 roots 386 -> 270, 96 roots 428 -> 380; depth-2 tree 1 root 81 -> 57, 128 roots 110 -> 95; 64 mixed roots to
-// depth 5 368 -> 240.  Tried: all children's rows requested at once instead of one child ahead (211 -> 231; with a
-// branch per child 218).
+// the prefix of the sorted ranges while eight take the card scans), rows are requested one child ahead, the parent's
+// before the first barrier, and a tier of work items costs one launch downwards and one upwards.  Microseconds per
+// iteration, three walks -> one over the same work items: three-raise river tree (105 nodes) 1 root 299 -> 211 (141
+// with the tree cut at every level), 64 roots 386 -> 270; depth-2 tree 1 root 81 -> 57, 128 roots 110 -> 95; 64 mixed
+// roots to depth 5 368 -> 240.  All these are roots with equal stacks, or happen to have no parent with two showdown
+// children: one such parent keeps the batch on the three walks.  Tried: all children's rows requested at once instead
+// of one child ahead (211 -> 231; with a branch per child 218).
 //
 // Why only few roots: the showdown's tables leave room for two workgroups per CU at most, and the barriers of a
 // family (fourteen) drain what rows are in flight.  4096 roots: 11.3 ms per iteration against 9.7 of the three walks,
-// although it moves 5-10 % fewer bytes (3.9 TB/s against 4.9); as four waves with six hands per lane and 256
+// although it moves 5 % fewer bytes (45.3 GB against 47.4); as four waves with six hands per lane and 256
 // registers the same walk took 11.7 ms there and 291 us on one root.
 #pragma once
 #include "cfr_iter.hip"

@@ -9,7 +9,7 @@ logic of ``CFREvaluator`` (src/p2/search/cfr_evaluator.py:285-303, :770-886, :12
 
 Two execution modes share the same state:
   * ``fused_iteration=True`` (default): ``cfr_iteration`` is ONE kernel launch
-    (``p2hip_cfr_iteration``), or two around the leaf network when the tree has
+    (``p2hip_cfr_iteration_shared``) per tier of work items, or two around the leaf network when the tree has
     non-terminal leaves and a leaf model is attached;
   * ``fused_iteration=False``: one launch per operation through the functions of
     ``fused_cfr_hip`` -- the call sequence of the reference's fused evaluator.
@@ -81,10 +81,12 @@ _PHASE_WHOLE = 256
 _PHASE_FUSED, _PHASE_FUSED_CFR_AVG = 64, 128
 FUSED_MAX_CHILDREN = 5
 # It shortens the chain of steps per family, at the cost of fewer workgroups per compute unit, so it is for launches
-# that leave the chip part empty: at most this many work items in a tier.  us per iteration, three walks -> one:
-# three-raise tree (9 items per root) 64 roots 386 -> 270, 96 roots 428 -> 380, 128 roots 465 -> 472, 192 roots 569 ->
-# 686; one-raise tree (4 per root) 128 roots 156 -> 134, 192 roots 171 -> 180; depth-2 tree (4 per root) 128 roots 110 ->
-# 95, 192 roots 128 -> 120, 300 roots 199 -> 223.
+# that leave the chip part empty: at most this many work items in a tier.  us per iteration, three walks -> one, below
+# the line: three-raise tree (9 items per root) 64 roots 386 -> 270; one-raise tree (4 per root) 128 roots 156 -> 134;
+# depth-2 tree (4 per root) 128 roots 110 -> 95.  Above it: one-raise tree 192 roots (768 items) 171 -> 180, three-raise
+# 128 roots (1152) 465 -> 472 and 192 roots 569 -> 686, depth-2 300 roots (1200) 199 -> 223 are losses; three-raise 96
+# roots (864) 428 -> 380, depth-2 192 roots (768) 128 -> 120 and 192 mixed roots to depth 5 (965) 512 -> 387 are gains
+# that one number for all trees does not take.
 FUSED_MAX_ITEMS = 640
 # While every family can have a compute unit of its own, the trees are cut at every level down to the fourth: the
 # chain of families inside an item goes (9 in the longest subtree of a three-raise tree), for two launches more per
@@ -562,7 +564,8 @@ class HipSparseCFREvaluator:
         # (whole tree tops), which makes fewer and longer workgroups of the same work.
         self._items_regret = (self._split_items(tree) if self._items is not None and len(self._items.tiers) > 2
                               else self._items)
-        # the one-walk kernel: few work items, at most one showdown child among siblings
+        # the one-walk kernel: few work items, at most one showdown child among siblings (of ANY parent of the batch:
+        # a call and an all-in that only calls, which unequal stacks bring, are two)
         showdown_parents = tree.parent_index[tree.showdown_mask]
         offs = tree.depth_offsets
         families = [int((tree.child_count[a:b] > 0).sum()) for a, b in zip(offs[:-1], offs[1:])]   # per level
@@ -961,7 +964,8 @@ class HipSparseCFREvaluator:
             return
         p = _lib.ptr
         shared = self._range_rows if phases & _PHASE_CONST else None      # every row is whole otherwise
-        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), p(shared), p(leaf_prev), p(leaf_next), n_items, self._max_children, phases, _lib.stream_ptr())
+        code = _lib.load().p2hip_cfr_iteration_shared(ctypes.byref(args), p(shared), p(leaf_prev), p(leaf_next), n_items,
+                                                      self._max_children, phases, _lib.stream_ptr())
         _lib.check(code, "p2hip_cfr_iteration_shared")
 
     def _swap_leaf_ranges(self) -> torch.Tensor:
