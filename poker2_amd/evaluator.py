@@ -270,7 +270,7 @@ class HipSparseCFREvaluator:
         self._iscal_host = (ctypes.c_int64 * 8)()
         self._iter_bundles: dict = {}
         self._reach_avg_alt = None
-        self._leaf_alt = None
+        self._leaf_alt = self._leaf_moved = None
         self._chance_helper = None
         self.subgame_serial = 0
 
@@ -394,7 +394,7 @@ class HipSparseCFREvaluator:
 
     _STATE_TENSORS = ("policy_probs", "policy_probs_avg", "policy_probs_sample", "cumulative_regrets",
                       "regret_weight_sums", "beliefs", "beliefs_avg", "self_reach", "self_reach_avg", "latest_values",
-                      "values_avg", "_scratch", "_reach_avg_alt", "_leaf_alt", "_leaf_home")
+                      "values_avg", "_scratch", "_reach_avg_alt", "_leaf_alt")
 
     def _drop_state(self) -> None:
         """Let go of the state tensors and their slabs (``reuse_state``), so that larger slabs can take
@@ -506,8 +506,8 @@ class HipSparseCFREvaluator:
         cc_dest = self.child_count[:tree.top].repeat_interleave(self.child_count[:tree.top])
         self.uniform_policy[N:] = (1.0 / cc_dest)[:, None].expand(-1, NUM_HANDS)
         self.beliefs, self.beliefs_avg = z2(), z2()
-        # the leaf ranges' own tensor: what every iteration but a one-walk one writes
-        self._leaf_home = self.beliefs_avg if self.cfr_avg else self.beliefs
+        # the name whose tensor and ``_leaf_alt`` a one-walk iteration has exchanged
+        self._leaf_moved: str | None = None
         self._walk_open = None         # the argument blocks of a one-walk iteration whose leaves a network evaluates
         self.root_pre_chance_beliefs = torch.zeros(N, 2, NUM_HANDS, dtype=self.float_dtype, device=dev)
         self.self_reach = z2()
@@ -577,7 +577,7 @@ class HipSparseCFREvaluator:
         self._items_walk = self._items
         if self._one_walk and cuttable and max(families[:FUSED_DEEP_CUT + 1]) <= FUSED_DEEP_MAX_ITEMS:
             self._items_walk = self._split_items(tree, list(range(1, FUSED_DEEP_CUT)), FUSED_DEEP_CUT)
-        self._leaf_alt = torch.zeros_like(self._leaf_home) if self._one_walk else None
+        self._leaf_alt = torch.zeros_like(self.beliefs) if self._one_walk else None
         self._root_items = None
         if self._items is None and T:
             # Roots of unequal size (mixed streets, stacks, pots): one work item per root, largest tree first, so
@@ -968,13 +968,23 @@ class HipSparseCFREvaluator:
                                                       self._max_children, phases, _lib.stream_ptr())
         _lib.check(code, "p2hip_cfr_iteration_shared")
 
+    @property
+    def _leaf_name(self) -> str:
+        """The evaluator's name for the leaf ranges."""
+        return "beliefs_avg" if self.cfr_avg else "beliefs"
+
+    @property
+    def _leaf_home(self) -> torch.Tensor:
+        """The leaf ranges' own tensor: what every iteration but a one-walk one writes."""
+        return self._leaf_alt if self._leaf_moved else getattr(self, self._leaf_name)
+
     def _swap_leaf_ranges(self) -> torch.Tensor:
-        """Let the evaluator's name for the leaf ranges (``beliefs``, ``beliefs_avg`` with CFR-AVG) stand for the
-        other of the two buffers; returns the one it stood for."""
-        name = "beliefs_avg" if self.cfr_avg else "beliefs"
+        """Let the name for the leaf ranges stand for the other of the two buffers; returns the one it stood for."""
+        name = self._leaf_moved or self._leaf_name
         before = getattr(self, name)
         setattr(self, name, self._leaf_alt)
         self._leaf_alt = before
+        self._leaf_moved = None if self._leaf_moved else name
         return before
 
     def _launch_walk(self, phases: int) -> None:
@@ -1006,9 +1016,10 @@ class HipSparseCFREvaluator:
         snapshot and the single operations go on from the state of a lean iteration as from an ordinary one.  (Rows
         that every lean iteration leaves stale stay so: reach and ranges of other childless rows, ``beliefs_avg``
         without CFR-AVG.)  Does nothing after an ordinary iteration, or in the middle of a one-walk one."""
-        moved = self._leaf_home is not (self.beliefs_avg if self.cfr_avg else self.beliefs)
+        moved = self._leaf_moved
         if self._walk_open is not None or not (moved or self._rows_short):
             return
+        by_average = (moved or self._leaf_name) == "beliefs_avg"
         tree, n = self.tree, self.root_nodes
         inner = np.nonzero(tree.child_count > 0)[0]
         inner = self._t(inner[inner >= n])
@@ -1016,22 +1027,23 @@ class HipSparseCFREvaluator:
         if moved:
             kept = torch.cat([torch.arange(n, device=self.device), inner, self.model_indices])
             before = self._swap_leaf_ranges()
-            self._leaf_home[kept] = before[kept]
-        tables = [(self.self_reach, inner), (self.self_reach_avg, inner), (self._leaf_home, torch.cat([inner, leaves]))]
-        if self.cfr_avg:
+            getattr(self, moved)[kept] = before[kept]
+        ranges = self.beliefs_avg if by_average else self.beliefs
+        tables = [(self.self_reach, inner), (self.self_reach_avg, inner), (ranges, torch.cat([inner, leaves]))]
+        if by_average:
             tables.append((self.beliefs, inner))
         for table, rows in tables:                     # the player who did not act on the way into the row
             source = self._range_rows[rows].long()
             flat = table.view(-1, NUM_HANDS)
             flat[2 * rows + source % 2] = flat[source]
         if self._walked:                               # the other player's range at the showdown leaves
-            reach, policy = ((self.self_reach_avg, self.policy_probs_avg) if self.cfr_avg
+            reach, policy = ((self.self_reach_avg, self.policy_probs_avg) if by_average
                              else (self.self_reach, self.policy_probs))
             actor = self.prev_actor[leaves]
             own = reach[self.parent_index[leaves], actor] * policy[leaves] * self.allowed_hands[leaves]
-            own *= self._leaf_home[self._root_index[leaves], actor]
+            own *= ranges[self._root_index[leaves], actor]
             total = own.sum(dim=-1, keepdim=True)
-            self._leaf_home[leaves, actor] = torch.where(total > 1e-5, own / total, self.allowed_hands_prob[leaves])
+            ranges[leaves, actor] = torch.where(total > 1e-5, own / total, self.allowed_hands_prob[leaves])
         folds = self._t(np.nonzero(tree.fold_mask & (tree.child_count == 0))[0])
         self.values_avg[folds] = self.values_avg[folds, :, :1].expand(-1, -1, NUM_HANDS)
         self._rows_short = self._walked = False
@@ -1098,6 +1110,8 @@ class HipSparseCFREvaluator:
         """``phases``: 1 = regrets, policy, reach, beliefs; 2 = leaf values and backup; 3 = both.
         ``lean``: store only what is read again (include/p2hip.h).  ``alternate``: write reach_avg into
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
+        if self._leaf_moved not in (None, self._leaf_name):        # CFR-AVG was switched on or off in between
+            self._complete_rows()
         watched = lean and self._rows_are_watched()
         if (self._walk_open is not None and not phases & _PHASE_12) or (
                 lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum and not watched):
@@ -1109,7 +1123,7 @@ class HipSparseCFREvaluator:
         alternate = alternate and bool(phases & _PHASE_12)
         # the three walks write the ranges' own tensor, wherever the one-walk iterations before left them
         leaf_prev = None
-        if phases & _PHASE_12 and self._leaf_home is not (self.beliefs_avg if self.cfr_avg else self.beliefs):
+        if phases & _PHASE_12 and self._leaf_moved:
             leaf_prev = self._swap_leaf_ranges()
             self._leaf_home[:self.root_nodes] = leaf_prev[:self.root_nodes]    # a caller may have written new ones
         b = self._iter_bundle(alternate)

@@ -111,3 +111,36 @@ def test_iteration_by_single_operations(cfr_type, cfr_avg, one_walk):
         ev.fused_iteration = False
         ev.cfr_iteration(4)
     assert_same(plain, lean)
+
+
+@pytest.mark.parametrize("one_walk", [False, True])
+@pytest.mark.parametrize("cfr_type,cfr_avg", CFR)
+def test_tensors_put_in_place_of_the_ranges(cfr_type, cfr_avg, one_walk):
+    """A caller may bind its own tensors to ``beliefs`` and ``beliefs_avg`` before the first iteration, and they stay bound."""
+    kept, bound = (build(cfr_type, cfr_avg, one_walk=one_walk) for _ in range(2))
+    for ev in (kept, bound):
+        for table in (ev.beliefs, ev.beliefs_avg):
+            table[:] = table.flip(1)
+    mine = {name: getattr(bound, name).clone() for name in ("beliefs", "beliefs_avg")}
+    for name, table in mine.items():
+        getattr(bound, name).fill_(float("nan"))
+        setattr(bound, name, table)
+    for t in range(6):
+        for ev in (kept, bound):
+            ev.cfr_iteration(t, lean=t in (1, 3, 4), alternate_reach_avg=True)
+        if t in (0, 2, 5):
+            assert_same(kept, bound)
+            assert all(getattr(bound, name) is table for name, table in mine.items())
+    assert torch.equal(kept._compute_exploitability().local_exploitability, bound._compute_exploitability().local_exploitability)
+
+
+@pytest.mark.parametrize("one_walk", [False, True])
+def test_cfr_avg_switched_off_between_iterations(one_walk):
+    plain, lean = (build("linear", True, one_walk=one_walk) for _ in range(2))
+    for t in range(4):
+        for ev in (plain, lean):
+            ev.cfr_avg = t < 1
+        plain.cfr_iteration(t)
+        lean.cfr_iteration(t, lean=t in (0, 2), alternate_reach_avg=True)
+        if t in (1, 3):
+            assert_same(plain, lean)
