@@ -271,6 +271,7 @@ class HipSparseCFREvaluator:
         self._iter_bundles: dict = {}
         self._reach_avg_alt = None
         self._leaf_alt = self._leaf_moved = None
+        self._replay_completes = False     # the graph being recorded is GraphedCFRIteration's, which sees to the rows itself
         self._chance_helper = None
         self.subgame_serial = 0
 
@@ -1110,16 +1111,21 @@ class HipSparseCFREvaluator:
         """``phases``: 1 = regrets, policy, reach, beliefs; 2 = leaf values and backup; 3 = both.
         ``lean``: store only what is read again (include/p2hip.h).  ``alternate``: write reach_avg into
         the other of two buffers; ``self_reach_avg`` names the new one when this returns."""
+        # Recorded into a graph of the caller's own: its replays run between iterations that know nothing of them.  So
+        # it reads rows where they are kept in any state, stores what a lean iteration must, and changes no note of
+        # the state, since nothing runs now; ranges that lie in the second buffer stay there for good.
+        recorded = torch.cuda.is_current_stream_capturing() and not self._replay_completes
+        if recorded and self._leaf_moved:
+            self._leaf_moved, self._iter_bundles = None, {}
         if self._leaf_moved not in (None, self._leaf_name):        # CFR-AVG was switched on or off in between
             self._complete_rows()
-        watched = lean and self._rows_are_watched()
+        watched = lean and (recorded or self._rows_are_watched())
         if (self._walk_open is not None and not phases & _PHASE_12) or (
                 lean and alternate and self._one_walk and phases & _PHASE_12 and not self.enforce_zero_sum and not watched):
             self._rows_short = self._walked = True
             self._launch_walk(phases)
             return
         self._walk_open = None
-        self._walked = self._walked and not phases & _PHASE_12
         alternate = alternate and bool(phases & _PHASE_12)
         # the three walks write the ranges' own tensor, wherever the one-walk iterations before left them
         leaf_prev = None
@@ -1127,10 +1133,11 @@ class HipSparseCFREvaluator:
             leaf_prev = self._swap_leaf_ranges()
             self._leaf_home[:self.root_nodes] = leaf_prev[:self.root_nodes]    # a caller may have written new ones
         b = self._iter_bundle(alternate)
-        self._rows_short = self._rows_short or lean
-        mode = (_PHASE_LEAN if lean else 0) | (_PHASE_CONST if self._rows_short else 0) | (_PHASE_WHOLE if watched else 0)
-        if phases & _PHASE_3:
-            self._rows_short = lean
+        mode = (_PHASE_LEAN if lean else 0) | (_PHASE_CONST if lean or self._rows_short or recorded else 0) | (
+            _PHASE_WHOLE if watched else 0)
+        if not recorded:
+            self._walked = self._walked and not phases & _PHASE_12
+            self._rows_short = lean or (self._rows_short and not phases & _PHASE_3)
         if self._items is None:
             self._launch_items(b.main, self.root_nodes, phases | mode, leaf_prev)
         else:
@@ -1589,6 +1596,7 @@ class GraphedCFRIteration:
         ev.prepare_replay(t_capture)
         prev = ev._skip_t_scalars_update
         ev._skip_t_scalars_update = True
+        ev._replay_completes = True
         try:
             s = torch.cuda.Stream()
             s.wait_stream(torch.cuda.current_stream())
@@ -1601,6 +1609,7 @@ class GraphedCFRIteration:
                 ev.cfr_iteration(t_capture)
         finally:
             ev._skip_t_scalars_update = prev
+            ev._replay_completes = False
         self._graph = graph
         self._captured_t = t_capture
         self._reach_avg = ev.self_reach_avg       # the one of two buffers that the graph updates in place

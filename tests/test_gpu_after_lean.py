@@ -144,3 +144,71 @@ def test_cfr_avg_switched_off_between_iterations(one_walk):
         lean.cfr_iteration(t, lean=t in (0, 2), alternate_reach_avg=True)
         if t in (1, 3):
             assert_same(plain, lean)
+
+
+def captured(ev, **kw):
+    """A graph of one iteration, recorded by the caller's own means; replayed for any t behind ``prepare_replay``."""
+    ev.prepare_replay(2)
+    ev._skip_t_scalars_update = True
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ev.cfr_iteration(2, **kw)
+    ev._skip_t_scalars_update = False
+
+    def replay(t):
+        ev.prepare_replay(t)
+        graph.replay()
+    return replay
+
+
+@pytest.mark.parametrize("lean", [False, True])        # what is recorded
+@pytest.mark.parametrize("alternate", [False, True])   # the two eager lean iterations before a replay
+@pytest.mark.parametrize("one_walk", [False, True])
+@pytest.mark.parametrize("cfr_type,cfr_avg", CFR)
+def test_graph_recorded_by_the_caller(cfr_type, cfr_avg, one_walk, alternate, lean):
+    """Replays between eager iterations, which cannot know that a replay ran; recording itself runs nothing."""
+    plain, ev = (build(cfr_type, cfr_avg, one_walk=one_walk) for _ in range(2))
+    kw = dict(lean=True, alternate_reach_avg=alternate)
+    for t in (2, 3):
+        plain.cfr_iteration(t)
+    ev.cfr_iteration(2)
+    ev.cfr_iteration(3, lean=alternate)
+    replay = captured(ev, lean=lean)                   # recorded behind a plain iteration and behind a lean one
+    t = 4
+    for eager in (alternate, 1, 2, 2, 1):              # a plain iteration, or a pair of lean ones, between replays
+        for _ in range(eager % 2):
+            plain.cfr_iteration(t)
+            ev.cfr_iteration(t)
+            assert_same(plain, ev)
+            t += 1
+        for _ in range(eager // 2 * 2):
+            plain.cfr_iteration(t)
+            ev.cfr_iteration(t, **kw)
+            t += 1
+        for _ in range(2):
+            plain.cfr_iteration(t)
+            replay(t)
+            if not lean:
+                assert_same(plain, ev)
+            t += 1
+    plain.cfr_iteration(t)
+    ev.cfr_iteration(t)
+    assert_same(plain, ev)
+
+
+@pytest.mark.parametrize("cfr_type,cfr_avg", CFR)
+def test_graph_recorded_while_the_ranges_lie_in_the_second_buffer(cfr_type, cfr_avg):
+    plain, ev = (build(cfr_type, cfr_avg, one_walk=True) for _ in range(2))
+    for t in (2, 3):
+        plain.cfr_iteration(t)
+        ev.cfr_iteration(t, lean=t == 3, alternate_reach_avg=True)
+    replay = captured(ev)
+    for t in range(4, 8):
+        plain.cfr_iteration(t)
+        replay(t)
+        assert_same(plain, ev)
+    for t in range(8, 11):
+        plain.cfr_iteration(t)
+        ev.cfr_iteration(t, lean=t < 10, alternate_reach_avg=t < 10)
+    assert_same(plain, ev)
