@@ -106,6 +106,23 @@ int p2hip_chance_expand_input(const float* pre_beliefs, const int64_t* root_indi
                               const int64_t* sample_offsets, int64_t source_rows, int64_t total_samples,
                               void* input_rows, int dtype, int64_t* board_samples, int64_t* root_lookup, void* stream);
 
+/* A single-card chance node and the value network behind it in one call, in float32: expected [n,2,H] =
+ * the mean over a state's samples (as p2hip_chance_expand makes them) of a network of `layers` linear
+ * layers with ReLU between them whose input is a row of p2hip_chance_expand_input.  host_weights[l]
+ * (device, [host_widths[l], columns] row-major, columns = 2704 for l = 0 and host_widths[l-1] after
+ * it), host_biases[l] (device, or NULL for none), all 16-byte aligned; the last width is 2 H, the
+ * others multiples of 32; 3 to P2HIP_NETWORK_MAX_LAYERS layers, at most P2HIP_NETWORK_MAX_SAMPLES samples.
+ * `workspace`: 256-byte aligned, of p2hip_chance_network_workspace(...) bytes (-1: not a network this
+ * call takes); its contents do not matter and mean nothing afterwards.  Everything that depends on the
+ * weights is derived anew in every call.  Replaces search/chance_node_helper.py:394-477 for such networks. */
+#define P2HIP_NETWORK_MAX_LAYERS 16
+#define P2HIP_NETWORK_MAX_SAMPLES ((1 << 23) - 1)
+int64_t p2hip_chance_network_workspace(int64_t n, int64_t total_samples, const int32_t* host_widths, int layers);
+int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, const int64_t* board, int64_t n,
+                         const int64_t* sample_offsets, int64_t source_rows, int64_t total_samples,
+                         const float* const* host_weights, const float* const* host_biases, const int32_t* host_widths,
+                         int layers, void* workspace, int64_t workspace_bytes, float* expected, void* stream);
+
 /* expected[i] = mean of hand_values [S,2,H] over samples sample_offsets[i] .. sample_offsets[i+1]
  * (index_add_ + divide of search/chance_node_helper.py:467-477). */
 int p2hip_chance_mean(const float* hand_values, const int64_t* sample_offsets, int64_t n, float* expected,

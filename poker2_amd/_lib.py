@@ -43,6 +43,8 @@ _SIGNATURES: dict[str, list] = {
     "p2hip_flop_expand": [_P, _P, _L, _P, _L, _P, _P],
     "p2hip_perm_mean": [_P, _L, _L, _P, _I, _P, _I, _P, _P, _I, _P],
     "p2hip_chance_mean": [_P, _P, _L, _P, _P],
+    "p2hip_chance_network_workspace": [_L, _L, _P, _I],
+    "p2hip_chance_network": [_P, _P, _P, _L, _P, _L, _L, _P, _P, _P, _I, _P, _L, _P, _P],
     "p2hip_orbit_mean": [_P, _L, _L, _P, _I, _P, _P, _I, _P],
     "p2hip_orbit_mean_static": [_P, _L, _L, _P, _I, _P, _I, _P],
     "p2hip_encode_context": [_P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _L, _P, _P, _P],
@@ -80,7 +82,7 @@ _SIGNATURES: dict[str, list] = {
     "p2hip_device_reserve": [_L, _P],
     "p2hip_device_release": [_P],
 }
-_RESTYPE = {"p2hip_error_string": ctypes.c_char_p, "p2hip_showdown_table_bytes": _L,
+_RESTYPE = {"p2hip_error_string": ctypes.c_char_p, "p2hip_showdown_table_bytes": _L, "p2hip_chance_network_workspace": _L,
             "p2hip_tree_node_columns": _L}
 
 

@@ -5,13 +5,15 @@ Mirror of ``ChanceNodeHelper.single_card_chance_values``
 to the network (src/p2/models/mlp/mlp_features.py:13-62): same names, arguments, sample
 order (state-major, next card ascending) and return value.  The masking / renormalising
 expansion and the per-state mean run as HIP kernels (``p2hip_chance_expand``,
-``p2hip_chance_mean``); the network itself stays an ordinary PyTorch module.
+``p2hip_chance_mean``); the network itself stays an ordinary PyTorch module, but one that is known to be plain float32
+layers is computed from its weights, node and network in one call (``p2hip_chance_network``).
 ``flop_chance_values`` (three-card chance nodes, :219-357) enumerates or samples the 1755
 suit-canonical flops (:76-216), expands through ``p2hip_flop_expand`` and averages each flop's
 answers over its suit orbit with ``p2hip_perm_mean``.
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Any
 
@@ -77,6 +79,23 @@ INPUT_ROW_WIDTH = 2 * NUM_HANDS + 52       # [ranges of both players | one-hot o
 _INPUT_DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 
+def _sample_offsets(board: torch.Tensor, roots: torch.Tensor, cards_on_board: int | None) -> tuple[torch.Tensor, int]:
+    """Where the samples of each selected state begin, [B + 1], and how many there are."""
+    b, dev = roots.numel(), roots.device
+    if cards_on_board is None:
+        on_board = ((board[roots] >= 0) & (board[roots] < 52)).sum(dim=1)
+        offsets = torch.zeros(b + 1, dtype=torch.int64, device=dev)
+        torch.cumsum(52 - on_board, dim=0, out=offsets[1:])
+        if b and int(on_board.max().item()) >= 5:
+            raise ValueError("single-card chance expansion needs an empty board slot (at most 4 cards dealt)")
+        return offsets, int(offsets[-1].item()) if b else 0
+    if not 0 <= cards_on_board <= 4:
+        raise ValueError("cards_on_board must be in 0..4")
+    per_state = 52 - cards_on_board
+    total = b * per_state
+    return torch.arange(0, total + 1, per_state, dtype=torch.int64, device=dev), total   # one launch, no board read
+
+
 def chance_expand(pre_chance_beliefs: torch.Tensor, root_indices: torch.Tensor, board_pre: torch.Tensor,
                   cards_on_board: int | None = None, check_rows: bool = True, input_dtype: torch.dtype | None = None):
     """Every (state, next card) sample of a single-card chance node.
@@ -107,19 +126,7 @@ def chance_expand(pre_chance_beliefs: torch.Tensor, root_indices: torch.Tensor, 
     source_rows = min(pre.shape[0], board.shape[0])
     if check_rows and _rows_out_of_range(roots, source_rows):
         raise IndexError("root_indices out of range")
-    if cards_on_board is None:
-        on_board = ((board[roots] >= 0) & (board[roots] < 52)).sum(dim=1)
-        offsets = torch.zeros(b + 1, dtype=torch.int64, device=dev)
-        torch.cumsum(52 - on_board, dim=0, out=offsets[1:])
-        if b and int(on_board.max().item()) >= 5:
-            raise ValueError("single-card chance expansion needs an empty board slot (at most 4 cards dealt)")
-        total = int(offsets[-1].item()) if b else 0
-    else:
-        if not 0 <= cards_on_board <= 4:
-            raise ValueError("cards_on_board must be in 0..4")
-        per_state = 52 - cards_on_board
-        total = b * per_state
-        offsets = torch.arange(0, total + 1, per_state, dtype=torch.int64, device=dev)   # one launch, no board read
+    offsets, total = _sample_offsets(board, roots, cards_on_board)
     # With ``cards_on_board`` given the sample count is taken on trust; the kernel gets the buffers'
     # size and writes nothing beyond it if a board holds fewer cards than claimed.  Where a state has
     # fewer samples than its share of the buffers (a board with MORE cards than claimed, no empty slot,
@@ -156,6 +163,71 @@ def chance_mean(hand_values: torch.Tensor, sample_offsets: torch.Tensor) -> torc
     out = torch.empty(b, 2, NUM_HANDS, dtype=torch.float32, device=hv.device)
     _lib.call("p2hip_chance_mean", _lib.ptr(hv), _lib.ptr(offsets), b, _lib.ptr(out), _lib.stream_ptr())
     return out
+
+
+# A float32 network of plain layers goes through ``p2hip_chance_network`` from this width on (ms per call, layer by layer
+# -> one call: 2 x 256, 1 state 0.26 -> 0.11, 35 states 0.20 -> 0.11, 2240 states 3.26 -> 0.29; 3 x 1536, 1 state 0.22 ->
+# 0.18, 35 states 0.51 -> 0.21, 2240 states 20.2 -> 3.4).  Narrower ones are what the product's tiles are not made for.
+NETWORK_MIN_WIDTH = 256
+
+
+def network_layers(model, device: torch.device) -> list[torch.nn.Linear] | None:
+    """The layers of ``model`` if its answer is what ``p2hip_chance_network`` computes from their weights as they are
+    now: linear layers with ReLU between them, read as float32 on ``device`` by nobody but ``torch.nn.Linear`` itself
+    (no hook on a layer, no subclass, no parametrisation, no autocast around the call).  None otherwise."""
+    stack = getattr(model, "relu_stack", None)
+    layers = stack() if callable(stack) else None
+    if layers is None or not 3 <= len(layers) <= 16 or torch.is_autocast_enabled("cuda"):
+        return None
+    everywhere = torch.nn.modules.module
+    if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks:
+        return None
+    columns = INPUT_ROW_WIDTH
+    for k, lin in enumerate(layers):
+        if type(lin) is not torch.nn.Linear or lin._forward_hooks or lin._forward_pre_hooks or "forward" in vars(lin):
+            return None
+        rows = lin.weight.shape[0]
+        last = k + 1 == len(layers)
+        if rows != 2 * NUM_HANDS if last else (rows < NETWORK_MIN_WIDTH or rows % 32 or rows > 65536):
+            return None
+        for t, shape in ((lin.weight, (rows, columns)), (lin.bias, (rows,))):
+            if t is None and len(shape) == 1:
+                continue
+            if type(t) not in (torch.nn.Parameter, torch.Tensor) or tuple(t.shape) != shape or t.device != device or \
+                    t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16:
+                return None
+        columns = rows
+    return layers
+
+
+def chance_network(pre_chance_beliefs: torch.Tensor, root_indices: torch.Tensor, board_pre: torch.Tensor,
+                   layers: list[torch.nn.Linear], cards_on_board: int | None = None, check_rows: bool = True) -> torch.Tensor:
+    """[B, 2, 1326]: the mean over the cards that can come next of the answers of the network made of ``layers``
+    (``network_layers``).  Arguments otherwise as in ``chance_expand``."""
+    _lib.require_gpu(pre_chance_beliefs, "chance_network")
+    dev = pre_chance_beliefs.device
+    pre = pre_chance_beliefs
+    _req(pre.dtype == torch.float32 and pre.is_contiguous() and tuple(pre.shape[1:]) == (2, NUM_HANDS),
+         "pre_chance_beliefs: contiguous float32 [rows, 2, 1326]")
+    _req(board_pre.dim() == 2 and board_pre.shape[1] == 5, "board_pre.dim() == 2 and board_pre.shape[1] == 5")
+    board = board_pre.to(device=dev, dtype=torch.int64).contiguous()
+    roots = root_indices.to(device=dev, dtype=torch.int64).contiguous()
+    b = roots.numel()
+    source_rows = min(pre.shape[0], board.shape[0])
+    if check_rows and _rows_out_of_range(roots, source_rows):
+        raise IndexError("root_indices out of range")
+    offsets, total = _sample_offsets(board, roots, cards_on_board)
+    expected = torch.empty(b, 2, NUM_HANDS, dtype=torch.float32, device=dev)
+    count = len(layers)
+    widths = (ctypes.c_int32 * count)(*(lin.weight.shape[0] for lin in layers))
+    weights = (ctypes.c_void_p * count)(*(lin.weight.data_ptr() for lin in layers))
+    biases = (ctypes.c_void_p * count)(*(_lib.ptr(lin.bias) for lin in layers))
+    size = _lib.load().p2hip_chance_network_workspace(b, total, widths, count)
+    _req(size >= 0, "a network and a number of samples that p2hip_chance_network takes")
+    workspace = torch.empty(size, dtype=torch.uint8, device=dev)
+    _lib.call("p2hip_chance_network", _lib.ptr(pre), _lib.ptr(roots), _lib.ptr(board), b, _lib.ptr(offsets), source_rows,
+              total, weights, biases, widths, count, _lib.ptr(workspace), size, _lib.ptr(expected), _lib.stream_ptr())
+    return expected
 
 
 def flop_expand(pre_chance_beliefs: torch.Tensor, root_indices: torch.Tensor, flops: torch.Tensor,
@@ -439,6 +511,12 @@ class ChanceNodeHelper:
         if getattr(model, "input_layout", None) == "ranges|board_onehot" and hasattr(model, "forward_input") \
                 and pre_chance_beliefs.dtype == torch.float32 and pre_chance_beliefs.is_contiguous() \
                 and pre_chance_beliefs.data_ptr() % 16 == 0:
+            layers = network_layers(model, pre_chance_beliefs.device) if self.autocast_dtype is None else None
+            if layers is not None:
+                if hasattr(model, "eval"):
+                    model.eval()
+                return chance_network(pre_chance_beliefs, root_indices, board_pre, layers, cards_on_board,
+                                      check_rows).to(self.float_dtype)
             # the network reads nothing but the ranges and the board: the expansion writes its input matrix
             in_dtype = self.autocast_dtype if self.autocast_dtype in _INPUT_DTYPES else torch.float32
             rows, _, _, offsets = chance_expand(pre_chance_beliefs, root_indices, board_pre, cards_on_board,

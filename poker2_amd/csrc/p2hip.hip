@@ -8,6 +8,7 @@
 #include "cfr_iter.hip"
 #include "cfr_search.hip"
 #include "chance.hip"
+#include "leaf_network.hip"
 #include "best_response.hip"
 #include "tree.hip"
 #include "datagen.hip"
@@ -16,7 +17,7 @@
 
 extern "C" {
 // Library / ABI version, bumped whenever an exported signature changes.
-int p2hip_abi_version(void) { return 5; }
+int p2hip_abi_version(void) { return 6; }
 // Number of visible HIP devices (0 when there is none); never throws.
 int p2hip_device_count(void) {
   int n = 0;

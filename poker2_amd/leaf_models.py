@@ -6,8 +6,9 @@ are evaluated on their own board; leaves where the round has ended and a card is
 come are expanded over every card that can come next (blocker masking, renormalisation,
 network, mean — the semantics of ``ChanceNodeHelper.single_card_chance_values``,
 src/p2/search/chance_node_helper.py:360-479), and leaves where the preflop round has ended
-over the canonical flops (``flop_chance_values``, :219-357).  The network stays ordinary PyTorch; only the
-expansion and the mean are HIP kernels.
+over the canonical flops (``flop_chance_values``, :219-357).  The network stays ordinary PyTorch; the
+expansion and the mean are HIP kernels, and ``RangeBoardMLP`` in float32 behind a single card as a whole is
+(``chance_node_helper.chance_network``).
 
 ``RangeBoardMLP`` is the network of the turn benchmark configuration: input 2 x 1326 ranges +
 52-dim board one-hot, three hidden ReLU layers, output 2 x 1326; orthogonal initialisation with
@@ -66,6 +67,11 @@ class RangeBoardMLP(torch.nn.Module):
         x = torch.zeros(board.shape[0], self.input_width, dtype=dtype, device=board.device)
         x[:, 2 * NUM_HANDS:] = onehot[:, :52]
         return x
+
+    def relu_stack(self) -> list[torch.nn.Linear] | None:
+        """The layers, if ``forward_input`` is these with ReLU between them: None once it has been replaced."""
+        own = type(self).forward_input is RangeBoardMLP.forward_input and "forward_input" not in vars(self)
+        return list(self.linears) if own else None
 
     def forward_input(self, x: torch.Tensor) -> SimpleNamespace:
         for lin in self.linears[:-1]:
