@@ -76,6 +76,11 @@ int p2hip_showdown_setup_sorted(const int32_t* c1_sorted, const int32_t* c2_sort
 int p2hip_showdown_both(const float* beliefs, const uint8_t* tables, const int64_t* table_row,
                         const float* potential, const float* scale, int64_t m, float* out, void* stream);
 
+/* The same on rows of a node table: state k reads beliefs row node_rows[k] and writes out row node_rows[k], both
+ * [rows,2,H] (NULL = identity); the rows are taken on trust. */
+int p2hip_showdown_rows(const float* beliefs, const uint8_t* tables, const int64_t* table_row, const int64_t* node_rows,
+                        const float* potential, const float* scale, int64_t m, float* out, void* stream);
+
 /* ---- single-card chance node around the leaf network --------------------------------- */
 
 /* For each of n public states (state i reads row root_indices[i] of pre_beliefs [*,2,H] and of
@@ -360,6 +365,48 @@ int p2hip_deep_beliefs(float* out, const float* root_beliefs, const float* reach
  * search/fused_sparse_cfr_evaluator.py:494-499 */
 int p2hip_sample_snapshot(const float* policy_probs, float* policy_probs_sample, const int64_t* t_sample,
                           const int64_t* t_now, int64_t total, void* stream);
+
+/* ---- a family, or a level of the tree, per launch ------------------------------------ */
+
+/* What the methods of search/fused_sparse_cfr_evaluator.py compose of the operations above, in the same roundings, for
+ * a whole tree: children of a parent p are rows child_offsets[p] .. + child_count[p] - 1, at most max_children <= 8. */
+
+/* compute_instantaneous_regrets (:312-349): achieved, expected, beliefs [T,2,H] -> regrets [T,H]; parents < top, rows <
+ * bottom zero */
+int p2hip_family_regrets(const float* achieved, const float* expected, const float* beliefs, const int64_t* to_act,
+                         const int64_t* prev_actor, const int64_t* child_offsets, const int64_t* child_count,
+                         int64_t bottom, int64_t top, float* regrets, void* stream);
+
+/* the same, added to the cumulative regrets as p2hip_dcfr_update does instead of stored */
+int p2hip_family_regret_update(const float* achieved, const float* expected, const float* beliefs, const int64_t* to_act,
+                               const int64_t* prev_actor, const int64_t* child_offsets, const int64_t* child_count,
+                               int64_t bottom, int64_t top, float* cumulative, float* weights, const float* t_alpha_num,
+                               const float* t_beta_num, const float* t_alpha_den, const float* t_beta_den, int apply_dcfr,
+                               int cfr_plus, void* stream);
+
+/* the regret matching of update_policy (:201-218): policy[c] = max(cumulative[c], 0) / family sum, fallback[c] where
+ * that is <= eps */
+int p2hip_family_regret_matching(const float* cumulative, const float* fallback, const int64_t* child_offsets,
+                                 const int64_t* child_count, int64_t top, int max_children, float eps, float* policy,
+                                 void* stream);
+
+/* update_average_policy (:355-398): the mix, then its division by the family sum; weights as device scalars */
+int p2hip_family_average_policy(const float* policy, float* policy_avg, const float* reach, const float* reach_avg,
+                                const int64_t* to_act, const int64_t* child_offsets, const int64_t* child_count,
+                                const float* old_w, const float* new_w, const float* total_w, int64_t bottom, int64_t top,
+                                int max_children, float eps, void* stream);
+
+/* reach weights and ranges of every row below the n_roots roots (_calculate_reach_weights and _propagate_all_beliefs of a
+ * whole tree of at most 64 levels); the nodes of a root share their allowed hands */
+#define P2HIP_TREE_MAX_DEPTH 64
+int p2hip_tree_reach_beliefs(float* reach, const float* policy, const uint8_t* allowed, const float* allowed_prob,
+                             const int64_t* parent_index, const int64_t* prev_actor, const int64_t* root_index,
+                             float* beliefs, int64_t n_roots, int64_t total, int depth, float eps, void* stream);
+
+/* compute_expected_values (:242-306) of parents base .. base + n - 1, all of one level, from the level below */
+int p2hip_level_expected_values(float* values, const float* policy, const float* beliefs, const int64_t* to_act,
+                                const int64_t* child_offsets, const int64_t* child_count, int64_t base, int64_t n,
+                                int max_children, float eps, void* stream);
 
 /* ---- one kernel = one CFR iteration ------------------------------------------------- */
 

@@ -33,6 +33,13 @@ _SIGNATURES: dict[str, list] = {
     "p2hip_showdown_setup": [_P, _I, _L, _I, _P, _P, _P, _P],
     "p2hip_showdown_setup_sorted": [_P, _P, _P, _P, _L, _P, _P, _P],
     "p2hip_showdown_both": [_P, _P, _P, _P, _P, _L, _P, _P],
+    "p2hip_showdown_rows": [_P, _P, _P, _P, _P, _P, _L, _P, _P],
+    "p2hip_family_regrets": [_P, _P, _P, _P, _P, _P, _P, _L, _L, _P, _P],
+    "p2hip_family_regret_matching": [_P, _P, _P, _P, _L, _I, _F, _P, _P],
+    "p2hip_family_average_policy": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _F, _P],
+    "p2hip_family_regret_update": [_P, _P, _P, _P, _P, _P, _P, _L, _L, _P, _P, _P, _P, _P, _P, _I, _I, _P],
+    "p2hip_tree_reach_beliefs": [_P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _F, _P],
+    "p2hip_level_expected_values": [_P, _P, _P, _P, _P, _P, _L, _L, _I, _F, _P],
     "p2hip_best_response_level": [_P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _P],
     "p2hip_upload_floats": [_P, _P, _I, _P],
     "p2hip_tree_node_columns": [],

@@ -5,6 +5,7 @@
 #include "unblocked.hip"
 #include "showdown.hip"
 #include "cfr_ops.hip"
+#include "cfr_families.hip"
 #include "cfr_iter.hip"
 #include "cfr_search.hip"
 #include "chance.hip"

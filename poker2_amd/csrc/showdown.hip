@@ -642,6 +642,7 @@ __device__ __forceinline__ void showdown_eval(const float (&vk)[2][SD_PPT], cons
 __global__ __launch_bounds__(SD_BLOCK, 3) void showdown_both_kernel(const float* __restrict__ beliefs,
                                                                      const uint8_t* __restrict__ tables,
                                                                      const int64_t* __restrict__ table_row,
+                                                                     const int64_t* __restrict__ node_rows,
                                                                      const float* __restrict__ potential,
                                                                      const float* __restrict__ scale, int64_t m,
                                                                      float* __restrict__ out) {
@@ -652,27 +653,31 @@ __global__ __launch_bounds__(SD_BLOCK, 3) void showdown_both_kernel(const float*
   ShowdownRegs R, Rn;
   float vk[2][SD_PPT], vkn[2][SD_PPT];
   int64_t n = blockIdx.x;
+  auto row_of = [&](int64_t k) { return node_rows ? node_rows[k] : k; };
+  int64_t row = 0, next_row = n < m ? row_of(n) : 0;
   if (n < m) {
     showdown_load_regs(tables + (table_row ? table_row[n] : n) * SD_TABLE_BYTES, Rn, ab_lds);
-    showdown_gather(beliefs + n * 2 * P2_H, beliefs + n * 2 * P2_H + P2_H, Rn, vkn);
+    showdown_gather(beliefs + next_row * 2 * P2_H, beliefs + next_row * 2 * P2_H + P2_H, Rn, vkn);
   }
   for (; n < m; n += gridDim.x) {
     R = Rn;
+    row = next_row;
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int i = 0; i < SD_PPT; ++i) vk[p][i] = vkn[p][i];
     const int64_t nn = n + gridDim.x;
     const bool more = nn < m;
+    if (more) next_row = row_of(nn);
     if (more) showdown_load_regs(tables + (table_row ? table_row[nn] : nn) * SD_TABLE_BYTES, Rn, ab_lds);
     const float mul0 = potential[2 * n], mul1 = potential[2 * n + 1], div = scale[n];
     showdown_scans(vk, R, s);
-    if (more) showdown_gather(beliefs + nn * 2 * P2_H, beliefs + nn * 2 * P2_H + P2_H, Rn, vkn);
+    if (more) showdown_gather(beliefs + next_row * 2 * P2_H, beliefs + next_row * 2 * P2_H + P2_H, Rn, vkn);
     // the EVs go over the sorted ranges, which are dead once the card scans are done
     showdown_finish(vk, R, s, s.v, mul0, mul1, div);
     p2_sync_lds();
-    float2* o0 = p2_row2(out, n * 2);
-    float2* o1 = p2_row2(out, n * 2 + 1);
+    float2* o0 = p2_row2(out, row * 2);
+    float2* o1 = p2_row2(out, row * 2 + 1);
     for (int i = threadIdx.x; i < P2_HPAIRS; i += SD_BLOCK) {
       const float2 x = s.v[2 * i], y = s.v[2 * i + 1];   // hands 2i, 2i+1: (hero 0, hero 1) each
       o0[i] = make_float2(x.x, y.x);
@@ -715,16 +720,21 @@ int p2hip_showdown_setup_sorted(const int32_t* c1_sorted, const int32_t* c2_sort
   return 0;
 }
 
-int p2hip_showdown_both(const float* beliefs, const uint8_t* tables, const int64_t* table_row,
+int p2hip_showdown_rows(const float* beliefs, const uint8_t* tables, const int64_t* table_row, const int64_t* node_rows,
                         const float* potential, const float* scale, int64_t m, float* out, void* stream) {
   if (m < 0 || (m > 0 && (!beliefs || !tables || !potential || !scale || !out))) return P2_EINVAL;
   if (m == 0) return 0;
   if (!p2_aligned8(tables) || !p2_aligned4(beliefs) || !p2_aligned8(out)) return P2_EINVAL;
   const int64_t cap = 256 * 3;  // three resident workgroups (43 KB of LDS each) on each of the 256 CUs
   hipLaunchKernelGGL(p2::showdown_both_kernel, dim3((unsigned)(m < cap ? m : cap)), dim3(p2::SD_BLOCK), 0,
-                     (hipStream_t)stream, beliefs, tables, table_row, potential, scale, m, out);
+                     (hipStream_t)stream, beliefs, tables, table_row, node_rows, potential, scale, m, out);
   P2_LAUNCH_CHECK();
   return 0;
+}
+
+int p2hip_showdown_both(const float* beliefs, const uint8_t* tables, const int64_t* table_row,
+                        const float* potential, const float* scale, int64_t m, float* out, void* stream) {
+  return p2hip_showdown_rows(beliefs, tables, table_row, nullptr, potential, scale, m, out, stream);
 }
 
 }  // extern "C"

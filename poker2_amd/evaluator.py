@@ -263,7 +263,6 @@ class HipSparseCFREvaluator:
         self._t_scalars = F.TScalars(self.device, dtype=self.float_dtype)
         self._skip_t_scalars_update = False
         self._skip_record_stats = True
-        self._fused_positive_regrets_buf = None
         self._fscal = self._t_scalars.floats      # the one-kernel iteration reads the first eight
         self._iscal = self._t_scalars.ints
         self._fscal_host = (ctypes.c_float * 8)()
@@ -769,22 +768,24 @@ class HipSparseCFREvaluator:
     def update_policy(self, t: int) -> None:
         """fused_sparse_cfr_evaluator.py:201-236."""
         self._complete_rows()
-        bottom, top = self.depth_offsets[1], self.depth_offsets[-2]
-        if self._fused_positive_regrets_buf is None or \
-                self._fused_positive_regrets_buf.shape != self.cumulative_regrets.shape:
-            self._fused_positive_regrets_buf = torch.empty_like(self.cumulative_regrets)
-        pos = self._fused_positive_regrets_buf
-        torch.clamp(self.cumulative_regrets, min=0.0, out=pos)
-        parent_sum = F.fused_parent_sum(pos, self.child_offsets[:top].contiguous(),
-                                        self.child_count[:top].contiguous(), max_children=self.num_actions)
-        F.fused_divide_by_parent_sum_(pos=pos[bottom:], fallback=self.uniform_policy[bottom:], parent_sum=parent_sum,
-                                      parent_index=self.parent_index[bottom:].contiguous(),
-                                      out=self.policy_probs[bottom:])
-        self._calculate_reach_weights(self.self_reach, self.policy_probs)
-        self._propagate_all_beliefs(self.beliefs, self.self_reach)
+        F.family_regret_matching_(self.policy_probs, self.cumulative_regrets, self.uniform_policy, self.child_offsets,
+                                  self.child_count, self.depth_offsets[-2], self._max_children)
+        self._push_down(self.self_reach, self.policy_probs, self.beliefs)
         self.update_average_policy(t)
-        self._calculate_reach_weights(self.self_reach_avg, self.policy_probs_avg)
-        self._propagate_all_beliefs(self.beliefs_avg, self.self_reach_avg)
+        self._push_down(self.self_reach_avg, self.policy_probs_avg, self.beliefs_avg)
+
+    def _own_methods(self, *names: str) -> bool:
+        """Whether these methods are this class's: a pass that replaces them must not pass an override by."""
+        return all(getattr(getattr(self, name), "__func__", None) is getattr(HipSparseCFREvaluator, name) for name in names)
+
+    def _push_down(self, reach: torch.Tensor, policy: torch.Tensor, beliefs: torch.Tensor) -> None:
+        """``_calculate_reach_weights`` and ``_propagate_all_beliefs`` in one launch."""
+        if self.tree_depth > F.TREE_MAX_DEPTH or not self._own_methods("_calculate_reach_weights", "_propagate_all_beliefs"):
+            self._calculate_reach_weights(reach, policy)
+            self._propagate_all_beliefs(beliefs, reach)
+            return
+        F.tree_reach_beliefs_(reach, beliefs, policy, self.allowed_hands, self.allowed_hands_prob, self.parent_index,
+                              self.prev_actor, self._root_index, self.root_nodes, self.tree_depth)
 
     def update_average_policy(self, t: int) -> None:
         """fused_sparse_cfr_evaluator.py:355-398."""
@@ -792,18 +793,10 @@ class HipSparseCFREvaluator:
         if self._avg_policy_copies(t):
             self.policy_probs_avg[:] = self.policy_probs
             return
-        N, top = self.root_nodes, self.depth_offsets[-2]
-        F.fused_average_policy_mix_with_tensors_(
-            policy_probs_avg=self.policy_probs_avg, policy_probs=self.policy_probs, self_reach=self.self_reach,
-            self_reach_avg=self.self_reach_avg, to_act=self.env.to_act, parent_index=self.parent_index,
-            old=self._t_scalars.mix_old, new=self._t_scalars.mix_new, total_weight=self._t_scalars.mix_total,
-            bottom=N)
-        parent_sum = F.fused_parent_sum(self.policy_probs_avg, self.child_offsets[:top].contiguous(),
-                                        self.child_count[:top].contiguous(), max_children=self.num_actions)
-        child = self.policy_probs_avg[N:]
-        F.fused_divide_by_parent_sum_(pos=child, fallback=child, parent_sum=parent_sum,
-                                      parent_index=self.parent_index[N:].contiguous(), out=child, eps=1e-5)
-        self.policy_probs_avg[:N] = 0.0
+        F.family_average_policy_(self.policy_probs_avg, self.policy_probs, self.self_reach, self.self_reach_avg,
+                                 self.env.to_act, self.child_offsets, self.child_count, self._t_scalars.mix_old,
+                                 self._t_scalars.mix_new, self._t_scalars.mix_total, self.root_nodes,
+                                 self.depth_offsets[-2], self._max_children)
 
     def compute_instantaneous_regrets(self, values_achieved: torch.Tensor,
                                       values_expected: torch.Tensor | None = None) -> torch.Tensor:
@@ -811,16 +804,9 @@ class HipSparseCFREvaluator:
         self._complete_rows()
         if values_expected is None:
             values_expected = values_achieved
-        bottom, top = self.depth_offsets[1], self.depth_offsets[-2]
-        beliefs = self.beliefs_avg if self.cfr_avg else self.beliefs
-        regrets = torch.zeros_like(self.policy_probs)
-        src_weights = F.unblocked_mass_opp_at_parents_triton(beliefs, self.env.to_act, top)
-        rows = torch.arange(top, device=self.device)
-        actor_values = values_expected[:top][rows, self.env.to_act[:top], :].contiguous()
-        F.fused_regret_tail_(regrets=regrets, values_achieved=values_achieved.contiguous(), actor_values=actor_values,
-                             src_weights=src_weights, parent_index=self.parent_index, prev_actor=self.prev_actor,
-                             bottom=bottom)
-        return regrets
+        return F.family_regrets(values_achieved.contiguous(), values_expected.contiguous(),
+                                self.beliefs_avg if self.cfr_avg else self.beliefs, self.env.to_act, self.prev_actor,
+                                self.child_offsets, self.child_count, self.depth_offsets[1], self.depth_offsets[-2])
 
     def compute_expected_values(self, policy=None, beliefs=None, leaf_values=None, values=None) -> None:
         """fused_sparse_cfr_evaluator.py:242-306."""
@@ -831,20 +817,10 @@ class HipSparseCFREvaluator:
         values = leaf_values if values is None else values
         if leaf_values is not values:
             torch.where(self.leaf_mask[:, None, None], leaf_values, torch.zeros_like(values), out=values)
-        bottom, top = self.depth_offsets[1], self.depth_offsets[-2]
-        rows = torch.arange(top, device=self.device)
-        actor_beliefs = beliefs[:top][rows, self.env.to_act[:top], :].contiguous()
-        marginal = actor_beliefs.index_select(0, self.parent_index[bottom:]) * policy[bottom:]
-        occ = torch.zeros_like(policy)
-        occ[bottom:] = F.unblocked_mass_ratio_indirect_triton(
-            numer_target=marginal.contiguous(), denom_target=actor_beliefs,
-            parent_index=self.parent_index[bottom:].contiguous())
+        policy, beliefs = policy.contiguous(), beliefs.contiguous()
         for depth in range(self.tree_depth - 1, -1, -1):
-            base, end = self.depth_offsets[depth], self.depth_offsets[depth + 1]
-            F.fused_weighted_parent_sum(values=values, prev_actor=self.prev_actor, policy_hero=policy, policy_opp=occ,
-                                        child_offsets=self.child_offsets[base:end].contiguous(),
-                                        child_count=self.child_count[base:end].contiguous(), parent_base=base,
-                                        max_children=self.num_actions)
+            F.level_expected_values_(values, policy, beliefs, self.env.to_act, self.child_offsets, self.child_count,
+                                     self.depth_offsets[depth], self.depth_offsets[depth + 1], self._max_children)
 
     def update_average_values(self, t: int) -> None:
         """fused_sparse_cfr_evaluator.py:404-414."""
@@ -929,7 +905,13 @@ class HipSparseCFREvaluator:
         if beliefs is None:
             beliefs = self.beliefs_avg if self.cfr_avg else self.beliefs
         self._set_model_values_impl(t, beliefs)
-        if showdown and self.showdown_indices.numel():
+        if not showdown or self.showdown_indices.numel() == 0:
+            return
+        if self._own_methods("_showdown_value_both") and beliefs.is_contiguous() and beliefs.dtype == torch.float32 \
+                and beliefs.shape == self.latest_values.shape:
+            rules_hip.showdown_value_rows_(self.latest_values, beliefs, self.showdown_indices, self.hand_rank_data,
+                                           self._showdown_potential_f, self._showdown_scale, self._showdown_rows)
+        else:
             self.latest_values[self.showdown_indices] = self._showdown_value_both(beliefs[self.showdown_indices])
 
     # ------------------------------------------------------------------ iteration
@@ -1099,8 +1081,7 @@ class HipSparseCFREvaluator:
         """Whether code from outside this package runs between the parts of an iteration, and so may look at any row
         that a lean iteration has to store: an overridden method, or a leaf model other than those that say of their
         ``leaf_values`` / ``leaf_values_from_nodes`` (by ``reads_given_rows_only``) that they read no other row."""
-        if any(getattr(getattr(self, name), "__func__", None) is not getattr(HipSparseCFREvaluator, name)
-               for name in self._ITERATION_HOOKS):
+        if not self._own_methods(*self._ITERATION_HOOKS):
             return True
         if self.model is None or not self._has_model_leaves:
             return False
@@ -1173,17 +1154,25 @@ class HipSparseCFREvaluator:
                 self._launch_iteration(3, lean, alternate_reach_avg)
             return
         F.fused_sample_snapshot_(self.policy_probs_sample, self.policy_probs, self.t_sample, self._t_scalars.t_tensor)
-        regrets = self.compute_instantaneous_regrets(self.latest_values)
+        s = self._t_scalars
+        update = dict(t_alpha_num=s.t_alpha_num, t_beta_num=s.t_beta_num, t_alpha_den=s.t_alpha_den,
+                      t_beta_den=s.t_beta_den, cfr_plus=self.cfr_plus,
+                      apply_dcfr=self.cfr_type in (CFRType.discounted, CFRType.discounted_plus))
         if self.cfr_type == CFRType.linear:
+            regrets = self.compute_instantaneous_regrets(self.latest_values)
             regrets.masked_fill_(self.prev_actor[:, None] == t % self.num_players, 0.0)
             self.regret_weight_sums += 1
             self.cumulative_regrets += regrets
+        elif self._own_methods("compute_instantaneous_regrets"):
+            self._complete_rows()
+            F.family_regret_update_(self.cumulative_regrets, self.regret_weight_sums, self.latest_values, self.latest_values,
+                                    self.beliefs_avg if self.cfr_avg else self.beliefs, self.env.to_act, self.prev_actor,
+                                    self.child_offsets, self.child_count, self.depth_offsets[1], self.depth_offsets[-2],
+                                    **update)
         else:
-            F.fused_dcfr_update_with_tensors_(
-                cumulative_regrets=self.cumulative_regrets, regret_weight_sums=self.regret_weight_sums,
-                regrets=regrets, t_alpha_num=self._t_scalars.t_alpha_num, t_beta_num=self._t_scalars.t_beta_num,
-                t_alpha_den=self._t_scalars.t_alpha_den, t_beta_den=self._t_scalars.t_beta_den,
-                apply_dcfr=self.cfr_type in (CFRType.discounted, CFRType.discounted_plus), cfr_plus=self.cfr_plus)
+            F.fused_dcfr_update_with_tensors_(cumulative_regrets=self.cumulative_regrets,
+                                              regret_weight_sums=self.regret_weight_sums,
+                                              regrets=self.compute_instantaneous_regrets(self.latest_values), **update)
         self.update_policy(t)
         self.set_leaf_values(t)
         self.compute_expected_values()

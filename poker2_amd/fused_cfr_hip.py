@@ -578,6 +578,103 @@ def fused_deep_beliefs_(out, root_beliefs, reach_weights, allowed_prob, root_ind
               int(n), total, float(eps), _S())
 
 
+# --------------------------------------------------------------------------- a family or a level per launch
+# What the evaluator's methods compose of the operations above, in the same roundings (csrc/cfr_families.hip).
+def _family_args(total: int, top: int, bottom: int, max_children: int, child_offsets, child_count, **index) -> None:
+    _need()
+    _i64(total, child_offsets=child_offsets, child_count=child_count, **index)
+    _req(0 <= int(top) <= total and 0 <= int(bottom) <= total, f"top={top} or bottom={bottom} outside the {total} rows")
+    _req(0 <= int(max_children) <= 8, "at most 8 children per parent")
+
+
+def _same_rows(total: int, one: dict, both: dict) -> None:
+    for name, t in one.items():
+        _req(tuple(t.shape) == (total, _H), f"{name}.shape == (total, 1326)")
+    for name, t in both.items():
+        _req(tuple(t.shape) == (total, 2, _H), f"{name}.shape == (total, 2, 1326)")
+    _f32(**one, **both)
+
+
+def family_regrets(achieved, expected, beliefs, to_act, prev_actor, child_offsets, child_count, bottom: int,
+                   top: int) -> torch.Tensor:
+    """regrets [total, 1326] of every child of a parent < ``top`` (fused_sparse_cfr_evaluator.py:312-349); rows below
+    ``bottom`` are zero."""
+    total = beliefs.shape[0]
+    _family_args(total, top, bottom, 0, child_offsets, child_count, to_act=to_act, prev_actor=prev_actor)
+    _same_rows(total, {}, dict(achieved=achieved, expected=expected, beliefs=beliefs))
+    regrets = torch.empty(total, _H, dtype=torch.float32, device=beliefs.device)
+    _lib.call("p2hip_family_regrets", _p(achieved), _p(expected), _p(beliefs), _p(to_act), _p(prev_actor),
+              _p(child_offsets), _p(child_count), int(bottom), int(top), _p(regrets), _S())
+    return regrets
+
+
+def family_regret_update_(cumulative, weights, achieved, expected, beliefs, to_act, prev_actor, child_offsets, child_count,
+                          bottom: int, top: int, t_alpha_num, t_beta_num, t_alpha_den, t_beta_den, apply_dcfr: bool,
+                          cfr_plus: bool) -> None:
+    """``fused_dcfr_update_with_tensors_`` of ``family_regrets`` without the tensor between them."""
+    total = beliefs.shape[0]
+    _family_args(total, top, bottom, 0, child_offsets, child_count, to_act=to_act, prev_actor=prev_actor)
+    _same_rows(total, dict(cumulative=cumulative, weights=weights), dict(achieved=achieved, expected=expected, beliefs=beliefs))
+    _scalar_ptrs(t_alpha_num=t_alpha_num, t_beta_num=t_beta_num, t_alpha_den=t_alpha_den, t_beta_den=t_beta_den)
+    _lib.call("p2hip_family_regret_update", _p(achieved), _p(expected), _p(beliefs), _p(to_act), _p(prev_actor),
+              _p(child_offsets), _p(child_count), int(bottom), int(top), _p(cumulative), _p(weights), _p(t_alpha_num),
+              _p(t_beta_num), _p(t_alpha_den), _p(t_beta_den), int(apply_dcfr), int(cfr_plus), _S())
+
+
+def family_regret_matching_(policy, cumulative, fallback, child_offsets, child_count, top: int, max_children: int,
+                            eps: float = 1e-8) -> None:
+    """policy[child] = its share of the family's positive regrets, ``fallback`` where there are none
+    (fused_sparse_cfr_evaluator.py:201-218)."""
+    total = policy.shape[0]
+    _family_args(total, top, 0, max_children, child_offsets, child_count)
+    _same_rows(total, dict(policy=policy, cumulative=cumulative, fallback=fallback), {})
+    _lib.call("p2hip_family_regret_matching", _p(cumulative), _p(fallback), _p(child_offsets), _p(child_count), int(top),
+              int(max_children), float(eps), _p(policy), _S())
+
+
+def family_average_policy_(policy_avg, policy, reach, reach_avg, to_act, child_offsets, child_count, old, new,
+                           total_weight, bottom: int, top: int, max_children: int, eps: float = 1e-5) -> None:
+    """The reach-weighted average policy, renormalised per family (fused_sparse_cfr_evaluator.py:355-398)."""
+    total = policy.shape[0]
+    _family_args(total, top, bottom, max_children, child_offsets, child_count, to_act=to_act)
+    _same_rows(total, dict(policy=policy, policy_avg=policy_avg), dict(reach=reach, reach_avg=reach_avg))
+    _scalar_ptrs(old=old, new=new, total_weight=total_weight)
+    _lib.call("p2hip_family_average_policy", _p(policy), _p(policy_avg), _p(reach), _p(reach_avg), _p(to_act),
+              _p(child_offsets), _p(child_count), _p(old), _p(new), _p(total_weight), int(bottom), int(top),
+              int(max_children), float(eps), _S())
+
+
+TREE_MAX_DEPTH = 64       # P2HIP_TREE_MAX_DEPTH
+
+
+def tree_reach_beliefs_(reach, beliefs, policy, allowed_mask, allowed_prob, parent_index, prev_actor, root_index,
+                        num_roots: int, depth: int, eps: float = 1e-5) -> None:
+    """``fused_reach_weights_depth_`` of every level and ``fused_deep_beliefs_`` in one launch, for a tree of at most
+    ``TREE_MAX_DEPTH`` levels below its roots whose nodes share their root's allowed hands."""
+    total = policy.shape[0]
+    _need()
+    _i64(total, parent_index=parent_index, prev_actor=prev_actor, root_index=root_index)
+    _same_rows(total, dict(policy=policy, allowed_prob=allowed_prob), dict(reach=reach, beliefs=beliefs))
+    _req(tuple(allowed_mask.shape) == (total, _H) and allowed_mask.dtype == torch.bool and allowed_mask.is_contiguous() and
+         allowed_mask.device.type == "cuda", "allowed_mask: contiguous bool [total, 1326] on the GPU")
+    _req(0 <= int(num_roots) <= total and 0 <= int(depth) <= TREE_MAX_DEPTH, "num_roots or depth out of range")
+    _lib.call("p2hip_tree_reach_beliefs", _p(reach), _p(policy), _p(allowed_mask), _p(allowed_prob), _p(parent_index),
+              _p(prev_actor), _p(root_index), _p(beliefs), int(num_roots), total, int(depth), float(eps), _S())
+
+
+def level_expected_values_(values, policy, beliefs, to_act, child_offsets, child_count, base: int, end: int,
+                           max_children: int, eps: float = 1e-5) -> None:
+    """values[p] of parents p in [base, end), all of one level, from their children's: the actor's weighted by ``policy``,
+    the other player's by where the actor's compatible range goes (fused_sparse_cfr_evaluator.py:242-306)."""
+    total = policy.shape[0]
+    _family_args(total, end, base, max_children, child_offsets, child_count, to_act=to_act)
+    _req(int(base) <= int(end), f"rows [{base}, {end})")
+    _same_rows(total, dict(policy=policy), dict(values=values, beliefs=beliefs))
+    _lib.call("p2hip_level_expected_values", _p(values), _p(policy), _p(beliefs), _p(to_act), _p(child_offsets),
+              _p(child_count), int(base), int(end) - int(base), int(max_children), float(eps), _S())
+
+
+
 def showdown_ev_triton(b_opp_sorted, c1_sorted, c2_sorted, L_idx, R_idx, eps: float = 1e-8, block_k: int = 32,
                        block_j: int = 128) -> torch.Tensor:
     """Showdown EV per hand, in strength order, from strength-sorted inputs: the villain range

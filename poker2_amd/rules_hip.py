@@ -246,3 +246,24 @@ def showdown_value_both(beliefs: torch.Tensor, tables: torch.Tensor, potential: 
     _lib.call("p2hip_showdown_both", _lib.ptr(beliefs), _lib.ptr(tables), _lib.ptr(table_row),
               _lib.ptr(potential), _lib.ptr(scale), m, _lib.ptr(out), _lib.stream_ptr())
     return out
+
+
+def showdown_value_rows_(values: torch.Tensor, beliefs: torch.Tensor, rows: torch.Tensor, tables: torch.Tensor,
+                         potential: torch.Tensor, scale: torch.Tensor, table_row: torch.Tensor) -> None:
+    """``values[rows] = showdown_value_both(beliefs[rows], ...)`` on node tables [total, 2, 1326], without the copies of
+    the rows.  ``rows`` are taken on trust."""
+    _require_backend()
+    _lib.require_gpu(beliefs, "showdown_value_rows_")
+    m = rows.numel()
+    for t in (values, beliefs):
+        _req(t.dtype == torch.float32 and t.is_contiguous() and t.dim() == 3 and tuple(t.shape[1:]) == (2, NUM_HANDS),
+             "values, beliefs: contiguous float32 [total, 2, 1326]")
+    _req(values.shape == beliefs.shape and values.data_ptr() != beliefs.data_ptr(), "two tables of the same rows")
+    for t, shape in ((potential, (m, 2)), (scale, (m,))):
+        _req(t.dtype == torch.float32 and t.is_contiguous() and tuple(t.shape) == shape, "potential [M, 2], scale [M]: float32")
+    for t in (rows, table_row):
+        _req(t.dtype == torch.int64 and t.is_contiguous() and tuple(t.shape) == (m,), "rows, table_row: contiguous int64 [M]")
+    _req(tables.is_contiguous() and tables.dtype == torch.uint8 and tables.shape[1] == showdown_table_bytes(),
+         "tables.is_contiguous() and tables.dtype == torch.uint8 and tables.shape[1] == showdown_table_bytes()")
+    _lib.call("p2hip_showdown_rows", _lib.ptr(beliefs), _lib.ptr(tables), _lib.ptr(table_row), _lib.ptr(rows),
+              _lib.ptr(potential), _lib.ptr(scale), m, _lib.ptr(values), _lib.stream_ptr())
