@@ -408,6 +408,34 @@ int p2hip_level_expected_values(float* values, const float* policy, const float*
                                 const int64_t* child_offsets, const int64_t* child_count, int64_t base, int64_t n,
                                 int max_children, float eps, void* stream);
 
+/* ---- before the first iteration and after the last ------------------------------------ */
+
+/* constant rows of a new state of `total` nodes, the first n_roots of them roots: uniform [T,H] = 1 / children of the
+ * parent (0 for roots); reach, reach_avg [T,2,H] = 1 for roots, else 0; latest, values_avg [T,2,H] = reward, -reward of
+ * the two players at folds, else 0 (search/sparse_cfr_evaluator.py:240-306) */
+int p2hip_subgame_rows(const int64_t* parent_index, const int64_t* child_count, const uint8_t* fold_mask,
+                       const float* reward, int64_t n_roots, int64_t total, float* uniform, float* reach, float* reach_avg,
+                       float* latest, float* values_avg, void* stream);
+
+/* board [roots,5] (-1 = not dealt): allowed [T,H] = no card of the hand on the board of row r's root, prob [T,H] uniform
+ * over these hands (search/cfr_evaluator.py:780-815) */
+int p2hip_allowed_hands(const int64_t* board, const int64_t* root_index, int64_t total, uint8_t* allowed, float* prob,
+                        void* stream);
+
+/* initialize_policy_and_beliefs (search/cfr_evaluator.py:830-886) for a uniform policy over the legal actions
+ * (legal_mask [T,actions]) of a tree of `depth` <= P2HIP_TREE_MAX_DEPTH levels: roots [n_roots,2,H] = the roots' ranges
+ * (not the rows of `beliefs`), root rows of `reach` read, everything else of the six tensors written */
+int p2hip_uniform_start(const float* roots, const uint8_t* allowed, const float* allowed_prob, const int64_t* parent_index,
+                        const int64_t* prev_actor, const int64_t* root_index, const uint8_t* legal_mask, int actions,
+                        int64_t n_roots, int64_t total, int depth, float eps, float* policy, float* policy_avg,
+                        float* reach, float* reach_avg, float* beliefs, float* beliefs_avg, void* stream);
+
+/* out [T,2,H] = values at leaves (clamped to [-1,1] if `clamp`), 0 elsewhere */
+int p2hip_leaf_rows(const float* values, const uint8_t* leaf_mask, int64_t total, int clamp, float* out, void* stream);
+
+/* *found = 1 if one of n (even) floats is infinite or NaN, else untouched */
+int p2hip_any_nonfinite(const float* x, int64_t n, int32_t* found, void* stream);
+
 /* ---- one kernel = one CFR iteration ------------------------------------------------- */
 
 /* Device pointers of one subgame batch.  Tree arrays and state tensors are the evaluator's

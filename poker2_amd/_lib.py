@@ -40,6 +40,11 @@ _SIGNATURES: dict[str, list] = {
     "p2hip_family_regret_update": [_P, _P, _P, _P, _P, _P, _P, _L, _L, _P, _P, _P, _P, _P, _P, _I, _I, _P],
     "p2hip_tree_reach_beliefs": [_P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _F, _P],
     "p2hip_level_expected_values": [_P, _P, _P, _P, _P, _P, _L, _L, _I, _F, _P],
+    "p2hip_subgame_rows": [_P, _P, _P, _P, _L, _L, _P, _P, _P, _P, _P, _P],
+    "p2hip_allowed_hands": [_P, _P, _L, _P, _P, _P],
+    "p2hip_uniform_start": [_P, _P, _P, _P, _P, _P, _P, _I, _L, _L, _I, _F, _P, _P, _P, _P, _P, _P, _P],
+    "p2hip_leaf_rows": [_P, _P, _L, _I, _P, _P],
+    "p2hip_any_nonfinite": [_P, _L, _P, _P],
     "p2hip_best_response_level": [_P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _P],
     "p2hip_upload_floats": [_P, _P, _I, _P],
     "p2hip_tree_node_columns": [],

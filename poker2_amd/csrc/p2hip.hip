@@ -6,6 +6,7 @@
 #include "showdown.hip"
 #include "cfr_ops.hip"
 #include "cfr_families.hip"
+#include "subgame.hip"
 #include "cfr_iter.hip"
 #include "cfr_search.hip"
 #include "chance.hip"

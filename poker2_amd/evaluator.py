@@ -40,7 +40,7 @@ import torch
 from . import _lib
 from . import fused_cfr_hip as F
 from . import rules_hip
-from .card_utils import NUM_HANDS, combo_to_onehot_tensor
+from .card_utils import NUM_HANDS
 from .fused_cfr_hip import CFRType
 from .chance_node_helper import ChanceNodeHelper
 from .rebel_batch import RebelBatch
@@ -293,8 +293,9 @@ class HipSparseCFREvaluator:
         rows = min(nbytes // 10 // 256 * 256 // (4 * NUM_HANDS), 12288)
         return float(ms.value) * 1e6 / rows
 
-    def _place_state(self, shapes: list[tuple[int, ...]]) -> list[torch.Tensor]:
-        """Zero-filled float tensors of the given shapes: the state of a search.
+    def _place_state(self, shapes: list[tuple[int, ...]], written: tuple[int, ...] = ()) -> list[torch.Tensor]:
+        """Zero-filled float tensors of the given shapes: the state of a search.  (Those at the places ``written`` are
+        written in full by the caller and may come as they are.)
 
         The iteration kernel writes about ten of them at once, and the card's memory takes that faster when
         the written tensors lie in two different thirds (~96 GiB each) of its physical address space than when
@@ -332,7 +333,8 @@ class HipSparseCFREvaluator:
         self.state_placement = {"placed": False}
         place = self.spread_state and min(slab_bytes) >= max(STATE_SPREAD_MIN_SLAB_BYTES, 2 * _PROBE_MIN_BYTES)
         if not place and not self.reuse_state:
-            return [torch.zeros(*sh, dtype=self.float_dtype, device=dev) for sh in shapes]
+            return [(torch.empty if k in written else torch.zeros)(*sh, dtype=self.float_dtype, device=dev)
+                    for k, sh in enumerate(shapes)]
         if self.reuse_state:
             slab_bytes = [(b + b // 4 + 255) // 256 * 256 for b in slab_bytes]
         first = torch.empty(slab_bytes[0], dtype=torch.uint8, device=dev)
@@ -484,7 +486,8 @@ class HipSparseCFREvaluator:
         # tensors, six [T, 2, H], the scratch rows, and the second reach_avg buffer of a lean search
         one, two = (T, NUM_HANDS), (T, 2, NUM_HANDS)
         with_alt = self.fused_iteration and self.lean_search
-        pool = self._place_state([one] * 5 + [two] * 6 + [one] + ([two] if with_alt else []))
+        # (7 to 10: reaches and values, written by p2hip_subgame_rows)
+        pool = self._place_state([one] * 5 + [two] * 6 + [one] + ([two] if with_alt else []), written=(7, 8, 9, 10))
         self._reach_avg_alt = pool.pop() if with_alt else None
         if with_alt:
             self._reach_avg_alt[:N] = 1.0
@@ -502,23 +505,18 @@ class HipSparseCFREvaluator:
 
         self.policy_probs, self.policy_probs_avg, self.policy_probs_sample = z1(), z1(), z1()
         self.cumulative_regrets, self.regret_weight_sums = z1(), z1()
-        self.uniform_policy = torch.zeros(T, NUM_HANDS, dtype=self.float_dtype, device=dev)
-        cc_dest = self.child_count[:tree.top].repeat_interleave(self.child_count[:tree.top])
-        self.uniform_policy[N:] = (1.0 / cc_dest)[:, None].expand(-1, NUM_HANDS)
         self.beliefs, self.beliefs_avg = z2(), z2()
         # the name whose tensor and ``_leaf_alt`` a one-walk iteration has exchanged
         self._leaf_moved: str | None = None
         self._walk_open = None         # the argument blocks of a one-walk iteration whose leaves a network evaluates
         self.root_pre_chance_beliefs = torch.zeros(N, 2, NUM_HANDS, dtype=self.float_dtype, device=dev)
-        self.self_reach = z2()
-        self.self_reach[:N] = 1.0
-        self.self_reach_avg = z2().copy_(self.self_reach)
-        self.latest_values = z2()
-        folded = tt("fold_mask", tree.fold_mask)
-        rew = tt("reward", tree.reward)
-        self.latest_values[folded, 0] = rew[folded][:, None]
-        self.latest_values[folded, 1] = -rew[folded][:, None]
-        self.values_avg = z2().copy_(self.latest_values)
+        self.self_reach, self.self_reach_avg, self.latest_values, self.values_avg = z2(), z2(), z2(), z2()
+        self.uniform_policy = torch.empty(T, NUM_HANDS, dtype=self.float_dtype, device=dev)
+        p = _lib.ptr
+        folded, reward = tt("fold_mask", tree.fold_mask).contiguous(), tt("reward", tree.reward).float().contiguous()
+        _lib.call("p2hip_subgame_rows", p(self.parent_index), p(self.child_count), p(folded), p(reward), N, T,
+                  p(self.uniform_policy), p(self.self_reach), p(self.self_reach_avg), p(self.latest_values),
+                  p(self.values_avg), _lib.stream_ptr())
         self.last_model_values = None
         self._scratch = z1()
         flags = np.zeros(T, dtype=np.uint8)
@@ -627,16 +625,11 @@ class HipSparseCFREvaluator:
         self.self_reach[:N] = 1.0
         self.self_reach_avg[:N] = 1.0
         board = self._t(self.tree.board)
-        onehot = combo_to_onehot_tensor(device=self.device).float()
-        board_mask = torch.zeros(N, 52, dtype=self.float_dtype, device=self.device)
-        valid = board >= 0
-        rows = torch.arange(N, device=self.device)[:, None].expand_as(board)
-        board_mask[rows[valid], board[valid]] = 1.0
-        root_allowed = (onehot @ board_mask.T).T < 0.5
-        root_prob = root_allowed.float()
-        root_prob /= root_prob.sum(dim=-1, keepdim=True).clamp(min=1.0)
-        self.allowed_hands = root_allowed[self._root_index].contiguous()
-        self.allowed_hands_prob = root_prob[self._root_index].contiguous()
+        T, p = self.total_nodes, _lib.ptr
+        self.allowed_hands = torch.empty(T, NUM_HANDS, dtype=torch.bool, device=self.device)
+        self.allowed_hands_prob = torch.empty(T, NUM_HANDS, dtype=self.float_dtype, device=self.device)
+        _lib.call("p2hip_allowed_hands", p(board), p(self._root_index), T, p(self.allowed_hands),
+                  p(self.allowed_hands_prob), _lib.stream_ptr())
         self._init_hand_rank_data()
         self.t_sample = torch.full((self.total_nodes,), -1, dtype=torch.long, device=self.device)
         self.stats["evaluator_total_nodes"] = float(self.total_nodes)
@@ -816,7 +809,7 @@ class HipSparseCFREvaluator:
         leaf_values = self.latest_values if leaf_values is None else leaf_values
         values = leaf_values if values is None else values
         if leaf_values is not values:
-            torch.where(self.leaf_mask[:, None, None], leaf_values, torch.zeros_like(values), out=values)
+            self._leaf_rows(leaf_values, out=values)
         policy, beliefs = policy.contiguous(), beliefs.contiguous()
         for depth in range(self.tree_depth - 1, -1, -1):
             F.level_expected_values_(values, policy, beliefs, self.env.to_act, self.child_offsets, self.child_count,
@@ -1180,11 +1173,29 @@ class HipSparseCFREvaluator:
             self.update_average_values(t)
 
     # ------------------------------------------------------------------ whole search
+    def _starts_uniform(self) -> bool:
+        """Whether the initial policy is known to be uniform over the legal actions (no model, or one that has none) and
+        the steps that follow from it are this class's own."""
+        policy = getattr(self.model, "policy_logits", None)
+        known = policy is None or getattr(self.model, "policy_is_uniform", False)
+        state = (self.policy_probs, self.policy_probs_avg, self.self_reach, self.self_reach_avg, self.beliefs,
+                 self.beliefs_avg, self.allowed_hands, self.allowed_hands_prob, self.legal_mask)
+        return (known and self.tree_depth <= F.TREE_MAX_DEPTH and all(t.is_contiguous() for t in state)
+                and self._own_methods("_normalize_beliefs", "_calculate_reach_weights"))
+
     @torch.no_grad()
     def initialize_policy_and_beliefs(self) -> None:
         """cfr_evaluator.py:830-886: initial policy from the model's logits (uniform over the
         legal actions without a model), beliefs pushed down level by level."""
         self._complete_rows()
+        if self._starts_uniform():
+            roots, p = self.beliefs[:self.root_nodes].clone(), _lib.ptr
+            _lib.call("p2hip_uniform_start", p(roots), p(self.allowed_hands), p(self.allowed_hands_prob),
+                      p(self.parent_index), p(self.prev_actor), p(self._root_index), p(self.legal_mask), self.num_actions,
+                      self.root_nodes, self.total_nodes, self.tree_depth, 1e-5, p(self.policy_probs),
+                      p(self.policy_probs_avg), p(self.self_reach), p(self.self_reach_avg), p(self.beliefs),
+                      p(self.beliefs_avg), _lib.stream_ptr())
+            return
         self.policy_probs.zero_()
         if self.tree_depth == 0:
             self._normalize_beliefs()
@@ -1218,12 +1229,10 @@ class HipSparseCFREvaluator:
         regret of every action against each player's best-response values, scaled by
         warm_start_iterations x warm_start_multiplier."""
         self.set_leaf_values(0)
-        if not torch.isfinite(self.latest_values).all():
-            raise ValueError("Non-finite values in latest_values after set_leaf_values")
+        self._require_finite_values("set_leaf_values")
         self.compute_expected_values(policy=self.policy_probs, beliefs=self.beliefs, leaf_values=self.latest_values,
                                      values=self.latest_values)
-        if not torch.isfinite(self.latest_values).all():
-            raise ValueError("Non-finite values in latest_values after compute_expected_values")
+        self._require_finite_values("compute_expected_values")
         self._record_initial_exploitability()
         t_ws = self.warm_start_iterations
         scale = float(t_ws) * self.warm_start_multiplier
@@ -1246,6 +1255,23 @@ class HipSparseCFREvaluator:
         self.cumulative_regrets += scale * regrets
         self.regret_weight_sums += scale
         self.update_policy(t_ws)
+
+    def _require_finite_values(self, after: str) -> None:
+        found = torch.zeros(1, dtype=torch.int32, device=self.device)
+        _lib.call("p2hip_any_nonfinite", _lib.ptr(self.latest_values), self.latest_values.numel(), _lib.ptr(found),
+                  _lib.stream_ptr())
+        if bool(found.item()):
+            raise ValueError(f"Non-finite values in latest_values after {after}")
+
+    def _leaf_rows(self, values: torch.Tensor, clamp: bool = False, out: torch.Tensor | None = None) -> torch.Tensor:
+        """``values`` at the leaves, clamped to [-1, 1] if asked, and zero at every other node."""
+        values = values.to(self.float_dtype).contiguous()
+        _req(tuple(values.shape) == (self.total_nodes, 2, NUM_HANDS), "values: [total, 2, 1326]")
+        out = torch.empty_like(values) if out is None else out
+        _req(out.shape == values.shape and out.dtype == values.dtype and out.is_contiguous(), "out: like values")
+        _lib.call("p2hip_leaf_rows", _lib.ptr(values), _lib.ptr(self.leaf_mask), self.total_nodes, int(clamp),
+                  _lib.ptr(out), _lib.stream_ptr())
+        return out
 
     def _record_initial_exploitability(self) -> None:
         """cfr_evaluator.py:1618-1633 (mean over roots; no per-street split)."""
@@ -1486,10 +1512,11 @@ class HipSparseCFREvaluator:
         return per_root.index_select(0, self._root_index)
 
     def _best_response_values(self, policy: torch.Tensor, beliefs: torch.Tensor, base_values: torch.Tensor,
-                              deviating_player: torch.Tensor | None = None) -> torch.Tensor:
+                              deviating_player: torch.Tensor | None = None, *, clamp: bool = False) -> torch.Tensor:
         """Values when ``deviating_player`` (per node; default: the root's player to act) plays a
         per-hand best response and the other player follows ``policy``
-        (cfr_evaluator.py:603-716).  One kernel launch per tree level, deepest first."""
+        (cfr_evaluator.py:603-716).  One kernel launch per tree level, deepest first.  ``clamp``: leaf values are cut to
+        [-1, 1]."""
         n = self.root_nodes
         if deviating_player is None:
             deviating_player = self._fan_out_deep(self.env.to_act[:n])
@@ -1497,7 +1524,7 @@ class HipSparseCFREvaluator:
         _req(deviating_player.shape == (self.total_nodes,), "deviating_player.shape == (self.total_nodes,)")
         policy = policy.contiguous()
         beliefs = beliefs.contiguous()
-        values_br = torch.where(self.leaf_mask[:, None, None], base_values, torch.zeros_like(base_values)).contiguous()
+        values_br = self._leaf_rows(base_values, clamp)
         for depth in range(self.tree_depth - 1, -1, -1):
             base, end = self.depth_offsets[depth], self.depth_offsets[depth + 1]
             _lib.call("p2hip_best_response_level", _lib.ptr(values_br), _lib.ptr(policy), _lib.ptr(beliefs),
@@ -1515,13 +1542,12 @@ class HipSparseCFREvaluator:
                                        torch.empty(0, 2, device=self.device, dtype=self.float_dtype))
         self._complete_rows()
         policy, beliefs = self.policy_probs_avg, self.beliefs_avg
-        leaf_values = self.values_avg.clamp(-1.0, 1.0)
-        base_values = torch.zeros_like(leaf_values)
-        self.compute_expected_values(policy=policy, beliefs=beliefs, leaf_values=leaf_values, values=base_values)
+        base_values = self._leaf_rows(self.values_avg, clamp=True)
+        self.compute_expected_values(policy=policy, beliefs=beliefs, leaf_values=base_values, values=base_values)
         improvements, br_agg = [], []
         for player in range(2):
             deviator = torch.full((n,), player, device=self.device, dtype=torch.int64)
-            br = self._best_response_values(policy, beliefs, leaf_values, self._fan_out_deep(deviator))
+            br = self._best_response_values(policy, beliefs, self.values_avg, self._fan_out_deep(deviator), clamp=True)
             root_beliefs = beliefs[:n, player]
             improvements.append(((br[:n, player] - base_values[:n, player]) * root_beliefs).sum(dim=-1))
             br_agg.append((br[:n, player] * root_beliefs).sum(dim=-1))

@@ -121,6 +121,12 @@ class NetworkLeafModel:
                 return self.net(feats, **kw)
         return self.net(feats, **kw)
 
+    @property
+    def policy_is_uniform(self) -> bool:
+        """Whether ``policy_logits`` is known to answer zeros, a uniform policy over the legal actions, without asking."""
+        own = type(self).policy_logits is NetworkLeafModel.policy_logits and "policy_logits" not in vars(self)
+        return own and not self._policy_keyword
+
     @torch.no_grad()
     def policy_logits(self, beliefs: torch.Tensor, rows: torch.Tensor, ev) -> torch.Tensor:
         """[K, 1326, actions] logits of the network at node rows ``rows`` (cfr_evaluator.py:305-319);
