@@ -127,13 +127,19 @@ def declared_symbols() -> list[str]:
     return list(_SIGNATURES)
 
 
+_available = False
+
+
 def hip_is_available() -> bool:
-    """True when the library loads and a GPU is visible to torch."""
-    try:
-        load()
-    except (P2HipError, OSError):
-        return False
-    return torch.cuda.is_available()
+    """True when the library loads and a GPU is visible to torch.  (A yes stays one: neither goes away.)"""
+    global _available
+    if not _available:
+        try:
+            load()
+        except (P2HipError, OSError):
+            return False
+        _available = torch.cuda.is_available()
+    return _available
 
 
 def check(code: int, what: str) -> None:
@@ -146,8 +152,16 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The current stream as the raw pointer that a launch takes, without the torch.cuda.Stream object around it: 0.2 us of
+# host time instead of 2.75 in every launch.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _current_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def require_gpu(t: torch.Tensor, name: str) -> None:
@@ -156,5 +170,6 @@ def require_gpu(t: torch.Tensor, name: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    lib = load()
-    check(getattr(lib, name)(*args), name)
+    code = getattr(_lib or load(), name)(*args)
+    if code:
+        check(code, name)

@@ -54,14 +54,13 @@ def _require_backend() -> None:
 
 
 def _planes_i8(ab_batch: torch.Tensor, tail: tuple[int, ...]) -> torch.Tensor:
-    if ab_batch.dim() != len(tail) + 1 or tuple(ab_batch.shape[1:]) != tail:
+    if ab_batch.shape[1:] != tail:
         raise ValueError(f"Expected [N, {', '.join(map(str, tail))}] input, got {tuple(ab_batch.shape)}")
-    if ab_batch.device.type != "cuda":
+    if not ab_batch.is_cuda:
         raise ValueError("The HIP hand evaluator requires a GPU tensor.")
-    x = ab_batch.contiguous()
-    if x.dtype in (torch.bool, torch.int8, torch.uint8):
-        return x.view(torch.uint8)            # one byte per card already: no copy (non-zero = present)
-    return (x != 0).view(torch.uint8)
+    if ab_batch.dtype in (torch.bool, torch.int8, torch.uint8):
+        return ab_batch.contiguous()          # one byte per card already: no copy (non-zero = present)
+    return (ab_batch != 0).contiguous()
 
 
 def _compare_planes(ab_batch: torch.Tensor, flush_first: int) -> torch.Tensor:
