@@ -209,6 +209,9 @@ struct SetupLds {
   uint16_t head_before[SD_HWORDS], head_after[SD_HWORDS], heads_in[SD_HWORDS];
   __align__(4) uint16_t clist[P2_CARDS * 51];
   int bcards[5];
+  int singles;                                 // hands scored one by one
+  int32_t pair_score[169];                     // by two ranks, 13 low + high
+  uint32_t pair_code[169];
 };
 
 // Combos of card c at sorted positions below `bound`.
@@ -227,7 +230,8 @@ __device__ __forceinline__ int card_below(const SetupLds& S, int c, int bound) {
 // Bound by vector issue and LDS.  Sorting 64-bit keys through LDS (66 steps with a barrier each), ranking every card's
 // combos against each other (52 x 51 x 51 look-ups) and binary searches for the tie groups took 544 us for 4096
 // boards; keys of 32 bits sorted in registers, and positions kept as bit sets whose prefix counts answer "how
-// many below", take 100 us (1 board: 20 us).
+// many below", take 102 us (1 board: 20 us); with scores by pairs of ranks 92.  2600 vector instructions a wave, 76 %
+// of the issue slots: 1000 of them sort, 1000 rank, 560 write the table.
 __global__ __launch_bounds__(SD_BLOCK) void showdown_setup_kernel(const void* __restrict__ boards, int elem_size,
                                                                    int mode, int32_t* __restrict__ ranks_out,
                                                                    int64_t* __restrict__ order_out,
@@ -252,29 +256,88 @@ __global__ __launch_bounds__(SD_BLOCK) void showdown_setup_kernel(const void* __
     if (c < 52u) { bs[c / 13u] |= 1u << (c % 13u); board_bits |= 1ull << c; }
     if (c < 52u && mode != 0) board_acc.add((int)c);   // the order of the cards does not matter: the board goes first, once
   }
+  // Without a flush a hand's score is that of its two ranks, 91 pairs of them.  Scored one by one are only the hands that
+  // may hold a flush (45 where the board has three cards of a suit) and those that hold a board card; where the board
+  // repeats a card or holds a flush itself, all of them.
+  auto score = [&](int a, int b) {
+    if (mode == 0) {
+      uint32_t s[4] = {bs[0], bs[1], bs[2], bs[3]};
+      s[a / 13] |= 1u << (a % 13);
+      s[b / 13] |= 1u << (b % 13);
+      return score_hand(hand_from_suits(s[0], s[1], s[2], s[3]), false);
+    }
+    CardAcc acc = board_acc;
+    acc.add(a);
+    acc.add(b);
+    return score_hand(acc.finish(), true);
+  };
+  auto put_score = [&](int h, int32_t sc, uint32_t code) {
+    if (mode != 0 && ranks_out) ranks_out[m * P2_H + h] = sc;
+    S.keys[h] = (code << 11) | (uint32_t)h;      // any order does: the keys are distinct
+  };
+  const int suited[4] = {popc(bs[0]), popc(bs[1]), popc(bs[2]), popc(bs[3])};
+  int flush_suit = -1;                           // of which the board holds three cards or more
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (suited[q] >= 3) flush_suit = q;
+  const int needed = flush_suit < 0 ? 3 : 5 - (flush_suit == 0 ? suited[0] : flush_suit == 1 ? suited[1] : flush_suit == 2 ? suited[2] : suited[3]);
+  const bool by_ranks = __popcll(board_bits) == 5 && needed > 0;
+  if (t == 0) S.singles = 0;
+  for (int h = P2_H + t; h < SORT_N; h += SD_BLOCK) S.keys[h] = ~0u;
+  p2_sync_lds();
+  uint32_t pair_of[6];                           // where the hands' scores will be: 13 x low rank + high rank
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const int h = t + i * SD_BLOCK;
+    const bool in = h < P2_H;
+    const int a = in ? p2_combo.a[h] : 0, b = in ? p2_combo.b[h] : 1;
+    const int sa = (a * 79) >> 10, sb = (b * 79) >> 10;                      // / 13 for 0 .. 51
+    const int ra = a - 13 * sa, rb = b - 13 * sb;
+    const bool single = in && (!by_ranks || (((board_bits >> a) | (board_bits >> b)) & 1ull) ||
+                               (int)(sa == flush_suit) + (int)(sb == flush_suit) >= needed);
+    pair_of[i] = in && !single ? (uint32_t)(ra < rb ? ra * 13 + rb : rb * 13 + ra) : 255u;
+    const unsigned long long who = __ballot(single);
+    int first = 0;
+    if (lane == 0 && who) first = atomicAdd(&S.singles, __popcll(who));
+    first = __builtin_amdgcn_readfirstlane(first);
+    if (single) S.clist[first + __popcll(who & ((1ull << lane) - 1ull))] = (uint16_t)h;   // (the lists come later)
+  }
+  p2_sync_lds();
+  // The pairs take two waves, the hands of the list (290 where the board has three of a suit) five turns of a wave: dealt
+  // from a wave that changes with the board, or the first SIMD of every CU had twice the work of the last.
+  const int turn = ((t >> 6) + (int)m) & 3;
+  if (by_ranks && turn < 2 && turn * 64 + lane < 91) {
+    // the unordered pairs of 13 ranks: those 0 to 6 apart, cyclically
+    const int e = turn * 64 + lane, step = e / 13, r = e - step * 13, r2 = r + step < 13 ? r + step : r + step - 13;
+    CardAcc acc = board_acc;
+    if (mode == 0)
+      for (int j = 0; j < 5; ++j) acc.add(S.bcards[j]);
+    acc.add(r);
+    acc.add(r2);
+    Hand h = acc.finish();
+    h.s0 = h.s1 = h.s2 = h.s3 = 0;               // no suits: planes that cannot hold a flush
+    const int32_t sc = score_hand(h, true);
+    const int at = r < r2 ? r * 13 + r2 : r2 * 13 + r;
+    S.pair_score[at] = sc;
+    S.pair_code[at] = score_code(sc);
+  }
+  for (int e = (((turn + 2) & 3) << 6) + lane; e < S.singles; e += SD_BLOCK) {
+    const int h = S.clist[e];
+    const int32_t sc = score(p2_combo.a[h], p2_combo.b[h]);
+    put_score(h, sc, score_code(sc));
+  }
+  p2_sync_lds();
+#pragma unroll
+  for (int i = 0; i < 6; ++i)
+    if (pair_of[i] != 255u) put_score(t + i * SD_BLOCK, S.pair_score[pair_of[i]], S.pair_code[pair_of[i]]);
+  p2_sync_lds();
   uint32_t key[SORT_PER];
 #pragma unroll
-  for (int i = 0; i < SORT_PER; ++i) {
-    const int h = t + i * SD_BLOCK;              // any order does: the keys are distinct
-    key[i] = ~0u;
-    if (h < P2_H) {
-      const int a = p2_combo.a[h], b = p2_combo.b[h];
-      int32_t sc;
-      if (mode == 0) {
-        uint32_t s[4] = {bs[0], bs[1], bs[2], bs[3]};
-        s[a / 13] |= 1u << (a % 13);
-        s[b / 13] |= 1u << (b % 13);
-        sc = score_hand(hand_from_suits(s[0], s[1], s[2], s[3]), false);
-      } else {
-        CardAcc acc = board_acc;
-        acc.add(a);
-        acc.add(b);
-        sc = score_hand(acc.finish(), true);
-        if (ranks_out) ranks_out[m * P2_H + h] = sc;
-      }
-      key[i] = (score_code(sc) << 11) | (uint32_t)h;
-    }
+  for (int r = 0; r < SORT_PER; r += 4) {
+    const uint4 x = *reinterpret_cast<const uint4*>(S.keys + t * SORT_PER + r);
+    key[r] = x.x; key[r + 1] = x.y; key[r + 2] = x.z; key[r + 3] = x.w;
   }
+  p2_sync_lds();                                 // the sort writes there
   sort_2048(key, S.keys);  // ties resolve by combo index: a stable argsort
 
   uint32_t hk[6], ab[6];   // this lane's positions t + 256 i

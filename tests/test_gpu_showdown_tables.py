@@ -51,3 +51,26 @@ def test_tables_match_numpy(triton_order, extra):
         assert np.array_equal(order[k], np.argsort(ranks[k], kind="stable"))
         want = expected_table(board, order[k], ranks[k])
         assert np.array_equal(tables[k, :want.size], want), board
+
+
+@pytest.mark.parametrize("triton_order", [True, False])
+@pytest.mark.parametrize("suited", [1, 2, 3, 4, 5])
+def test_scores_by_ranks_and_one_by_one_agree_with_the_oracle(triton_order, suited):
+    """Boards with every number of cards of one suit, paired or not: which hands take the score of their two ranks and
+    which are scored one by one depends on these."""
+    from poker2_amd import rules_hip as K
+    rng = np.random.default_rng(suited)
+    boards = []
+    for k in range(12):
+        suit, ranks = int(rng.integers(0, 4)), rng.permutation(13)
+        cards = [13 * suit + r for r in ranks[:suited]]
+        others = [13 * s + r for s in range(4) if s != suit for r in (ranks[:3] if k % 2 else range(13))]   # odd: pairs
+        cards += [int(c) for c in rng.permutation(others)][:5 - suited]
+        boards.append(rng.permutation(cards))
+    boards = np.array(boards, dtype=np.int64)
+    device = torch.from_numpy(boards).cuda()
+    ranks, order = (x.cpu().numpy() for x in (K.rank_hands_triton(device) if triton_order else K.rank_hands(device)))
+    want_ranks, want_order = (ORK.rank_hands_cards if triton_order else ORK.rank_hands)(boards)
+    assert np.array_equal(ranks, want_ranks) and np.array_equal(order, want_order)
+    alone = K.rank_hands_triton(device[5:6])[0] if triton_order else K.rank_hands(device[5:6])[0]
+    assert np.array_equal(alone.cpu().numpy()[0], want_ranks[5])        # the dealing of work changes with the board's place
