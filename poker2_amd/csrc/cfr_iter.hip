@@ -406,6 +406,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 
   const float f_an = A.fscal[0], f_bn = A.fscal[1], f_ad = A.fscal[2], f_bd = A.fscal[3];
   const float mix_old = A.fscal[4], mix_new = A.fscal[5], mix_total = A.fscal[6], mix_inv = A.fscal[7];
+  const float y_ad = p2_recip_wide(f_ad), y_bd = p2_recip_wide(f_bd), y_mix = p2_recip_wide(mix_total);
   const int64_t t_now = A.iscal[0];
   const bool apply_dcfr = A.iscal[1] != 0, cfr_plus = A.iscal[2] != 0, avg_copy = A.iscal[3] != 0;
   const bool enforce_zs = A.iscal[4] != 0, update_avg = A.iscal[5] != 0;
@@ -430,7 +431,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
         for (int e = 0; e < 2; ++e) {
           if (apply_dcfr) {
             ww[e] = ww[e] * f_bn;
-            ww[e] = ww[e] / f_bd;
+            ww[e] = p2_quotient(ww[e], f_bd, y_bd);
           }
           ww[e] = ww[e] + 1.0f;
         }
@@ -519,10 +520,11 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                     if (apply_dcfr) {
                       const bool positive = cc[e] > 0.f;
                       const float num = positive ? f_an : f_bn, den = positive ? f_ad : f_bd;
+                      const float inv = positive ? y_ad : y_bd;
                       cc[e] = cc[e] * num;
-                      cc[e] = cc[e] / den;
+                      cc[e] = p2_quotient(cc[e], den, inv);
                       ww[e] = ww[e] * num;
-                      ww[e] = ww[e] / den;
+                      ww[e] = p2_quotient(ww[e], den, inv);
                     }
                     ww[e] = ww[e] + 1.0f;
                     cc[e] = cc[e] + rg[e];
@@ -546,8 +548,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           if (k < cnt) {
             float2 pol[IT_PPT];
             IT_FOR(j) {
-              pol[j].x = sum[j].x > 1e-8f ? pos[k][j].x / fmaxf(sum[j].x, 1e-8f) : uniform;
-              pol[j].y = sum[j].y > 1e-8f ? pos[k][j].y / fmaxf(sum[j].y, 1e-8f) : uniform;
+              pol[j].x = p2_matched(pos[k][j].x, sum[j].x, uniform);
+              pol[j].y = p2_matched(pos[k][j].y, sum[j].y, uniform);
             }
             st(A.policy, first + k, pol, ln);
           }
@@ -647,8 +649,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                 const float reach_a = rao[e] * mix_old, reach_n = rr[e] * mix_new;
                 const float num = reach_a * aa[e] + reach_n * cc[e];
                 const float den = reach_a + reach_n;
-                const float unweighted = (mix_old * aa[e] + mix_new * cc[e]) / mix_total;
-                o[e] = den > 1e-5f ? num / den : unweighted;
+                const float unweighted = p2_quotient(mix_old * aa[e] + mix_new * cc[e], mix_total, y_mix);
+                o[e] = den > 1e-5f ? p2_div(num, den) : unweighted;
               }
               pav[k][j] = make_float2(o[0], o[1]);
               psum[j].x += o[0];
@@ -662,8 +664,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
         if (k < cnt) {
           if (!avg_copy) {
             IT_FOR(j) {
-              if (psum[j].x > 1e-5f) pav[k][j].x = pav[k][j].x / fmaxf(psum[j].x, 1e-5f);
-              if (psum[j].y > 1e-5f) pav[k][j].y = pav[k][j].y / fmaxf(psum[j].y, 1e-5f);
+              if (psum[j].x > 1e-5f) pav[k][j].x = p2_div(pav[k][j].x, fmaxf(psum[j].x, 1e-5f));
+              if (psum[j].y > 1e-5f) pav[k][j].y = p2_div(pav[k][j].y, fmaxf(psum[j].y, 1e-5f));
             }
           }
           st(A.policy_avg, first + k, pav[k], ln);
@@ -765,8 +767,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       float2 bo[IT_PPT], boa[IT_PPT];
       IT_FOR(j) {
         const float2 vb = mul2(rb_opp[j], rn_opp[j]), vba = mul2(rba_opp[j], ran_opp[j]);
-        bo[j] = so > 1e-5f ? make_float2(vb.x / so, vb.y / so) : ap[j];
-        boa[j] = soa > 1e-5f ? make_float2(vba.x / soa, vba.y / soa) : ap[j];
+        bo[j] = so > 1e-5f ? make_float2(p2_div(vb.x, so), p2_div(vb.y, so)) : ap[j];
+        boa[j] = soa > 1e-5f ? make_float2(p2_div(vba.x, soa), p2_div(vba.y, soa)) : ap[j];
       }
 #pragma unroll
       for (int k = 0; k < MAXC; ++k) {
@@ -777,7 +779,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           from_lds(xa, L.u.vecs[k], ln);
           IT_FOR(j) {
             const float2 vb = mul2(rb_act[j], xa[j]);
-            o[j] = sa > 1e-5f ? make_float2(vb.x / sa, vb.y / sa) : ap[j];
+            o[j] = sa > 1e-5f ? make_float2(p2_div(vb.x, sa), p2_div(vb.y, sa)) : ap[j];
           }
           st(A.beliefs, c * 2 + actor, o, ln);
           if ((opp_rows >> (2 * k)) & 1) st(A.beliefs, c * 2 + 1 - actor, bo, ln);
@@ -792,7 +794,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           float2 oa[IT_PPT];
           IT_FOR(j) {
             const float2 vba = mul2(rba_act[j], pav[k][j]);
-            oa[j] = saa > 1e-5f ? make_float2(vba.x / saa, vba.y / saa) : ap[j];
+            oa[j] = saa > 1e-5f ? make_float2(p2_div(vba.x, saa), p2_div(vba.y, saa)) : ap[j];
           }
           st(A.beliefs_avg, c * 2 + actor, oa, ln);
           if (bavg_all || ((opp_rows >> (2 * k)) & 1)) st(A.beliefs_avg, c * 2 + 1 - actor, boa, ln);
@@ -955,8 +957,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                 unblocked_regs(nm, mg, L.cs + (1 + k) * P2_CARDS, card_total(L.cs + (1 + k) * P2_CARDS), ln);
               }
               IT_FOR(j) {
-                occ[j].x = dn[j].x > 1e-5f ? nm[j].x / dn[j].x : 0.f;
-                occ[j].y = dn[j].y > 1e-5f ? nm[j].y / dn[j].y : 0.f;
+                occ[j].x = dn[j].x > 1e-5f ? p2_div(nm[j].x, dn[j].x) : 0.f;
+                occ[j].y = dn[j].y > 1e-5f ? p2_div(nm[j].y, dn[j].y) : 0.f;
               }
               IT_FOR(j) {
                 const float2 wa = polk[k][j], wo = occ[j];

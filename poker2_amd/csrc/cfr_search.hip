@@ -297,6 +297,7 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
 
   const float f_an = A.fscal[0], f_bn = A.fscal[1], f_ad = A.fscal[2], f_bd = A.fscal[3];
   const float mix_old = A.fscal[4], mix_new = A.fscal[5], mix_total = A.fscal[6], mix_inv = A.fscal[7];
+  const float y_ad = p2_recip_wide(f_ad), y_bd = p2_recip_wide(f_bd), y_mix = p2_recip_wide(mix_total);
   const int64_t t_now = A.iscal[0];
   const bool apply_dcfr = A.iscal[1] != 0, cfr_plus = A.iscal[2] != 0, avg_copy = A.iscal[3] != 0;
   const bool update_avg = A.iscal[5] != 0, linear = A.iscal[7] != 0;
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
       }
       const float2 pk = sget(L.pol[k], ln);
       const float2 nm = sunblocked(mul2(ab, pk), L.cs + (1 + k) * P2_CARDS, card_total(L.cs + (1 + k) * P2_CARDS), cards);
-      const float2 wo = make_float2(dn.x > 1e-5f ? nm.x / dn.x : 0.f, dn.y > 1e-5f ? nm.y / dn.y : 0.f);
+      const float2 wo = make_float2(dn.x > 1e-5f ? p2_div(nm.x, dn.x) : 0.f, dn.y > 1e-5f ? p2_div(nm.y, dn.y) : 0.f);
       const float2 w0 = actor == 0 ? pk : wo, w1 = actor == 0 ? wo : pk;
       vp[0].x += u0.x * w0.x; vp[0].y += u0.y * w0.y;
       vp[1].x += u1.x * w1.x; vp[1].y += u1.y * w1.y;
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
       float2 ws = sld(A.wsum, r, ln);
       if (apply_dcfr) {
         ws = make_float2(ws.x * f_bn, ws.y * f_bn);
-        ws = make_float2(ws.x / f_bd, ws.y / f_bd);
+        ws = make_float2(p2_quotient(ws.x, f_bd, y_bd), p2_quotient(ws.y, f_bd, y_bd));
       }
       sst(A.wsum, r, make_float2(ws.x + 1.0f, ws.y + 1.0f), ln);
     }
@@ -441,10 +442,11 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
           if (apply_dcfr) {
             const bool positive = cc[e] > 0.f;
             const float num = positive ? f_an : f_bn, den = positive ? f_ad : f_bd;
+            const float inv = positive ? y_ad : y_bd;
             cc[e] = cc[e] * num;
-            cc[e] = cc[e] / den;
+            cc[e] = p2_quotient(cc[e], den, inv);
             ww[e] = ww[e] * num;
-            ww[e] = ww[e] / den;
+            ww[e] = p2_quotient(ww[e], den, inv);
           }
           ww[e] = ww[e] + 1.0f;
           cc[e] = cc[e] + rg[e];
@@ -472,8 +474,8 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
           if (take_sample) sst(A.policy_sample, first + k, sld(A.policy, first + k, ln), ln);
           const float2 pos = sget(L.pol[k], ln);
           float2 pol;
-          pol.x = sum.x > 1e-8f ? pos.x / fmaxf(sum.x, 1e-8f) : uniform;
-          pol.y = sum.y > 1e-8f ? pos.y / fmaxf(sum.y, 1e-8f) : uniform;
+          pol.x = p2_matched(pos.x, sum.x, uniform);
+          pol.y = p2_matched(pos.y, sum.y, uniform);
           sst(A.policy, first + k, pol, ln);
           sput(L.pol[k], pol, ln);
           if (avg_copy) {
@@ -487,8 +489,8 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
               const float reach_a = rao[e] * mix_old, reach_n = rr[e] * mix_new;
               const float num = reach_a * aa[e] + reach_n * cc[e];
               const float den = reach_a + reach_n;
-              const float unweighted = (mix_old * aa[e] + mix_new * cc[e]) / mix_total;
-              o[e] = den > 1e-5f ? num / den : unweighted;
+              const float unweighted = p2_quotient(mix_old * aa[e] + mix_new * cc[e], mix_total, y_mix);
+              o[e] = den > 1e-5f ? p2_div(num, den) : unweighted;
             }
             pav[k] = make_float2(o[0], o[1]);
             psum.x += o[0];
@@ -521,8 +523,8 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
       for (int k = 0; k < MAXC; ++k) {
         if (k < cnt) {
           if (!avg_copy) {
-            if (psum.x > 1e-5f) pav[k].x = pav[k].x / fmaxf(psum.x, 1e-5f);
-            if (psum.y > 1e-5f) pav[k].y = pav[k].y / fmaxf(psum.y, 1e-5f);
+            if (psum.x > 1e-5f) pav[k].x = p2_div(pav[k].x, fmaxf(psum.x, 1e-5f));
+            if (psum.y > 1e-5f) pav[k].y = p2_div(pav[k].y, fmaxf(psum.y, 1e-5f));
           }
           sst(A.policy_avg, first + k, pav[k], ln);
           pav[k] = allowed2(mul2(ran_act, pav[k]));    // the child's average reach from here on
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(SR_BLOCK, 3) void cfr_search_kernel(IterArgs A, Sea
       search_sums<NS>(sums, L);
       // ---- rows other families read: reach, average reach, ranges of children that have children
       auto normalised = [&](float2 v, float s) {
-        return s > 1e-5f ? make_float2(v.x / s, v.y / s) : sld(A.allowed_prob, r, ln);
+        return s > 1e-5f ? make_float2(p2_div(v.x, s), p2_div(v.y, s)) : sld(A.allowed_prob, r, ln);
       };
       if (sdbits | opp_rows) lo = normalised(lo, sums[0]);
       float2 own = make_float2(0.f, 0.f);  // the showdown child's range of the actor
