@@ -102,6 +102,23 @@ struct IterArgs {
   int whole_rows;        // a lean iteration stores the rows that range_rows and const_rows spare all the same
 };
 
+// The kernel's arguments.  A lean iteration's sweeps each read them ANEW from the argument segment and keep the
+// handful that they use.  Read once at the start, the forty pointers do not fit into the scalar registers next to the
+// schedule's factors; the compiler then parks them in lanes of vector registers, in runs of sixteen, and brings back
+// a whole run wherever one is used: 2260 of the kernel's 9700 vector instructions (five children).  River roots, in
+// ms: 192, 16 iterations, 10.16 -> 9.93; 1003 small trees, 12 iterations, 6.45 -> 6.23; the search of 192, 44.7 ->
+// 44.0; one and 4096 the same within 0.4 %.  Asking anew for every family was slower than parking (one root, 32
+// iterations, 4.46 -> 4.56): the scalar loads were waited for there.  An ordinary iteration (192 in a graph, 5.87)
+// spilled vector registers with it (5.93), so there the compiler places the reads (5.87).
+// (The empty asm only hides from the compiler that the address is the one it has already loaded from.)
+typedef const __attribute__((address_space(4))) IterArgs IterArgsConst;
+template <bool ANEW>
+__device__ __forceinline__ IterArgsConst& iter_args() {
+  uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  if (ANEW) asm volatile("" : "+s"(at));
+  return *(IterArgsConst*)at;
+}
+
 // Which sweeps a launch runs.  Sweep 1 of a family reads its parent's beliefs, values and reach_avg
 // as the PREVIOUS iteration left them; sweep 2 needs sweep 1 of its family and sweep 2 of its
 // ancestors (it rewrites the rows sweep 1 of the families below reads); sweep 3 needs sweep 2 of its
@@ -301,8 +318,8 @@ struct FamWin {
 // bit 2k + 1 = its ranges feed a leaf evaluation, bit 16 + 2k = that evaluation reads both of the child's own
 // range rows (a leaf network), bit 17 + 2k = the child's values do not depend on the hand.
 // SH: the launch shares rows (range_rows or const_rows given); without, none of that costs anything.
-template <int MAXC, bool KINDS, bool SH>
-__device__ __forceinline__ void fam_load(FamWin& F, const IterArgs& A, int64_t pp0, int nfam, int base) {
+template <int MAXC, bool KINDS, bool SH, class Args>
+__device__ __forceinline__ void fam_load(FamWin& F, Args& A, int64_t pp0, int nfam, int base) {
   const int l = base + (int)(threadIdx.x & 63);
   F.base = base;
   F.p = 0;
@@ -364,7 +381,7 @@ struct SdWin {
   int base;
 };
 template <bool SH>
-__device__ __forceinline__ void sd_load(SdWin& S, const IterArgs& A, int64_t sd0, int nsd, int base) {
+__device__ __forceinline__ void sd_load(SdWin& S, IterArgsConst& A, int64_t sd0, int nsd, int base) {
   const int l = base + (int)(threadIdx.x & 63);
   S.base = base;
   S.c = S.rs = 0;
@@ -383,8 +400,13 @@ __device__ __forceinline__ float readlane_f(float v, int s) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s));
 }
 
+__device__ __forceinline__ float first_lane_f(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
 template <int MAXC, bool LEAN, bool ALT, bool SH>
-__global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iteration_kernel(IterArgs A) {
+__global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iteration_kernel(IterArgs) {
+  IterArgsConst& A = iter_args<LEAN>();
   constexpr int IT_CHUNK = ItChunk<MAXC>::value;
   // how many rows are requested together: parents staged for the card sums, children of a family in
   // the regret sweep, children of a family in the value sweep
@@ -406,7 +428,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 
   const float f_an = A.fscal[0], f_bn = A.fscal[1], f_ad = A.fscal[2], f_bd = A.fscal[3];
   const float mix_old = A.fscal[4], mix_new = A.fscal[5], mix_total = A.fscal[6], mix_inv = A.fscal[7];
-  const float y_ad = p2_recip_wide(f_ad), y_bd = p2_recip_wide(f_bd), y_mix = p2_recip_wide(mix_total);
+  const float y_ad = first_lane_f(p2_recip_wide(f_ad)), y_bd = first_lane_f(p2_recip_wide(f_bd));
+  const float y_mix = first_lane_f(p2_recip_wide(mix_total));
   const int64_t t_now = A.iscal[0];
   const bool apply_dcfr = A.iscal[1] != 0, cfr_plus = A.iscal[2] != 0, avg_copy = A.iscal[3] != 0;
   const bool enforce_zs = A.iscal[4] != 0, update_avg = A.iscal[5] != 0;
@@ -417,14 +440,17 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
   const float* leaf_beliefs = cfr_avg ? A.beliefs_avg : A.beliefs;
 
   if (A.phases & (PHASE_12 | PHASE_1)) {
+    IterArgsConst& A = iter_args<LEAN>();
     // ---------------- sweep 1: regrets -> DCFR -> regret matching ----------------
+    float *const policy = A.policy, *const cum = A.cum, *const wsum = A.wsum, *const latest = A.latest;
+    const float* const ranges = A.leaf_prev ? A.leaf_prev : leaf_beliefs;
     PROF_BEGIN(t_s1);
     const bool take_sample = A.t_sample[r] == t_now;
     if (top) {
       // The root row takes part in the flat DCFR update like every other row: its regret is
       // zero (never positive), so only its weight sum moves.
       float2 ws[IT_PPT];
-      ld(ws, A.wsum, r, ln);
+      ld(ws, wsum, r, ln);
       IT_FOR(j) {
         float ww[2] = {ws[j].x, ws[j].y};
 #pragma unroll
@@ -437,7 +463,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
         }
         ws[j] = make_float2(ww[0], ww[1]);
       }
-      st(A.wsum, r, ws, ln);
+      st(wsum, r, ws, ln);
     }
     for (int i0 = 0; i0 < nfam; i0 += IT_CHUNK) {
       const int nch = (nfam - i0) < IT_CHUNK ? (nfam - i0) : IT_CHUNK;
@@ -454,7 +480,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           for (int uu = 0; uu < SB; ++uu) {
             const int u = u0 + uu < nch ? u0 + uu : nch - 1;
             const Fam f = fam_get<LEAN, SH>(F, i0 + u);
-            ld(bo[uu], A.leaf_prev ? A.leaf_prev : leaf_beliefs, row_of(f, 1 - f.actor), ln);
+            ld(bo[uu], ranges, row_of(f, 1 - f.actor), ln);
             if (stash) ld(ra[uu], A.reach_avg, row_of(f, f.actor), ln);  // the mix in sweep 2 needs the pre-update value
           }
 #pragma unroll
@@ -478,12 +504,12 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
         if (take_sample) {
           for (int k = 0; k < cnt; ++k) {
             float2 tmp[IT_PPT];
-            ld(tmp, A.policy, first + k, ln);
+            ld(tmp, policy, first + k, ln);
             st(A.policy_sample, first + k, tmp, ln);
           }
         }
         float2 ex[IT_PPT], pos[MAXC][IT_PPT], sum[IT_PPT], wgt[IT_PPT];
-        ld(ex, A.latest, f.p * 2 + actor, ln);
+        ld(ex, latest, f.p * 2 + actor, ln);
         IT_FOR(j) sum[j] = make_float2(0.f, 0.f);
 #pragma unroll
         for (int g0 = 0; g0 < MAXC; g0 += GRP) {
@@ -494,9 +520,9 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
               const int k = g0 + kk;
               if (k < MAXC && k < cnt) {
                 const int64_t c = first + k;
-                ld_masked(ach[kk], A.latest, c * 2 + actor, ln, mask_of(f, k));
-                ld(cu[kk], A.cum, c, ln);
-                ld(ws[kk], A.wsum, c, ln);
+                ld_masked(ach[kk], latest, c * 2 + actor, ln, mask_of(f, k));
+                ld(cu[kk], cum, c, ln);
+                ld(ws[kk], wsum, c, ln);
               }
             }
             if (g0 == 0) {
@@ -536,8 +562,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                   sum[j].x += pos[k][j].x;
                   sum[j].y += pos[k][j].y;
                 }
-                st(A.cum, c, cu[kk], ln);
-                st(A.wsum, c, ws[kk], ln);
+                st(cum, c, cu[kk], ln);
+                st(wsum, c, ws[kk], ln);
               }
             }
           }
@@ -551,7 +577,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
               pol[j].x = p2_matched(pos[k][j].x, sum[j].x, uniform);
               pol[j].y = p2_matched(pos[k][j].y, sum[j].y, uniform);
             }
-            st(A.policy, first + k, pol, ln);
+            st(policy, first + k, pol, ln);
           }
         }
       }
@@ -561,8 +587,14 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
   }
 
   if (A.phases & (PHASE_12 | PHASE_2)) {
+    IterArgsConst& A = iter_args<LEAN>();
     PROF_BEGIN(t_s2);
     // ---------------- sweep 2: reach, beliefs, average policy ----------------
+    float *const reach = A.reach, *const reach_avg = A.reach_avg;
+    float *const beliefs = A.beliefs, *const beliefs_avg = A.beliefs_avg;
+    float *const policy = A.policy, *const policy_avg = A.policy_avg, *const scratch = A.scratch;
+    const float* const reach_avg_prev = A.reach_avg_prev;
+    const bool given_rows = !LEAN || !SH || !A.range_rows || A.whole_rows;
     // (re-reads policy / reach rows that the same lane wrote: no cross-lane hand-off)
     // The root's ranges scale every belief below it.  Where the LDS vectors have four slots to spare
     // next to a family's children they wait there (in this lane's own slots: no barrier) instead of
@@ -573,11 +605,11 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
     const bool bavg_all = !LEAN || enforce_zs, bavg_any = bavg_all || cfr_avg;
     float2 rbk[2][IT_PPT], rbak[2][IT_PPT], ap[IT_PPT];
     uchar2 am[IT_PPT];
-    ld(rbk[0], A.beliefs, r * 2, ln);
-    ld(rbk[1], A.beliefs, r * 2 + 1, ln);
+    ld(rbk[0], beliefs, r * 2, ln);
+    ld(rbk[1], beliefs, r * 2 + 1, ln);
     if (bavg_any) {
-      ld(rbak[0], A.beliefs_avg, r * 2, ln);
-      ld(rbak[1], A.beliefs_avg, r * 2 + 1, ln);
+      ld(rbak[0], beliefs_avg, r * 2, ln);
+      ld(rbak[1], beliefs_avg, r * 2 + 1, ln);
     } else {
       IT_FOR(j) rbak[0][j] = rbak[1][j] = make_float2(0.f, 0.f);
     }
@@ -605,29 +637,29 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // The player who does not act keeps the rows of the parent's range row: a lean iteration stores them
       // again only right under the root (whose own rows are given, not computed) and where a leaf network
       // reads a leaf's two rows side by side.
-      const int opp_all = !LEAN || !SH || !A.range_rows || A.whole_rows || (top && i == 0) ? 0x5555 : 0;
+      const int opp_all = given_rows || (top && i == 0) ? 0x5555 : 0;
       const int opp_rows = opp_all | (f.kinds >> 16);
       const int keep_ba = bavg_all ? 0x5555 : (cfr_avg ? (has_children | leaf_eval) : 0);
       float2 rn[2][IT_PPT], ran[2][IT_PPT], ra_old[IT_PPT];
       float2 cur[MAXC][IT_PPT], pav[MAXC][IT_PPT];
       const int64_t row0 = row_of(f, 0), row1 = row_of(f, 1);
-      ld(rn[0], A.reach, row0, ln);
-      ld(rn[1], A.reach, row1, ln);
+      ld(rn[0], reach, row0, ln);
+      ld(rn[1], reach, row1, ln);
       // the average reach of the player who does not act is only handed on, or normalised into beliefs_avg
       const bool opp_avg = (opp_all | keep_ba) != 0;
-      if (opp_avg || actor == 0) ld(ran[0], A.reach_avg, row0, ln);
+      if (opp_avg || actor == 0) ld(ran[0], reach_avg, row0, ln);
       else IT_FOR(j) ran[0][j] = make_float2(0.f, 0.f);
-      if (opp_avg || actor == 1) ld(ran[1], A.reach_avg, row1, ln);
+      if (opp_avg || actor == 1) ld(ran[1], reach_avg, row1, ln);
       else IT_FOR(j) ran[1][j] = make_float2(0.f, 0.f);
-      if (stash) ld(ra_old, A.scratch, p, ln);
-      else ld(ra_old, A.reach_avg_prev, actor == 0 ? row0 : row1, ln);
+      if (stash) ld(ra_old, scratch, p, ln);
+      else ld(ra_old, reach_avg_prev, actor == 0 ? row0 : row1, ln);
 #pragma unroll
       for (int k = 0; k < MAXC; ++k)
-        if (k < cnt) ld(cur[k], A.policy, first + k, ln);
+        if (k < cnt) ld(cur[k], policy, first + k, ln);
       if (!avg_copy) {
 #pragma unroll
         for (int k = 0; k < MAXC; ++k)
-          if (k < cnt) ld(pav[k], A.policy_avg, first + k, ln);   // the old average; mixed in place below
+          if (k < cnt) ld(pav[k], policy_avg, first + k, ln);   // the old average; mixed in place below
       }
 
       float2 rn_act[IT_PPT];  // new reach of the acting player at the parent
@@ -668,7 +700,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
               if (psum[j].y > 1e-5f) pav[k][j].y = p2_div(pav[k][j].y, fmaxf(psum[j].y, 1e-5f));
             }
           }
-          st(A.policy_avg, first + k, pav[k], ln);
+          st(policy_avg, first + k, pav[k], ln);
         }
       }
       // From here on a child's policy is only needed as its new reach x = reach(actor) * policy
@@ -750,8 +782,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           const int64_t c = first + k;
           float2 xa[IT_PPT];
           from_lds(xa, L.u.vecs[k], ln);
-          st(A.reach, c * 2 + actor, xa, ln);
-          if (opp_all) st(A.reach, c * 2 + 1 - actor, rn_opp, ln);
+          st(reach, c * 2 + actor, xa, ln);
+          if (opp_all) st(reach, c * 2 + 1 - actor, rn_opp, ln);
         }
       }
       // reach_avg
@@ -759,8 +791,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       for (int k = 0; k < MAXC; ++k) {
         if (k < cnt && ((has_children >> (2 * k)) & 1)) {
           const int64_t c = first + k;
-          st(A.reach_avg, c * 2 + actor, pav[k], ln);
-          if (opp_all) st(A.reach_avg, c * 2 + 1 - actor, ran_opp, ln);
+          st(reach_avg, c * 2 + actor, pav[k], ln);
+          if (opp_all) st(reach_avg, c * 2 + 1 - actor, ran_opp, ln);
         }
       }
       // beliefs
@@ -781,8 +813,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
             const float2 vb = mul2(rb_act[j], xa[j]);
             o[j] = sa > 1e-5f ? make_float2(p2_div(vb.x, sa), p2_div(vb.y, sa)) : ap[j];
           }
-          st(A.beliefs, c * 2 + actor, o, ln);
-          if ((opp_rows >> (2 * k)) & 1) st(A.beliefs, c * 2 + 1 - actor, bo, ln);
+          st(beliefs, c * 2 + actor, o, ln);
+          if ((opp_rows >> (2 * k)) & 1) st(beliefs, c * 2 + 1 - actor, bo, ln);
         }
       }
       // beliefs_avg
@@ -796,8 +828,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
             const float2 vba = mul2(rba_act[j], pav[k][j]);
             oa[j] = saa > 1e-5f ? make_float2(p2_div(vba.x, saa), p2_div(vba.y, saa)) : ap[j];
           }
-          st(A.beliefs_avg, c * 2 + actor, oa, ln);
-          if (bavg_all || ((opp_rows >> (2 * k)) & 1)) st(A.beliefs_avg, c * 2 + 1 - actor, boa, ln);
+          st(beliefs_avg, c * 2 + actor, oa, ln);
+          if (bavg_all || ((opp_rows >> (2 * k)) & 1)) st(beliefs_avg, c * 2 + 1 - actor, boa, ln);
         }
       }
     }
@@ -805,6 +837,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
   }
 
   if (A.phases & PHASE_3) {
+    IterArgsConst& A = iter_args<LEAN>();
     // ---------------- sweep 3a: showdown leaves ----------------
     PROF_BEGIN(t_s3);
     const int64_t sd0 = A.root_showdown_offsets[w];
@@ -863,8 +896,12 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
     }
 
     // ---------------- sweep 3b: backup, bottom-up ----------------
+    IterArgsConst& backup = iter_args<LEAN>();
+    float *const policy = backup.policy, *const beliefs = backup.beliefs;
+    float *const latest = backup.latest, *const values_avg = backup.values_avg;
+    const bool whole_rows = backup.whole_rows;
     for (int i = nfam - 1; i >= 0; --i) {
-      if (i < F.base || i >= F.base + 64) fam_load<MAXC, LEAN, SH>(F, A, pp0, nfam, i > 63 ? i - 63 : 0);
+      if (i < F.base || i >= F.base + 64) fam_load<MAXC, LEAN, SH>(F, backup, pp0, nfam, i > 63 ? i - 63 : 0);
       const Fam f = fam_get<LEAN, SH>(F, i);
       const int64_t p = f.p, first = f.first;
       const int cnt = f.cnt, actor = f.actor;
@@ -872,10 +909,10 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
       // actor beliefs at the parent and the marginal of every action, card-summed in one pass
       PROF_BEGIN(t_c3);
       float2 ab[IT_PPT], dn[IT_PPT], polk[MAXC][IT_PPT];
-      ld(ab, A.beliefs, row_of(f, actor), ln);
+      ld(ab, beliefs, row_of(f, actor), ln);
 #pragma unroll
       for (int k = 0; k < MAXC; ++k)
-        if (k < cnt) ld(polk[k], A.policy, first + k, ln);
+        if (k < cnt) ld(polk[k], policy, first + k, ln);
       to_lds(L.u.vecs[0], ab, ln);
 #pragma unroll
       for (int k = 0; k < MAXC; ++k) {
@@ -901,11 +938,11 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
             const int k = g0 + kk < cnt ? g0 + kk : cnt - 1;
             const int64_t c = first + k;
             const int m = mask_of(f, k);
-            ld_masked(v[kk][0], A.latest, c * 2, ln, m);
-            ld_masked(v[kk][1], A.latest, c * 2 + 1, ln, m);
+            ld_masked(v[kk][0], latest, c * 2, ln, m);
+            ld_masked(v[kk][1], latest, c * 2 + 1, ln, m);
             if (update_avg) {
-              ld_masked(av[kk][0], A.values_avg, c * 2, ln, m);
-              ld_masked(av[kk][1], A.values_avg, c * 2 + 1, ln, m);
+              ld_masked(av[kk][0], values_avg, c * 2, ln, m);
+              ld_masked(av[kk][1], values_avg, c * 2 + 1, ln, m);
             }
           }
           if (g0 == 0) {
@@ -927,26 +964,26 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                                                         (av[kk][pl][j].y * mix_old + v[kk][pl][j].y * mix_new) * mix_inv);
                   if (enforce_zs) {
                     float2 ba[IT_PPT];
-                    ld(ba, A.beliefs_avg, c * 2 + pl, ln);
+                    ld(ba, backup.beliefs_avg, c * 2 + pl, ln);
                     IT_FOR(j) s4[0] += av[kk][pl][j].x * ba[j].x + av[kk][pl][j].y * ba[j].y;
                   }
                 }
                 float shift = 0.f;
                 if (enforce_zs) {
                   block_sum4(s4, L.red[0]);
-                  shift = (A.node_flags[c] & NODE_DONE) ? 0.f : 0.5f * s4[0];
+                  shift = (backup.node_flags[c] & NODE_DONE) ? 0.f : 0.5f * s4[0];
                 }
 #pragma unroll
                 for (int pl = 0; pl < 2; ++pl) {
                   IT_FOR(j) av[kk][pl][j] = make_float2(av[kk][pl][j].x - shift, av[kk][pl][j].y - shift);
-                  if (LEAN && !A.whole_rows && mask_of(f, k) == 0) {
+                  if (LEAN && !whole_rows && mask_of(f, k) == 0) {
                     // (the other waves read the pair for nothing: whichever of its two values they see is dropped)
-                    if (threadIdx.x == 0) p2_row2(A.values_avg, c * 2 + pl)[0] = av[kk][pl][0];
+                    if (threadIdx.x == 0) p2_row2(values_avg, c * 2 + pl)[0] = av[kk][pl][0];
                   } else {
                     // Every wave mixes the row's first pair, which the first wave is about to overwrite: all of
                     // them have read it, for both players, before the first of its two rows is stored.
                     if (SH && pl == 0 && mask_of(f, k) == 0) sync_loads();
-                    st(A.values_avg, c * 2 + pl, av[kk][pl], ln);
+                    st(values_avg, c * 2 + pl, av[kk][pl], ln);
                   }
                 }
               }
@@ -974,8 +1011,8 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
           }
         }
       }
-      st(A.latest, p * 2, vp[0], ln);
-      st(A.latest, p * 2 + 1, vp[1], ln);
+      st(latest, p * 2, vp[0], ln);
+      st(latest, p * 2 + 1, vp[1], ln);
       if (i == 0 && update_avg && top) {
         // the root is nobody's child: update its average values here
         float2 nv[2][IT_PPT];
@@ -983,24 +1020,24 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl) {
           float2 av[IT_PPT];
-          ld(av, A.values_avg, p * 2 + pl, ln);
+          ld(av, values_avg, p * 2 + pl, ln);
           IT_FOR(j) nv[pl][j] = make_float2((av[j].x * mix_old + vp[pl][j].x * mix_new) * mix_inv,
                                             (av[j].y * mix_old + vp[pl][j].y * mix_new) * mix_inv);
           if (enforce_zs) {
             float2 ba[IT_PPT];
-            ld(ba, A.beliefs_avg, p * 2 + pl, ln);
+            ld(ba, backup.beliefs_avg, p * 2 + pl, ln);
             IT_FOR(j) s4[0] += nv[pl][j].x * ba[j].x + nv[pl][j].y * ba[j].y;
           }
         }
         float shift = 0.f;
         if (enforce_zs) {
           block_sum4(s4, L.red[0]);
-          shift = (A.node_flags[p] & NODE_DONE) ? 0.f : 0.5f * s4[0];
+          shift = (backup.node_flags[p] & NODE_DONE) ? 0.f : 0.5f * s4[0];
         }
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl) {
           IT_FOR(j) nv[pl][j] = make_float2(nv[pl][j].x - shift, nv[pl][j].y - shift);
-          st(A.values_avg, p * 2 + pl, nv[pl], ln);
+          st(values_avg, p * 2 + pl, nv[pl], ln);
         }
       }
       p2_sync_lds();  // the staged vectors and L.cs are rewritten by the next family
