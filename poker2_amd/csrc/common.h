@@ -180,8 +180,8 @@ __device__ __forceinline__ double p2_block_sum(double v, double* red) {
 // correctly rounded quotient, for divisors from 2^-126 to 2^126, equal to `/` on 1.6e9 random pairs of operands and
 // the special ones.  A dividend below 2^-102 can lose its remainder to rounding, and its quotient then a unit in the
 // last place.  Divisors that several quotients share (a family's sum, a range's mass, the schedule's) are inverted
-// once.  River roots: one, 32 iterations, 4.63 -> 4.45 ms; 192, 16 iterations,
-// 10.2 -> 10.0 ms; 4096, 4 iterations, 43.1 -> 42.2 ms.
+// once.  River roots: one, 32 iterations, 4.63 -> 4.45 ms; 192, eight
+// ordinary iterations, 5.93 -> 5.87, 16 lean ones 10.23 -> 10.16; 4096, 4 iterations, 44.1 -> 44.0.
 __device__ __forceinline__ float p2_recip(float b) {
   const float y = __builtin_amdgcn_rcpf(b);
   return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
