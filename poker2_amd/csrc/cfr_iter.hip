@@ -297,12 +297,6 @@ __device__ __forceinline__ int opaque(int x) {
   return x;
 }
 
-// Workgroup barrier that no wave enters with a load of its own still under way (p2_sync_lds orders LDS traffic only).
-__device__ __forceinline__ void sync_loads() {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-}
-
 __device__ __forceinline__ float2 mul2(float2 a, float2 b) { return make_float2(a.x * b.x, a.y * b.y); }
 
 // A window of 64 consecutive entries of a work item's family list, one per lane: the parent row, the
@@ -982,7 +976,7 @@ __global__ __launch_bounds__(IT_BLOCK, ItTune<MAXC>::min_waves) void cfr_iterati
                   } else {
                     // Every wave mixes the row's first pair, which the first wave is about to overwrite: all of
                     // them have read it, for both players, before the first of its two rows is stored.
-                    if (SH && pl == 0 && mask_of(f, k) == 0) sync_loads();
+                    if (SH && pl == 0 && mask_of(f, k) == 0) p2_sync_loads();
                     st(values_avg, c * 2 + pl, av[kk][pl], ln);
                   }
                 }

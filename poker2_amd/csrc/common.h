@@ -144,6 +144,13 @@ __device__ __forceinline__ void p2_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Workgroup barrier that no wave enters with a load of its own still under way.  It also hands over what was loaded
+// straight into LDS: such loads are counted by vmcnt, and neither p2_sync_lds nor __syncthreads waits for those.
+__device__ __forceinline__ void p2_sync_loads() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 // Block-wide sum of one float per thread; `red` needs >= blockDim/64 floats.
 // All threads get the result.  Contains two barriers.
 template <int NWAVES>

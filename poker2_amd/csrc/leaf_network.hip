@@ -488,15 +488,15 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void ln_gemm_kernel(LnGemm g) {
   fetch(buf0, 0);
   int kb = 0;
   for (; kb + 2 <= g.blocks; kb += 2) {
-    __syncthreads();                                       // block kb is there, and everyone is done with buf1
+    p2_sync_loads();                                       // block kb is there, and everyone is done with buf1
     fetch(buf1, kb + 1);
     multiply(buf0);
-    __syncthreads();
+    p2_sync_loads();
     fetch(buf0, kb + 2 < g.blocks ? kb + 2 : kb + 1);      // past the end: a block nobody uses
     multiply(buf1);
     if ((kb & 6) == 6) carry();
   }
-  __syncthreads();
+  p2_sync_loads();
   if (kb < g.blocks) multiply(buf0);
   carry();
 
@@ -758,19 +758,19 @@ __global__ __launch_bounds__(LN_FIRST_THREADS, 4) void ln_first_kernel(LnFirst g
     }
     const int next = c + 1 < c1 ? c + 1 : c;
     static_assert(LN_CARD_BLOCKS == 4, "a card is two rounds of the two buffers");
-    __syncthreads();
+    p2_sync_loads();
     fetch(buf1, c, off_a, 1);
     multiply(buf0);
-    __syncthreads();
+    p2_sync_loads();
     fetch(buf0, c, off_a, 2);
     const uint32_t off_next = sample_of(next);
 #pragma unroll
     for (int i = 0; i < TM; ++i) wt[i] = row[i] >= 0 ? g.weight[row[i]] : make_float2(0.f, 0.f);
     multiply(buf1);
-    __syncthreads();
+    p2_sync_loads();
     fetch(buf1, c, off_a, 3);
     multiply(buf0);
-    __syncthreads();
+    p2_sync_loads();
     off_a = off_next;
     fetch(buf0, next, off_a, 0);
     multiply(buf1);
@@ -798,7 +798,7 @@ __global__ __launch_bounds__(LN_FIRST_THREADS, 4) void ln_first_kernel(LnFirst g
       }
     }
   }
-  __syncthreads();                                         // the last fetch has landed before the LDS is given back
+  p2_sync_loads();                                         // the last fetch has landed before the LDS is given back
 }
 
 // The samples whose first layer is taken whole: those of `whole` (a device count of them).  Four at a time their input
