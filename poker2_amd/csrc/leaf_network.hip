@@ -86,32 +86,96 @@ __device__ __forceinline__ float ln_block_max(float v, float* red) {
 }
 
 // ---- weights ------------------------------------------------------------------------------------
-// One workgroup per row of weights, all layers in one launch, and a few more that clear the maxima kept below.
-// A row n of the first layer [width, 2704] is cut up the way its products need it, all of it under one scale:
+// Two networks are the same function if a hidden unit's weights and bias are divided by a power of two u and the column
+// that reads it is multiplied by u.  The network is computed as the one whose units all answer with about 1: a row of
+// answers has ONE scale, and a unit far below the largest would lose its low bits to float16's smallest number (with
+// units 2^N(0, 4) apart, 3 x 768: 8e-2 off, like this 4.4e-8 as with units of one size).  u is the power of two below
+// sqrt(sum of absolute weights x largest) + |bias|, which lies between the weights' 2-norm and their sum: in the first layer
+// the largest weight + |bias|.  A unit that is always 0 gets the smallest u, so that what reads it sets no row's scale.
+// A layer's weights are therefore prepared behind those of the layer in front of it.
+__device__ __forceinline__ float ln_unit(float size) {
+  int e = (int)((__builtin_bit_cast(uint32_t, size) >> 23) & 255u) - 127;
+  e = e > 96 ? 96 : (e < -96 ? -96 : e);
+  return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+}
+__device__ __forceinline__ float ln_inverse(float power_of_two) {
+  return __builtin_bit_cast(float, 0x7F000000u - __builtin_bit_cast(uint32_t, power_of_two));
+}
+
+// A layer as its product needs it, a workgroup per row.  `inv`, `bias` and `bound` are those of the answers in units of u;
+// `bound` is what an answer can reach for inputs of at most 1, without the bias (the sum of absolute weights).
+struct LnLayerWeights {
+  const float *w, *b;          // as given; b: none if the layer has no bias
+  const float* column_unit;    // u of the units that the layer reads
+  char* out;                   // split rows
+  float *inv, *bound, *bias, *unit;
+  int columns, hidden;         // the last layer's answers are not `hidden`: u = 1
+};
+__global__ __launch_bounds__(LN_THREADS) void ln_weights_kernel(LnLayerWeights a) {
+  __shared__ float red[LN_THREADS / 64];
+  __shared__ float red_sum[LN_THREADS / 64];
+  const int64_t r = blockIdx.x;
+  const int units = a.columns / 8;                        // columns are a multiple of 32
+  const float4* src = reinterpret_cast<const float4*>(a.w + r * a.columns);
+  const float4* of = reinterpret_cast<const float4*>(a.column_unit);
+  auto load = [&](int u) {
+    const float4 v = src[u], c = of[u];
+    return make_float4(v.x * c.x, v.y * c.y, v.z * c.z, v.w * c.w);
+  };
+  float mx = 0.f, l1 = 0.f;
+  for (int u = threadIdx.x; u < units; u += LN_THREADS)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const float4 v = load(2 * u + q);
+      mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+      l1 += (fabsf(v.x) + fabsf(v.y)) + (fabsf(v.z) + fabsf(v.w));
+    }
+  l1 = p2_wave_sum(l1);
+  if ((threadIdx.x & 63) == 0) red_sum[threadIdx.x >> 6] = l1;
+  mx = ln_block_max(mx, red);
+  const LnScale s = ln_scale(mx);
+  if (threadIdx.x == 0) {
+    const float sum = (red_sum[0] + red_sum[1]) + (red_sum[2] + red_sum[3]), b = a.b ? a.b[r] : 0.f;
+    const float unit = a.hidden ? ln_unit(sqrtf(sum) * sqrtf(mx) + fabsf(b)) : 1.0f, down = ln_inverse(unit);
+    a.inv[r] = s.down * down;
+    a.bound[r] = sum * down;
+    a.bias[r] = b * down;
+    a.unit[r] = unit;
+  }
+  char* out = a.out + r * (units / 4) * (int64_t)LN_BLOCK_BYTES;
+  for (int u = threadIdx.x; u < units; u += LN_THREADS) {
+    const float4 v = load(2 * u), w = load(2 * u + 1);
+    const float y[8] = {v.x * s.up, v.y * s.up, v.z * s.up, v.w * s.up, w.x * s.up, w.y * s.up, w.z * s.up, w.w * s.up};
+    ln_store8(out, 8 * u, y);
+  }
+}
+
+// The first layer [width, 2704], a row cut up the way its products need it, all of it under one scale:
 //   ranges  [2][width] split rows of 1326 columns, a player each;
 //   cards   [52][width] split rows of 103 columns: the hands of player 0, then of player 1, that hold the card (in the
 //           order of the partner card), then the card's own board column;
-//   board   [52][width] float: the board columns.
-// `bound`: per row what its answer can reach for inputs of at most 1 (the sum of absolute weights).  In the first layer
-// a sample's ranges add up to 1 each and its board holds at most five cards: seven times the largest weight.
-struct LnLayerWeights {
-  const float* w;
-  char* out;             // split rows (not for the first layer)
-  float *inv, *bound;    // [rows]
-  int columns, first_block;
-};
-struct LnWeights {
-  LnLayerWeights layer[LN_MAX_LAYERS];
+//   board   [52][width] float: the board columns, in units of u.
+// `bound`: a sample's ranges add up to 1 each and its board holds at most five cards, seven times the largest weight.
+// A few more workgroups clear the maxima that are kept below.
+struct LnFirstWeights {
+  LnLayerWeights layer;        // without `out`, `column_unit`
   char *ranges, *cards;
   float* board;
   uint4* clear;
   int64_t clear_units;
-  int layers, width, clear_blocks;     // `width` of the first layer
+  int width, clear_blocks;
 };
-
-__device__ __forceinline__ void ln_first_weights(const LnWeights& a, int64_t n, float* row, float* red) {
-  const int64_t width = a.width;
-  const float4* src = reinterpret_cast<const float4*>(a.layer[0].w + n * LN_INPUT);
+__global__ __launch_bounds__(LN_THREADS) void ln_first_weights_kernel(LnFirstWeights a) {
+  __shared__ __align__(16) float row[LN_INPUT];
+  __shared__ float red[LN_THREADS / 64];
+  if ((int)blockIdx.x >= a.width) {
+    for (int64_t k = (int64_t)((int)blockIdx.x - a.width) * LN_THREADS + threadIdx.x; k < a.clear_units;
+         k += (int64_t)a.clear_blocks * LN_THREADS)
+      a.clear[k] = make_uint4(0u, 0u, 0u, 0u);
+    return;
+  }
+  const int64_t n = blockIdx.x, width = a.width;
+  const float4* src = reinterpret_cast<const float4*>(a.layer.w + n * LN_INPUT);
   float mx = 0.f;
   for (int k = threadIdx.x; k < LN_INPUT / 4; k += LN_THREADS) {
     const float4 v = src[k];
@@ -120,9 +184,12 @@ __device__ __forceinline__ void ln_first_weights(const LnWeights& a, int64_t n, 
   }
   mx = ln_block_max(mx, red);                             // its barriers cover `row` too
   const LnScale s = ln_scale(mx);
+  const float b = a.layer.b ? a.layer.b[n] : 0.f, unit = ln_unit(mx + fabsf(b)), down = ln_inverse(unit);
   if (threadIdx.x == 0) {
-    a.layer[0].inv[n] = s.down;
-    a.layer[0].bound[n] = 7.f * mx;
+    a.layer.inv[n] = s.down * down;
+    a.layer.bound[n] = 7.f * (mx * down);
+    a.layer.bias[n] = b * down;
+    a.layer.unit[n] = unit;
   }
   for (int u = threadIdx.x; u < 2 * LN_RANGE_BLOCKS * 4; u += LN_THREADS) {
     const int p = u / (LN_RANGE_BLOCKS * 4), f = 8 * (u - p * (LN_RANGE_BLOCKS * 4));
@@ -144,51 +211,7 @@ __device__ __forceinline__ void ln_first_weights(const LnWeights& a, int64_t n, 
     }
     ln_store8(a.cards + (c * width + n) * (LN_CARD_BLOCKS * LN_BLOCK_BYTES), f, y);
   }
-  if (threadIdx.x < P2_CARDS) a.board[threadIdx.x * width + n] = row[2 * P2_H + threadIdx.x];
-}
-
-__global__ __launch_bounds__(LN_THREADS) void ln_weights_kernel(LnWeights a) {
-  __shared__ __align__(16) float row[LN_INPUT];
-  __shared__ float red[LN_THREADS / 64];
-  __shared__ float red_sum[LN_THREADS / 64];
-  if ((int)blockIdx.x < a.width) {
-    ln_first_weights(a, blockIdx.x, row, red);
-    return;
-  }
-  const int cleared = (int)gridDim.x - a.clear_blocks;
-  if ((int)blockIdx.x >= cleared) {
-    for (int64_t k = (int64_t)(blockIdx.x - cleared) * LN_THREADS + threadIdx.x; k < a.clear_units;
-         k += (int64_t)a.clear_blocks * LN_THREADS)
-      a.clear[k] = make_uint4(0u, 0u, 0u, 0u);
-    return;
-  }
-  int l = 1;
-  while (l + 1 < a.layers && (int)blockIdx.x >= a.layer[l + 1].first_block) ++l;
-  const int64_t r = (int)blockIdx.x - a.layer[l].first_block;
-  const int units = a.layer[l].columns / 8;               // columns are a multiple of 32
-  const float4* src = reinterpret_cast<const float4*>(a.layer[l].w + r * a.layer[l].columns);
-  float mx = 0.f, l1 = 0.f;
-  for (int u = threadIdx.x; u < units; u += LN_THREADS)
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const float4 v = src[2 * u + q];
-      mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
-      l1 += (fabsf(v.x) + fabsf(v.y)) + (fabsf(v.z) + fabsf(v.w));
-    }
-  l1 = p2_wave_sum(l1);
-  if ((threadIdx.x & 63) == 0) red_sum[threadIdx.x >> 6] = l1;
-  mx = ln_block_max(mx, red);
-  const LnScale s = ln_scale(mx);
-  if (threadIdx.x == 0) {
-    a.layer[l].inv[r] = s.down;
-    a.layer[l].bound[r] = (red_sum[0] + red_sum[1]) + (red_sum[2] + red_sum[3]);
-  }
-  char* out = a.layer[l].out + r * (units / 4) * (int64_t)LN_BLOCK_BYTES;
-  for (int u = threadIdx.x; u < units; u += LN_THREADS) {
-    const float4 v = src[2 * u], w = src[2 * u + 1];
-    const float y[8] = {v.x * s.up, v.y * s.up, v.z * s.up, v.w * s.up, w.x * s.up, w.y * s.up, w.z * s.up, w.w * s.up};
-    ln_store8(out, 8 * u, y);
-  }
+  if (threadIdx.x < P2_CARDS) a.board[threadIdx.x * width + n] = row[2 * P2_H + threadIdx.x] * down;
 }
 
 // What is known of a sample.  `inv`: 1 / the mass left to a player, 0 where the uniform range takes its place.
@@ -311,7 +334,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_states_kernel(
 // Workgroup l of the first `layers`: stats[2 l], stats[2 l + 1] = the largest bound and bias of layer l.  The others, a
 // state each: base[i][n] = the first layer's bias + the columns of the cards on the state's board.
 struct LnBounds {
-  const float *bound[LN_MAX_LAYERS], *bias[LN_MAX_LAYERS];
+  const float *bound[LN_MAX_LAYERS], *bias[LN_MAX_LAYERS];   // in units of u
   int rows[LN_MAX_LAYERS];
 };
 __global__ __launch_bounds__(LN_THREADS) void ln_base_kernel(LnBounds bounds, int layers, float* __restrict__ stats,
@@ -326,7 +349,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_base_kernel(LnBounds bounds, in
     float m = 0.f, b = 0.f;
     for (int k = threadIdx.x; k < bounds.rows[l]; k += LN_THREADS) {
       m = fmaxf(m, bound[k]);
-      if (bias) b = fmaxf(b, fabsf(bias[k]));
+      b = fmaxf(b, fabsf(bias[k]));
     }
     m = ln_block_max(m, red);
     b = ln_block_max(b, red);
@@ -339,7 +362,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_base_kernel(LnBounds bounds, in
   uint64_t bits = 0;
   if (root >= 0 && root < source_rows) chance_board(board + root * 5, bcards, bits);
   for (int k = threadIdx.x; k < width; k += LN_THREADS) {
-    float v = bounds.bias[0] ? bounds.bias[0][k] : 0.f;
+    float v = bounds.bias[0][k];
     for (uint64_t b = bits; b; b &= b - 1) v += columns[(__ffsll((unsigned long long)b) - 1) * width + k];
     base[i * width + k] = v;
   }
@@ -810,8 +833,8 @@ constexpr int LN_WHOLE = 4, LN_WHOLE_GRID = 64, LN_WHOLE_COLS = 64;
 __global__ __launch_bounds__(LN_THREADS) void ln_whole_samples_kernel(
     const float* __restrict__ pre_beliefs, const int64_t* __restrict__ root_indices, const int64_t* __restrict__ board,
     int64_t source_rows, const LnSample* __restrict__ samples, const int32_t* __restrict__ whole,
-    const int32_t* __restrict__ whole_count, const float* __restrict__ w, const float* __restrict__ bias, int width,
-    const float* __restrict__ stats, char* __restrict__ out_split, float* __restrict__ out_inv) {
+    const int32_t* __restrict__ whole_count, const float* __restrict__ w, const float* __restrict__ bias,
+    const float* __restrict__ unit, int width, const float* __restrict__ stats, char* __restrict__ out_split, float* __restrict__ out_inv) {
   __shared__ __align__(16) float x[LN_WHOLE][LN_INPUT];
   const int count = *whole_count, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const LnScale scale = ln_scale(stats[0] + stats[1]);
@@ -856,7 +879,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_whole_samples_kernel(
       }
 #pragma unroll
       for (int k = 0; k < LN_WHOLE; ++k) {
-        const float v = ln_relu(p2_wave_sum(acc[k]) + (bias ? bias[n] : 0.f));
+        const float v = ln_relu(p2_wave_sum(acc[k]) * ln_inverse(unit[n]) + bias[n]);
         if (lane == k && first + k < count) {
           _Float16 h, l;
           ln_split(v * scale.up, h, l);
@@ -946,7 +969,7 @@ struct LnPlan {
   float* out_max[2];                       // these two and the count are cleared first, one run
   int32_t* whole_count;
   int64_t cleared;
-  float *stats, *w_inv[LN_MAX_LAYERS], *w_bound[LN_MAX_LAYERS];
+  float *stats, *w_inv[LN_MAX_LAYERS], *w_bound[LN_MAX_LAYERS], *bias[LN_MAX_LAYERS], *unit[LN_MAX_LAYERS];
   char *first_ranges, *first_cards, *weights[LN_MAX_LAYERS];
   float *first_board, *products, *base;
   char *ranges, *gone, *hidden[2], *means;
@@ -971,6 +994,8 @@ static LnPlan ln_plan(void* base, int64_t states, int64_t samples, const int32_t
   for (int l = 0; l < layers; ++l) {
     p.w_inv[l] = w.take<float>(widths[l]);
     p.w_bound[l] = w.take<float>(widths[l]);
+    p.bias[l] = w.take<float>(widths[l]);
+    p.unit[l] = w.take<float>(widths[l]);
     p.weights[l] = l ? w.take<char>((int64_t)widths[l] * (widths[l - 1] / 32) * LN_BLOCK_BYTES) : nullptr;
   }
   for (int k = 0; k < 2; ++k) {
@@ -1050,17 +1075,21 @@ int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, 
   hipStream_t s = (hipStream_t)stream;
   const int w0 = widths[0];
   {
-    LnWeights a = {};
-    int blocks = 0;
+    LnFirstWeights a = {};
     for (int l = 0; l < layers; ++l) {
-      a.layer[l] = LnLayerWeights{weights[l], p.weights[l], p.w_inv[l], p.w_bound[l], l ? (int)widths[l - 1] : LN_INPUT, blocks};
-      blocks += widths[l];
+      const LnLayerWeights g = {weights[l], biases[l], l ? p.unit[l - 1] : nullptr, p.weights[l], p.w_inv[l], p.w_bound[l],
+                                p.bias[l], p.unit[l], l ? (int)widths[l - 1] : LN_INPUT, l + 1 < layers};
+      if (l == 0) {
+        a.layer = g;
+        a.ranges = p.first_ranges; a.cards = p.first_cards; a.board = p.first_board;
+        a.clear = (uint4*)workspace; a.clear_units = p.cleared / 16;
+        a.width = w0; a.clear_blocks = (int)ln_clear_grid(a.clear_units);
+        hipLaunchKernelGGL(ln_first_weights_kernel, dim3((unsigned)(w0 + a.clear_blocks)), dim3(LN_THREADS), 0, s, a);
+      } else {
+        hipLaunchKernelGGL(ln_weights_kernel, dim3((unsigned)widths[l]), dim3(LN_THREADS), 0, s, g);
+      }
+      P2_LAUNCH_CHECK();
     }
-    a.ranges = p.first_ranges; a.cards = p.first_cards; a.board = p.first_board;
-    a.clear = (uint4*)workspace; a.clear_units = p.cleared / 16;
-    a.layers = layers; a.width = w0; a.clear_blocks = (int)ln_clear_grid(a.clear_units);
-    hipLaunchKernelGGL(ln_weights_kernel, dim3((unsigned)(blocks + a.clear_blocks)), dim3(LN_THREADS), 0, s, a);
-    P2_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(ln_states_kernel, dim3((unsigned)n), dim3(LN_THREADS), 0, s, pre_beliefs, root_indices, board,
                      sample_offsets, source_rows, total_samples, p.ranges, p.ranges_inv, p.gone, p.weight, p.samples,
@@ -1068,7 +1097,7 @@ int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, 
   P2_LAUNCH_CHECK();
   {
     LnBounds b = {};
-    for (int l = 0; l < layers; ++l) { b.bound[l] = p.w_bound[l]; b.bias[l] = biases[l]; b.rows[l] = widths[l]; }
+    for (int l = 0; l < layers; ++l) { b.bound[l] = p.w_bound[l]; b.bias[l] = p.bias[l]; b.rows[l] = widths[l]; }
     hipLaunchKernelGGL(ln_base_kernel, dim3((unsigned)(layers + n)), dim3(LN_THREADS), 0, s, b, layers, p.stats,
                        root_indices, board, source_rows, p.first_board, w0, p.base);
     P2_LAUNCH_CHECK();
@@ -1093,13 +1122,13 @@ int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, 
     P2_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(ln_whole_samples_kernel, dim3(LN_WHOLE_GRID, (unsigned)((w0 + LN_WHOLE_COLS - 1) / LN_WHOLE_COLS)), dim3(LN_THREADS), 0, s, pre_beliefs, root_indices,
-                     board, source_rows, p.samples, p.whole, p.whole_count, weights[0], biases[0], w0, p.stats,
+                     board, source_rows, p.samples, p.whole, p.whole_count, weights[0], p.bias[0], p.unit[0], w0, p.stats,
                      p.hidden[0], p.hidden_inv[0]);
   P2_LAUNCH_CHECK();
   for (int l = 1; l + 1 < layers; ++l) {
     const int in = (l - 1) & 1, out = l & 1;
     LnGemm g = {};
-    g.a = p.hidden[in]; g.b = p.weights[l]; g.a_inv = p.hidden_inv[in]; g.b_inv = p.w_inv[l]; g.bias = biases[l];
+    g.a = p.hidden[in]; g.b = p.weights[l]; g.a_inv = p.hidden_inv[in]; g.b_inv = p.w_inv[l]; g.bias = p.bias[l];
     g.m = total_samples; g.n = widths[l]; g.blocks = widths[l - 1] / 32; g.batches = 1;
     if (l + 2 < layers) {
       const bool measured = l + 3 < layers;                // the hidden layer after this one needs a bound on its answer
@@ -1121,7 +1150,7 @@ int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, 
   }
   LnGemm g = {};
   const int l = layers - 1;
-  g.a = p.means; g.b = p.weights[l]; g.a_inv = p.means_inv; g.b_inv = p.w_inv[l]; g.bias = biases[l];
+  g.a = p.means; g.b = p.weights[l]; g.a_inv = p.means_inv; g.b_inv = p.w_inv[l]; g.bias = p.bias[l];
   g.m = n; g.n = widths[l]; g.blocks = widths[l - 1] / 32; g.batches = 1; g.out = expected;
   return ln_launch<LN_PLAIN>(g, s);
 }

@@ -104,6 +104,41 @@ def test_matches_float64(hidden, layers, n, kind, on_board, bias):
     assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -22 * len(stack)
 
 
+def rescale_units(net, kind):
+    """The same function with hidden units that answer in other sizes: what they are multiplied by is taken out of the
+    columns that read them."""
+    gen = torch.Generator().manual_seed(11)
+    with torch.no_grad():
+        for lin, reader in zip(net.linears[:-1], net.linears[1:]):
+            power = torch.zeros(lin.weight.shape[0])
+            if kind == "all":
+                power = (torch.randn(power.shape, generator=gen) * 6).round()
+            elif kind == "dead":                        # a unit that is always 0, with outgoing weights out of proportion
+                lin.weight[3], lin.bias[3] = 0.0, 0.0
+                reader.weight[:, 3] *= 2.0 ** 30
+            else:
+                power[5] = kind
+            up = torch.exp2(power).to(lin.weight)
+            lin.weight.mul_(up[:, None])
+            lin.bias.mul_(up)
+            reader.weight.div_(up)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ranges", ["gamma", "one hand"])
+@pytest.mark.parametrize("kind", [8, 12, 16, 20, 24, 40, -30, "all", "dead"])
+def test_units_of_unequal_size(kind, ranges):
+    """As close as with units of one size (``test_matches_float64``), which is as close as float32 products are."""
+    net = make_net(320, 4)
+    rescale_units(net, kind)
+    pre, boards = make_inputs(3, ranges, seed=21, on_board=4)
+    with torch.no_grad():
+        got = K.chance_network(pre, torch.arange(3).cuda(), boards, K.network_layers(net, pre.device), 4)
+        want, tol = reference(net, pre, boards)
+    assert bool(((got.double() - want).abs() <= tol).all())
+    assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -22 * len(net.linears)
+
+
 @pytest.mark.gpu
 def test_256_row_tiles_and_a_selection_of_rows():
     """Enough samples for the largest tiles (4 per CU), taken from a table through ``root_indices``; a few states of it
