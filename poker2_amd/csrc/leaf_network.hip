@@ -214,7 +214,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_first_weights_kernel(LnFirstWei
   if (threadIdx.x < P2_CARDS) a.board[threadIdx.x * width + n] = row[2 * P2_H + threadIdx.x] * down;
 }
 
-// What is known of a sample.  `inv`: 1 / the mass left to a player, 0 where the uniform range takes its place.
+// What is known of a sample.  `inv`: 1 / the mass left to a player, -1 where the uniform range takes its place.
 struct LnSample {
   float inv0, inv1;
   int32_t state;   // among the call's states
@@ -222,7 +222,7 @@ struct LnSample {
 };
 
 // A player's hands with the dealt card may hold nearly all of his mass.  T minus their share would then cancel: above
-// this share the sample is taken whole (`ln_whole_samples_kernel`), at most seven cards per player.
+// this share the sample is taken whole (`ln_whole_kernel`), at most seven cards per player.
 constexpr double LN_HEAVY_SHARE = 0.25;
 
 // One workgroup per state: the ranges without the board's hands as split rows [2][states], and for each of its samples
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_states_kernel(
       for (int p = 0; p < 2; ++p) {
         const float sum = (float)(total[p] - cs[p * P2_CARDS + c]);
         const bool ok = sum > 1e-12f;
-        inv[p] = ok ? 1.0f / fmaxf(sum, 1e-12f) : 0.f;
+        inv[p] = ok ? 1.0f / fmaxf(sum, 1e-12f) : -1.0f;
         // (negated, so that a NaN makes the sample a whole one)
         heavy = heavy || (!empty[p] && !(ok && cs[p * P2_CARDS + c] <= LN_HEAVY_SHARE * total[p]));
         (p ? wt.y : wt.x) = empty[p] ? uniform : inv[p];
@@ -824,73 +824,203 @@ __global__ __launch_bounds__(LN_FIRST_THREADS, 4) void ln_first_kernel(LnFirst g
   p2_sync_loads();                                         // the last fetch has landed before the LDS is given back
 }
 
-// The samples whose first layer is taken whole: those of `whole` (a device count of them).  Four at a time their input
-// rows lie in LDS and every wave takes a row of the weights; float32 throughout.  Runs behind the product that wrote
-// the same rows of `out_split` from zero weights.  Ranges of one hand each, 4 of 48 samples to be taken whole: 35 states
-// 1.91 ms a call with all columns in one workgroup, 0.42 with 64 (0.21 without such samples); 2240 states 16.0 and
-// 15.3 (3.4).  Without any the launch takes 5 us.
-constexpr int LN_WHOLE = 4, LN_WHOLE_GRID = 64, LN_WHOLE_COLS = 64;
-__global__ __launch_bounds__(LN_THREADS) void ln_whole_samples_kernel(
-    const float* __restrict__ pre_beliefs, const int64_t* __restrict__ root_indices, const int64_t* __restrict__ board,
-    int64_t source_rows, const LnSample* __restrict__ samples, const int32_t* __restrict__ whole,
-    const int32_t* __restrict__ whole_count, const float* __restrict__ w, const float* __restrict__ bias,
-    const float* __restrict__ unit, int width, const float* __restrict__ stats, char* __restrict__ out_split, float* __restrict__ out_inv) {
-  __shared__ __align__(16) float x[LN_WHOLE][LN_INPUT];
-  const int count = *whole_count, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const LnScale scale = ln_scale(stats[0] + stats[1]);
-  const int n0 = blockIdx.y * LN_WHOLE_COLS, n1 = n0 + LN_WHOLE_COLS < width ? n0 + LN_WHOLE_COLS : width;
-  for (int first = blockIdx.x * LN_WHOLE; first < count; first += LN_WHOLE_GRID * LN_WHOLE) {
-    __syncthreads();
-    for (int k = 0; k < LN_WHOLE; ++k) {
-      LnSample sm = {0.f, 0.f, 0, -1};
-      if (first + k < count) sm = samples[whole[first + k]];
-      const int64_t root = root_indices ? root_indices[sm.state] : sm.state;
-      int bcards[5];
-      uint64_t bits = 0;
-      const bool dealt = sm.card >= 0 && root >= 0 && root < source_rows;
-      const int ncards = dealt ? chance_board(board + root * 5, bcards, bits) : 5;
-      const int left = P2_CARDS - ncards - 1;
-      const float uniform = 1.0f / fmaxf((float)(left * (left - 1) / 2), 1.0f);
-      const uint64_t gone = dealt ? bits | (1ull << sm.card) : 0ull;
-      for (int j = threadIdx.x; j < LN_INPUT; j += LN_THREADS) {
-        float v = 0.f;
-        if (dealt && j < 2 * P2_H) {
-          const int p = j >= P2_H, h = j - p * P2_H;
-          const float inv = p ? sm.inv1 : sm.inv0;
-          if (!(((gone >> p2_combo.a[h]) | (gone >> p2_combo.b[h])) & 1ull))
-            v = inv == 0.f ? uniform : pre_beliefs[root * (2 * P2_H) + j] * inv;
-        } else if (dealt) {
-          v = ((gone >> (j - 2 * P2_H)) & 1ull) ? 1.f : 0.f;
-        }
-        x[k][j] = v;
+// The samples whose first layer is taken whole: those of `whole` (a device count of them).  Their ranges are masked,
+// normalised and split on the way into LDS, 64 samples against 128 columns a tile, and multiplied by the ranges' columns
+// as LN_PLAIN does; the board's columns come from `base` and `columns`.  Runs behind ln_first_kernel, which wrote the
+// same rows of `out_split` from zero weights.  A fixed number of workgroups takes the tiles in turn, each XCD a run of
+// them, columns outermost, so that it keeps its columns' weights in its L2.
+// 3 x 1536, ms a call, float32 on the vector units (four samples at a time) -> here: 2240 states with three hands per
+// range (up to 12 of 48 samples whole) 21.4 -> 5.1, with one hand 9.8 -> 4.2, smooth ranges 3.7 -> 3.6; 35 states with three
+// hands 0.66 -> 0.39.  The network layer by layer: 20.6 and 0.56.  Bound: for few samples the 84 steps, one after the other,
+// 0.1 ms; for many the splitting, which the vector units do again for every stripe of columns.
+struct LnWhole {
+  const float* pre_beliefs;
+  const int64_t *root_indices, *board;
+  int64_t source_rows;
+  const LnSample* samples;
+  const int32_t *whole, *whole_count;
+  const char* ranges;           // [2][width] split rows
+  const float *b_inv, *bias, *base, *columns, *stats;
+  int width;
+  char* out_split;
+  float* out_inv;
+};
+constexpr int LN_WHOLE_ROWS = 64, LN_WHOLE_COLS = 128, LN_WHOLE_THREADS = 512, LN_WHOLE_GRID = 512;
+__global__ __launch_bounds__(LN_WHOLE_THREADS, 4) void ln_whole_kernel(LnWhole g) {
+  constexpr int TM = 2, TN = 2, BM = LN_WHOLE_ROWS, BN = LN_WHOLE_COLS, STEPS = 2 * LN_RANGE_BLOCKS;
+  static_assert(STEPS % 2 == 0, "steps in pairs, a buffer each");
+  __shared__ __align__(128) char buf0[(BM + BN) * LN_BLOCK_BYTES];
+  __shared__ __align__(128) char buf1[(BM + BN) * LN_BLOCK_BYTES];
+  const int count = *g.whole_count;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 2, wn = wave & 3;                 // waves 2 x 4, 32 x 32 each
+  const int fr = lane & 15, fq = lane >> 4, turn = (fr >> 1) & 7;
+  const LnScale scale = ln_scale(g.stats[0] + g.stats[1]);
+  const int64_t row_bytes = LN_RANGE_BLOCKS * LN_BLOCK_BYTES, out_bytes = (int64_t)(g.width / 32) * LN_BLOCK_BYTES;
+  const unsigned tiles_m = (unsigned)((count + BM - 1) / BM), tiles_n = (unsigned)((g.width + BN - 1) / BN);
+  const unsigned tiles = tiles_m * tiles_n, xcd = blockIdx.x & 7, per = tiles >> 3, more = tiles & 7;
+  const unsigned mine = per + (xcd < more ? 1 : 0), start = xcd * per + (xcd < more ? xcd : more);
+  for (unsigned turn_of = blockIdx.x >> 3; turn_of < mine; turn_of += gridDim.x >> 3) {
+    const unsigned tile = start + turn_of, tm = tile % tiles_m, tn = tile / tiles_m;
+    const int m0 = (int)tm * BM, n0 = (int)tn * BN;
+    const int cols_left = g.width - n0 < BN ? g.width - n0 : BN;
+
+    // this thread's part of the samples: row threadIdx.x / 8, four hands of every block
+    const int a_row = threadIdx.x >> 3, a_col = (threadIdx.x & 7) * 4;
+    const float* range = g.stats;                          // (of an input of zeros: one number, not used)
+    bool dealt = false;
+    float inv[2] = {0.f, 0.f}, uniform = 0.f;
+    uint64_t gone = 0;
+    if (m0 + a_row < count) {
+      const LnSample sm = g.samples[g.whole[m0 + a_row]];
+      const int64_t root = g.root_indices ? g.root_indices[sm.state] : sm.state;
+      if (sm.card >= 0 && root >= 0 && root < g.source_rows) {
+        int bcards[5];
+        const int left = P2_CARDS - chance_board(g.board + root * 5, bcards, gone) - 1;
+        gone |= 1ull << sm.card;
+        uniform = 1.0f / fmaxf((float)(left * (left - 1) / 2), 1.0f);
+        range = g.pre_beliefs + root * (2 * P2_H);
+        dealt = true;
+        inv[0] = sm.inv0;
+        inv[1] = sm.inv1;
       }
     }
-    __syncthreads();
-    for (int n = n0 + wave; n < n1; n += LN_THREADS / 64) {
-      float acc[LN_WHOLE] = {};
-      const float4* row = reinterpret_cast<const float4*>(w + (int64_t)n * LN_INPUT);
-      for (int j = lane; j < LN_INPUT / 4; j += 64) {
-        const float4 c = row[j];
+    float x[4];
+    uint32_t ca[4], cb[4];                                 // the hands' cards
+    auto load = [&](int step) {
+      const int p = step >= LN_RANGE_BLOCKS, h = (step - p * LN_RANGE_BLOCKS) * 32 + a_col;
 #pragma unroll
-        for (int k = 0; k < LN_WHOLE; ++k) {
-          const float4 y = reinterpret_cast<const float4*>(x[k])[j];
-          acc[k] = fmaf(c.x, y.x, fmaf(c.y, y.y, fmaf(c.z, y.z, fmaf(c.w, y.w, acc[k]))));
-        }
+      for (int e = 0; e < 4; ++e) {
+        const int hand = h + e < P2_H ? h + e : 0;         // (selected, not branched on: the loads go out together)
+        ca[e] = p2_combo.a[hand];
+        cb[e] = p2_combo.b[hand];
+        x[e] = range[dealt ? p * P2_H + hand : 0];
+      }
+    };
+    auto store = [&](char* buf, int step) {
+      const int p = step >= LN_RANGE_BLOCKS, h = (step - p * LN_RANGE_BLOCKS) * 32 + a_col;
+      const float scaled = p ? inv[1] : inv[0];
+      ln_half4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool off = (((gone >> ca[e]) | (gone >> cb[e])) & 1ull) | !dealt | (h + e >= P2_H);
+        const float v = off ? 0.f : (scaled < 0.f ? uniform : x[e] * scaled);
+        _Float16 a, b;
+        ln_split(v * LN_SAMPLE_SCALE, a, b);
+        hi[e] = a;
+        lo[e] = b;
+      }
+      char* row = buf + a_row * LN_BLOCK_BYTES;
+      const int chunk = a_col >> 3, half = (a_col & 4) * 2, swap = (a_row >> 1) & 7;
+      *reinterpret_cast<ln_half4*>(row + ((chunk ^ swap) << 4) + half) = hi;
+      *reinterpret_cast<ln_half4*>(row + (((chunk + 4) ^ swap) << 4) + half) = lo;
+    };
+    // and of the weights: 16 bytes of rows threadIdx.x / 8 and 64 + threadIdx.x / 8
+    uint32_t off_b[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = a_row + 64 * i;
+      off_b[i] = (uint32_t)((r < cols_left ? r : cols_left - 1) * (int)row_bytes + (((lane & 7) ^ ((a_row >> 1) & 7)) * 16));
+    }
+    auto fetch = [&](char* buf, int step) {
+      const int p = step >= LN_RANGE_BLOCKS;
+      const char* from = g.ranges + ((int64_t)p * g.width + n0) * row_bytes + (step - p * LN_RANGE_BLOCKS) * LN_BLOCK_BYTES;
+      ln_to_lds(from + off_b[0], buf + (BM + wave * 8) * LN_BLOCK_BYTES);
+      ln_to_lds(from + off_b[1], buf + (BM + 64 + wave * 8) * LN_BLOCK_BYTES);
+      load(step);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    ln_float4 acc[TM][TN] = {}, sum[TM][TN] = {};
+    // A step's operands are read before the next step's loads go out: behind them the compiler waits for those first.
+    ln_half8 wh[TN], wl[TN], xh[TM], xl[TM];
+    auto take = [&](const char* buf) {
+      const int ch = (fq ^ turn) * 16, cl = ((4 + fq) ^ turn) * 16;
+      const char* la = buf + (wm * TM * 16 + fr) * LN_BLOCK_BYTES;
+      const char* lb = buf + (BM + wn * TN * 16 + fr) * LN_BLOCK_BYTES;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        wl[j] = *reinterpret_cast<const ln_half8*>(lb + j * 16 * LN_BLOCK_BYTES + cl);
+        wh[j] = *reinterpret_cast<const ln_half8*>(lb + j * 16 * LN_BLOCK_BYTES + ch);
       }
 #pragma unroll
-      for (int k = 0; k < LN_WHOLE; ++k) {
-        const float v = ln_relu(p2_wave_sum(acc[k]) * ln_inverse(unit[n]) + bias[n]);
-        if (lane == k && first + k < count) {
+      for (int i = 0; i < TM; ++i) {
+        xh[i] = *reinterpret_cast<const ln_half8*>(la + i * 16 * LN_BLOCK_BYTES + ch);
+        xl[i] = *reinterpret_cast<const ln_half8*>(la + i * 16 * LN_BLOCK_BYTES + cl);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&]() {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          ln_float4 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], xl[i], ln_float4{}, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], xh[i], t, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xl[i], t, 0, 0, 0);
+          acc[i][j] += __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xh[i], t, 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);                   // (`store` waits for the loads)
+    };
+    auto carry = [&]() {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = ln_float4{};
+        }
+    };
+    fetch(buf0, 0);
+    store(buf0, 0);
+    for (int step = 0; step < STEPS; step += 2) {
+      p2_sync_loads();                                     // `step` is there, and everyone is done with buf1
+      take(buf0);
+      fetch(buf1, step + 1);
+      multiply();
+      store(buf1, step + 1);
+      p2_sync_loads();
+      const int next = step + 2 < STEPS ? step + 2 : step + 1;   // past the end: a block nobody uses
+      take(buf1);
+      fetch(buf0, next);
+      multiply();
+      store(buf0, next);
+      if ((step & 6) == 6) carry();
+    }
+    p2_sync_loads();                                       // everyone is done with the buffers
+    carry();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int r = m0 + (wm * TM + i) * 16 + fr;
+      if (r >= count) continue;
+      const int32_t s = g.whole[r];
+      const LnSample sm = g.samples[s];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int n = n0 + (wn * TN + j) * 16 + fq * 4;
+        if (n >= g.width) continue;
+        const ln_float4 bi = *reinterpret_cast<const ln_float4*>(g.b_inv + n);
+        ln_float4 rest;                                    // what does not come from the ranges
+        if (sm.card >= 0) {
+          rest = *reinterpret_cast<const ln_float4*>(g.base + (int64_t)sm.state * g.width + n);
+          rest += *reinterpret_cast<const ln_float4*>(g.columns + (int64_t)sm.card * g.width + n);
+        } else {
+          rest = *reinterpret_cast<const ln_float4*>(g.bias + n);
+        }
+        ln_half4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = sum[i][j][e] * (bi[e] * (1.0f / LN_SAMPLE_SCALE)) + rest[e];
           _Float16 h, l;
-          ln_split(v * scale.up, h, l);
-          char* at = out_split + (int64_t)whole[first + k] * ((width / 32) * (int64_t)LN_BLOCK_BYTES) +
-                     (n >> 5) * LN_BLOCK_BYTES + (n & 31) * 2;
-          *reinterpret_cast<_Float16*>(at) = h;
-          *reinterpret_cast<_Float16*>(at + 64) = l;
+          ln_split(ln_relu(v) * scale.up, h, l);
+          hi[e] = h;
+          lo[e] = l;
         }
+        char* at = g.out_split + s * out_bytes + (n >> 5) * LN_BLOCK_BYTES + (n & 31) * 2;
+        *reinterpret_cast<ln_half4*>(at) = hi;
+        *reinterpret_cast<ln_half4*>(at + 64) = lo;
+        if (n == 0) g.out_inv[s] = scale.down;
       }
     }
-    if (n0 == 0 && threadIdx.x < LN_WHOLE && first + (int)threadIdx.x < count) out_inv[whole[first + threadIdx.x]] = scale.down;
   }
 }
 
@@ -1121,10 +1251,14 @@ int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, 
     hipLaunchKernelGGL(ln_first_kernel, dim3((unsigned)(squares * g.groups)), dim3(LN_FIRST_THREADS), 0, s, g);
     P2_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(ln_whole_samples_kernel, dim3(LN_WHOLE_GRID, (unsigned)((w0 + LN_WHOLE_COLS - 1) / LN_WHOLE_COLS)), dim3(LN_THREADS), 0, s, pre_beliefs, root_indices,
-                     board, source_rows, p.samples, p.whole, p.whole_count, weights[0], p.bias[0], p.unit[0], w0, p.stats,
-                     p.hidden[0], p.hidden_inv[0]);
-  P2_LAUNCH_CHECK();
+  {
+    const LnWhole g = {pre_beliefs, root_indices, board, source_rows, p.samples, p.whole, p.whole_count, p.first_ranges,
+                       p.w_inv[0], p.bias[0], p.base, p.first_board, p.stats, w0, p.hidden[0], p.hidden_inv[0]};
+    const int64_t most = ((total_samples + LN_WHOLE_ROWS - 1) / LN_WHOLE_ROWS) * ((w0 + LN_WHOLE_COLS - 1) / LN_WHOLE_COLS);
+    hipLaunchKernelGGL(ln_whole_kernel, dim3((unsigned)(most < LN_WHOLE_GRID ? (most + 7) / 8 * 8 : LN_WHOLE_GRID)),
+                       dim3(LN_WHOLE_THREADS), 0, s, g);
+    P2_LAUNCH_CHECK();
+  }
   for (int l = 1; l + 1 < layers; ++l) {
     const int in = (l - 1) & 1, out = l & 1;
     LnGemm g = {};

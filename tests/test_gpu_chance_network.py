@@ -37,6 +37,14 @@ def make_inputs(n, kind, seed, on_board=None):
         x[:] = 0
         x[np.arange(n), 0, rng.integers(0, H, n)] = 1.0
         x[np.arange(n), 1, rng.integers(0, H, n)] = 0.25
+    elif kind == "three hands":                # six cards of a player hold a third of his range each
+        x[:] = 0
+        for _ in range(3):
+            x[np.arange(n), 0, rng.integers(0, H, n)] = 1.0
+            x[np.arange(n), 1, rng.integers(0, H, n)] = 1.0
+    elif kind == "one hand against none":
+        x[:] = 0
+        x[np.arange(n), np.arange(n) % 2, rng.integers(0, H, n)] = 1.0
     elif kind == "some empty":
         x[::2, 0] = 0
         x[1::3, 1] = 0
@@ -90,6 +98,8 @@ def reference(net, pre, boards):
     (256, 4, 7, "some empty", None, True),
     (1536, 3, 6, "gamma", 4, True),
     (512, 2, 180, "gamma", 4, True),           # states across tiles of 128 rows
+    (288, 2, 40, "three hands", None, True),   # several tiles of samples taken whole, the last of both kinds no full one
+    (256, 2, 9, "one hand against none", 4, True),
 ])
 def test_matches_float64(hidden, layers, n, kind, on_board, bias):
     net = make_net(hidden, layers, bias)
@@ -140,12 +150,14 @@ def test_units_of_unequal_size(kind, ranges):
 
 
 @pytest.mark.gpu
-def test_256_row_tiles_and_a_selection_of_rows():
-    """Enough samples for the largest tiles (4 per CU), taken from a table through ``root_indices``; a few states of it
-    against float64, all against the network sample by sample in float32."""
+@pytest.mark.parametrize("kind", ["gamma", "three hands"])
+def test_256_row_tiles_and_a_selection_of_rows(kind):
+    """Enough samples for the largest tiles (4 per CU), taken from a table through ``root_indices``, and enough of them
+    taken whole for several tiles per workgroup; a few states against float64, all against the network sample by sample
+    in float32."""
     n = 1400
     net = make_net(1024, 2)
-    pre, boards = make_inputs(n + 3, "gamma", seed=1, on_board=4)
+    pre, boards = make_inputs(n + 3, kind, seed=1, on_board=4)
     roots = torch.randperm(n + 3, generator=torch.Generator().manual_seed(2))[:n].cuda()
     with torch.no_grad():
         got = K.chance_network(pre, roots, boards, K.network_layers(net, pre.device), 4, check_rows=False)
