@@ -828,11 +828,14 @@ __global__ __launch_bounds__(LN_FIRST_THREADS, 4) void ln_first_kernel(LnFirst g
 // normalised and split on the way into LDS, 64 samples against 128 columns a tile, and multiplied by the ranges' columns
 // as LN_PLAIN does; the board's columns come from `base` and `columns`.  Runs behind ln_first_kernel, which wrote the
 // same rows of `out_split` from zero weights.  A fixed number of workgroups takes the tiles in turn, each XCD a run of
-// them, columns outermost, so that it keeps its columns' weights in its L2.
+// them, columns outermost, so that it keeps its columns' weights in its L2.  Where the tiles leave workgroups over, a
+// tile's steps are cut into as many parts as there are workgroups for, and another launch adds them up (the last
+// workgroup of a tile doing that, behind fences of the whole device, took 50 us more).
 // 3 x 1536, ms a call, float32 on the vector units (four samples at a time) -> here: 2240 states with three hands per
-// range (up to 12 of 48 samples whole) 21.4 -> 5.1, with one hand 9.8 -> 4.2, smooth ranges 3.7 -> 3.6; 35 states with three
-// hands 0.66 -> 0.39.  The network layer by layer: 20.6 and 0.56.  Bound: for few samples the 84 steps, one after the other,
-// 0.1 ms; for many the splitting, which the vector units do again for every stripe of columns.
+// range (up to 12 of 48 samples whole) 21.4 -> 5.4, with one hand 9.8 -> 4.4, smooth ranges 3.7; 35 states with three
+// hands 0.66 -> 0.31 (a tile in one part 0.39), smooth 0.27.  The network layer by layer: 20.4 and 0.56.  Bound: for few
+// samples the chain of steps, 1.2 us each; for many the splitting, which the vector units do again for every stripe of
+// columns.
 struct LnWhole {
   const float* pre_beliefs;
   const int64_t *root_indices, *board;
@@ -842,12 +845,66 @@ struct LnWhole {
   const char* ranges;           // [2][width] split rows
   const float *b_inv, *bias, *base, *columns, *stats;
   int width;
+  ln_float4* parts;             // [LN_WHOLE_GRID][4][LN_WHOLE_THREADS]
   char* out_split;
   float* out_inv;
 };
 constexpr int LN_WHOLE_ROWS = 64, LN_WHOLE_COLS = 128, LN_WHOLE_THREADS = 512, LN_WHOLE_GRID = 512;
+// A tile of the ranges' share becomes rows of `out_split`: element e of sum[i][j] is row (wave / 4 TM + i) 16 + lane % 16,
+// column (wave % 4 TN + j) 16 + 4 (lane / 16) + e.
+constexpr int LN_WHOLE_TM = 2, LN_WHOLE_TN = 2;
+__device__ __forceinline__ void ln_whole_store(const LnWhole& g, const ln_float4 (&sum)[LN_WHOLE_TM][LN_WHOLE_TN], int count,
+                                               int m0, int n0) {
+  constexpr int TM = LN_WHOLE_TM, TN = LN_WHOLE_TN;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave >> 2, wn = wave & 3, fr = lane & 15, fq = lane >> 4;
+  const LnScale scale = ln_scale(g.stats[0] + g.stats[1]);
+  const int64_t out_bytes = (int64_t)(g.width / 32) * LN_BLOCK_BYTES;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int r = m0 + (wm * TM + i) * 16 + fr;
+        if (r >= count) continue;
+        const int32_t s = g.whole[r];
+        const LnSample sm = g.samples[s];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int n = n0 + (wn * TN + j) * 16 + fq * 4;
+          if (n >= g.width) continue;
+          const ln_float4 bi = *reinterpret_cast<const ln_float4*>(g.b_inv + n);
+          ln_float4 rest;                                    // what does not come from the ranges
+          if (sm.card >= 0) {
+            rest = *reinterpret_cast<const ln_float4*>(g.base + (int64_t)sm.state * g.width + n);
+            rest += *reinterpret_cast<const ln_float4*>(g.columns + (int64_t)sm.card * g.width + n);
+          } else {
+            rest = *reinterpret_cast<const ln_float4*>(g.bias + n);
+          }
+          ln_half4 hi, lo;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = sum[i][j][e] * (bi[e] * (1.0f / LN_SAMPLE_SCALE)) + rest[e];
+            _Float16 h, l;
+            ln_split(ln_relu(v) * scale.up, h, l);
+            hi[e] = h;
+            lo[e] = l;
+          }
+          char* at = g.out_split + s * out_bytes + (n >> 5) * LN_BLOCK_BYTES + (n & 31) * 2;
+          *reinterpret_cast<ln_half4*>(at) = hi;
+          *reinterpret_cast<ln_half4*>(at + 64) = lo;
+          if (n == 0) g.out_inv[s] = scale.down;
+        }
+      }
+}
+
+// Into how many parts the steps of a tile are cut, each a divisor of them that leaves an even number: as many as there are
+// workgroups for.
+__device__ __forceinline__ unsigned ln_whole_split(unsigned tiles) {
+  unsigned split = 14;
+  while (split > 1 && tiles * split > LN_WHOLE_GRID) split = split == 14 ? 7 : split == 7 ? 6 : split / 2;
+  return split;
+}
+
 __global__ __launch_bounds__(LN_WHOLE_THREADS, 4) void ln_whole_kernel(LnWhole g) {
-  constexpr int TM = 2, TN = 2, BM = LN_WHOLE_ROWS, BN = LN_WHOLE_COLS, STEPS = 2 * LN_RANGE_BLOCKS;
+  constexpr int TM = LN_WHOLE_TM, TN = LN_WHOLE_TN, BM = LN_WHOLE_ROWS, BN = LN_WHOLE_COLS, STEPS = 2 * LN_RANGE_BLOCKS;
   static_assert(STEPS % 2 == 0, "steps in pairs, a buffer each");
   __shared__ __align__(128) char buf0[(BM + BN) * LN_BLOCK_BYTES];
   __shared__ __align__(128) char buf1[(BM + BN) * LN_BLOCK_BYTES];
@@ -855,14 +912,15 @@ __global__ __launch_bounds__(LN_WHOLE_THREADS, 4) void ln_whole_kernel(LnWhole g
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;                 // waves 2 x 4, 32 x 32 each
   const int fr = lane & 15, fq = lane >> 4, turn = (fr >> 1) & 7;
-  const LnScale scale = ln_scale(g.stats[0] + g.stats[1]);
-  const int64_t row_bytes = LN_RANGE_BLOCKS * LN_BLOCK_BYTES, out_bytes = (int64_t)(g.width / 32) * LN_BLOCK_BYTES;
+  const int64_t row_bytes = LN_RANGE_BLOCKS * LN_BLOCK_BYTES;
   const unsigned tiles_m = (unsigned)((count + BM - 1) / BM), tiles_n = (unsigned)((g.width + BN - 1) / BN);
-  const unsigned tiles = tiles_m * tiles_n, xcd = blockIdx.x & 7, per = tiles >> 3, more = tiles & 7;
+  const unsigned split = ln_whole_split(tiles_m * tiles_n);
+  const int steps = STEPS / (int)split;
+  const unsigned items = tiles_m * tiles_n * split, xcd = blockIdx.x & 7, per = items >> 3, more = items & 7;
   const unsigned mine = per + (xcd < more ? 1 : 0), start = xcd * per + (xcd < more ? xcd : more);
   for (unsigned turn_of = blockIdx.x >> 3; turn_of < mine; turn_of += gridDim.x >> 3) {
-    const unsigned tile = start + turn_of, tm = tile % tiles_m, tn = tile / tiles_m;
-    const int m0 = (int)tm * BM, n0 = (int)tn * BN;
+    const unsigned item = start + turn_of, part = item % split, tile = item / split, tm = tile % tiles_m, tn = tile / tiles_m;
+    const int first = (int)part * steps, m0 = (int)tm * BM, n0 = (int)tn * BN;
     const int cols_left = g.width - n0 < BN ? g.width - n0 : BN;
 
     // this thread's part of the samples: row threadIdx.x / 8, four hands of every block
@@ -970,16 +1028,16 @@ __global__ __launch_bounds__(LN_WHOLE_THREADS, 4) void ln_whole_kernel(LnWhole g
           acc[i][j] = ln_float4{};
         }
     };
-    fetch(buf0, 0);
-    store(buf0, 0);
-    for (int step = 0; step < STEPS; step += 2) {
+    fetch(buf0, first);
+    store(buf0, first);
+    for (int step = first; step < first + steps; step += 2) {
       p2_sync_loads();                                     // `step` is there, and everyone is done with buf1
       take(buf0);
       fetch(buf1, step + 1);
       multiply();
       store(buf1, step + 1);
       p2_sync_loads();
-      const int next = step + 2 < STEPS ? step + 2 : step + 1;   // past the end: a block nobody uses
+      const int next = step + 2 < first + steps ? step + 2 : step + 1;   // past the end: a block nobody uses
       take(buf1);
       fetch(buf0, next);
       multiply();
@@ -988,40 +1046,35 @@ __global__ __launch_bounds__(LN_WHOLE_THREADS, 4) void ln_whole_kernel(LnWhole g
     }
     p2_sync_loads();                                       // everyone is done with the buffers
     carry();
+    if (split > 1) {
+      ln_float4* at = g.parts + (int64_t)item * (TM * TN) * LN_WHOLE_THREADS + threadIdx.x;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int r = m0 + (wm * TM + i) * 16 + fr;
-      if (r >= count) continue;
-      const int32_t s = g.whole[r];
-      const LnSample sm = g.samples[s];
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = n0 + (wn * TN + j) * 16 + fq * 4;
-        if (n >= g.width) continue;
-        const ln_float4 bi = *reinterpret_cast<const ln_float4*>(g.b_inv + n);
-        ln_float4 rest;                                    // what does not come from the ranges
-        if (sm.card >= 0) {
-          rest = *reinterpret_cast<const ln_float4*>(g.base + (int64_t)sm.state * g.width + n);
-          rest += *reinterpret_cast<const ln_float4*>(g.columns + (int64_t)sm.card * g.width + n);
-        } else {
-          rest = *reinterpret_cast<const ln_float4*>(g.bias + n);
-        }
-        ln_half4 hi, lo;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float v = sum[i][j][e] * (bi[e] * (1.0f / LN_SAMPLE_SCALE)) + rest[e];
-          _Float16 h, l;
-          ln_split(ln_relu(v) * scale.up, h, l);
-          hi[e] = h;
-          lo[e] = l;
-        }
-        char* at = g.out_split + s * out_bytes + (n >> 5) * LN_BLOCK_BYTES + (n & 31) * 2;
-        *reinterpret_cast<ln_half4*>(at) = hi;
-        *reinterpret_cast<ln_half4*>(at + 64) = lo;
-        if (n == 0) g.out_inv[s] = scale.down;
-      }
+        for (int j = 0; j < TN; ++j) at[(i * TN + j) * LN_WHOLE_THREADS] = sum[i][j];
+      continue;
     }
+    ln_whole_store(g, sum, count, m0, n0);
   }
+}
+
+// Adds up the parts of the tiles that ln_whole_kernel has cut, in their order, and finishes them.
+__global__ __launch_bounds__(LN_WHOLE_THREADS) void ln_whole_parts_kernel(LnWhole g) {
+  constexpr int TM = LN_WHOLE_TM, TN = LN_WHOLE_TN;
+  const int count = *g.whole_count;
+  const unsigned tiles_m = (unsigned)((count + LN_WHOLE_ROWS - 1) / LN_WHOLE_ROWS);
+  const unsigned tiles = tiles_m * (unsigned)((g.width + LN_WHOLE_COLS - 1) / LN_WHOLE_COLS), split = ln_whole_split(tiles);
+  const unsigned tile = blockIdx.x;
+  if (split == 1 || tile >= tiles) return;
+  const ln_float4* at = g.parts + (int64_t)tile * split * (TM * TN) * LN_WHOLE_THREADS + threadIdx.x;
+  ln_float4 sum[TM][TN] = {};
+#pragma unroll 2
+  for (unsigned k = 0; k < split; ++k, at += (TM * TN) * LN_WHOLE_THREADS)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) sum[i][j] += at[(i * TN + j) * LN_WHOLE_THREADS];
+  ln_whole_store(g, sum, count, (int)(tile % tiles_m) * LN_WHOLE_ROWS, (int)(tile / tiles_m) * LN_WHOLE_COLS);
 }
 
 // The means over the samples of each state as split rows: the last layer's input.
@@ -1108,6 +1161,7 @@ struct LnPlan {
   float2* weight;
   LnSample* samples;
   int32_t *row_of, *whole;
+  ln_float4* whole_parts;
   int64_t size;
 };
 
@@ -1147,6 +1201,7 @@ static LnPlan ln_plan(void* base, int64_t states, int64_t samples, const int32_t
   p.samples = early.take<LnSample>(samples);
   p.row_of = early.take<int32_t>(P2_CARDS * states);
   p.whole = early.take<int32_t>(samples);
+  p.whole_parts = early.take<ln_float4>((int64_t)LN_WHOLE_GRID * 4 * LN_WHOLE_THREADS);
   const int64_t early_end = (int64_t)((uintptr_t)p.hidden[1] - (uintptr_t)base) + early.size;
   if (w.size < early_end) w.size = early_end;
   const int last = widths[layers - 2];
@@ -1253,10 +1308,10 @@ int p2hip_chance_network(const float* pre_beliefs, const int64_t* root_indices, 
   }
   {
     const LnWhole g = {pre_beliefs, root_indices, board, source_rows, p.samples, p.whole, p.whole_count, p.first_ranges,
-                       p.w_inv[0], p.bias[0], p.base, p.first_board, p.stats, w0, p.hidden[0], p.hidden_inv[0]};
-    const int64_t most = ((total_samples + LN_WHOLE_ROWS - 1) / LN_WHOLE_ROWS) * ((w0 + LN_WHOLE_COLS - 1) / LN_WHOLE_COLS);
-    hipLaunchKernelGGL(ln_whole_kernel, dim3((unsigned)(most < LN_WHOLE_GRID ? (most + 7) / 8 * 8 : LN_WHOLE_GRID)),
-                       dim3(LN_WHOLE_THREADS), 0, s, g);
+                       p.w_inv[0], p.bias[0], p.base, p.first_board, p.stats, w0, p.whole_parts, p.hidden[0], p.hidden_inv[0]};
+    hipLaunchKernelGGL(ln_whole_kernel, dim3(LN_WHOLE_GRID), dim3(LN_WHOLE_THREADS), 0, s, g);
+    P2_LAUNCH_CHECK();
+    hipLaunchKernelGGL(ln_whole_parts_kernel, dim3(LN_WHOLE_GRID / 2), dim3(LN_WHOLE_THREADS), 0, s, g);
     P2_LAUNCH_CHECK();
   }
   for (int l = 1; l + 1 < layers; ++l) {
