@@ -165,10 +165,16 @@ def chance_mean(hand_values: torch.Tensor, sample_offsets: torch.Tensor) -> torc
     return out
 
 
-# A float32 network of plain layers goes through ``p2hip_chance_network`` from this width on (ms per call, layer by layer
-# -> one call: 2 x 256, 1 state 0.26 -> 0.11, 35 states 0.20 -> 0.11, 2240 states 3.26 -> 0.29; 3 x 1536, 1 state 0.22 ->
-# 0.18, 35 states 0.51 -> 0.21, 2240 states 20.2 -> 3.4).  Narrower ones are what the product's tiles are not made for.
+# Narrower float32 networks go layer by layer: the product's tiles are not made for them.
 NETWORK_MIN_WIDTH = 256
+# A call prepares all weights before it uses them, whatever its size, and some ranges need another product besides
+# (samples taken whole).  Three or more hidden layers of at most 512 units gain all the same, two of 256 too; others from
+# this many samples on.  ms a call of three hidden layers, layer by layer -> one call, smooth ranges / three hands a
+# player: 512 wide, 48 samples 0.19 -> 0.17 / 0.19 (two layers 0.165 -> 0.161 / 0.179); 1024 wide, 48 0.19 -> 0.20 / 0.22, 768 0.21 -> 0.21 / 0.23, 960 0.24 -> 0.21 / 0.24; 1536 wide, 48 0.19 -> 0.23 / 0.25,
+# 768 0.28 -> 0.24 / 0.27, 960 0.34 -> 0.25 / 0.28; 4096 wide, 48 0.19 -> 0.60 / 0.63, 960 0.89 -> 0.68 / 0.75; 1536 wide,
+# 107 520 samples 20.5 -> 3.6 / 5.1.
+NETWORK_ANY_SAMPLES_WIDTH, NETWORK_ANY_SAMPLES_WIDTH_OF_TWO = 512, 256
+NETWORK_MIN_SAMPLES = 960
 
 
 def network_layers(model, device: torch.device) -> list[torch.nn.Linear] | None:
@@ -198,6 +204,16 @@ def network_layers(model, device: torch.device) -> list[torch.nn.Linear] | None:
                 return None
         columns = rows
     return layers
+
+
+def network_takes(layers: list[torch.nn.Linear], states: int, samples: int) -> bool:
+    """Whether ``chance_network`` is the way to compute that many samples: it takes no more than the library says (larger
+    calls go layer by layer, as far as memory goes), and has to be the faster one."""
+    widths = (ctypes.c_int32 * len(layers))(*(lin.weight.shape[0] for lin in layers))
+    if _lib.load().p2hip_chance_network_workspace(states, samples, widths, len(layers)) < 0:
+        return False
+    narrow = NETWORK_ANY_SAMPLES_WIDTH if len(layers) > 3 else NETWORK_ANY_SAMPLES_WIDTH_OF_TWO
+    return samples >= NETWORK_MIN_SAMPLES or max(widths[:-1]) <= narrow
 
 
 def chance_network(pre_chance_beliefs: torch.Tensor, root_indices: torch.Tensor, board_pre: torch.Tensor,
@@ -511,10 +527,11 @@ class ChanceNodeHelper:
         if getattr(model, "input_layout", None) == "ranges|board_onehot" and hasattr(model, "forward_input") \
                 and pre_chance_beliefs.dtype == torch.float32 and pre_chance_beliefs.is_contiguous() \
                 and pre_chance_beliefs.data_ptr() % 16 == 0:
+            if hasattr(model, "eval"):
+                model.eval()
             layers = network_layers(model, pre_chance_beliefs.device) if self.autocast_dtype is None else None
-            if layers is not None:
-                if hasattr(model, "eval"):
-                    model.eval()
+            states = root_indices.numel()
+            if layers is not None and network_takes(layers, states, states * (52 - (cards_on_board or 0))):
                 return chance_network(pre_chance_beliefs, root_indices, board_pre, layers, cards_on_board,
                                       check_rows).to(self.float_dtype)
             # the network reads nothing but the ranges and the board: the expansion writes its input matrix
@@ -524,8 +541,6 @@ class ChanceNodeHelper:
             if rows.shape[0] == 0:
                 return torch.zeros(root_indices.numel(), self.num_players, NUM_HANDS, device=self.device,
                                    dtype=self.float_dtype)
-            if hasattr(model, "eval"):
-                model.eval()
             if self.autocast_dtype is not None:
                 with torch.autocast(device_type="cuda", dtype=self.autocast_dtype):
                     hv = model.forward_input(rows).hand_values

@@ -253,6 +253,30 @@ def test_which_networks_take_this_path():
         torch.set_autocast_enabled("cuda", False)
 
 
+@pytest.mark.parametrize("hidden,layers,states,cards_on_board,one_call", [
+    (256, 2, 1, 4, True), (288, 2, 1, 4, False), (512, 3, 1, None, True), (544, 3, 1, 4, False), (1536, 3, 19, 4, False),
+    (1536, 3, 20, 4, True), (1536, 3, 1, None, False), (256, 2, 174762, 4, True),
+    (256, 2, 174763, 4, False),                # more samples than the library's limit, 8388607
+    (1536, 3, 170000, None, False),            # the same if every board is empty
+])
+def test_which_calls_take_this_path(monkeypatch, hidden, layers, states, cards_on_board, one_call):
+    taken = []
+
+    def note(name):
+        def stop(*args, **kw):
+            taken.append(name)
+            raise StopIteration
+        return stop
+    monkeypatch.setattr(K, "chance_network", note("one call"))
+    monkeypatch.setattr(K, "chance_expand", note("layer by layer"))
+    cpu = torch.device("cpu")
+    helper = K.ChanceNodeHelper(cpu, torch.float32, 2, make_net(hidden, layers, device="cpu"), autocast_dtype=None)
+    with pytest.raises(StopIteration):
+        helper.single_card_chance_values(torch.zeros(states, dtype=torch.int64), None, torch.zeros(1, 2, H),
+                                         torch.full((1, 5), -1), cards_on_board=cards_on_board)
+    assert taken == ["one call" if one_call else "layer by layer"]
+
+
 def test_library_refuses_what_it_does_not_take():
     import ctypes
     from poker2_amd import _lib
