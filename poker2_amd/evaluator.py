@@ -1512,11 +1512,10 @@ class HipSparseCFREvaluator:
         return per_root.index_select(0, self._root_index)
 
     def _best_response_values(self, policy: torch.Tensor, beliefs: torch.Tensor, base_values: torch.Tensor,
-                              deviating_player: torch.Tensor | None = None, *, clamp: bool = False) -> torch.Tensor:
+                              deviating_player: torch.Tensor | None = None) -> torch.Tensor:
         """Values when ``deviating_player`` (per node; default: the root's player to act) plays a
         per-hand best response and the other player follows ``policy``
-        (cfr_evaluator.py:603-716).  One kernel launch per tree level, deepest first.  ``clamp``: leaf values are cut to
-        [-1, 1]."""
+        (cfr_evaluator.py:603-716).  One kernel launch per tree level, deepest first."""
         n = self.root_nodes
         if deviating_player is None:
             deviating_player = self._fan_out_deep(self.env.to_act[:n])
@@ -1524,7 +1523,7 @@ class HipSparseCFREvaluator:
         _req(deviating_player.shape == (self.total_nodes,), "deviating_player.shape == (self.total_nodes,)")
         policy = policy.contiguous()
         beliefs = beliefs.contiguous()
-        values_br = self._leaf_rows(base_values, clamp)
+        values_br = self._leaf_rows(base_values)
         for depth in range(self.tree_depth - 1, -1, -1):
             base, end = self.depth_offsets[depth], self.depth_offsets[depth + 1]
             _lib.call("p2hip_best_response_level", _lib.ptr(values_br), _lib.ptr(policy), _lib.ptr(beliefs),
@@ -1542,12 +1541,15 @@ class HipSparseCFREvaluator:
                                        torch.empty(0, 2, device=self.device, dtype=self.float_dtype))
         self._complete_rows()
         policy, beliefs = self.policy_probs_avg, self.beliefs_avg
-        base_values = self._leaf_rows(self.values_avg, clamp=True)
-        self.compute_expected_values(policy=policy, beliefs=beliefs, leaf_values=base_values, values=base_values)
+        # this class's own methods look at the leaves alone and leave them as they are: one tensor serves both
+        own = self._own_methods("compute_expected_values", "_best_response_values")
+        leaf_values = self._leaf_rows(self.values_avg, clamp=True) if own else self.values_avg.clamp(-1.0, 1.0)
+        base_values = leaf_values if own else torch.zeros_like(leaf_values)
+        self.compute_expected_values(policy=policy, beliefs=beliefs, leaf_values=leaf_values, values=base_values)
         improvements, br_agg = [], []
         for player in range(2):
             deviator = torch.full((n,), player, device=self.device, dtype=torch.int64)
-            br = self._best_response_values(policy, beliefs, self.values_avg, self._fan_out_deep(deviator), clamp=True)
+            br = self._best_response_values(policy, beliefs, leaf_values, self._fan_out_deep(deviator))
             root_beliefs = beliefs[:n, player]
             improvements.append(((br[:n, player] - base_values[:n, player]) * root_beliefs).sum(dim=-1))
             br_agg.append((br[:n, player] * root_beliefs).sum(dim=-1))

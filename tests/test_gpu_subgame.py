@@ -138,3 +138,28 @@ def test_leaf_rows_and_finite_check(ev):
         with pytest.raises(ValueError, match="after here"):
             ev._require_finite_values("here")
         ev.latest_values.view(-1)[at] = old
+
+
+def test_exploitability_asks_overrides_as_the_reference_does():
+    """An overridden ``_best_response_values`` gets four arguments and the clamped values of every row, an overridden
+    ``compute_expected_values`` two tensors."""
+    ev = make(5, [0.5, 1.0], 5, [3], 4)
+    ev.initialize_policy_and_beliefs()
+    ev.values_avg.normal_(generator=torch.Generator(device="cuda").manual_seed(1))
+    want = ev._compute_exploitability()
+    seen = []
+    best, expected = ev._best_response_values, ev.compute_expected_values
+
+    def best_response(policy, beliefs, base_values, deviating_player=None):
+        seen.append(base_values.clone())
+        return best(policy, beliefs, base_values, deviating_player)
+
+    def expected_values(policy=None, beliefs=None, leaf_values=None, values=None):
+        assert leaf_values is not values and not bool(values.any())
+        expected(policy=policy, beliefs=beliefs, leaf_values=leaf_values, values=values)
+    for name, method in (("_best_response_values", best_response), ("compute_expected_values", expected_values)):
+        setattr(ev, name, method)
+        got = ev._compute_exploitability()
+        assert torch.equal(got.local_exploitability, want.local_exploitability)
+        assert torch.equal(got.local_best_response_values, want.local_best_response_values)
+    assert len(seen) == 4 and all(torch.equal(x, ev.values_avg.clamp(-1.0, 1.0)) for x in seen)
