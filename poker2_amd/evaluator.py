@@ -1264,9 +1264,8 @@ class HipSparseCFREvaluator:
             raise ValueError(f"Non-finite values in latest_values after {after}")
 
     def _leaf_rows(self, values: torch.Tensor, clamp: bool = False, out: torch.Tensor | None = None) -> torch.Tensor:
-        """``values`` at the leaves, clamped to [-1, 1] if asked, and zero at every other node."""
-        values = values.to(self.float_dtype).contiguous()
-        _req(tuple(values.shape) == (self.total_nodes, 2, NUM_HANDS), "values: [total, 2, 1326]")
+        """``values`` (or what broadcasts to it) at the leaves, clamped to [-1, 1] if asked, zero at every other node."""
+        values = values.to(self.float_dtype).expand(self.total_nodes, 2, NUM_HANDS).contiguous()
         out = torch.empty_like(values) if out is None else out
         _req(out.shape == values.shape and out.dtype == values.dtype and out.is_contiguous(), "out: like values")
         _lib.call("p2hip_leaf_rows", _lib.ptr(values), _lib.ptr(self.leaf_mask), self.total_nodes, int(clamp),

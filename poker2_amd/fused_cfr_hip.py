@@ -595,13 +595,21 @@ def _same_rows(total: int, one: dict, both: dict) -> None:
     _f32(**one, **both)
 
 
+def _parent_rows(top: int, **both) -> None:
+    """Tensors that are read at parents alone may end behind the last of them."""
+    for name, t in both.items():
+        _req(t.dim() == 3 and tuple(t.shape[1:]) == (2, _H) and t.shape[0] >= int(top), f"{name}: [>= {int(top)}, 2, 1326]")
+    _f32(**both)
+
+
 def family_regrets(achieved, expected, beliefs, to_act, prev_actor, child_offsets, child_count, bottom: int,
                    top: int) -> torch.Tensor:
     """regrets [total, 1326] of every child of a parent < ``top`` (fused_sparse_cfr_evaluator.py:312-349); rows below
     ``bottom`` are zero."""
-    total = beliefs.shape[0]
+    total = prev_actor.shape[0]
     _family_args(total, top, bottom, 0, child_offsets, child_count, to_act=to_act, prev_actor=prev_actor)
-    _same_rows(total, {}, dict(achieved=achieved, expected=expected, beliefs=beliefs))
+    _same_rows(total, {}, dict(achieved=achieved))
+    _parent_rows(top, expected=expected, beliefs=beliefs)
     regrets = torch.empty(total, _H, dtype=torch.float32, device=beliefs.device)
     _lib.call("p2hip_family_regrets", _p(achieved), _p(expected), _p(beliefs), _p(to_act), _p(prev_actor),
               _p(child_offsets), _p(child_count), int(bottom), int(top), _p(regrets), _S())
@@ -612,9 +620,10 @@ def family_regret_update_(cumulative, weights, achieved, expected, beliefs, to_a
                           bottom: int, top: int, t_alpha_num, t_beta_num, t_alpha_den, t_beta_den, apply_dcfr: bool,
                           cfr_plus: bool) -> None:
     """``fused_dcfr_update_with_tensors_`` of ``family_regrets`` without the tensor between them."""
-    total = beliefs.shape[0]
+    total = prev_actor.shape[0]
     _family_args(total, top, bottom, 0, child_offsets, child_count, to_act=to_act, prev_actor=prev_actor)
-    _same_rows(total, dict(cumulative=cumulative, weights=weights), dict(achieved=achieved, expected=expected, beliefs=beliefs))
+    _same_rows(total, dict(cumulative=cumulative, weights=weights), dict(achieved=achieved))
+    _parent_rows(top, expected=expected, beliefs=beliefs)
     _scalar_ptrs(t_alpha_num=t_alpha_num, t_beta_num=t_beta_num, t_alpha_den=t_alpha_den, t_beta_den=t_beta_den)
     _lib.call("p2hip_family_regret_update", _p(achieved), _p(expected), _p(beliefs), _p(to_act), _p(prev_actor),
               _p(child_offsets), _p(child_count), int(bottom), int(top), _p(cumulative), _p(weights), _p(t_alpha_num),
@@ -669,7 +678,8 @@ def level_expected_values_(values, policy, beliefs, to_act, child_offsets, child
     total = policy.shape[0]
     _family_args(total, end, base, max_children, child_offsets, child_count, to_act=to_act)
     _req(int(base) <= int(end), f"rows [{base}, {end})")
-    _same_rows(total, dict(policy=policy), dict(values=values, beliefs=beliefs))
+    _same_rows(total, dict(policy=policy), dict(values=values))
+    _parent_rows(end, beliefs=beliefs)
     _lib.call("p2hip_level_expected_values", _p(values), _p(policy), _p(beliefs), _p(to_act), _p(child_offsets),
               _p(child_count), int(base), int(end) - int(base), int(max_children), float(eps), _S())
 

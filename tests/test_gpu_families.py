@@ -64,6 +64,10 @@ def test_regrets(ev):
     junk = torch.full_like(want, float("nan"))
     del junk                                             # the result may get its memory: every row has to be written
     assert torch.equal(ev.compute_instantaneous_regrets(achieved, expected), want)
+    # what is read at parents may end behind the last of them
+    assert torch.equal(ev.compute_instantaneous_regrets(achieved, expected[:top]), want)
+    with pytest.raises(AssertionError):
+        ev.compute_instantaneous_regrets(achieved, expected[:top - 1])
 
 
 @pytest.mark.parametrize("cfr", ["standard", "discounted", "discounted_plus"])
@@ -144,8 +148,18 @@ def test_expected_values(ev):
                                     child_offsets=ev.child_offsets[base:end].contiguous(),
                                     child_count=ev.child_count[base:end].contiguous(), parent_base=base,
                                     max_children=ev.num_actions)
+    start = ev.latest_values.clone()
+    ev.compute_expected_values(beliefs=ev.beliefs[:top], values=start, leaf_values=start)
+    assert torch.equal(start, want)
     ev.compute_expected_values()
     assert torch.equal(ev.latest_values, want)
+    # one value for a row, or for all
+    leaf = ev.leaf_mask[:, None, None]
+    for values in (ev.latest_values[:, :, :1], torch.tensor(0.5, device="cuda")):
+        a, b = torch.empty_like(want), torch.where(leaf, values, torch.zeros_like(want))
+        ev.compute_expected_values(leaf_values=values, values=a)
+        ev.compute_expected_values(leaf_values=b, values=b)
+        assert torch.equal(a, b)
 
 
 def test_showdown_rows(ev):
