@@ -369,7 +369,8 @@ int p2hip_sample_snapshot(const float* policy_probs, float* policy_probs_sample,
 /* ---- a family, or a level of the tree, per launch ------------------------------------ */
 
 /* What the methods of search/fused_sparse_cfr_evaluator.py compose of the operations above, in the same roundings, for
- * a whole tree: children of a parent p are rows child_offsets[p] .. + child_count[p] - 1, at most max_children <= 8. */
+ * a whole tree: children of a parent p are rows child_offsets[p] .. + child_count[p] - 1, at most max_children <= 8 (a
+ * parent that has more children than claimed may be left alone). */
 
 /* compute_instantaneous_regrets (:312-349): achieved, expected, beliefs [T,2,H] -> regrets [T,H]; parents < top, rows <
  * bottom zero */

@@ -17,6 +17,7 @@ namespace p2 {
 
 static_assert(UB_BLOCK == OPS_BLOCK && UB_PPT == OPS_PAIRS_PER_THREAD, "a lane's pairs of a row");
 constexpr int FAM_MAX_CHILDREN = 8;
+// (Where a kernel keeps MAXC children in registers or LDS, a family larger than the caller's max_children is left alone.)
 
 __device__ __forceinline__ void fam_load(const float* __restrict__ base, int64_t row, float2 (&v)[UB_PPT]) {
   const float2* r = p2_row2(base, row);
@@ -155,8 +156,9 @@ __global__ __launch_bounds__(UB_BLOCK) void family_regret_matching_kernel(const 
                                                                            const int64_t* __restrict__ child_offsets,
                                                                            const int64_t* __restrict__ child_count,
                                                                            float eps, float* __restrict__ policy) {
-  const int count = (int)child_count[blockIdx.x];
-  if (count <= 0) return;
+  const int64_t count64 = child_count[blockIdx.x];
+  if (count64 <= 0 || count64 > MAXC) return;
+  const int count = (int)count64;
   const int64_t first = child_offsets[blockIdx.x];
   float2 v[MAXC][UB_PPT], sum[UB_PPT];
   fam_load_children(cumulative, first, count, v);
@@ -195,8 +197,9 @@ __global__ __launch_bounds__(UB_BLOCK) void family_average_policy_kernel(
     const float2 none[UB_PPT] = {};
     fam_store(policy_avg, p, none);
   }
-  const int count = p < top ? (int)child_count[p] : 0;
-  if (count <= 0) return;
+  const int64_t count64 = p < top ? child_count[p] : 0;
+  if (count64 <= 0 || count64 > MAXC) return;
+  const int count = (int)count64;
   const int64_t first = child_offsets[p], row = 2 * p + to_act[p];
   float2 r[UB_PPT], ra[UB_PPT], cur[MAXC][UB_PPT], avg[MAXC][UB_PPT], sum[UB_PPT];
   fam_load(reach, row, r);
@@ -325,10 +328,11 @@ __global__ __launch_bounds__(UB_BLOCK) void level_expected_values_kernel(
   __shared__ double cs[(MAXC + 1) * P2_CARDS];
   __shared__ double totals[MAXC + 1];
   const int64_t p = base + blockIdx.x;
-  const int count = (int)child_count[p];
+  const int64_t count64 = child_count[p];
+  if (count64 <= 0 || count64 > MAXC) return;               // a leaf keeps its values
+  const int count = (int)count64;
   const int64_t first = child_offsets[p];
   const int actor = (int)to_act[p];
-  if (count <= 0) return;                                   // a leaf keeps its values
   float2 range[UB_PPT], w[MAXC][UB_PPT], own[UB_PPT], other[UB_PPT];
   fam_load(beliefs, 2 * p + actor, range);
   fam_load_children(policy, first, count, w);

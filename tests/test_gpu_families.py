@@ -192,3 +192,38 @@ def test_wrappers_refuse_what_would_index_out_of_bounds(ev):
     with pytest.raises(AssertionError):
         F.family_regrets(ev.latest_values[:-1], ev.latest_values, ev.beliefs, ev.env.to_act, ev.prev_actor,
                          ev.child_offsets, ev.child_count, 1, 1)
+
+
+def test_a_family_larger_than_claimed_is_left_alone():
+    from poker2_amd import fused_cfr_hip as F
+    ev = make(*CASES[2])
+    ev.prepare_replay(3)
+    n, top, base = ev.root_nodes, ev.depth_offsets[-2], ev.depth_offsets[-3]
+    large = ev.child_count[:top] > 5
+    assert bool(large.any()) and bool((ev.child_count[:top] == 5).any())
+    of_large = torch.zeros(ev.total_nodes, dtype=torch.bool, device="cuda")
+    of_large[n:] = large[ev.parent_index[n:]]
+
+    def run(names, call):
+        start, ends = {k: getattr(ev, k).clone() for k in names}, []
+        for claim in (5, 8):
+            for k in names:
+                getattr(ev, k).copy_(start[k])
+            call(claim)
+            ends.append({k: getattr(ev, k).clone() for k in names})
+        return start, *ends
+    tree = (ev.child_offsets, ev.child_count)
+    s = ev._t_scalars
+    for name, call in (
+            ("policy_probs", lambda claim: F.family_regret_matching_(ev.policy_probs, ev.cumulative_regrets,
+                                                                     ev.uniform_policy, *tree, top, claim)),
+            ("policy_probs_avg", lambda claim: F.family_average_policy_(
+                ev.policy_probs_avg, ev.policy_probs, ev.self_reach, ev.self_reach_avg, ev.env.to_act, *tree, s.mix_old,
+                s.mix_new, s.mix_total, n, top, claim))):
+        start, small, whole = run((name,), call)
+        assert torch.equal(small[name][of_large], start[name][of_large])
+        assert torch.equal(small[name][~of_large], whole[name][~of_large])
+    start, small, whole = run(("latest_values",), lambda claim: F.level_expected_values_(
+        ev.latest_values, ev.policy_probs, ev.beliefs, ev.env.to_act, *tree, base, top, claim))
+    want = torch.where(large[base:, None, None], start["latest_values"][base:top], whole["latest_values"][base:top])
+    assert torch.equal(small["latest_values"][base:top], want)
