@@ -772,8 +772,9 @@ class HipSparseCFREvaluator:
         return all(getattr(getattr(self, name), "__func__", None) is getattr(HipSparseCFREvaluator, name) for name in names)
 
     def _push_down(self, reach: torch.Tensor, policy: torch.Tensor, beliefs: torch.Tensor) -> None:
-        """``_calculate_reach_weights`` and ``_propagate_all_beliefs`` in one launch."""
-        if self.tree_depth > F.TREE_MAX_DEPTH or not self._own_methods("_calculate_reach_weights", "_propagate_all_beliefs"):
+        """``_calculate_reach_weights`` and ``_propagate_all_beliefs``, in one launch where that is faster."""
+        if self.total_nodes > F.TREE_ONE_LAUNCH_ROWS or self.tree_depth > F.TREE_MAX_DEPTH or \
+                not self._own_methods("_calculate_reach_weights", "_propagate_all_beliefs"):
             self._calculate_reach_weights(reach, policy)
             self._propagate_all_beliefs(beliefs, reach)
             return

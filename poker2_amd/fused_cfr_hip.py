@@ -654,6 +654,11 @@ def family_average_policy_(policy_avg, policy, reach, reach_avg, to_act, child_o
 
 
 TREE_MAX_DEPTH = 64       # P2HIP_TREE_MAX_DEPTH
+# Up to this many rows tree_reach_beliefs_ is faster than an operation per level (us, levels -> one launch): 64 roots 8 levels
+# deep, 1088 rows, 113 -> 25; 50 roots, 7 levels, 19 100 rows, 252 -> 219.  Beyond, the launches of the levels no longer show
+# and a row reads one policy instead of all on its way: 25 000 rows of 12 levels 293 and 300, 61 400 rows of 10 levels 652 and
+# 754, 376 000 rows of 5 levels 3434 and 3758.
+TREE_ONE_LAUNCH_ROWS = 20_000
 
 
 def tree_reach_beliefs_(reach, beliefs, policy, allowed_mask, allowed_prob, parent_index, prev_actor, root_index,

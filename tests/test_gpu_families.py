@@ -95,7 +95,7 @@ def test_regret_update(ev, cfr, plus):
         assert torch.equal(runs[0][k], runs[1][k]) and not torch.equal(runs[0][k], start[k]), k
 
 
-def test_policies_reach_and_ranges(ev):
+def test_policies_reach_and_ranges(ev, monkeypatch):
     from poker2_amd import fused_cfr_hip as F
     n, bottom, top = ev.root_nodes, ev.depth_offsets[1], ev.depth_offsets[-2]
 
@@ -125,6 +125,15 @@ def test_policies_reach_and_ranges(ev):
     ev.update_policy(3)
     for k in names:
         assert torch.equal(getattr(ev, k), want[k]), k
+    # a tree too large for the walk down from the roots: an operation per level
+    for k in names:
+        getattr(ev, k).copy_(start[k])
+    monkeypatch.setattr(F, "TREE_ONE_LAUNCH_ROWS", ev.total_nodes - 1)
+    monkeypatch.setattr(F, "tree_reach_beliefs_", None)
+    ev.update_policy(3)
+    for k in names:
+        assert torch.equal(getattr(ev, k), want[k]), k
+    monkeypatch.undo()
     # an override of one of the two steps is not passed by
     calls = []
     ev._calculate_reach_weights = lambda *a: calls.append("reach")
