@@ -288,14 +288,16 @@ __global__ __launch_bounds__(SD_BLOCK) void showdown_setup_kernel(const void* __
   uint32_t pair_of[6];                           // where the hands' scores will be: 13 x low rank + high rank
 #pragma unroll
   for (int i = 0; i < 6; ++i) {
+    pair_of[i] = 255u;
+    if (!by_ranks) continue;   // (for the whole workgroup: all hands through the list took 8192 boards 199 us, like this 187)
     const int h = t + i * SD_BLOCK;
     const bool in = h < P2_H;
     const int a = in ? p2_combo.a[h] : 0, b = in ? p2_combo.b[h] : 1;
     const int sa = (a * 79) >> 10, sb = (b * 79) >> 10;                      // / 13 for 0 .. 51
     const int ra = a - 13 * sa, rb = b - 13 * sb;
-    const bool single = in && (!by_ranks || (((board_bits >> a) | (board_bits >> b)) & 1ull) ||
+    const bool single = in && ((((board_bits >> a) | (board_bits >> b)) & 1ull) ||
                                (int)(sa == flush_suit) + (int)(sb == flush_suit) >= needed);
-    pair_of[i] = in && !single ? (uint32_t)(ra < rb ? ra * 13 + rb : rb * 13 + ra) : 255u;
+    if (in && !single) pair_of[i] = (uint32_t)(ra < rb ? ra * 13 + rb : rb * 13 + ra);
     const unsigned long long who = __ballot(single);
     int first = 0;
     if (lane == 0 && who) first = atomicAdd(&S.singles, __popcll(who));
@@ -321,8 +323,9 @@ __global__ __launch_bounds__(SD_BLOCK) void showdown_setup_kernel(const void* __
     S.pair_score[at] = sc;
     S.pair_code[at] = score_code(sc);
   }
-  for (int e = (((turn + 2) & 3) << 6) + lane; e < S.singles; e += SD_BLOCK) {
-    const int h = S.clist[e];
+  const int singles = by_ranks ? S.singles : P2_H;
+  for (int e = (((turn + 2) & 3) << 6) + lane; e < singles; e += SD_BLOCK) {
+    const int h = by_ranks ? S.clist[e] : e;
     const int32_t sc = score(p2_combo.a[h], p2_combo.b[h]);
     put_score(h, sc, score_code(sc));
   }
