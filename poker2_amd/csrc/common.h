@@ -183,18 +183,21 @@ __device__ __forceinline__ double p2_block_sum(double v, double* red) {
 // far from the ends of the exponent's range; the kernels divide four to ten times per row and hand, and their
 // launches are bound by the vector units (59 % busy in the subtree launch of 192 roots).  Here the reciprocal is the
 // hardware's, within one unit in the last place, with one Newton step, and the quotient is corrected once by its
-// exact remainder (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990): the
-// correctly rounded quotient, for divisors from 2^-126 to 2^126, equal to `/` on 1.6e9 random pairs of operands and
-// the special ones.  A dividend below 2^-102 can lose its remainder to rounding, and its quotient then a unit in the
-// last place.  Divisors that several quotients share (a family's sum, a range's mass, the schedule's) are inverted
-// once.  River roots: one, 32 iterations, 4.63 -> 4.45 ms; 192, eight
-// ordinary iterations, 5.93 -> 5.87, 16 lean ones 10.23 -> 10.16; 4096, 4 iterations, 44.1 -> 44.0.
+// exact remainder (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  Equal
+// to `/` for dividends from 2^-102 and divisors from 2^-126 to 2^126 whose quotient is a normal number: the oracle
+// (oracle/quotient.c) goes through every mantissa of a divisor with every reciprocal that hardware may start from.
+// Outside of that: a smaller dividend can lose its remainder to rounding, and its quotient then a unit in the last place,
+// and so can a subnormal quotient.  A quotient that overflows becomes NaN, not infinity; none of the kernels' can: their
+// dividends are at most their divisors (a regret and its family's sum, a hand and its range's mass, a mix and its
+// weights) or the divisor is at least 1 (the schedule's).  The launch-per-operation path divides by `/`.
+// Divisors that several quotients share (a family's sum, a range's mass, the schedule's) are inverted once.  One river
+// root, 32 iterations, 4.63 -> 4.45 ms; the sizes that fill the chip gain about as much as two runs of them differ.
 __device__ __forceinline__ float p2_recip(float b) {
   const float y = __builtin_amdgcn_rcpf(b);
   return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
 }
 
-// The same for divisors up to the largest float, whose reciprocal is subnormal.
+// The same for divisors from 2^-94 up to the largest float, whose reciprocal is subnormal.
 __device__ __forceinline__ float p2_recip_wide(float b) {
   const float y = __builtin_amdgcn_rcpf(b * 0x1p-32f) * 0x1p-32f;
   return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);

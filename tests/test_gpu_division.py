@@ -1,13 +1,41 @@
 """The iteration kernels' quotient (p2_div in csrc/common.h) against IEEE division: regret matching's policy is the
 quotient of the regrets that the same iteration leaves, bit for bit, from sums at the threshold to sums whose
 reciprocal is subnormal.  A dividend below 2^-102 has a remainder that can be subnormal and is rounded to a multiple of
-2^-149: its quotient may be off by half of that over the divisor and by the rounding of the product."""
+2^-149: its quotient may be off by half of that over the divisor and by the rounding of the product.  The quotients of
+the discounts and of the average policy's mix, which share their reciprocals, against the launch-per-operation path,
+which divides as IEEE does.  (What of this needs no GPU: tests/test_oracle_quotient.py.)"""
 import pytest
 import torch
 
-from tests.test_gpu_families import make
+from tests.test_gpu_families import CASES, make
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", CASES, ids=["one root", "five", "eight"])
+@pytest.mark.parametrize("cfr", ["standard", "discounted", "discounted_plus", "linear"])
+@pytest.mark.parametrize("t", [1, 7, 300])
+def test_discounts_and_mixes_are_those_of_ieee_division(shape, cfr, t):
+    from poker2_amd.evaluator import STATE_NAMES
+    from poker2_amd.fused_cfr_hip import CFRType
+    print(shape, cfr, t, flush=True)
+    ev = make(*shape)
+    ev.cfr_type = CFRType[cfr]
+    ev.dcfr_beta_initial = -1.0
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    ev.regret_weight_sums.uniform_(generator=gen)
+    start = {k: getattr(ev, k).clone() for k in STATE_NAMES}
+    ends = []
+    for fused in (False, True):
+        for k, v in start.items():
+            getattr(ev, k).copy_(v)
+        ev.fused_iteration = fused
+        ev.prepare_replay(t)
+        ev.cfr_iteration(t)
+        ends.append({k: getattr(ev, k).clone() for k in STATE_NAMES})
+    n = ev.root_nodes                                    # (make() leaves root rows that no search would)
+    for k in ("cumulative_regrets", "regret_weight_sums", "policy_probs", "policy_probs_avg", "self_reach", "self_reach_avg"):
+        assert torch.equal(ends[0][k][n:], ends[1][k][n:]) and not torch.equal(ends[1][k], start[k]), k
 
 
 @pytest.mark.parametrize("scale", [2e-8, 1.0, 1e30, 1.2e38])
