@@ -90,8 +90,10 @@ __device__ __forceinline__ float ln_block_max(float v, float* red) {
 // that reads it is multiplied by u.  The network is computed as the one whose units all answer with about 1: a row of
 // answers has ONE scale, and a unit far below the largest would lose its low bits to float16's smallest number (with
 // units 2^N(0, 4) apart, 3 x 768: 8e-2 off, like this 4.4e-8 as with units of one size).  u is the power of two below
-// sqrt(sum of absolute weights x largest) + |bias|, which lies between the weights' 2-norm and their sum: in the first layer
-// the largest weight + |bias|.  A unit that is always 0 gets the smallest u, so that what reads it sets no row's scale.
+// sqrt(sum of absolute weights x largest) + bias, which lies between the weights' 2-norm and their sum: in the first layer
+// the largest weight + bias.  A negative bias makes no answer larger and does not count, here or in a row's bound: a unit
+// may be switched off by one of any size, -infinity too.  A unit that is always 0 gets the smallest u, so that what reads
+// it sets no row's scale.
 // A layer's weights are therefore prepared behind those of the layer in front of it.
 __device__ __forceinline__ float ln_unit(float size) {
   int e = (int)((__builtin_bit_cast(uint32_t, size) >> 23) & 255u) - 127;
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_weights_kernel(LnLayerWeights a
   const LnScale s = ln_scale(mx);
   if (threadIdx.x == 0) {
     const float sum = (red_sum[0] + red_sum[1]) + (red_sum[2] + red_sum[3]), b = a.b ? a.b[r] : 0.f;
-    const float unit = a.hidden ? ln_unit(sqrtf(sum) * sqrtf(mx) + fabsf(b)) : 1.0f, down = ln_inverse(unit);
+    const float unit = a.hidden ? ln_unit(sqrtf(sum) * sqrtf(mx) + fmaxf(b, 0.f)) : 1.0f, down = ln_inverse(unit);
     a.inv[r] = s.down * down;
     a.bound[r] = sum * down;
     a.bias[r] = b * down;
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_first_weights_kernel(LnFirstWei
   }
   mx = ln_block_max(mx, red);                             // its barriers cover `row` too
   const LnScale s = ln_scale(mx);
-  const float b = a.layer.b ? a.layer.b[n] : 0.f, unit = ln_unit(mx + fabsf(b)), down = ln_inverse(unit);
+  const float b = a.layer.b ? a.layer.b[n] : 0.f, unit = ln_unit(mx + fmaxf(b, 0.f)), down = ln_inverse(unit);
   if (threadIdx.x == 0) {
     a.layer.inv[n] = s.down * down;
     a.layer.bound[n] = 7.f * (mx * down);
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_states_kernel(
   }
 }
 
-// Workgroup l of the first `layers`: stats[2 l], stats[2 l + 1] = the largest bound and bias of layer l.  The others, a
+// Workgroup l of the first `layers`: stats[2 l], stats[2 l + 1] = the largest bound and bias (0 at least) of layer l.  The others, a
 // state each: base[i][n] = the first layer's bias + the columns of the cards on the state's board.
 struct LnBounds {
   const float *bound[LN_MAX_LAYERS], *bias[LN_MAX_LAYERS];   // in units of u
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(LN_THREADS) void ln_base_kernel(LnBounds bounds, in
     float m = 0.f, b = 0.f;
     for (int k = threadIdx.x; k < bounds.rows[l]; k += LN_THREADS) {
       m = fmaxf(m, bound[k]);
-      b = fmaxf(b, fabsf(bias[k]));
+      b = fmaxf(b, bias[k]);
     }
     m = ln_block_max(m, red);
     b = ln_block_max(b, red);
@@ -380,7 +382,7 @@ struct LnGemm {
   int64_t m;
   int n, blocks, batches;
   float* out;               // LN_PLAIN: [batch][m][n]
-  // LN_HIDDEN: the next layer's input.  The answer is at most stats[0] * (largest entry of the input) + stats[1], the
+  // LN_HIDDEN: the next layer's input.  An answer is at most stats[0] * (largest entry of the input) + stats[1], the
   // input at most a_max[row] or, without that, first_stats[0] + first_stats[1].
   const float *stats, *first_stats, *a_max;
   char* out_split;

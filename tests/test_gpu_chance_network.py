@@ -150,6 +150,22 @@ def test_units_of_unequal_size(kind, ranges):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bias", [-1e4, -3e38, -float("inf")])
+def test_units_switched_off_by_their_bias(bias):
+    """As if nothing read them."""
+    net, without = make_net(320, 4), make_net(320, 4)
+    with torch.no_grad():
+        for k in range(4):
+            net.linears[k].bias[k::50] = bias
+            without.linears[k + 1].weight[:, k::50] = 0
+        pre, boards = make_inputs(3, "three hands", seed=22, on_board=4)
+        got = K.chance_network(pre, torch.arange(3).cuda(), boards, K.network_layers(net, pre.device), 4)
+        want, tol = reference(without, pre, boards)
+    assert bool(((got.double() - want).abs() <= tol).all())
+    assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -22 * len(net.linears)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["gamma", "three hands"])
 def test_256_row_tiles_and_a_selection_of_rows(kind):
     """Enough samples for the largest tiles (4 per CU), taken from a table through ``root_indices``, and enough of them
