@@ -180,12 +180,12 @@ __device__ __forceinline__ double p2_block_sum(double v, double* red) {
 }
 
 // Quotients of the iteration kernels.  IEEE division costs eleven operations, and two scalings of operands that are
-// far from the ends of the exponent's range; the kernels divide four to ten times per row and hand, and their
-// launches are bound by the vector units (59 % busy in the subtree launch of 192 roots).  Here the reciprocal is the
+// far from the ends of the exponent's range; the kernels divide four to ten times per row and hand, each time in the
+// chain of a family's steps that nothing covers while few workgroups run.  Here the reciprocal is the
 // hardware's, within one unit in the last place, with one Newton step, and the quotient is corrected once by its
 // exact remainder (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  Equal
-// to `/` for dividends from 2^-102 and divisors from 2^-126 to 2^126 whose quotient is a normal number: the oracle
-// (oracle/quotient.c) goes through every mantissa of a divisor with every reciprocal that hardware may start from.
+// to `/` for dividends from 2^-102 and divisors from 2^-126 to 2^126 whose quotient is a normal number: a test restates
+// it on the CPU and goes through every mantissa of a divisor, with every reciprocal that hardware may start from.
 // Outside of that: a smaller dividend can lose its remainder to rounding, and its quotient then a unit in the last place,
 // and so can a subnormal quotient.  A quotient that overflows becomes NaN, not infinity; none of the kernels' can: their
 // dividends are at most their divisors (a regret and its family's sum, a hand and its range's mass, a mix and its
