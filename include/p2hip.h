@@ -119,7 +119,9 @@ int p2hip_chance_expand_input(const float* pre_beliefs, const int64_t* root_indi
  * others multiples of 32; 3 to P2HIP_NETWORK_MAX_LAYERS layers, at most P2HIP_NETWORK_MAX_SAMPLES samples.
  * `workspace`: 256-byte aligned, of p2hip_chance_network_workspace(...) bytes (-1: not a network this
  * call takes); its contents do not matter and mean nothing afterwards.  Everything that depends on the
- * weights is derived anew in every call.  Replaces search/chance_node_helper.py:394-477 for such networks. */
+ * weights is derived anew in every call.  Products are three of float16 halves under powers of two, a hidden unit's own
+ * among them: errors as of float32 products for finite numbers, but an infinity may turn into NaN.  Every state needs a
+ * sample (with total_samples = 0 nothing is written).  Replaces search/chance_node_helper.py:394-477 for such networks. */
 #define P2HIP_NETWORK_MAX_LAYERS 16
 #define P2HIP_NETWORK_MAX_SAMPLES ((1 << 23) - 1)
 int64_t p2hip_chance_network_workspace(int64_t n, int64_t total_samples, const int32_t* host_widths, int layers);

@@ -6,7 +6,7 @@ to the network (src/p2/models/mlp/mlp_features.py:13-62): same names, arguments,
 order (state-major, next card ascending) and return value.  The masking / renormalising
 expansion and the per-state mean run as HIP kernels (``p2hip_chance_expand``,
 ``p2hip_chance_mean``); the network itself stays an ordinary PyTorch module, but one that is known to be plain float32
-layers is computed from its weights, node and network in one call (``p2hip_chance_network``).
+layers is computed from its weights, node and network in one call (``p2hip_chance_network``), where that is faster.
 ``flop_chance_values`` (three-card chance nodes, :219-357) enumerates or samples the 1755
 suit-canonical flops (:76-216), expands through ``p2hip_flop_expand`` and averages each flop's
 answers over its suit orbit with ``p2hip_perm_mean``.

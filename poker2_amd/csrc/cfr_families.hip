@@ -235,7 +235,8 @@ __global__ __launch_bounds__(UB_BLOCK) void family_average_policy_kernel(
 // range x reach normalised, allowed_prob where the sum is at most eps.  The nodes of a root share their allowed hands.
 // A row reads the policies on its way instead of the reach above it, so that all levels are one launch: they are read by
 // many rows and come from the caches (8400 rows: five launches of 22 us, a level at a time, or one of 105; neighbouring rows
-// on one XCD, so that they share the policies in its L2: 113, the stores like neighbours on different XCDs better).
+// on one XCD, so that they share the policies in its L2: 113, the stores like neighbours on different XCDs better).  From
+// some 20 000 rows on the levels are faster, and the evaluator takes those.
 constexpr int FAM_MAX_DEPTH = 64;
 constexpr int FAM_BATCH = 4;                                // rows of policy requested together
 __global__ __launch_bounds__(UB_BLOCK) void tree_reach_beliefs_kernel(

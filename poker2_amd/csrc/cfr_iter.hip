@@ -105,11 +105,11 @@ struct IterArgs {
 // The kernel's arguments.  A lean iteration's sweeps each read them ANEW from the argument segment and keep the
 // handful that they use.  Read once at the start, the forty pointers do not fit into the scalar registers next to the
 // schedule's factors; the compiler then parks them in lanes of vector registers, in runs of sixteen, and brings back
-// a whole run wherever one is used: 2260 of the kernel's 9700 vector instructions (five children).  River roots, in
-// ms: 192, 16 iterations, 10.16 -> 9.93; 1003 small trees, 12 iterations, 6.45 -> 6.23; the search of 192, 44.7 ->
-// 44.0; one and 4096 the same within 0.4 %.  Asking anew for every family was slower than parking (one root, 32
-// iterations, 4.46 -> 4.56): the scalar loads were waited for there.  An ordinary iteration (192 in a graph, 5.87)
-// spilled vector registers with it (5.93), so there the compiler places the reads (5.87).
+// a whole run wherever one is used: 2359 reads of a lane among 10961 vector instructions (five children; now 89 among
+// 7376, the quotients' share included).  192 river roots, 16 iterations, 10.16 -> 9.93 ms, their search 44.7 -> 44.0; one
+// root, 4096 and 1003 small trees the same within what two runs differ.  Asking anew for every family was slower than
+// parking (one root, 32 iterations, 4.46 -> 4.56): the scalar loads were waited for there.  An ordinary iteration spilled
+// vector registers with it and was no faster, so there the compiler places the reads.
 // (The empty asm only hides from the compiler that the address is the one it has already loaded from.)
 typedef const __attribute__((address_space(4))) IterArgs IterArgsConst;
 template <bool ANEW>

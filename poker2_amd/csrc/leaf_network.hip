@@ -16,9 +16,13 @@
 // hi hi + hi lo + lo hi, added up in float32.  What is dropped (lo lo and the bits below lo) is 2^-22 of a product, below
 // what adding 1536 of them in float32 rounds away: against 64 bits such a layer is 1.6e-7 off (norm over norm, 1536
 // wide), the library's float32 product 5.0e-7.  The whole call, 3 x 1536, against 64 bits, before (library, mean of the
-// answers) and now: 1.70e-7 / 1.56e-7 over Gamma(1/2) ranges, 1.87e-7 / 1.62e-7 over their eighth powers, 1.71e-7 /
-// 1.60e-7 over single hands.
-// 2240 states x 48 cards, 3 x 1536: 20.2 -> 3.4 ms (the hidden layers 1.24 + 1.31, the first 0.6); 1 state 0.22 -> 0.18.
+// answers) and now: 1.72e-7 / 1.61e-7 over Gamma(1/2) ranges, 1.91e-7 / 1.67e-7 over their eighth powers, 1.79e-7 /
+// 1.65e-7 over single hands; with torch's own initial weights 1.12e-7 / 0.57e-7.  An answer's error is bounded against
+// what its unit's weights can reach, not against the answer itself: hence a scale per unit (below), since units that
+// share one lose their bits to the largest.
+// 2240 states x 48 cards, 3 x 1536: 20.4 -> 3.7 ms (the hidden layers 1.36 + 1.59, the first 0.5).  Every call prepares
+// all weights, which is what few samples pay for: 35 states 0.56 -> 0.27 ms, 1 state 0.19 -> 0.23 (the caller's rule,
+// chance_node_helper.py, sends those through the layers).
 //
 // Numbers that are not finite stay so on the way through, but an infinity may turn into NaN (its low part does).
 #pragma once
@@ -409,9 +413,9 @@ __device__ __forceinline__ void ln_to_lds(const char* from, char* to) {   // 16 
 // The three products of a step start from zero and are added to the sum by the vector ALU, a row of squares behind the
 // matrix instructions: added up inside them the result is 4.4e-7 off, like this 1.6e-7, for 8 % of the time.  LN_PLAIN
 // (few rows, and the layer whose error nothing averages) also keeps sums of 256 columns apart and takes lo lo along.
-// 107 520 x 1536 x 1536, 6 x as many float16 operations: 1.41 ms = 1075 TFLOP/s (32 x 32 squares, one sum 1.37; 16 x 16,
-// one sum 1.27; the library's float32 product 3.6-3.7 ms, its plain bfloat16 products reach 1144 on this card).  Bound:
-// the card's power; it runs them at 1.5-1.9 GHz, the matrix cores busy 56-60 % of the cycles.
+// 107 520 x 1536 x 1536, 6 x as many float16 operations: 1.36-1.41 ms = 1075-1121 TFLOP/s (32 x 32 squares, one sum 1.37;
+// 16 x 16, one sum 1.27; the library's float32 product 3.6-3.7 ms, its plain bfloat16 products reach 1144 on this card).
+// Bound: the card's power; it runs them at 1.8-2.0 GHz, the matrix cores busy 53-57 % of the cycles, no bank conflicts.
 // 256 x 256 tiles need 128 KiB of LDS (one workgroup per CU); 128 x 128 tiles make it 1.93 ms at that size, but 2240 x
 // 2652 x 1536 goes from 0.109 to 0.067 and 8192 x 1536 x 1536 from 0.118 to 0.112 (first version): the smaller tile below
 // four large ones per CU, and 64 x 64 where even those leave CUs idle.
@@ -673,9 +677,11 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void ln_gemm_kernel(LnGemm g) {
 
 // The first layer's answers.  A workgroup keeps T of both players and the base of 64 states x 128 columns (registers, LDS)
 // and goes through its cards: a product of 103 columns, the card's rows of `gone` against the card's columns of the
-// weights, one 128-byte block of every row at a time as above, the next one (of the next card too) in flight.  T read
-// again for every card, as the epilogue of a product over cards, made the layer 560-590 us at 2240 states x 48 cards x
-// 1536 (830 us with 16-byte loads of sixteen rows at a time), this 505.
+// weights, one 128-byte block of every row at a time as above, the next one (of the next card too) sent ahead.  (In two of
+// a card's four steps the compiler cannot tell the buffers apart and waits for those loads before it reads the step's
+// operands; they overlap with the products in the other two only.)  T read again for every card, as the epilogue of a
+// product over cards, made the layer 560-590 us at 2240 states x 48 cards x 1536 (830 us with 16-byte loads of sixteen rows
+// at a time), this 505-515; the matrix cores are busy 12 % of it.
 // The cards are dealt to as many workgroups as fill the chip twice; those of one stripe of columns follow each other on
 // one XCD and share the weights in its L2.
 struct LnFirst {

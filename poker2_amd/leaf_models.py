@@ -7,8 +7,8 @@ come are expanded over every card that can come next (blocker masking, renormali
 network, mean — the semantics of ``ChanceNodeHelper.single_card_chance_values``,
 src/p2/search/chance_node_helper.py:360-479), and leaves where the preflop round has ended
 over the canonical flops (``flop_chance_values``, :219-357).  The network stays ordinary PyTorch; the
-expansion and the mean are HIP kernels, and ``RangeBoardMLP`` in float32 behind a single card as a whole is
-(``chance_node_helper.chance_network``).
+expansion and the mean are HIP kernels, and ``RangeBoardMLP`` in float32 behind a single card as a whole is, from some
+size on (``chance_node_helper.network_takes``).
 
 ``RangeBoardMLP`` is the network of the turn benchmark configuration: input 2 x 1326 ranges +
 52-dim board one-hot, three hidden ReLU layers, output 2 x 1326; orthogonal initialisation with
