@@ -186,6 +186,28 @@ def test_256_row_tiles_and_a_selection_of_rows(kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("row_tiles", [1, 4, 5, 9, 10, 11, 21, 22])
+def test_tiles_of_whole_samples_in_parts(row_tiles):
+    """Tiles are 64 samples by 128 of 1024 columns; their steps are cut into 14, 14, 7, 7, 6, 3, 3 and 1 parts, as many as
+    512 workgroups take."""
+    net = make_net(1024, 2)
+    pre, boards = make_inputs(240, "three hands", seed=31, on_board=4)
+    cards = hand_combos_tensor().cuda()
+    on = torch.zeros(240, 52, device="cuda").scatter_(1, boards[:, :4], 1.0)
+    left = pre * (1 - on[:, cards].amax(2))[:, None]
+    held = torch.stack([(left * (cards == c).any(1)).sum(2) for c in range(52)], dim=2)
+    whole = ((held > 0.25 * left.sum(2, keepdim=True)).any(1) & (on == 0)).sum(1).cumsum(0)
+    n = int((whole <= 64 * (row_tiles - 1)).sum()) + 1   # the first state that needs the last tile
+    assert -(-int(whole[n - 1]) // 64) == row_tiles
+    roots = torch.arange(n).cuda()
+    with torch.no_grad():
+        got = K.chance_network(pre, roots, boards, K.network_layers(net, pre.device), 4)
+        rows, _, _, offsets = K.chance_expand(pre, roots, boards, 4, input_dtype=torch.float32)
+        want = K.chance_mean(net.forward_input(rows).hand_values, offsets)
+    assert float((got - want).norm() / want.norm()) < 2e-6
+
+
+@pytest.mark.gpu
 def test_a_wrong_card_count_claim_and_a_row_outside_the_table():
     """The rest of a state's share is samples with an input of zeros, as the expansion writes them."""
     net = make_net(256, 2)
