@@ -170,9 +170,12 @@ NETWORK_MIN_WIDTH = 256
 # A call prepares all weights before it uses them, whatever its size, and some ranges need another product besides
 # (samples taken whole).  Three or more hidden layers of at most 512 units gain all the same, two of 256 too; others from
 # this many samples on.  ms a call of three hidden layers, layer by layer -> one call, smooth ranges / three hands a
-# player: 512 wide, 48 samples 0.19 -> 0.17 / 0.19 (two layers 0.165 -> 0.161 / 0.179); 1024 wide, 48 0.19 -> 0.20 / 0.22, 768 0.21 -> 0.21 / 0.23, 960 0.24 -> 0.21 / 0.24; 1536 wide, 48 0.19 -> 0.23 / 0.25,
-# 768 0.28 -> 0.24 / 0.27, 960 0.34 -> 0.25 / 0.28; 4096 wide, 48 0.19 -> 0.60 / 0.63, 960 0.89 -> 0.68 / 0.75; 1536 wide,
-# 107 520 samples 20.5 -> 3.6 / 5.1.
+# player:
+#    512 wide, 48 samples 0.19 -> 0.17 / 0.19 (two layers 0.165 -> 0.161 / 0.179);
+#   1024 wide, 48 samples 0.19 -> 0.20 / 0.22, 768 samples 0.21 -> 0.21 / 0.23, 960 samples 0.24 -> 0.21 / 0.24;
+#   1536 wide, 48 samples 0.19 -> 0.23 / 0.25, 768 samples 0.28 -> 0.24 / 0.27, 960 samples 0.34 -> 0.25 / 0.28,
+#     107 520 samples 20.5 -> 3.6 / 5.1;
+#   4096 wide, 48 samples 0.19 -> 0.60 / 0.63, 960 samples 0.89 -> 0.68 / 0.75.
 NETWORK_ANY_SAMPLES_WIDTH, NETWORK_ANY_SAMPLES_WIDTH_OF_TWO = 512, 256
 NETWORK_MIN_SAMPLES = 960
 

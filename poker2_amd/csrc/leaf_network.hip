@@ -337,8 +337,8 @@ __global__ __launch_bounds__(LN_THREADS) void ln_states_kernel(
   }
 }
 
-// Workgroup l of the first `layers`: stats[2 l], stats[2 l + 1] = the largest bound and bias (0 at least) of layer l.  The others, a
-// state each: base[i][n] = the first layer's bias + the columns of the cards on the state's board.
+// Workgroup l of the first `layers`: stats[2 l], stats[2 l + 1] = the largest bound and bias (0 at least) of layer l.  The
+// others, a state each: base[i][n] = the first layer's bias + the columns of the cards on the state's board.
 struct LnBounds {
   const float *bound[LN_MAX_LAYERS], *bias[LN_MAX_LAYERS];   // in units of u
   int rows[LN_MAX_LAYERS];
@@ -869,38 +869,38 @@ __device__ __forceinline__ void ln_whole_store(const LnWhole& g, const ln_float4
   const LnScale scale = ln_scale(g.stats[0] + g.stats[1]);
   const int64_t out_bytes = (int64_t)(g.width / 32) * LN_BLOCK_BYTES;
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int r = m0 + (wm * TM + i) * 16 + fr;
-        if (r >= count) continue;
-        const int32_t s = g.whole[r];
-        const LnSample sm = g.samples[s];
+  for (int i = 0; i < TM; ++i) {
+    const int r = m0 + (wm * TM + i) * 16 + fr;
+    if (r >= count) continue;
+    const int32_t s = g.whole[r];
+    const LnSample sm = g.samples[s];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int n = n0 + (wn * TN + j) * 16 + fq * 4;
-          if (n >= g.width) continue;
-          const ln_float4 bi = *reinterpret_cast<const ln_float4*>(g.b_inv + n);
-          ln_float4 rest;                                    // what does not come from the ranges
-          if (sm.card >= 0) {
-            rest = *reinterpret_cast<const ln_float4*>(g.base + (int64_t)sm.state * g.width + n);
-            rest += *reinterpret_cast<const ln_float4*>(g.columns + (int64_t)sm.card * g.width + n);
-          } else {
-            rest = *reinterpret_cast<const ln_float4*>(g.bias + n);
-          }
-          ln_half4 hi, lo;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float v = sum[i][j][e] * (bi[e] * (1.0f / LN_SAMPLE_SCALE)) + rest[e];
-            _Float16 h, l;
-            ln_split(ln_relu(v) * scale.up, h, l);
-            hi[e] = h;
-            lo[e] = l;
-          }
-          char* at = g.out_split + s * out_bytes + (n >> 5) * LN_BLOCK_BYTES + (n & 31) * 2;
-          *reinterpret_cast<ln_half4*>(at) = hi;
-          *reinterpret_cast<ln_half4*>(at + 64) = lo;
-          if (n == 0) g.out_inv[s] = scale.down;
-        }
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + (wn * TN + j) * 16 + fq * 4;
+      if (n >= g.width) continue;
+      const ln_float4 bi = *reinterpret_cast<const ln_float4*>(g.b_inv + n);
+      ln_float4 rest;                                    // what does not come from the ranges
+      if (sm.card >= 0) {
+        rest = *reinterpret_cast<const ln_float4*>(g.base + (int64_t)sm.state * g.width + n);
+        rest += *reinterpret_cast<const ln_float4*>(g.columns + (int64_t)sm.card * g.width + n);
+      } else {
+        rest = *reinterpret_cast<const ln_float4*>(g.bias + n);
       }
+      ln_half4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = sum[i][j][e] * (bi[e] * (1.0f / LN_SAMPLE_SCALE)) + rest[e];
+        _Float16 h, l;
+        ln_split(ln_relu(v) * scale.up, h, l);
+        hi[e] = h;
+        lo[e] = l;
+      }
+      char* at = g.out_split + s * out_bytes + (n >> 5) * LN_BLOCK_BYTES + (n & 31) * 2;
+      *reinterpret_cast<ln_half4*>(at) = hi;
+      *reinterpret_cast<ln_half4*>(at + 64) = lo;
+      if (n == 0) g.out_inv[s] = scale.down;
+    }
+  }
 }
 
 // Into how many parts the steps of a tile are cut, each a divisor of them that leaves an even number: as many as there are
